@@ -218,6 +218,17 @@ typedef struct ltr_attn_bwd_args {
 int ltr_attn_bwd(const ltr_attn_bwd_args *args, void *stream);
 
 /*
+ * ltr_attn_bwd_ws - ltr_attn_bwd with a workspace of the caller's for launches that have fewer key tiles than the device has
+ * compute units: several blocks then share a key tile's queries, leave partial dK / dV in the workspace, and one more kernel
+ * sums them (in a fixed order: results stay reproducible, but differ from ltr_attn_bwd's in the order of fp32 additions).
+ * ltr_attn_bwd_workspace (host only; sizes, positions, dtype and flags of args are read) says in *bytes how much this problem
+ * can use: 0 when sharing does not pay.  A NULL or smaller workspace makes the call the same as ltr_attn_bwd.  The
+ * workspace (16-byte aligned) need not be cleared, holds nothing between calls and must not be shared by calls that overlap.
+ */
+int ltr_attn_bwd_ws(const ltr_attn_bwd_args *args, void *workspace, int64_t workspace_bytes, void *stream);
+int ltr_attn_bwd_workspace(const ltr_attn_bwd_args *args, int64_t *bytes);
+
+/*
  * ltr_attn_bwd_noalloc - ltr_attn_bwd for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  It has
  * no counterpart in the reference.  Same arguments and results as ltr_attn_bwd with

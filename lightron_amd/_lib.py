@@ -20,7 +20,7 @@ LTR_FWD_ROWS_256, LTR_FWD_ROWS_512 = 8192, 16384
 LTR_FWD_F32_SCALAR = 32768
 LTR_BWD_F32_SCALAR = 65536
 
-EXPORTS = ("ltr_attn_fwd", "ltr_attn_bwd_delta", "ltr_attn_bwd", "ltr_attn_bwd_noalloc", "ltr_attn_plan", "ltr_cast_f32_to_bf16",
+EXPORTS = ("ltr_attn_fwd", "ltr_attn_bwd_delta", "ltr_attn_bwd", "ltr_attn_bwd_ws", "ltr_attn_bwd_workspace", "ltr_attn_bwd_noalloc", "ltr_attn_plan", "ltr_cast_f32_to_bf16",
            "ltr_rope_apply", "ltr_abi_version", "ltr_strerror")
 # the bench-only measurement library (include/ltr_probe.h); not part of the attention path
 PROBE_LIB_PATH = os.path.join(HERE, "csrc", "libltr_probe.so")
@@ -114,6 +114,10 @@ def load():
     lib.ltr_attn_bwd_delta.restype = ctypes.c_int
     lib.ltr_attn_bwd.argtypes = [ctypes.POINTER(BwdArgs), ctypes.c_void_p]
     lib.ltr_attn_bwd.restype = ctypes.c_int
+    lib.ltr_attn_bwd_ws.argtypes = [ctypes.POINTER(BwdArgs), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+    lib.ltr_attn_bwd_ws.restype = ctypes.c_int
+    lib.ltr_attn_bwd_workspace.argtypes = [ctypes.POINTER(BwdArgs), ctypes.POINTER(ctypes.c_int64)]
+    lib.ltr_attn_bwd_workspace.restype = ctypes.c_int
     lib.ltr_attn_bwd_noalloc.argtypes = [ctypes.POINTER(BwdArgs), ctypes.c_void_p]
     lib.ltr_attn_bwd_noalloc.restype = ctypes.c_int
     lib.ltr_cast_f32_to_bf16.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]

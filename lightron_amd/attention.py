@@ -201,9 +201,16 @@ def attn_delta(o: torch.Tensor, do: torch.Tensor) -> torch.Tensor:
     return delta
 
 
+def _partials(lib, ref, device):
+    """Workspace for the partial dK / dV of blocks that share key tiles (None: this problem does not use one)."""
+    n = ctypes.c_int64(0)
+    _lib.check(lib.ltr_attn_bwd_workspace(ref, ctypes.byref(n)), "ltr_attn_bwd_workspace")
+    return torch.empty(n.value, dtype=torch.uint8, device=device) if n.value else None
+
+
 def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_accs, q_pos0=0, q_split=None,
                         causal=False, scale=None, do_dq=True, do_dkdv=True, o=None, library_scratch=False, dq_rope=None,
-                        dkdv_keys=None, dq_rows=None, f32_scalar=False):
+                        dkdv_keys=None, dq_rows=None, f32_scalar=False, share_keys=False):
     """Adds this Q chunk's contribution into the fp32 accumulators dq_acc / dk_accs / dv_accs.
     do_dq / do_dkdv select which of the two backward kernels are enqueued.  dq_acc may instead be a bf16
     tensor: it then RECEIVES dQ (LTR_DQ_BF16), which is only right when ks / vs hold every KV chunk these
@@ -219,7 +226,9 @@ def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_a
     kernel's epilogue rotates dQ back by the conjugate angles (LTR_ROPE_DQ): dq is the gradient of the un-rotated q.
     dkdv_keys: None (the library chooses), 128 or 256 keys per block of the dK/dV kernel (256: bf16 with head dim 64 only).
     dq_rows: None, 256 or 512 query rows per block of the dQ kernel (512: bf16 with head dim 64 only).
-    f32_scalar: fp32 inputs only - the scalar fp32 kernels instead of the matrix-pipe ones (LTR_BWD_F32_SCALAR)."""
+    f32_scalar: fp32 inputs only - the scalar fp32 kernels instead of the matrix-pipe ones (LTR_BWD_F32_SCALAR).
+    share_keys: launches with few key tiles may let several dK/dV blocks share a tile and sum their partials from a workspace
+    allocated here (ltr_attn_bwd_ws); dK / dV then differ from the unshared ones in the order of fp32 additions."""
     lib = _lib.load()
     if library_scratch and (o is None or not do_dq):
         raise RuntimeError("library_scratch needs o (DELTA is computed from it) and do_dq")
@@ -300,7 +309,9 @@ def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_a
             if library_scratch:
                 _lib.check(lib.ltr_attn_bwd_noalloc(ctypes.byref(a), stream), "ltr_attn_bwd_noalloc")
             else:
-                _lib.check(lib.ltr_attn_bwd(ctypes.byref(a), stream), "ltr_attn_bwd")
+                part = _partials(lib, ctypes.byref(a), q.device) if share_keys and do_dkdv else None
+                _lib.check(lib.ltr_attn_bwd_ws(ctypes.byref(a), None if part is None else part.data_ptr(), 0 if part is None else part.numel(),
+                                               stream), "ltr_attn_bwd")
 
 
 def attn_plan(B: int, Hq: int, Hkv: int, D: int, Sq: int, chunk_lens: Sequence[int], k_pos0: Sequence[int], q_pos0=0,
@@ -399,7 +410,7 @@ class BlockAttentionFunction(torch.autograd.Function):
             # accumulators and cast once at the end, instead of one bf16 rounding per node: nothing flows to k, v here
             dk_accs, dv_accs = ctx.kv_grad_acc
             attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_accs, q_pos0, q_split, causal,
-                                scale, o=o if fuse else None, dq_rope=ctx.q_rope)
+                                scale, o=o if fuse else None, dq_rope=ctx.q_rope, share_keys=True)
             dq = dq_acc if (direct or f32) else cast_to_bf16(dq_acc)
             return (dq, None, None, None, None, None, None, None, None, None, None) + (None,) * (2 * n_chunks)
         lens = [k.shape[1] for k in ks]
@@ -414,7 +425,7 @@ class BlockAttentionFunction(torch.autograd.Function):
         dk_accs = [dk_buf[:, o_:o_ + n_] for o_, n_ in zip(offs, lens)]
         dv_accs = [dv_buf[:, o_:o_ + n_] for o_, n_ in zip(offs, lens)]
         attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_accs, q_pos0, q_split, causal, scale,
-                            o=o if fuse else None, dq_rope=ctx.q_rope)
+                            o=o if fuse else None, dq_rope=ctx.q_rope, share_keys=True)
         dq = dq_acc if (direct or f32) else cast_to_bf16(dq_acc)
         dk16, dv16 = dk_buf, dv_buf
         dks = [dk16[:, o_:o_ + n_] for o_, n_ in zip(offs, lens)]
@@ -540,7 +551,8 @@ class SingleChunkAttentionFunction(torch.autograd.Function):
         if q_rope is not None:
             a.rope_freqs = q_rope.data_ptr()
         with _on_device(dev):
-            rc = lib.ltr_attn_bwd(ref, _stream_ptr(dev))
+            part = _partials(lib, ref, dev)
+            rc = lib.ltr_attn_bwd_ws(ref, None if part is None else part.data_ptr(), 0 if part is None else part.numel(), _stream_ptr(dev))
         if rc:
             _lib.check(rc, "ltr_attn_bwd")
         return dq, dk, dv, None

@@ -29,6 +29,7 @@
 //                        read from LDS feeds two MFMAs, and a block's transfers and per-step costs are spread over
 //                        twice the matrix work.  The registers allow it at head dim 64 only; chosen by the host
 //                        when the blocks are long and still many (or forced with LTR_DKDV_KEYS_256).
+//   bwd_dkdv_reduce_kernel<D, KW>  sums the partial dK / dV of blocks that share a key tile (see KvSplit).
 //   bwd_dq_kernel<D, RB> forward-shaped: a block owns 256 * RB query rows, loops over K/V tiles
 //                        (same direct-to-LDS tiles as the forward), recomputes S and dP and
 //                        accumulates dQ^T in registers.  No atomics anywhere: results are
@@ -119,6 +120,10 @@ struct BwdParams {
     unsigned flags;
     int n_chunks;
     int tiles_total;  // key tiles over all chunks
+    int split_log2;   // log2 of the blocks that share one key tile of the dK/dV kernel (0: a block owns its keys alone), see KvSplit
+    int share_log2;   // log2 of those that share out the q tiles of a head; the others share out the group's q heads,
+    int n_reps;       // of which a block walks this many
+    float *part;      // n_split > 1: the blocks' partial dK / dV, summed by bwd_dkdv_reduce_kernel
     int n_slots;      // slots of 256-row q tiles of the dQ kernel (see q_tile_slots)
     const float *rope;     // LTR_ROPE_DQ: (cos, sin) rows, D floats per position, row 0 = position rope_pos0
     int rope_pos0;
@@ -1395,6 +1400,20 @@ __device__ __forceinline__ unsigned bwd_ds_pair(unsigned pu, const f32x16 &dpm, 
     return pack2_bf16(p0 * dpm[2 * j], p1 * dpm[2 * j + 1]);
 }
 
+// A wave's D x 32 accumulator tile as it lies in its registers: 16 bytes per lane and instruction, 1 KB runs.
+template <int D>
+__device__ __forceinline__ void store_partial(float *dst, int lane, const f32x16 (&acc)[D / 32], float mul) {
+#pragma unroll
+    for (int i = 0; i < D / 32; i++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = acc[i][4 * g + e] * mul;
+            *(f32x4 *)(dst + ((i * 4 + g) * 64 + lane) * 4) = v;
+        }
+}
+
 template <int D, int KW>
 __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
     using L = BwdLds<D, KW>;   // KW = 32-key halves per wave
@@ -1415,15 +1434,18 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
     int idx = blockIdx.x, pair, rest;
     const int P = p.B * p.Hkv;
     if ((P & 7) == 0) {
-        int xcd = idx & 7, j = idx >> 3;
-        pair = (j / p.tiles_total) * 8 + xcd;
-        rest = j % p.tiles_total;
+        const int xcd = idx & 7, j = idx >> 3, n = p.tiles_total << p.split_log2;
+        pair = (j / n) * 8 + xcd;
+        rest = j % n;
     } else {
         pair = idx % P;
         rest = idx / P;
     }
+    // blocks that share a key tile follow each other: each takes n_reps of the q heads and, of a head's visible q tiles, every
+    // 2^share_log2-th
+    const int split = rest & ((1 << p.split_log2) - 1), tile = rest >> p.split_log2;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
-    int c = 0, kt = rest;
+    int c = 0, kt = tile;
     for (; c < p.n_chunks; c++) {
         int n = (p.chunk[c].sk + BN - 1) / BN;
         if (kt < n) break;
@@ -1447,7 +1469,7 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
         q_pos_range(0, (int)p.Sq - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], q_lo, q_hi);
         if (q_hi < tile_kpos_lo) {
             for (int k = 0; k < KW; k++)
-            if ((p.flags & LTR_DKDV_BF16) && key_ok[k]) {   // results, not accumulators: these keys get zeros
+            if ((p.flags & LTR_DKDV_BF16) && p.split_log2 == 0 && key_ok[k]) {   // results, not accumulators: these keys get zeros
                 __bf16 *gz = p_role ? (__bf16 *)p.chunk[c].dv + b * p.dvs[0] + (long long)my_key[k] * p.dvs[1] + hkv * p.dvs[2]
                                     : (__bf16 *)p.chunk[c].dk + b * p.dks[0] + (long long)my_key[k] * p.dks[1] + hkv * p.dks[2];
                 for (int d = 8 * hh; d < D; d += 16) *(uint4 *)(gz + d) = make_uint4(0, 0, 0, 0);
@@ -1502,10 +1524,19 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
     unsigned short *const tlist = (unsigned short *)(smem + L::LIST_OFF);     // [2][MAX_QTILES]
     int *const tcount = (int *)(smem + L::LIST_OFF + 2 * L::MAX_QTILES * 2);
     if (w == 0) {
+        // a block that shares its keys lists every n_share-th visible tile, counted from its own offset
+        const int n_share = 1 << p.share_log2;
         int n1 = 0, n2 = 0;
+        int skip = split & (n_share - 1);   // visible tiles to pass over before the next one of this block
         for (int base = 0; base < p.n_qtiles; base += 64) {
             const int qt = base + lane;
-            const int cls = qt < p.n_qtiles ? tile_class(qt) : 0;
+            int cls = qt < p.n_qtiles ? tile_class(qt) : 0;
+            if (n_share > 1) {
+                const unsigned long long vis = __builtin_amdgcn_ballot_w64(cls != 0);
+                const int rank = __builtin_popcountll(vis & ((1ull << lane) - 1ull)), n = __builtin_popcountll(vis);
+                if (((rank - skip) & (n_share - 1)) != 0 || rank < skip) cls = 0;
+                skip = (skip - n) & (n_share - 1);
+            }
             const unsigned long long m1 = __builtin_amdgcn_ballot_w64(cls == 1), m2 = __builtin_amdgcn_ballot_w64(cls == 2);
             const unsigned long long below = (1ull << lane) - 1ull;
             if (cls == 1) tlist[n1 + __builtin_popcountll(m1 & below)] = (unsigned short)qt;
@@ -1534,8 +1565,9 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
     }
     const __bf16 *qp_head = nullptr, *dop_head = nullptr;
     const float *sp_head = nullptr;   // LSE (wave 0) or DELTA - BM (wave 1) of the head's rows, indexed by row0 + tid
+    const int h_first = hkv * p.n_rep + (split >> p.share_log2) * p.n_reps;   // first of the n_reps q heads this block walks
     auto set_head = [&](int rep) __attribute__((always_inline)) {
-        const int h = hkv * p.n_rep + rep;
+        const int h = h_first + rep;
         qp_head = (const __bf16 *)p.q + b * p.qs[0] + h * p.qs[2];
         dop_head = (const __bf16 *)p.d_o + b * p.dos[0] + h * p.dos[2];
         const long long so = ((long long)b * p.Hq + h) * p.Sq;
@@ -1560,7 +1592,7 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
         auto advance = [&](int &rep, int &qt) {   // next tile of this class after (rep, qt); false when done
             if (++li_ >= cnt) {
                 li_ = 0;
-                if (++rep >= p.n_rep) return false;
+                if (++rep >= p.n_reps) return false;
                 set_head(rep);
             }
             qt = __builtin_amdgcn_readfirstlane((int)pre);
@@ -1833,6 +1865,13 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
     run_pass(std::false_type{});
     run_pass(std::true_type{});
 
+    if (p.split_log2) {   // a share of the keys' gradients: stored as it lies in registers, summed by the reduction kernel
+        float *const part = p.part + (((((long long)pair * p.tiles_total + tile) << p.split_log2) + split) * 8 + w) * (KW * 32 * D);
+        const float mul = p_role ? 1.f : p.scale;
+#pragma unroll
+        for (int k = 0; k < KW; k++) store_partial<D>(part + k * 32 * D, lane, acc[k], mul);
+        return;
+    }
     // dV^T (P wave) / dK^T (dS wave) tile of the wave's 32 keys: added to the fp32 accumulators in whole rows, through the
     // wave's LDS staging area (every wave is past the last barrier: tiles, slots and lists are no longer read)
 #pragma unroll
@@ -1875,6 +1914,85 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
             it++;
         });
     }
+}
+
+// Sum of the partial dK / dV that the blocks sharing a key tile left in p.part (bf16 and fp32 kernels alike), in the order of
+// the shares: results do not depend on which block finished first.  A wave takes 64 columns of one 32-key slice of dK or dV
+// (slots 0-3 of a tile's partials are dV of its four slices, 4-7 dK) and writes them the way the dK/dV kernels do.  Bound:
+// the partials' traffic, which was written just before and mostly still lies in L2 / the memory-side cache.
+template <int D, int KW>
+__global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const BwdParams p) {
+    __shared__ __attribute__((aligned(16))) unsigned char stage_mem[4 * WaveStage<64>::BYTES];
+    constexpr int BN = 128 * KW, WPT = 8 * KW * (D / 64), BPT = WPT / 4;   // waves and blocks per key tile
+    const int lane = threadIdx.x & 63, w4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int idx = blockIdx.x, pair, rest;
+    const int P = p.B * p.Hkv;
+    if ((P & 7) == 0) {   // the XCD that wrote the partials reads them
+        const int j = idx >> 3, n = p.tiles_total * BPT;
+        pair = (j / n) * 8 + (idx & 7);
+        rest = j % n;
+    } else {
+        pair = idx % P;
+        rest = idx / P;
+    }
+    const int tile = rest / BPT, item = (rest % BPT) * 4 + w4;
+    const int half = item % (D / 64), k = (item / (D / 64)) % KW, slot = item / (D / 64 * KW);
+    const bool is_dv = slot < 4;
+    const int b = pair / p.Hkv, hkv = pair % p.Hkv;
+    int c = 0, kt = tile;
+    for (; c < p.n_chunks; c++) {
+        const int n = (p.chunk[c].sk + BN - 1) / BN;
+        if (kt < n) break;
+        kt -= n;
+    }
+    if (c >= p.n_chunks) return;
+    const int sk = p.chunk[c].sk, key_base = kt * BN + (slot & 3) * 32 * KW + 32 * k;
+    const bool out_bf16 = (p.flags & LTR_DKDV_BF16) != 0;
+    bool seen = true;
+    if (p.flags & LTR_CAUSAL) {   // a tile that no query sees: its blocks left nothing
+        int q_lo, q_hi;
+        q_pos_range(0, p.Sq - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], q_lo, q_hi);
+        seen = q_hi >= p.chunk[c].pos0 + kt * BN;
+    }
+    if (key_base >= sk || (!seen && !out_bf16)) return;
+    f32x16 acc[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
+    if (seen) {
+        const float *src = p.part + ((((long long)pair * p.tiles_total + tile) << p.split_log2) * 8 + slot) * (KW * 32 * D) + k * 32 * D + half * 2048;
+        for (int s = 0; s < 1 << p.split_log2; s++, src += 8 * KW * 32 * D)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const f32x4 v = *(const f32x4 *)(src + (i * 64 + lane) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[i / 4][4 * (i % 4) + e] += v[e];
+            }
+    }
+    const long long stride = is_dv ? p.dvs[1] : p.dks[1];
+    const long long off = (is_dv ? b * p.dvs[0] + hkv * p.dvs[2] : b * p.dks[0] + hkv * p.dks[2]) + (key_base + lane / 16) * stride +
+                          64 * half + 4 * (lane % 16);
+    unsigned char *const stage = stage_mem + w4 * WaveStage<64>::BYTES;
+    float *gp = (is_dv ? p.chunk[c].dv : p.chunk[c].dk) + (out_bf16 ? 0 : off);
+    __bf16 *gb = (__bf16 *)(is_dv ? p.chunk[c].dv : p.chunk[c].dk) + (out_bf16 ? off : 0);
+    wave_tile_rowmajor<64>(stage, lane, acc, 1.f, [&](int row, int, f32x4 val) {
+        if (key_base + row < sk) {
+            if (out_bf16) {
+                bf16x4 y;
+#pragma unroll
+                for (int e = 0; e < 4; e++) y[e] = (__bf16)val[e];
+                *(bf16x4 *)gb = y;
+            } else {
+                const f32x4 old = *(const f32x4 *)gp;
+#pragma unroll
+                for (int e = 0; e < 4; e++) val[e] += old[e];
+                *(f32x4 *)gp = val;
+            }
+        }
+        gp += 4 * stride;
+        gb += 4 * stride;
+    });
 }
 
 // dQ: same block / wave / lane roles as the forward (a lane owns one query row), so LSE and DELTA are
@@ -2656,8 +2774,10 @@ __global__ __launch_bounds__(256) void bwd_dkdv_f32_mfma_kernel(const BwdParams 
     const bool causal = p.flags & LTR_CAUSAL;
     // block -> (batch, kv head, chunk, 128-key tile)
     const int P = p.B * p.Hkv;
-    const int pair = blockIdx.x % P;
-    int c = 0, kt = blockIdx.x / P;
+    const int pair = blockIdx.x % P, rest = blockIdx.x / P;
+    const int step = 1 << p.split_log2;                            // blocks that share a key tile take every step-th q tile
+    const int split = rest & (step - 1), tile = rest >> p.split_log2;
+    int c = 0, kt = tile;
     for (; c < p.n_chunks; c++) {
         const int n = (p.chunk[c].sk + BN - 1) / BN;
         if (kt < n) break;
@@ -2709,7 +2829,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_f32_mfma_kernel(const BwdParams 
         return hi >= blk_kpos_lo;
     };
     auto next_visible = [&](int it) {
-        while (it < total && !visible(it)) it++;
+        while (it < total && !visible(it)) it += step;
         return it;
     };
     const int st_row = lane / CPR, st_pc = lane % CPR;
@@ -2742,12 +2862,12 @@ __global__ __launch_bounds__(256) void bwd_dkdv_f32_mfma_kernel(const BwdParams 
             }
         }
     };
-    int it = next_visible(0);
+    int it = next_visible(split);
     if (it < total) gload(it, 0);
     tile_barrier();
     int par = 0;
     while (it < total) {
-        const int nxt = next_visible(it + 1);
+        const int nxt = next_visible(it + step);
         if (nxt < total) gload(nxt, par ^ 1);
         const float *Qs = (const float *)(smem + par * L::BUF_BYTES), *dOs = Qs + TILE;
         const float *st = dOs + TILE;
@@ -2811,6 +2931,12 @@ __global__ __launch_bounds__(256) void bwd_dkdv_f32_mfma_kernel(const BwdParams 
         tile_barrier();
         par ^= 1;
         it = nxt;
+    }
+    if (p.split_log2) {   // a share of the keys' gradients, summed by the reduction kernel
+        float *const part = p.part + (((((long long)pair * p.tiles_total + tile) << p.split_log2) + split) * 8 + w) * (32 * D);
+        store_partial<D>(part, lane, dvacc, 1.f);
+        store_partial<D>(part + 4 * 32 * D, lane, dkacc, p.scale);
+        return;
     }
     // dK^T / dV^T of the wave's 32 keys: added to the fp32 accumulators in whole rows through the wave's staging area
     unsigned char *stage = smem + w * WaveStage<D>::BYTES;
@@ -3053,6 +3179,63 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Sq, int q_s
     return pl;
 }
 
+// Blocks that share one key tile of the dK/dV kernel.  A launch with fewer key tiles than the device has CUs (few kv heads, a
+// short or single sequence, one ring step's half-chunk) leaves CUs idle while each block walks all q heads of its group and
+// all q tiles; n blocks per tile then take a share of the (q head, q tile) steps each and leave partial sums in a workspace,
+// which bwd_dkdv_reduce_kernel adds up.  The choice compares launch times of n = 1, 2, 4 ...: a block costs its steps plus a fixed
+// part worth `fixed` steps, the blocks run longest first, one per CU, and the partials are written and read once.  The
+// constants are fitted to measured launches of 22 shapes with every n forced (each choice within 3 % of the best n):
+// B=1, 32/8 heads, D=128, causal S=1237: n=1 123 us, 2 75, 4 52, 8 67; S=4096: 374, 262, 281, 360; the half-filled ring
+// step of 2048 keys x 4096 rows: 184, 129, 138, 158; enough key tiles (B=1, 32 heads, S=2048, 512 tiles): 100, 115, 197, 344;
+// fp32, 4/16 heads, D=128, S=700: 870, 445, 233, 128, 83 (n=16).
+struct KvSplit {
+    int n, reps;      // blocks per key tile; how many of them share out the q heads (the largest power of two that divides both)
+};
+struct KvSplitCost {
+    int rows;                        // q rows per step
+    double step_us, fixed;           // time of a step; a block's fixed part in steps
+    double part_bytes_per_us;        // rate at which partials move (each is written and read)
+};
+KvSplit kv_split(const KvSplitCost &cost, int D, int keys, bool causal, int B, int Hkv, int n_rep, int Sq, int q_split, const int *q_pos0,
+                 const ChunkDev *chunk, int n_chunks) {
+    auto steps_at = [&](long long kpos) -> long long {   // steps of one q head that see the key at position kpos
+        long long rows = Sq;
+        if (causal)
+            rows = std::min<long long>(std::max<long long>(q_pos0[0] + (long long)q_split - kpos, 0), q_split) +
+                   std::min<long long>(std::max<long long>(q_pos0[1] + (long long)(Sq - q_split) - kpos, 0), Sq - q_split);
+        return (rows + cost.rows - 1) / cost.rows;
+    };
+    const long long q_last = std::max(q_split > 0 ? q_pos0[0] + (long long)q_split - 1 : -1,
+                                      Sq > q_split ? q_pos0[1] + (long long)(Sq - q_split) - 1 : -1);
+    long long tiles = 0, longest = 0;
+    double total = 0;
+    for (int c = 0; c < n_chunks; c++) {
+        const long long seen = causal ? std::min<long long>(chunk[c].sk, q_last - chunk[c].pos0 + 1) : chunk[c].sk;
+        if (seen <= 0) continue;
+        const long long n = (seen + keys - 1) / keys, first = steps_at(chunk[c].pos0), last = steps_at(chunk[c].pos0 + (n - 1) * keys);
+        tiles += n;
+        total += 0.5 * n * (first + last);
+        longest = std::max(longest, first);
+    }
+    KvSplit best{1, 1};
+    if (tiles == 0) return best;
+    const double cus = device_cus(), blocks = (double)tiles * B * Hkv, avg = total / tiles * n_rep, most = (double)longest * n_rep;
+    double best_us = 0;
+    for (int n = 1; n <= 32 && n <= most; n *= 2) {
+        const double one = avg / n + cost.fixed, max_one = (double)(((long long)most + n - 1) / n) + cost.fixed;
+        const double launch = std::max(max_one, blocks * n * one / cus + 0.25 * one);
+        const double bytes = blocks * n * keys * D * 8.0;
+        double us = launch * cost.step_us;
+        if (n > 1) us += 2.0 + 2.0 * bytes / cost.part_bytes_per_us;   // 2 us: the reduction's launch
+        if (n == 1 || (us < best_us && bytes <= 512e6)) {
+            best_us = us;
+            best.n = n;
+        }
+    }
+    while (best.reps * 2 <= best.n && n_rep % (best.reps * 2) == 0) best.reps *= 2;
+    return best;
+}
+
 // The same for the two backward kernels.
 struct BwdPlan {
     int f32_ks;         // fp32: 0 = scalar kernels, else the key shares per row group of bwd_dq_f32_mfma_kernel
@@ -3060,14 +3243,23 @@ struct BwdPlan {
     int keys_per_block;
     long long kv_tiles; // key blocks over all chunks of one (batch, kv head)
     long long kv_blocks;
+    KvSplit split;      // blocks per key tile (1 unless the caller brought a workspace for their partial sums)
+    int64_t part_bytes; // workspace they need
     bool wide_q;        // dQ kernel: 512 rows per block
     int dq_rows, dq_qtiles, dq_slots;
     long long dq_blocks;
 };
 BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
-                 int n_chunks) {
+                 int n_chunks, bool may_split = false) {
     BwdPlan pl;
     pl.f32_ks = 0;
+    pl.split = KvSplit{1, 1};
+    pl.part_bytes = 0;
+    may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
+    auto split_keys = [&](const KvSplitCost &cost) {
+        if (may_split) pl.split = kv_split(cost, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks);
+        if (pl.split.n > 1) pl.part_bytes = (int64_t)pl.kv_blocks * pl.split.n * pl.keys_per_block * D * 2 * 4;
+    };
     if (f32) {
         pl.wide_kv = pl.wide_q = false;
         if (flags & LTR_BWD_F32_SCALAR) {
@@ -3086,6 +3278,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         pl.kv_tiles = 0;
         for (int c = 0; c < n_chunks; c++) pl.kv_tiles += (chunk[c].sk + pl.keys_per_block - 1) / pl.keys_per_block;
         pl.kv_blocks = pl.kv_tiles * B * Hkv;
+        split_keys(D == 128 ? KvSplitCost{32, 9.0, 2.0, 6e6} : KvSplitCost{32, 4.5, 1.5, 6e6});
         pl.dq_qtiles = pl.dq_slots = (Sq + pl.dq_rows - 1) / pl.dq_rows;
         pl.dq_blocks = (long long)pl.dq_qtiles * B * Hq;
         return pl;
@@ -3114,6 +3307,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.kv_tiles = 0;
     for (int c = 0; c < n_chunks; c++) pl.kv_tiles += (chunk[c].sk + pl.keys_per_block - 1) / pl.keys_per_block;
     pl.kv_blocks = pl.kv_tiles * B * Hkv;
+    split_keys(D == 128 ? KvSplitCost{64, 1.4, 8.0, 8e6} : KvSplitCost{64, wide ? 1.9 : 1.0, wide ? 6.0 : 8.0, 6e6});
     // query rows per block of the dQ kernel: 512 (two 32-row blocks per wave) pays at head dim 64 when the wider blocks still
     // fill the device, and under a causal mask only on sequences long enough that the diagonal does not dominate
     bool wide_q = (flags & LTR_DQ_ROWS_512) != 0;
@@ -3317,8 +3511,8 @@ extern "C" int ltr_attn_bwd_delta(const ltr_attn_delta_args *a, void *stream) {
 
 namespace {
 // ltr_attn_bwd (DELTA is the caller's buffer) and ltr_attn_bwd_noalloc (use_scratch: DELTA lives in the library's fixed
-// scratch array; flags already carry LTR_DELTA_FROM_O)
-int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, void *stream) {
+// scratch array; flags already carry LTR_DELTA_FROM_O); work: the caller's workspace for partial dK / dV, or nullptr
+int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, void *stream, void *work = nullptr, int64_t work_bytes = 0) {
     float *delta = use_scratch ? nullptr : a->delta;
     if (!a->q || !a->d_o || !a->lse || (!use_scratch && !delta)) return LTR_EINVAL;
     const bool do_dq = !(flags & LTR_NO_DQ), do_dkdv = !(flags & LTR_NO_DKDV);
@@ -3413,9 +3607,15 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     p.scale = a->scale;
     p.flags = flags;
     p.n_chunks = a->n_chunks;
-    const BwdPlan pl = plan_bwd(a->D, f32, flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks);
-    if (pl.kv_blocks > 0x7fffffffLL || pl.dq_blocks > 0x7fffffffLL) return LTR_EINVAL;
+    BwdPlan pl = plan_bwd(a->D, f32, flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks, work != nullptr);
+    if (pl.part_bytes > work_bytes) pl.split = KvSplit{1, 1};
+    const long long kv_grid = pl.kv_blocks * pl.split.n, reduce_grid = pl.kv_blocks * (pl.keys_per_block / 128) * (a->D / 32);
+    if (kv_grid > 0x7fffffffLL || reduce_grid > 0x7fffffffLL || pl.dq_blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.tiles_total = (int)pl.kv_tiles;
+    p.split_log2 = __builtin_ctz(pl.split.n);
+    p.share_log2 = __builtin_ctz(pl.split.n / pl.split.reps);
+    p.n_reps = p.n_rep / pl.split.reps;
+    p.part = (float *)work;
     p.n_slots = pl.dq_slots;
     hipStream_t st = (hipStream_t)stream;
     if (f32 && pl.f32_ks) {   // fp32 on the matrix pipe
@@ -3431,9 +3631,13 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
                                       : launch((const void *)bwd_dq_f32_mfma_kernel<64, 4>, pl.dq_blocks, 256, F32Mfma<64, 4>::LDS, st, p);
             if (rc) return rc;
         }
-        if (do_dkdv)
-            rc = a->D == 128 ? launch((const void *)bwd_dkdv_f32_mfma_kernel<128>, pl.kv_blocks, 256, F32DkdvLds<128>::LDS, st, p)
-                             : launch((const void *)bwd_dkdv_f32_mfma_kernel<64>, pl.kv_blocks, 256, F32DkdvLds<64>::LDS, st, p);
+        if (do_dkdv) {
+            rc = a->D == 128 ? launch((const void *)bwd_dkdv_f32_mfma_kernel<128>, kv_grid, 256, F32DkdvLds<128>::LDS, st, p)
+                             : launch((const void *)bwd_dkdv_f32_mfma_kernel<64>, kv_grid, 256, F32DkdvLds<64>::LDS, st, p);
+            if (rc || pl.split.n == 1) return rc;
+            rc = a->D == 128 ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
+                             : launch((const void *)bwd_dkdv_reduce_kernel<64, 1>, reduce_grid, 256, 0, st, p);
+        }
         return rc;
     }
     if (f32) {
@@ -3467,9 +3671,13 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
         // the tail (the sums inside a block do not depend on the table's order).
         if (flags & LTR_CAUSAL)
             std::stable_sort(p.chunk, p.chunk + p.n_chunks, [](const ChunkDev &x, const ChunkDev &y) { return x.pos0 < y.pos0; });
-        if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, pl.kv_blocks, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
-        else if (pl.wide_kv) rc = launch((const void *)bwd_dkdv_kernel<64, 2>, pl.kv_blocks, BwdLds<64, 2>::NT, BwdLds<64, 2>::TOTAL, st, p);
-        else rc = launch((const void *)bwd_dkdv_kernel<64, 1>, pl.kv_blocks, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
+        if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, kv_grid, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
+        else if (pl.wide_kv) rc = launch((const void *)bwd_dkdv_kernel<64, 2>, kv_grid, BwdLds<64, 2>::NT, BwdLds<64, 2>::TOTAL, st, p);
+        else rc = launch((const void *)bwd_dkdv_kernel<64, 1>, kv_grid, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
+        if (rc || pl.split.n == 1) return rc;
+        rc = a->D == 128 ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
+             : pl.wide_kv ? launch((const void *)bwd_dkdv_reduce_kernel<64, 2>, reduce_grid, 256, 0, st, p)
+                          : launch((const void *)bwd_dkdv_reduce_kernel<64, 1>, reduce_grid, 256, 0, st, p);
     }
     return rc;
 }
@@ -3478,6 +3686,31 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
 extern "C" int ltr_attn_bwd(const ltr_attn_bwd_args *a, void *stream) {
     if (!a) return LTR_EINVAL;
     return bwd_launch(a, a->flags, false, stream);
+}
+
+extern "C" int ltr_attn_bwd_ws(const ltr_attn_bwd_args *a, void *workspace, int64_t workspace_bytes, void *stream) {
+    if (!a || workspace_bytes < 0) return LTR_EINVAL;
+    if (workspace && !aligned16(workspace)) return LTR_EALIGN;
+    return bwd_launch(a, a->flags, false, stream, workspace, workspace_bytes);
+}
+
+// Host-only: sizes, positions and flags are read, no pointer.
+extern "C" int ltr_attn_bwd_workspace(const ltr_attn_bwd_args *a, int64_t *bytes) {
+    if (!a || !bytes) return LTR_EINVAL;
+    *bytes = 0;
+    if (a->B <= 0 || a->Hq <= 0 || a->Hkv <= 0 || a->Sq <= 0 || a->Hq % a->Hkv || a->n_chunks < 1 || a->n_chunks > LTR_MAX_CHUNKS) return LTR_EINVAL;
+    if (a->D != 64 && a->D != 128) return LTR_EUNSUP;
+    if (!fits_i32(a->Sq) || a->q_split < 0 || a->q_split > a->Sq) return LTR_EINVAL;
+    if (!fits_i32(a->q_pos0[0] + a->Sq) || !fits_i32(a->q_pos0[1] + a->Sq)) return LTR_EINVAL;
+    ChunkDev chunk[LTR_MAX_CHUNKS];
+    for (int c = 0; c < a->n_chunks; c++) {
+        if (a->chunk[c].sk <= 0 || !fits_i32(a->chunk[c].sk) || !fits_i32(a->chunk[c].pos0 + a->chunk[c].sk)) return LTR_EINVAL;
+        chunk[c].sk = (int)a->chunk[c].sk;
+        chunk[c].pos0 = (int)a->chunk[c].pos0;
+    }
+    const int q_pos0[2] = {(int)a->q_pos0[0], (int)a->q_pos0[1]};
+    *bytes = plan_bwd(a->D, a->io_dtype == LTR_F32, a->flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks, true).part_bytes;
+    return LTR_OK;
 }
 
 // Host-only: nothing is enqueued, no pointer is read.

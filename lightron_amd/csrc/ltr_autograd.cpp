@@ -158,7 +158,12 @@ class SingleChunkNode : public torch::autograd::Function<SingleChunkNode> {
             a.rope_pos0 = 0;
             a.rope_len = rope.size(0);
         }
-        check_rc(ltr_attn_bwd(&a, (void *)ctx->saved_data["stream"].toInt()), "ltr_attn_bwd");
+        // few key tiles: blocks share them and leave partial sums in a workspace (from torch's caching allocator)
+        int64_t part_bytes = 0;
+        check_rc(ltr_attn_bwd_workspace(&a, &part_bytes), "ltr_attn_bwd_workspace");
+        Tensor part;
+        if (part_bytes > 0) part = torch::empty({part_bytes}, q.options().dtype(at::kByte));
+        check_rc(ltr_attn_bwd_ws(&a, part_bytes > 0 ? part.data_ptr() : nullptr, part_bytes, (void *)ctx->saved_data["stream"].toInt()), "ltr_attn_bwd");
         out[0] = dq;
         out[1] = dk;
         out[2] = dv;
