@@ -510,27 +510,79 @@ __device__ __forceinline__ void lds_tr_gemm_kw(const __bf16 *T, int row0, int la
 }
 
 // keys per K / V tile of the forward and dQ kernels
-template <int D, int RB = 1>
+template <int D, int RB = 1, int KS = 1>
 struct FwdTile {
-    static constexpr int BN = (D == 64 && RB == 1) ? 128 : 64;   // two row blocks per wave: S^T of 128 keys would be 128 registers
+    // two row blocks per wave: S^T of 128 keys would be 128 registers; key shares: the tile is KS times as long (LDS)
+    static constexpr int BN = KS > 1 ? (D == 128 && KS == 4 ? 32 : 64) : (D == 64 && RB == 1) ? 128 : 64;
 };
+
+// Key shares of the forward and dQ kernels (KS waves per 32-row group, each with its own keys): at the end every wave collects CW of
+// the D result columns from the KS partial results, which lie in LDS as they lie in registers (4 KB per 32 x 32 tile).
+template <int D, int KS>
+struct KeyShares {
+    static constexpr int CW = D / KS > 32 ? D / KS : 32;
+    static constexpr int PART_OFF = 8 * 64 * 4;                                    // after the forward's references and sums
+    static constexpr int BYTES = KS > 1 ? PART_OFF + 8 * (D / 32) * 4096 : 0;
+};
+template <int D, int KS>
+__device__ __forceinline__ void collect_shares(unsigned char *smem, int w, int ks, int lane, const f32x16 (&acc)[D / 32], float mul,
+                                               f32x16 (&own)[KeyShares<D, KS>::CW / 32]) {
+    constexpr int ND = D / 32, NC = KeyShares<D, KS>::CW / 32;
+    float *const parts = (float *)(smem + KeyShares<D, KS>::PART_OFF);
+#pragma unroll
+    for (int j = 0; j < NC; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) own[j][r] = 0.f;
+#pragma unroll
+    for (int i = 0; i < ND; i++) {
+        if (i / NC == ks) {   // wave-uniform
+#pragma unroll
+            for (int r = 0; r < 16; r++) own[i % NC][r] = acc[i][r] * mul;
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                f32x4 v;
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = acc[i][4 * g + e] * mul;
+                *(f32x4 *)(parts + (((w * ND + i) * 4 + g) * 64 + lane) * 4) = v;
+            }
+        }
+    }
+    __syncthreads();
+    if (ks * NC >= ND) return;
+#pragma unroll
+    for (int k = 1; k < KS; k++) {
+        const int other = w - ks + ((ks + k) & (KS - 1));
+#pragma unroll
+        for (int j = 0; j < NC; j++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const f32x4 v = *(const f32x4 *)(parts + (((other * ND + ks * NC + j) * 4 + g) * 64 + lane) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) own[j][4 * g + e] += v[e];
+            }
+    }
+}
 
 // ------------------------------------------------------------------------------ forward, bf16
 // RB = 32-row blocks per wave.  With two (head dim 64) every K / V operand read from LDS feeds two MFMAs and a tile of
 // 64 keys serves 512 query rows: half the LDS reads and half the tile transfers per MFMA.
-template <int D, int RB>
-__global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
-    constexpr int NW = 8, BM = 32 * RB * NW;   // 8 waves (two per SIMD) share every K / V tile
-    constexpr int BN = FwdTile<D, RB>::BN, NB = BN / 32;   // keys per tile: 32 KB (16 KB with two row blocks per wave)
+// KS = waves that share a 32-row group: each takes its own BN keys of every tile of KS * BN keys, and their partial (reference, row
+// sum, O) are merged through LDS at the end.  For launches with too few query rows to give every CU a block (see FwdPlan).
+template <int D, int RB, int KS>
+__device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
+    constexpr int NW = 8, RG = NW / KS, BM = 32 * RB * RG;   // 8 waves (two per SIMD) share every K / V tile
+    constexpr int BN = FwdTile<D, RB, KS>::BN, NB = BN / 32, BNT = BN * KS;   // keys per wave and per tile
     constexpr int CPR = D / 8;   // 16-byte chunks per row
     constexpr int RPI = 64 / CPR;            // rows filled by one wave-wide 16-byte-per-lane LDS-direct load (1 KB)
-    constexpr int NI = BN / (RPI * NW);       // such loads per wave, per tensor and per tile
+    constexpr int NI = BNT / (RPI * NW);      // such loads per wave, per tensor and per tile
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // two {K tile, V tile} buffers,
-    constexpr int TILE = BN * D;             // rows unpadded, 16-byte chunks XOR-swizzled (lds_swz)
+    constexpr int TILE = BNT * D;            // rows unpadded, 16-byte chunks XOR-swizzled (lds_swz)
     constexpr int BUF_ELEMS = 2 * TILE;
 
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = w / KS, ks = w % KS;      // row group and key share of the wave
     const bool causal = p.flags & LTR_CAUSAL;
 
     // block -> (batch, kv head, q head of the group, q tile).  Consecutive block ids go to
@@ -566,18 +618,18 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
     const int lane = lane_of_part, l32 = lane & 31, hh = lane >> 5;
 
     const int row0 = qt * BM;
-    int my_row[RB], my_pos[RB];   // row block rb of wave w: rows row0 + 32 * (RB * w + rb) ..
+    int my_row[RB], my_pos[RB];   // row block rb of row group rg: rows row0 + 32 * (RB * rg + rb) ..
     bool row_ok[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
-        my_row[rb] = row0 + (w * RB + rb) * 32 + l32;
+        my_row[rb] = row0 + (rg * RB + rb) * 32 + l32;
         row_ok[rb] = my_row[rb] < p.Sq;
         my_pos[rb] = q_position(my_row[rb], p.q_split, p.q_pos0[0], p.q_pos0[1]);
     }
     int blk_lo, blk_hi, w_lo, w_hi;
     q_pos_range(row0, min(row0 + BM, p.Sq) - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], blk_lo, blk_hi);
     {
-        int wr0 = row0 + w * 32 * RB, wr1 = min(wr0 + 32 * RB, p.Sq) - 1;
+        int wr0 = row0 + rg * 32 * RB, wr1 = min(wr0 + 32 * RB, p.Sq) - 1;
         if (wr1 >= wr0) q_pos_range(wr0, wr1, p.q_split, p.q_pos0[0], p.q_pos0[1], w_lo, w_hi);
         else { w_lo = 0x7fffffff; w_hi = -0x7fffffff; }  // wave has no valid row
     }
@@ -597,7 +649,7 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
         // by the angles of the row's global position; the rotated row can be stored for the backward
         if ((p.flags & LTR_ROPE_Q) && row_ok[rb]) {
             const float *fr = p.rope + (long long)(my_pos[rb] - p.rope_pos0) * D + 8 * hh;
-            __bf16 *qr = p.q_rot ? (__bf16 *)p.q_rot + b * p.qrs[0] + (long long)my_row[rb] * p.qrs[1] + h * p.qrs[2] + 8 * hh : nullptr;
+            __bf16 *qr = p.q_rot && ks == 0 ? (__bf16 *)p.q_rot + b * p.qrs[0] + (long long)my_row[rb] * p.qrs[1] + h * p.qrs[2] + 8 * hh : nullptr;
 #pragma unroll
             for (int kb = 0; kb < D / 16; kb++) {
                 qreg[rb][kb] = rope_rotate8(qreg[rb][kb], *(const f32x4 *)(fr + 16 * kb), *(const f32x4 *)(fr + 16 * kb + 4));
@@ -645,7 +697,7 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
                 ld_kb = (const __bf16 *)p.chunk[c].k + b * p.ks[0] + hkv * p.ks[2];
                 ld_vb = (const __bf16 *)p.chunk[c].v + b * p.vs[0] + hkv * p.vs[2];
                 const int nvis = causal ? max(0, min(ld_sk, blk_hi - ld_pos0 + 1)) : ld_sk;
-                nt = (nvis + BN - 1) / BN;
+                nt = (nvis + BNT - 1) / BNT;
             }
         }
     };
@@ -662,7 +714,7 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
         const int i = j % NI;
         const unsigned dst = lds_address(smem) + buf * BUF_ELEMS * 2 + (j / NI) * TILE * 2 + RPI * (NI * w + i) * D * 2;
         const int row = RPI * (NI * w + i) + st_row;
-        const int key = min(ti * BN + row, ld_sk - 1);
+        const int key = min(ti * BNT + row, ld_sk - 1);
         const int chunk = st_pc ^ lds_swz<D>(row);
         const __bf16 *src = j < NI ? ld_kb + (long long)(key * (int)p.ks[1] + chunk * 8)
                                    : ld_vb + (long long)(key * (int)p.vs[1] + chunk * 8);
@@ -671,7 +723,7 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
     auto gload_begin = [&](int ti) {   // scalar state of the tile whose transfers are issued next
         nx_sk = ld_sk;
         nx_pos0 = ld_pos0;
-        nx_key0 = ti * BN;
+        nx_key0 = ti * BNT;
     };
 
     // Double-buffered LDS, one barrier per tile: tile t+1 streams into the other buffer (whose readers all
@@ -690,8 +742,8 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
     // per-lane register plus an immediate offset (no address arithmetic between the MFMAs).
     auto tile_step = [&](auto par_tag) {
         constexpr int par = decltype(par_tag)::value;
-        const int sk = nx_sk, pos0 = nx_pos0, key0 = nx_key0;
-        const __bf16 *Ks = (const __bf16 *)smem + par * BUF_ELEMS, *Vs = Ks + TILE;
+        const int sk = nx_sk, pos0 = nx_pos0, key0 = nx_key0 + (KS > 1 ? ks * BN : 0);
+        const __bf16 *Ks = (const __bf16 *)smem + par * BUF_ELEMS + (KS > 1 ? ks * BN * D : 0), *Vs = Ks + TILE;
         t++;
         settle();
         const bool have_next = c < p.n_chunks;
@@ -706,18 +758,22 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
 
         // A wave whose 32 rows all precede the tile's first key (upper part of a diagonal tile, rows past the end) has
         // nothing to add: it only takes part in the transfers and the barrier.
-        if (!causal || pos0 + key0 <= w_hi) {
+        if ((!causal || pos0 + key0 <= w_hi) && (KS == 1 || key0 < sk)) {
         // S^T of the two 32-key blocks of the tile.  The wave raises its priority while it issues MFMAs: the
         // other wave of the SIMD then fills the gaps with its softmax arithmetic instead of delaying them.
         __builtin_amdgcn_s_setprio(1);
         f32x16 s[NB][RB];
         if constexpr (RB == 1) {
 #pragma unroll
-            for (int nb = 0; nb < NB; nb += 2) {
+            for (int nb = 0; nb + 1 < NB; nb += 2) {
                 s[nb][0] = zero16;
                 s[nb + 1][0] = zero16;
                 lds_gemm_pair<D>(Ks + (nb * 32 + l32) * D, lds_swz<D>(nb * 32 + l32) ^ hh, Ks + (nb * 32 + 32 + l32) * D,
                                  lds_swz<D>(nb * 32 + 32 + l32) ^ hh, qreg[0], qreg[0], s[nb][0], s[nb + 1][0]);
+            }
+            if constexpr (NB == 1) {
+                s[0][0] = zero16;
+                lds_gemm_chain<D>(Ks + l32 * D, lds_swz<D>(l32) ^ hh, qreg[0], s[0][0]);
             }
         } else {
 #pragma unroll
@@ -834,17 +890,43 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
         tile_step(std::integral_constant<int, 1>{});
     }
 
+    // The KS partial results of a row group: the waves agree on a reference (the largest share's log2 of its own sum), scale their O to
+    // it, and each collects CW of the D columns from the others.  The tile buffers are no longer read: the last barrier is
+    // behind us.
+    constexpr int CW = KeyShares<D, KS>::CW;   // columns a wave writes, from column col0 on
+    const int col0 = KS > 1 ? ks * CW : 0;
+    f32x16 own[CW / 32];                       // KS > 1: those columns of O
+    float l_shared = 0.f, lse_before = 0.f;
+    if constexpr (KS > 1) {
+        static_assert(RB == 1, "key shares are built for one row block per wave");
+        if ((p.flags & LTR_MERGE) && row_ok[0]) lse_before = p.lse[((long long)b * p.Hq + h) * p.Sq + my_row[0]];   // before any wave writes it
+        float *const ml = (float *)smem + w * 64;   // [wave][32 references | 32 sums]
+        const float l_own = xhalf_sum(l_run[0]), ref_own = l_own > 0.f ? mc[0] + __log2f(l_own) : -INFINITY;
+        if (hh == 0) ml[l32] = ref_own;
+        __syncthreads();
+        float ref = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < KS; k++) ref = fmaxf(ref, ml[(k - ks) * 64 + l32]);
+        const float f_own = l_own > 0.f ? __builtin_amdgcn_exp2f(mc[0] - ref) : 0.f;
+        if (hh == 0) ml[32 + l32] = l_own * f_own;
+        collect_shares<D, KS>(smem, w, ks, lane, oacc[0], f_own, own);
+#pragma unroll
+        for (int k = 0; k < KS; k++) l_shared += ml[32 + (k - ks) * 64 + l32];
+        mc[0] = ref == -INFINITY ? 0.f : ref;
+        __syncthreads();                            // the partials are read: their memory becomes the staging areas
+        if (col0 >= D) continue;                    // more shares than 32-column groups: nothing left to write
+    }
     // epilogue: normalise, optional merge with the partial result already in (o, lse); one row block after the other
     // through the same staging area
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
-    const float l_tot = xhalf_sum(l_run[rb]);
+    const float l_tot = KS > 1 ? l_shared : xhalf_sum(l_run[rb]);
     float lse_new = (l_tot > 0.f) ? mc[rb] * LTR_LN2 + logf(l_tot) : -INFINITY;
     float w_cur = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
     float w_old = 0.f;
     float *lse_p = p.lse + ((long long)b * p.Hq + h) * p.Sq + my_row[rb];
     if ((p.flags & LTR_MERGE) && row_ok[rb]) {
-        const float lse_old = *lse_p;
+        const float lse_old = KS > 1 ? lse_before : *lse_p;
         const float mxl = fmaxf(lse_old, lse_new);
         if (mxl == -INFINITY) {
             w_cur = 0.f;
@@ -856,16 +938,16 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
             lse_new = mxl + logf(tot);
         }
     }
-    if (row_ok[rb] && hh == 0) *lse_p = lse_new;
+    if (row_ok[rb] && hh == 0 && col0 == 0) *lse_p = lse_new;
     // O through the wave's LDS staging area (the tiles are no longer read: the last barrier is behind us)
-    unsigned char *stage = smem + w * WaveStage<D>::BYTES;
-    float *row_w_old = (float *)(stage + 32 * WaveStage<D>::ROW_BYTES);
+    unsigned char *stage = smem + w * WaveStage<CW>::BYTES;
+    float *row_w_old = (float *)(stage + 32 * WaveStage<CW>::ROW_BYTES);
     if (hh == 0) row_w_old[l32] = w_old;
-    constexpr int LPR = D / 4, ROWS_PER_IT = 64 / LPR;      // see wave_tile_rowmajor
-    const int Sq_u = uniform32(p.Sq), wave_row0 = uniform32(row0 + (w * RB + rb) * 32);
+    constexpr int LPR = CW / 4, ROWS_PER_IT = 64 / LPR;      // see wave_tile_rowmajor
+    const int Sq_u = uniform32(p.Sq), wave_row0 = uniform32(row0 + (rg * RB + rb) * 32);
     const bool merge = uniform32(p.flags & LTR_MERGE) != 0, o_f32 = uniform32(p.o_f32) != 0;
     const long long os1 = uniform64(p.os[1]);
-    const long long off0 = uniform64(b * p.os[0] + h * p.os[2]) + (wave_row0 + lane / LPR) * os1 + 4 * (lane % LPR);
+    const long long off0 = uniform64(b * p.os[0] + h * p.os[2] + col0) + (wave_row0 + lane / LPR) * os1 + 4 * (lane % LPR);
     // merging: all reads of the earlier partial result first (independent loads in flight together), then the writes
     constexpr int NIT = 32 / ROWS_PER_IT;
     f32x4 old[NIT];
@@ -883,9 +965,13 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
         }
     }
     int it = 0;
+    auto &result = [&]() -> f32x16(&)[CW / 32] {
+        if constexpr (KS > 1) return own;
+        else return oacc[rb];
+    }();
     if (o_f32) {
         float *op = (float *)p.o + off0;
-        wave_tile_rowmajor<D>(stage, lane, oacc[rb], w_cur, [&](int row, int, f32x4 val) {
+        wave_tile_rowmajor<CW>(stage, lane, result, w_cur, [&](int row, int, f32x4 val) {
             if (wave_row0 + row < Sq_u) {
                 if (merge) {
                     const float wo = row_w_old[row];
@@ -899,7 +985,7 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
         });
     } else {
         __bf16 *op = (__bf16 *)p.o + off0;
-        wave_tile_rowmajor<D>(stage, lane, oacc[rb], w_cur, [&](int row, int, f32x4 val) {
+        wave_tile_rowmajor<CW>(stage, lane, result, w_cur, [&](int row, int, f32x4 val) {
             if (wave_row0 + row < Sq_u) {
                 if (merge) {
                     const float wo = row_w_old[row];
@@ -917,6 +1003,15 @@ __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
     }
     }   // row block
     }   // part
+}
+
+template <int D, int RB>
+__global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
+    fwd_bf16_body<D, RB, 1>(p);
+}
+template <int D, int KS>
+__global__ __launch_bounds__(512) void fwd_bf16_shares_kernel(const FwdParams p) {
+    fwd_bf16_body<D, 1, KS>(p);
 }
 
 // ------------------------------------------------------------------------------ forward, fp32
@@ -2053,18 +2148,21 @@ __device__ __forceinline__ void lds_tr_gemm_at_rb(const unsigned (&addr)[D / 32]
     }
 }
 
-template <int D, int RB>   // RB = 32-row blocks per wave: a lane owns RB query rows, a block 256 * RB
-__global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
-    constexpr int NW = 8, BM = 32 * RB * NW, BN = FwdTile<D>::BN;   // 8 waves (two per SIMD) share every K / V tile
+// RB = 32-row blocks per wave: a lane owns RB query rows, a block 256 * RB / KS; KS = key shares per row group as in the forward
+template <int D, int RB, int KS>
+__device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
+    constexpr int NW = 8, RG = NW / KS, BM = 32 * RB * RG;   // 8 waves (two per SIMD) share every K / V tile
+    constexpr int BN = FwdTile<D, 1, KS>::BN, BNT = BN * KS; // keys per wave and per tile
     constexpr int CPR = D / 8;
     constexpr int RPI = 64 / CPR;            // rows filled by one wave-wide 16-byte-per-lane LDS-direct load (1 KB)
-    constexpr int NI = BN / (RPI * NW);       // such loads per wave, per tensor and per tile
+    constexpr int NI = BNT / (RPI * NW);      // such loads per wave, per tensor and per tile
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // two {K tile, V tile} buffers,
-    constexpr int TILE = BN * D;             // rows unpadded, 16-byte chunks XOR-swizzled (lds_swz)
+    constexpr int TILE = BNT * D;            // rows unpadded, 16-byte chunks XOR-swizzled (lds_swz)
     constexpr int BUF_ELEMS = 2 * TILE;
 
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = w / KS, ks = w % KS;      // row group and key share of the wave
     const bool causal = p.flags & LTR_CAUSAL;
 
     int idx = blockIdx.x, pair, rest;
@@ -2097,14 +2195,14 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
     bool row_ok[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
-        my_row[rb] = row0 + w * 32 * RB + 32 * rb + l32;
+        my_row[rb] = row0 + rg * 32 * RB + 32 * rb + l32;
         row_ok[rb] = my_row[rb] < p.Sq;
         my_pos[rb] = q_position(my_row[rb], p.q_split, p.q_pos0[0], p.q_pos0[1]);
     }
     int blk_lo, blk_hi, w_lo, w_hi;
     q_pos_range(row0, min(row0 + BM, p.Sq) - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], blk_lo, blk_hi);
     {
-        int wr0 = row0 + w * 32 * RB, wr1 = min(wr0 + 32 * RB, p.Sq) - 1;
+        int wr0 = row0 + rg * 32 * RB, wr1 = min(wr0 + 32 * RB, p.Sq) - 1;
         if (wr1 >= wr0) q_pos_range(wr0, wr1, p.q_split, p.q_pos0[0], p.q_pos0[1], w_lo, w_hi);
         else { w_lo = -0x7fffffff; w_hi = -0x7fffffff; }  // wave has no valid row: everything masked
     }
@@ -2134,7 +2232,7 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
                 for (int e = 0; e < 8; e++) part += (float)ov[e] * (float)doreg[rb][kb][e];
             }
             dlt[rb] = xhalf_sum(part);
-            if (row_ok[rb] && hh == 0) p.delta[((long long)b * p.Hq + h) * p.Sq + my_row[rb]] = dlt[rb];
+            if (row_ok[rb] && hh == 0 && ks == 0) p.delta[((long long)b * p.Hq + h) * p.Sq + my_row[rb]] = dlt[rb];
         }
         if (row_ok[rb]) {
             // a row that saw no key has LSE = -inf: give it +inf like a row past the end, so that P = exp2(-inf) = 0
@@ -2178,7 +2276,7 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
                 ld_kb = (const __bf16 *)p.chunk[c].k + b * p.ks[0] + hkv * p.ks[2];
                 ld_vb = (const __bf16 *)p.chunk[c].v + b * p.vs[0] + hkv * p.vs[2];
                 const int nvis = causal ? max(0, min(ld_sk, blk_hi - ld_pos0 + 1)) : ld_sk;
-                nt = (nvis + BN - 1) / BN;
+                nt = (nvis + BNT - 1) / BNT;
             }
         }
     };
@@ -2191,12 +2289,12 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
     auto gload = [&](int ti, int buf) {
         nx_sk = ld_sk;
         nx_pos0 = ld_pos0;
-        nx_key0 = ti * BN;
+        nx_key0 = ti * BNT;
         const unsigned Kd = lds_address(smem) + buf * BUF_ELEMS * 2, Vd = Kd + TILE * 2;   // LDS byte addresses
 #pragma unroll
         for (int i = 0; i < NI; i++) {
             const int row = RPI * (NI * w + i) + st_row;
-            const int key = min(ti * BN + row, ld_sk - 1);
+            const int key = min(ti * BNT + row, ld_sk - 1);
             const int chunk = st_pc ^ lds_swz<D>(row);
             global_to_lds_b128(ld_kb + (long long)(key * (int)p.ks[1] + chunk * 8), Kd + RPI * (NI * w + i) * D * 2);
             global_to_lds_b128(ld_vb + (long long)(key * (int)p.vs[1] + chunk * 8), Vd + RPI * (NI * w + i) * D * 2);
@@ -2213,7 +2311,7 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
     static_assert((BUF_ELEMS * 2 & (BUF_ELEMS * 2 - 1)) == 0, "buffer size must be a power of two for the XOR flip");
     unsigned pa[D / 16], ta[D / 32][2];
     {
-        const unsigned lds0 = lds_address(smem);   // the only LDS object of the kernel: aligned far beyond the buffer size
+        const unsigned lds0 = lds_address(smem) + (KS > 1 ? ks * BN * D * 2 : 0);   // the only LDS object of the kernel: aligned far beyond the buffer size
         const int sw = lds_swz<D>(l32) ^ hh;        // rows l32 + 32 n share the swizzle word of row l32
 #pragma unroll
         for (int kb = 0; kb < D / 16; kb++) pa[kb] = lds0 + ((l32 * D + (((2 * kb) ^ sw) << 3)) << 1);
@@ -2228,7 +2326,7 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
     }
     int par = 0;
     while (have) {
-        const int sk = nx_sk, pos0 = nx_pos0, key0 = nx_key0;
+        const int sk = nx_sk, pos0 = nx_pos0, key0 = nx_key0 + (KS > 1 ? ks * BN : 0);
         t++;
         settle();
         const bool have_next = c < p.n_chunks;
@@ -2238,7 +2336,7 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
         // 32 keys at a time, one block after the other: one live (S^T, dP^T) tile pair keeps the kernel at two
         // waves per SIMD, and the other wave's MFMAs cover this wave's softmax arithmetic.  A wave whose rows all
         // precede the tile's first key has nothing to add (see the forward kernel).
-        if (!causal || pos0 + key0 <= w_hi) {
+        if ((!causal || pos0 + key0 <= w_hi) && (KS == 1 || key0 < sk)) {
 #pragma unroll
         for (int nb = 0; nb < BN / 32; nb++) {
             f32x16 s[RB], dp[RB];
@@ -2297,14 +2395,23 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
         have = have_next;
     }
 
+    constexpr int CW = KeyShares<D, KS>::CW;   // columns a wave writes, from column col0 on
+    const int col0 = KS > 1 ? ks * CW : 0;
+    f32x16 own[CW / 32];                       // KS > 1: those columns, summed over the shares
+    if constexpr (KS > 1) {
+        static_assert(RB == 1, "key shares are built for one row block per wave");
+        collect_shares<D, KS>(smem, w, ks, lane, dqacc[0], 1.f, own);
+        __syncthreads();                        // the partials are read: their memory becomes the staging areas
+        if (col0 >= D) continue;                // more shares than 32-column groups: nothing left to write
+    }
     // dQ in whole rows through the wave's LDS staging area (the tiles are no longer read: the last barrier is behind us)
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
-        constexpr int LPR = D / 4, ROWS_PER_IT = 64 / LPR;      // see wave_tile_rowmajor
-        unsigned char *stage = smem + w * WaveStage<D>::BYTES;
-        const int Sq_u = uniform32(p.Sq), wave_row0 = uniform32(row0 + w * 32 * RB + 32 * rb);
+        constexpr int LPR = CW / 4, ROWS_PER_IT = 64 / LPR;      // see wave_tile_rowmajor
+        unsigned char *stage = smem + w * WaveStage<CW>::BYTES;
+        const int Sq_u = uniform32(p.Sq), wave_row0 = uniform32(row0 + rg * 32 * RB + 32 * rb);
         const long long dqs1 = uniform64(p.dqs[1]);
-        const long long off0 = uniform64(b * p.dqs[0] + h * p.dqs[2]) + (wave_row0 + lane / LPR) * dqs1 + 4 * (lane % LPR);
+        const long long off0 = uniform64(b * p.dqs[0] + h * p.dqs[2] + col0) + (wave_row0 + lane / LPR) * dqs1 + 4 * (lane % LPR);
         // LTR_ROPE_DQ: q was rotated by the forward's prologue, so the gradient of the caller's un-rotated q is dQ rotated by
         // the conjugate angles of its row's position (the rotation is linear: it commutes with the accumulation over calls)
         const bool rope = uniform32(p.flags & LTR_ROPE_DQ) != 0;
@@ -2313,11 +2420,15 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
         auto unrotate = [&](int row, int col, f32x4 val) {
             if (!rope) return val;
             const int pos = q_position(wave_row0 + row, split_u, qp0, qp1);
-            return rope_conj4(val, *(const f32x4 *)(rope_tab + (long long)(pos - rope_p0) * D + col));
+            return rope_conj4(val, *(const f32x4 *)(rope_tab + (long long)(pos - rope_p0) * D + col0 + col));
         };
+        auto &result = [&]() -> f32x16(&)[CW / 32] {
+            if constexpr (KS > 1) return own;
+            else return dqacc[rb];
+        }();
         if (uniform32(p.flags & LTR_DQ_BF16)) {   // this call saw every key of these rows: store the result, no accumulator
             __bf16 *dqp = (__bf16 *)p.dq + off0;
-            wave_tile_rowmajor<D>(stage, lane, dqacc[rb], p.scale, [&](int row, int col, f32x4 val) {
+            wave_tile_rowmajor<CW>(stage, lane, result, p.scale, [&](int row, int col, f32x4 val) {
                 if (wave_row0 + row < Sq_u) {
                     val = unrotate(row, col, val);
                     bf16x4 y;
@@ -2337,7 +2448,7 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
                 if (wave_row0 + it * ROWS_PER_IT + lane / LPR < Sq_u) old[it] = *(const f32x4 *)(dqp + it * ROWS_PER_IT * dqs1);
             }
             int it = 0;
-            wave_tile_rowmajor<D>(stage, lane, dqacc[rb], p.scale, [&](int row, int col, f32x4 val) {
+            wave_tile_rowmajor<CW>(stage, lane, result, p.scale, [&](int row, int col, f32x4 val) {
                 if (wave_row0 + row < Sq_u) {
                     val = unrotate(row, col, val);
 #pragma unroll
@@ -2350,6 +2461,15 @@ __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
         }
     }
     }   // part
+}
+
+template <int D, int RB>
+__global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
+    bwd_dq_body<D, RB, 1>(p);
+}
+template <int D, int KS>
+__global__ __launch_bounds__(512) void bwd_dq_shares_kernel(const BwdParams p) {
+    bwd_dq_body<D, 1, KS>(p);
 }
 
 // ------------------------------------------------------------------------------ backward, fp32
@@ -2999,53 +3119,50 @@ constexpr int fwd_lds_bytes() {   // the K / V tile buffers, reused by the epilo
 }
 template <int D>
 constexpr int dq_lds_bytes() { return fwd_lds_bytes<D>(); }   // same tile buffers and staging areas as the forward
+template <int D, int KS>
+constexpr int shares_lds_bytes() {   // forward and dQ kernels with key shares: tile buffers, then the shares' partial results
+    return 2 * 2 * FwdTile<D, 1, KS>::BN * KS * D * 2 > KeyShares<D, KS>::BYTES ? 2 * 2 * FwdTile<D, 1, KS>::BN * KS * D * 2 : KeyShares<D, KS>::BYTES;
+}
+static_assert(shares_lds_bytes<128, 2>() <= 160 * 1024 && shares_lds_bytes<128, 4>() <= 160 * 1024 && shares_lds_bytes<64, 4>() <= 160 * 1024, "LDS of one CU");
+static_assert(8 * WaveStage<64>::BYTES <= shares_lds_bytes<128, 2>() && 8 * WaveStage<32>::BYTES <= shares_lds_bytes<64, 2>(), "staging areas");
 
 int enable_large_lds() {
     int dev = 0;
     if (current_device(&dev)) return LTR_EDEVICE;
     if (g_dev[dev].large_lds.load(std::memory_order_acquire) == 1) return LTR_OK;
-    bool ok = hipFuncSetAttribute((const void *)bwd_dkdv_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  BwdLds<128, 1>::TOTAL) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dkdv_kernel<64, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  BwdLds<64, 1>::TOTAL) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dkdv_kernel<64, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  BwdLds<64, 2>::TOTAL) == hipSuccess &&
-              hipFuncSetAttribute((const void *)fwd_bf16_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  fwd_lds_bytes<128>()) == hipSuccess &&
-              hipFuncSetAttribute((const void *)fwd_bf16_kernel<64, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  fwd_lds_bytes<64>()) == hipSuccess &&
-              hipFuncSetAttribute((const void *)fwd_bf16_kernel<64, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  fwd_lds_bytes<64, 2>()) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dq_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  dq_lds_bytes<128>()) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dq_kernel<64, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  dq_lds_bytes<64>()) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dq_kernel<64, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  dq_lds_bytes<64>()) == hipSuccess &&
-              hipFuncSetAttribute((const void *)fwd_f32_mfma_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<128, 1>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)fwd_f32_mfma_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<128, 2>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)fwd_f32_mfma_kernel<64, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<64, 1>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)fwd_f32_mfma_kernel<64, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<64, 2>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)fwd_f32_mfma_kernel<64, 4>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<64, 4>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dq_f32_mfma_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<128, 1>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dq_f32_mfma_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<128, 2>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dq_f32_mfma_kernel<64, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<64, 1>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dq_f32_mfma_kernel<64, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<64, 2>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dq_f32_mfma_kernel<64, 4>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32Mfma<64, 4>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dkdv_f32_mfma_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32DkdvLds<128>::LDS) == hipSuccess &&
-              hipFuncSetAttribute((const void *)bwd_dkdv_f32_mfma_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  F32DkdvLds<64>::LDS) == hipSuccess;
+    const struct { const void *kernel; int bytes; } large[] = {
+        {(const void *)bwd_dkdv_kernel<128, 1>, BwdLds<128, 1>::TOTAL},
+        {(const void *)bwd_dkdv_kernel<64, 1>, BwdLds<64, 1>::TOTAL},
+        {(const void *)bwd_dkdv_kernel<64, 2>, BwdLds<64, 2>::TOTAL},
+        {(const void *)fwd_bf16_kernel<128, 1>, fwd_lds_bytes<128>()},
+        {(const void *)fwd_bf16_kernel<64, 1>, fwd_lds_bytes<64>()},
+        {(const void *)fwd_bf16_kernel<64, 2>, fwd_lds_bytes<64, 2>()},
+        {(const void *)bwd_dq_kernel<128, 1>, dq_lds_bytes<128>()},
+        {(const void *)bwd_dq_kernel<64, 1>, dq_lds_bytes<64>()},
+        {(const void *)bwd_dq_kernel<64, 2>, dq_lds_bytes<64>()},
+        {(const void *)fwd_f32_mfma_kernel<128, 1>, F32Mfma<128, 1>::LDS},
+        {(const void *)fwd_f32_mfma_kernel<128, 2>, F32Mfma<128, 2>::LDS},
+        {(const void *)fwd_f32_mfma_kernel<64, 1>, F32Mfma<64, 1>::LDS},
+        {(const void *)fwd_f32_mfma_kernel<64, 2>, F32Mfma<64, 2>::LDS},
+        {(const void *)fwd_f32_mfma_kernel<64, 4>, F32Mfma<64, 4>::LDS},
+        {(const void *)bwd_dq_f32_mfma_kernel<128, 1>, F32Mfma<128, 1>::LDS},
+        {(const void *)bwd_dq_f32_mfma_kernel<128, 2>, F32Mfma<128, 2>::LDS},
+        {(const void *)bwd_dq_f32_mfma_kernel<64, 1>, F32Mfma<64, 1>::LDS},
+        {(const void *)bwd_dq_f32_mfma_kernel<64, 2>, F32Mfma<64, 2>::LDS},
+        {(const void *)bwd_dq_f32_mfma_kernel<64, 4>, F32Mfma<64, 4>::LDS},
+        {(const void *)bwd_dkdv_f32_mfma_kernel<128>, F32DkdvLds<128>::LDS},
+        {(const void *)bwd_dkdv_f32_mfma_kernel<64>, F32DkdvLds<64>::LDS},
+        {(const void *)fwd_bf16_shares_kernel<128, 2>, shares_lds_bytes<128, 2>()},
+        {(const void *)fwd_bf16_shares_kernel<128, 4>, shares_lds_bytes<128, 4>()},
+        {(const void *)fwd_bf16_shares_kernel<64, 2>, shares_lds_bytes<64, 2>()},
+        {(const void *)fwd_bf16_shares_kernel<64, 4>, shares_lds_bytes<64, 4>()},
+        {(const void *)bwd_dq_shares_kernel<128, 2>, shares_lds_bytes<128, 2>()},
+        {(const void *)bwd_dq_shares_kernel<128, 4>, shares_lds_bytes<128, 4>()},
+        {(const void *)bwd_dq_shares_kernel<64, 2>, shares_lds_bytes<64, 2>()},
+        {(const void *)bwd_dq_shares_kernel<64, 4>, shares_lds_bytes<64, 4>()},
+    };
+    bool ok = true;
+    for (const auto &k : large) ok = ok && hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, k.bytes) == hipSuccess;
     if (!ok) {
         (void)hipGetLastError();
         return LTR_ELAUNCH;
@@ -3129,18 +3246,69 @@ int q_tile_slots(int n_qtiles, long long blocks_per_tile, bool uneven) {
     return n * 10 >= rounds * cus * 9 ? n_slots : n_qtiles;
 }
 
+// Waves that share a row group's keys in the bf16 forward and dQ kernels.  Blocks of 256 rows leave CUs idle when a launch has few
+// rows (a short or single sequence, few heads), and the longest block of a causal launch then decides its time; with 2 or 4
+// waves per row group a block has 128 or 64 rows and each wave walks half or a quarter of the keys.  The price is more K / V
+// traffic per row and the merge at the end.  The choice compares launch times: a q tile costs its K / V tiles times step_us plus
+// fixed_us, blocks run longest first, one per CU.  Constants fitted to 24 shapes with every size forced; forward / dQ
+// kernel in us, shares 1, 2, 4 (with the launch gap):
+//   B=1 32 heads D=128 causal S=1237   38.1 / 48.1    26.7 / 32.9    36.3 / 43.3
+//   B=1  8 heads D=128 causal S=4096   99.0 / 128.7   64.8 / 81.3    52.7 / 66.1
+//   B=1  8 heads D=64  causal S=4096   64.9 / 72.8    40.4 / 46.6    34.5 / 40.8
+//   B=1 32 heads D=128 causal S=4096  135.1 / 183.9  158.5 / 204.6  203.2 / 256.8   (256-row blocks fill the device)
+struct ShareCost {
+    double step_us[3], fixed_us[3];   // per step (one K / V tile) and per block, for 1, 2 and 4 shares
+};
+int key_shares(const ShareCost &cost, int D, bool causal, long long BH, long long kv_heads, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks) {
+    const int cus = device_cus();
+    if (BH * ((Sq + 255) / 256) >= 4LL * cus) return 1;   // several rounds of 256-row blocks: they balance by themselves
+    int best = 1;
+    double best_us = 0;
+    for (int i = 0; i < 3; i++) {
+        const int ks = 1 << i, rows = 256 / ks, keys = ks * (D == 64 ? (ks == 1 ? 128 : 64) : (ks == 4 ? 32 : 64));
+        const int n = (Sq + rows - 1) / rows;
+        // more than one kv head per XCD and every CU busy: the extra K / V traffic of the shares shows (B=1, 32 kv heads, D=128,
+        // S=2048: 57 us with one share, 67 with two; with 8 kv heads 57 and 49)
+        const double step_us = cost.step_us[i] * (ks > 1 && BH * n > cus && kv_heads > 8 ? 1.25 : 1.0);
+        double sum = 0, most = 0;
+        for (int t = 0; t < n; t++) {
+            double steps = 0;
+            const int r0 = t * rows, r1 = std::min(Sq, r0 + rows) - 1;
+            int hi = r1 < q_split ? q_pos0[0] + r1 : q_pos0[1] + (r1 - q_split);
+            if (r0 < q_split && r1 >= q_split) hi = std::max(hi, q_pos0[0] + q_split - 1);
+            for (int c = 0; c < n_chunks; c++) {
+                const long long seen = causal ? std::min<long long>(std::max<long long>((long long)hi - chunk[c].pos0 + 1, 0), chunk[c].sk) : chunk[c].sk;
+                steps += (double)((seen + keys - 1) / keys);
+            }
+            const double us = steps * step_us + cost.fixed_us[i];
+            sum += us;
+            most = std::max(most, us);
+        }
+        const double us = BH * n <= cus ? most : std::max(most, sum * BH / cus + 0.25 * sum / n);
+        if (i == 0 || us < 0.97 * best_us) {
+            best_us = us;
+            best = ks;
+        }
+    }
+    return best;
+}
+constexpr ShareCost FWD_SHARES_128{{1.45, 1.8, 1.05}, {9.0, 8.0, 10.0}}, FWD_SHARES_64{{1.7, 0.95, 1.0}, {9.0, 8.0, 6.0}};
+constexpr ShareCost DQ_SHARES_128{{1.85, 2.2, 1.4}, {11.0, 10.0, 10.0}}, DQ_SHARES_64{{1.95, 1.15, 1.35}, {10.0, 9.0, 6.0}};
+
 // What a forward launch looks like: rows per block, q tiles, slots (see q_tile_slots), blocks.  One function decides for
 // ltr_attn_fwd and for ltr_attn_plan, so the plan a caller is shown is the launch it gets.
 struct FwdPlan {
     bool wide;          // 512-row blocks (two 32-row blocks per wave, head dim 64)
+    int ks;             // bf16: key shares per row group (1, or 2 / 4 with blocks of 256 / ks rows; see key_shares)
     int f32_ks;         // fp32: 0 = scalar kernel, else the key shares per row group of fwd_f32_mfma_kernel
     int rows, n_qtiles, n_slots;
     long long blocks;
 };
-FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
+FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
                  int n_chunks) {
     FwdPlan pl;
     pl.f32_ks = 0;
+    pl.ks = 1;
     if (f32) {
         pl.wide = false;
         if (flags & LTR_FWD_F32_SCALAR) {
@@ -3163,7 +3331,10 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Sq, int q_s
     // query rows per block: 512 (two 32-row blocks per wave, 64-key tiles) pays at head dim 64 under the conditions of
     // the dQ kernel's 512-row blocks (see plan_bwd)
     bool wide = (flags & LTR_FWD_ROWS_512) != 0;
-    if (!wide && !(flags & LTR_FWD_ROWS_256) && D == 64) {
+    if (!wide && !(flags & LTR_FWD_ROWS_256))
+        pl.ks = key_shares(D == 128 ? FWD_SHARES_128 : FWD_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
+                           n_chunks);
+    if (!wide && !(flags & LTR_FWD_ROWS_256) && D == 64 && pl.ks == 1) {
         const int tiles512 = (Sq + 511) / 512;
         const int slots512 = q_tile_slots(tiles512, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, 512, q_split, q_pos0, chunk, n_chunks));
         const long long blocks512 = (long long)slots512 * B * Hq, blocks256 = (long long)((Sq + 255) / 256) * B * Hq;
@@ -3172,6 +3343,12 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Sq, int q_s
                        : (cu_fill(blocks512, cus) * 1.07 >= cu_fill(blocks256, cus));
     }
     pl.wide = wide;
+    if (pl.ks > 1) {
+        pl.rows = 256 / pl.ks;
+        pl.n_qtiles = pl.n_slots = (Sq + pl.rows - 1) / pl.rows;
+        pl.blocks = (long long)pl.n_qtiles * B * Hq;
+        return pl;
+    }
     pl.rows = wide ? 512 : 256;
     pl.n_qtiles = (Sq + pl.rows - 1) / pl.rows;
     pl.n_slots = q_tile_slots(pl.n_qtiles, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, pl.rows, q_split, q_pos0, chunk, n_chunks));
@@ -3246,6 +3423,7 @@ struct BwdPlan {
     KvSplit split;      // blocks per key tile (1 unless the caller brought a workspace for their partial sums)
     int64_t part_bytes; // workspace they need
     bool wide_q;        // dQ kernel: 512 rows per block
+    int dq_ks;          // bf16 dQ kernel: key shares per row group, as in the forward
     int dq_rows, dq_qtiles, dq_slots;
     long long dq_blocks;
 };
@@ -3255,6 +3433,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.f32_ks = 0;
     pl.split = KvSplit{1, 1};
     pl.part_bytes = 0;
+    pl.dq_ks = 1;
     may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
     auto split_keys = [&](const KvSplitCost &cost) {
         if (may_split) pl.split = kv_split(cost, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks);
@@ -3278,6 +3457,9 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         pl.kv_tiles = 0;
         for (int c = 0; c < n_chunks; c++) pl.kv_tiles += (chunk[c].sk + pl.keys_per_block - 1) / pl.keys_per_block;
         pl.kv_blocks = pl.kv_tiles * B * Hkv;
+        // fp32 sums of more than 4096 rows keep their one serial order: its rounding reaches 1e-4 of single elements (measured at
+        // 27064 rows), and a sum in another order differs from it by as much
+        may_split = may_split && (long long)(Hq / Hkv) * Sq <= 4096;
         split_keys(D == 128 ? KvSplitCost{32, 9.0, 2.0, 6e6} : KvSplitCost{32, 4.5, 1.5, 6e6});
         pl.dq_qtiles = pl.dq_slots = (Sq + pl.dq_rows - 1) / pl.dq_rows;
         pl.dq_blocks = (long long)pl.dq_qtiles * B * Hq;
@@ -3311,7 +3493,10 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     // query rows per block of the dQ kernel: 512 (two 32-row blocks per wave) pays at head dim 64 when the wider blocks still
     // fill the device, and under a causal mask only on sequences long enough that the diagonal does not dominate
     bool wide_q = (flags & LTR_DQ_ROWS_512) != 0;
-    if (!wide_q && !(flags & LTR_DQ_ROWS_256) && D == 64 && !(flags & LTR_NO_DQ)) {
+    if (!wide_q && !(flags & (LTR_DQ_ROWS_256 | LTR_NO_DQ)))
+        pl.dq_ks = key_shares(D == 128 ? DQ_SHARES_128 : DQ_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
+                              n_chunks);
+    if (!wide_q && !(flags & LTR_DQ_ROWS_256) && D == 64 && !(flags & LTR_NO_DQ) && pl.dq_ks == 1) {
         const int tiles512 = (Sq + 511) / 512;
         const int slots512 = q_tile_slots(tiles512, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, 512, q_split, q_pos0, chunk, n_chunks));
         const long long blocks512 = (long long)slots512 * B * Hq;
@@ -3323,9 +3508,10 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
                          : (cu_fill(blocks512, cus) * 1.07 >= cu_fill(blocks256, cus));
     }
     pl.wide_q = wide_q;
-    pl.dq_rows = wide_q ? 512 : 256;
+    pl.dq_rows = wide_q ? 512 : 256 / pl.dq_ks;
     pl.dq_qtiles = (Sq + pl.dq_rows - 1) / pl.dq_rows;
-    pl.dq_slots = q_tile_slots(pl.dq_qtiles, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks));
+    pl.dq_slots = pl.dq_ks > 1 ? pl.dq_qtiles
+                               : q_tile_slots(pl.dq_qtiles, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks));
     pl.dq_blocks = (long long)pl.dq_slots * B * Hq;
     return pl;
 }
@@ -3453,13 +3639,19 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     p.n_chunks = a->n_chunks;
     hipStream_t st = (hipStream_t)stream;
     if ((a->flags & LTR_FWD_ROWS_512) && (a->D != 64 || a->io_dtype != LTR_BF16)) return LTR_EUNSUP;
-    const FwdPlan pl = plan_fwd(a->D, a->io_dtype == LTR_F32, a->flags, p.B, p.Hq, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks);
+    const FwdPlan pl = plan_fwd(a->D, a->io_dtype == LTR_F32, a->flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks);
     if (pl.blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.n_qtiles = pl.n_qtiles;
     p.n_slots = pl.n_slots;
     if (a->io_dtype == LTR_BF16) {
         rc = enable_large_lds();
         if (rc) return rc;
+        if (pl.ks == 2)
+            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 2>, pl.blocks, 512, shares_lds_bytes<128, 2>(), st, p)
+                               : launch((const void *)fwd_bf16_shares_kernel<64, 2>, pl.blocks, 512, shares_lds_bytes<64, 2>(), st, p);
+        if (pl.ks == 4)
+            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 4>, pl.blocks, 512, shares_lds_bytes<128, 4>(), st, p)
+                               : launch((const void *)fwd_bf16_shares_kernel<64, 4>, pl.blocks, 512, shares_lds_bytes<64, 4>(), st, p);
         if (a->D == 128) return launch((const void *)fwd_bf16_kernel<128, 1>, pl.blocks, 512, fwd_lds_bytes<128>(), st, p);
         if (pl.wide) return launch((const void *)fwd_bf16_kernel<64, 2>, pl.blocks, 512, fwd_lds_bytes<64, 2>(), st, p);
         return launch((const void *)fwd_bf16_kernel<64, 1>, pl.blocks, 512, fwd_lds_bytes<64>(), st, p);
@@ -3659,7 +3851,13 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     if (rc) return rc;
     // the dQ kernel goes first: with LTR_DELTA_FROM_O it produces the DELTA that the dK/dV kernel reads
     if (do_dq) {
-        if (a->D == 128) rc = launch((const void *)bwd_dq_kernel<128, 1>, pl.dq_blocks, 512, dq_lds_bytes<128>(), st, p);
+        if (pl.dq_ks == 2)
+            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 2>, pl.dq_blocks, 512, shares_lds_bytes<128, 2>(), st, p)
+                             : launch((const void *)bwd_dq_shares_kernel<64, 2>, pl.dq_blocks, 512, shares_lds_bytes<64, 2>(), st, p);
+        else if (pl.dq_ks == 4)
+            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 4>, pl.dq_blocks, 512, shares_lds_bytes<128, 4>(), st, p)
+                             : launch((const void *)bwd_dq_shares_kernel<64, 4>, pl.dq_blocks, 512, shares_lds_bytes<64, 4>(), st, p);
+        else if (a->D == 128) rc = launch((const void *)bwd_dq_kernel<128, 1>, pl.dq_blocks, 512, dq_lds_bytes<128>(), st, p);
         else if (pl.wide_q) rc = launch((const void *)bwd_dq_kernel<64, 2>, pl.dq_blocks, 512, dq_lds_bytes<64>(), st, p);
         else rc = launch((const void *)bwd_dq_kernel<64, 1>, pl.dq_blocks, 512, dq_lds_bytes<64>(), st, p);
         if (rc) return rc;
@@ -3739,7 +3937,7 @@ extern "C" int ltr_attn_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out) {
         chunk[c].pos0 = (int)ch.pos0;
     }
     const int q_pos0[2] = {(int)a->q_pos0[0], (int)a->q_pos0[1]};
-    const FwdPlan f = plan_fwd(a->D, f32, flags, a->B, a->Hq, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks);
+    const FwdPlan f = plan_fwd(a->D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks);
     const BwdPlan b = plan_bwd(a->D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks);
     out->compute_units = device_cus();
     out->fwd_rows = f.rows;
@@ -3761,8 +3959,10 @@ extern "C" int ltr_attn_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out) {
             snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_f32_kernel<%d, *>", a->D);
         }
     } else {
-        snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_kernel<%d, %d>", a->D, f.wide ? 2 : 1);
-        snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_kernel<%d, %d>", a->D, b.wide_q ? 2 : 1);
+        if (f.ks > 1) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_shares_kernel<%d, %d>", a->D, f.ks);
+        else snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_kernel<%d, %d>", a->D, f.wide ? 2 : 1);
+        if (b.dq_ks > 1) snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_shares_kernel<%d, %d>", a->D, b.dq_ks);
+        else snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_kernel<%d, %d>", a->D, b.wide_q ? 2 : 1);
         snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", a->D, b.wide_kv ? 2 : 1);
     }
     return LTR_OK;
