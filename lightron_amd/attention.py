@@ -558,9 +558,9 @@ class SingleChunkAttentionFunction(torch.autograd.Function):
         return dq, dk, dv, None
 
 
-# The single-chunk bf16 call has two host sides over the same two C-ABI calls: a C++ autograd node (_ltr_node.so, built by
-# lightron_amd.build: the backward then runs on the autograd thread without the interpreter) and SingleChunkAttentionFunction
-# (Python).  The C++ node is used when it has been built for this ABI version and the library is the in-tree one.
+# A call has two host sides over the same C-ABI calls: a C++ autograd node (_ltr_node.so, built by lightron_amd.build: arguments are
+# filled and the backward runs on the autograd thread without the interpreter) and the Python Functions above.  The C++ node is
+# used when it has been built for this ABI version and the library is the in-tree one.
 USE_CPP_NODE = True
 _node = None
 
@@ -577,6 +577,23 @@ def _cpp_node():
             except (ImportError, OSError):       # not built, or built against another torch: the Python node serves
                 pass
     return _node
+
+
+def chunk_table_attention(q, ks, vs, entries, q_pos0, q_split, causal, scale, stepwise, out_dtype, kv_grad_acc, q_rope):
+    """(O, LSE) through the C++ node, or None when it cannot serve the call (not built, host tensors, chunks whose strides differ).
+    entries: flat (index into ks / vs, first row, rows, global position of the first) per entry of the chunk table."""
+    node = _cpp_node() if USE_CPP_NODE else None
+    if not node or not q.is_cuda or q.shape[-1] not in (64, 128) or q.dtype not in _DT:
+        return None
+    out_dtype = out_dtype or q.dtype
+    if out_dtype not in _DT or (q.dtype == torch.float32 and out_dtype != torch.float32):
+        return None
+    qa, qb = q_pos0 if isinstance(q_pos0, (tuple, list)) else (q_pos0, q_pos0)
+    dk, dv = kv_grad_acc if kv_grad_acc is not None else ((), ())
+    res = node.chunks(q, [*ks, *vs], entries, int(qa), int(qb), q.shape[1] if q_split is None else int(q_split), bool(causal),
+                      scale if scale is not None else 1.0 / math.sqrt(q.shape[3]), _stream_ptr(q.device), int(stepwise),
+                      out_dtype == torch.float32, dk, dv, q_rope)
+    return res or None
 
 
 _warned_pad = False
@@ -650,5 +667,10 @@ def block_attention(q, ks, vs, k_pos0, q_pos0=0, q_split=None, causal=False, sca
                 raise RuntimeError("kv_grad_acc entries must be fp32 tensors shaped like their chunks")
     if q_rope is not None and q.dtype != torch.bfloat16:
         raise RuntimeError("the fused RoPE prologue is implemented for bf16 q")
+    if n:
+        res = chunk_table_attention(q, ks, vs, [x for i in range(n) for x in (i, 0, ks[i].shape[1], int(k_pos0[i]))], q_pos0, q_split, causal, scale,
+                                    stepwise, out_dtype, kv_grad_acc, q_rope)
+        if res is not None:
+            return res[0], res[1]
     return BlockAttentionFunction.apply(q, n, list(k_pos0), q_pos0, q_split, causal, scale, stepwise, out_dtype,
                                         kv_grad_acc, q_rope, *ks, *vs)

@@ -14,7 +14,7 @@ from typing import List, Optional, Sequence, Tuple
 
 import torch
 
-from .attention import block_attention
+from .attention import block_attention, chunk_table_attention
 
 
 class RingKVGrads:
@@ -25,20 +25,30 @@ class RingKVGrads:
 
     def __init__(self, kv: Sequence):
         self.kv = list(kv)
-        self.dk = [torch.zeros(k.shape, dtype=torch.float32, device=k.device) for k, _ in self.kv]
-        self.dv = [torch.zeros(v.shape, dtype=torch.float32, device=v.device) for _, v in self.kv]
+        # one buffer, cut at multiples of 64 elements: cleared by one fill, cast by one launch
+        tensors = [k for k, _ in self.kv] + [v for _, v in self.kv]
+        self._cuts, end = [], 0
+        for t in tensors:
+            self._cuts.append(end)
+            end += (t.numel() + 63) // 64 * 64
+        self._buf = torch.zeros(end, dtype=torch.float32, device=tensors[0].device if tensors else None)
+        acc = self._views(self._buf)
+        self.dk, self.dv = acc[:len(self.kv)], acc[len(self.kv):]
+
+    def _views(self, buf):
+        tensors = [k for k, _ in self.kv] + [v for _, v in self.kv]
+        return [buf[a:a + t.numel()].view(t.shape) for a, t in zip(self._cuts, tensors)]
 
     def zero_(self):
-        for t in self.dk + self.dv:
-            t.zero_()
+        self._buf.zero_()
 
     def finalize(self, assign: bool = True):
         """[(dK, dV)] per rank in the chunks' dtype; with assign=True also added to k.grad / v.grad of leaf tensors."""
         from .attention import cast_to_bf16
         out = []
-        for (k, v), dk, dv in zip(self.kv, self.dk, self.dv):
-            gk = cast_to_bf16(dk) if k.dtype == torch.bfloat16 else dk.to(k.dtype)
-            gv = cast_to_bf16(dv) if v.dtype == torch.bfloat16 else dv.to(v.dtype)
+        grads = self._views(cast_to_bf16(self._buf)) if all(t.dtype == torch.bfloat16 for kv in self.kv for t in kv) else self.dk + self.dv
+        for (k, v), dk, dv in zip(self.kv, grads[:len(self.kv)], grads[len(self.kv):]):
+            gk, gv = dk.to(k.dtype), dv.to(v.dtype)
             if assign:
                 for t, g in ((k, gk), (v, gv)):
                     if t.requires_grad and t.is_leaf:
@@ -141,12 +151,25 @@ def ring_attention_with_lse(local_q, local_k, local_v, cp_group) -> Tuple[torch.
         q_pos0, q_split = (ring.rank * hc, (2 * W - 1 - ring.rank) * hc), hc
     else:
         q_pos0, q_split = (ring.rank * S_local, ring.rank * S_local), S_local
-    ks, vs, pos, grad_acc = _chunk_table(ring, local_k, local_v, S_local)
-    if grad_acc is not None and ring.kv[ring.rank] is None:
+    if ring.kv_grads is not None and ring.kv[ring.rank] is None:
         raise RuntimeError("kv_grads needs the ring's own chunk in LocalRing.kv (entry %d is None)" % ring.rank)
     # a ring step delivers one rank's chunk: one table entry, or the two half-chunks of a zig-zag chunk in ONE launch (the
     # dK/dV and forward kernels then see twice the keys per launch: a block for every CU where a half-chunk leaves half idle)
     step = (2 if ring.layout == "zigzag" else 1) if ring.stepwise else False
+    # the ranks' tensors as they are, halves of a zig-zag chunk named by row offsets: no views, and one gradient per tensor
+    order = ring.order()
+    kv = [ring.kv[j] if ring.kv[j] is not None else (local_k, local_v) if j == ring.rank else None for j in order]
+    if None not in kv and all(k.shape[1] > (hc if ring.layout == "zigzag" else 0) for k, _ in kv):
+        if ring.layout == "zigzag":
+            entries = [x for t, j in enumerate(order) for x in (t, 0, hc, j * hc, t, hc, kv[t][0].shape[1] - hc, (2 * W - 1 - j) * hc)]
+        else:
+            entries = [x for t, j in enumerate(order) for x in (t, 0, kv[t][0].shape[1], j * S_local)]
+        acc = ring.kv_grads
+        res = chunk_table_attention(local_q, [k for k, _ in kv], [v for _, v in kv], entries, q_pos0, q_split, ring.causal, None, step,
+                                    ring.out_dtype, None if acc is None else ([acc.dk[j] for j in order], [acc.dv[j] for j in order]), None)
+        if res is not None:
+            return res[0], res[1]
+    ks, vs, pos, grad_acc = _chunk_table(ring, local_k, local_v, S_local)
     o, lse = block_attention(local_q, ks, vs, pos, q_pos0, q_split, ring.causal, None, step,
                              ring.out_dtype, grad_acc)
     return o, lse
