@@ -70,6 +70,10 @@ extern "C" {
 #define LTR_BWD_F32_SCALAR 65536u /* backward, fp32 only: the scalar fp32 kernels instead of the matrix-pipe ones (fallback and
                                     cross-check) */
 
+#define LTR_HEAD_COLS 131072u /* forward and backward, bf16: D may be any multiple of 8 up to 128; the kernels of the next width (64 or 128)
+                                run with their columns past D cleared on chip: no padded copies of the tensors.  scale is the caller's
+                                (1/sqrt of the true D); a RoPE table has D/2 pairs per row.  No 512-row / 256-key blocks. */
+
 /* error codes */
 #define LTR_OK 0
 #define LTR_EINVAL (-1)   /* null pointer, bad size, bad flag */
@@ -106,7 +110,7 @@ typedef struct ltr_attn_fwd_args {
     const void *q;      /* [B, Sq, Hq, D] by q strides; dtype io_dtype */
     void *o;            /* same logical shape by o strides; dtype o_dtype */
     float *lse;         /* [B, Hq, Sq] */
-    int32_t B, Hq, Hkv, D; /* D in {64, 128} */
+    int32_t B, Hq, Hkv, D; /* D in {64, 128}; others with LTR_HEAD_COLS */
     int64_t Sq;
     int64_t q_stride[3];  /* batch, seq, head */
     int64_t o_stride[3];
@@ -115,7 +119,7 @@ typedef struct ltr_attn_fwd_args {
     int64_t q_pos0[2];
     int64_t q_split;
     float scale;          /* 1/sqrt(D) at every reference call site (ring_attention.py:20) */
-    uint32_t flags;       /* LTR_CAUSAL | LTR_MERGE | LTR_ROPE_Q | LTR_FWD_ROWS_256 | LTR_FWD_ROWS_512 | LTR_FWD_F32_SCALAR */
+    uint32_t flags;       /* LTR_CAUSAL | LTR_MERGE | LTR_ROPE_Q | LTR_FWD_ROWS_256 | LTR_FWD_ROWS_512 | LTR_FWD_F32_SCALAR | LTR_HEAD_COLS */
     int32_t io_dtype;     /* LTR_BF16 or LTR_F32, of q/k/v */
     int32_t o_dtype;      /* LTR_BF16 or LTR_F32 */
     int32_t n_chunks;     /* 1..LTR_MAX_CHUNKS */
@@ -198,7 +202,8 @@ typedef struct ltr_attn_bwd_args {
     int64_t q_split;
     float scale;
     uint32_t flags;       /* LTR_CAUSAL | LTR_NO_DQ | LTR_NO_DKDV | LTR_DQ_BF16 | LTR_DELTA_FROM_O | LTR_DKDV_BF16 | LTR_ROPE_DQ |
-                             LTR_DKDV_KEYS_128 | LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR */
+                             LTR_DKDV_KEYS_128 | LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR |
+                             LTR_HEAD_COLS */
     int32_t io_dtype;     /* LTR_BF16 or LTR_F32, of q/k/v/dO (LTR_F32: fp32 kernels on v_mfma_f32_32x32x2_f32 for the 1e-4 cases;
                              LTR_DQ_BF16, LTR_DELTA_FROM_O and LTR_DKDV_BF16 are bf16 only and return LTR_EUNSUP with it) */
     int32_t n_chunks;

@@ -579,11 +579,24 @@ def _cpp_node():
     return _node
 
 
+def _native_cols(q, ks, vs, kv_grad_acc):
+    """Whether the kernels take these tensors of a head dim other than 64 / 128 as they are (LTR_HEAD_COLS): bf16, a multiple of 8
+    up to 128, rows that start 16-byte aligned."""
+    D = q.shape[-1]
+    if q.dtype != torch.bfloat16 or D % 8 or not 0 < D <= 128 or kv_grad_acc is not None:
+        return False
+    for t in (q, *ks, *vs):
+        b, s, h, d = t.stride()
+        if d != 1 or (b | s | h) % 8 or t.data_ptr() % 16:
+            return False
+    return True
+
+
 def chunk_table_attention(q, ks, vs, entries, q_pos0, q_split, causal, scale, stepwise, out_dtype, kv_grad_acc, q_rope):
     """(O, LSE) through the C++ node, or None when it cannot serve the call (not built, host tensors, chunks whose strides differ).
     entries: flat (index into ks / vs, first row, rows, global position of the first) per entry of the chunk table."""
     node = _cpp_node() if USE_CPP_NODE else None
-    if not node or not q.is_cuda or q.shape[-1] not in (64, 128) or q.dtype not in _DT:
+    if not node or not q.is_cuda or q.dtype not in _DT or (q.shape[-1] not in (64, 128) and not _native_cols(q, ks, vs, kv_grad_acc)):
         return None
     out_dtype = out_dtype or q.dtype
     if out_dtype not in _DT or (q.dtype == torch.float32 and out_dtype != torch.float32):
@@ -596,12 +609,17 @@ def chunk_table_attention(q, ks, vs, entries, q_pos0, q_split, causal, scale, st
     return res or None
 
 
+def _table(ks, k_pos0):
+    return [x for i, k in enumerate(ks) for x in (i, 0, k.shape[1], int(k_pos0[i]))]
+
+
 _warned_pad = False
 
 
 def _padded_head_dim(q, ks, vs, k_pos0, q_pos0, q_split, causal, scale, stepwise, out_dtype, kv_grad_acc, q_rope):
     """Head dims the kernels are not instantiated for (anything but 64 and 128; the reference hands any dim // n_heads to
-    SDPA, model/model.py:135, 193): a SLOW PATH that zero-pads q, k and v to the next instantiated head dim (one copy of
+    SDPA, model/model.py:135, 193) where the kernels cannot mask the missing columns themselves (_native_cols: fp32, unaligned
+    rows, no C++ node): a SLOW PATH that zero-pads q, k and v to the next instantiated head dim (one copy of
     each tensor per call, the gradients sliced back by autograd), keeps the scale of the TRUE head dim, and slices the
     result.  Zero columns change neither the scores nor the real columns of O.  Multiples of 8 up to 128."""
     D = q.shape[-1]
@@ -646,6 +664,9 @@ def block_attention(q, ks, vs, k_pos0, q_pos0=0, q_split=None, causal=False, sca
     per rank."""
     n = len(ks)
     if q.shape[-1] not in (64, 128):
+        res = n and chunk_table_attention(q, ks, vs, _table(ks, k_pos0), q_pos0, q_split, causal, scale, stepwise, out_dtype, kv_grad_acc, q_rope)
+        if res:
+            return res[0], res[1]
         return _padded_head_dim(q, ks, vs, k_pos0, q_pos0, q_split, causal, scale, stepwise, out_dtype, kv_grad_acc, q_rope)
     if (n == 1 and kv_grad_acc is None and not stepwise and q.dtype == torch.bfloat16 and out_dtype in (None, torch.bfloat16)
             and q.is_cuda and ks[0].is_cuda and vs[0].is_cuda):
@@ -668,8 +689,7 @@ def block_attention(q, ks, vs, k_pos0, q_pos0=0, q_split=None, causal=False, sca
     if q_rope is not None and q.dtype != torch.bfloat16:
         raise RuntimeError("the fused RoPE prologue is implemented for bf16 q")
     if n:
-        res = chunk_table_attention(q, ks, vs, [x for i in range(n) for x in (i, 0, ks[i].shape[1], int(k_pos0[i]))], q_pos0, q_split, causal, scale,
-                                    stepwise, out_dtype, kv_grad_acc, q_rope)
+        res = chunk_table_attention(q, ks, vs, _table(ks, k_pos0), q_pos0, q_split, causal, scale, stepwise, out_dtype, kv_grad_acc, q_rope)
         if res is not None:
             return res[0], res[1]
     return BlockAttentionFunction.apply(q, n, list(k_pos0), q_pos0, q_split, causal, scale, stepwise, out_dtype,

@@ -16,6 +16,8 @@
 //   fwd_f32_mfma_kernel<D, KS>  fp32 I/O and arithmetic on v_mfma_f32_32x32x2_f32: the forward of the 1e-4 cases (the reference's
 //                        acceptance dtype) on the matrix pipe; KS key shares per 32-row group for launches with few rows.
 //   fwd_f32_kernel<D>    the same in scalar fp32 (no MFMA): kept as the fallback, reached with LTR_FWD_F32_SCALAR.
+//                        fwd_bf16_shares_kernel<D, KS>, bwd_dq_shares_kernel<D, KS>: KS waves share a row group's keys (launches with
+//                        few rows, see key_shares); *_pad_kernel: head dims below the width D (LTR_HEAD_COLS).
 //   delta_kernel         DELTA = rowsum(dO * O).
 //   bwd_dkdv_kernel<D, KW>  a block of 8 waves owns 128 * KW keys of one kv head and loops over the
 //                        query heads of the GQA group and over 64-row query tiles taken from
@@ -87,6 +89,7 @@ struct FwdParams {
     void *o;
     float *lse;
     int B, Hq, Hkv, n_rep;
+    int cols;              // head dim of the tensors (the kernel's own width, or less: PAD kernels)
     int Sq, n_qtiles;
     int n_slots;           // q tiles are handed out in slots: n_qtiles of one tile, or (n_qtiles + 1) / 2 of two (see q_tile_slots)
     long long qs[3], os[3], ks[3], vs[3];
@@ -96,7 +99,7 @@ struct FwdParams {
     unsigned flags;
     int o_f32;
     int n_chunks;
-    const float *rope;     // LTR_ROPE_Q: (cos, sin) rows, D floats per position, row 0 = position rope_pos0
+    const float *rope;     // LTR_ROPE_Q: (cos, sin) rows, cols floats per position, row 0 = position rope_pos0
     int rope_pos0;
     void *q_rot;           // optional bf16 output: the rotated q
     long long qrs[3];
@@ -112,6 +115,7 @@ struct BwdParams {
     long long os_[3];
     void *dq;          // fp32 accumulator, or bf16 result with LTR_DQ_BF16
     int B, Hq, Hkv, n_rep;
+    int cols;          // head dim of the tensors (the kernel's own width, or less: PAD kernels)
     int Sq, n_qtiles;
     long long qs[3], dos[3], dqs[3], ks[3], vs[3], dks[3], dvs[3];
     int q_pos0[2];
@@ -125,7 +129,7 @@ struct BwdParams {
     int n_reps;       // of which a block walks this many
     float *part;      // n_split > 1: the blocks' partial dK / dV, summed by bwd_dkdv_reduce_kernel
     int n_slots;      // slots of 256-row q tiles of the dQ kernel (see q_tile_slots)
-    const float *rope;     // LTR_ROPE_DQ: (cos, sin) rows, D floats per position, row 0 = position rope_pos0
+    const float *rope;     // LTR_ROPE_DQ: (cos, sin) rows, cols floats per position, row 0 = position rope_pos0
     int rope_pos0;
     ChunkDev chunk[LTR_MAX_CHUNKS];
 };
@@ -137,6 +141,7 @@ struct DeltaParams {
     int B, Hq, D, Sq;
     long long os[3], dos[3];
     int o_f32, do_f32;
+    int vec;           // rows start 16-byte aligned: 16-byte loads
 };
 
 __device__ __forceinline__ int q_position(int row, int split, int p0, int p1) {
@@ -235,6 +240,17 @@ __device__ __forceinline__ void tile_barrier() {
     __builtin_amdgcn_s_waitcnt(0x0070);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+}
+
+// PAD kernels serve head dims between the two instantiated widths (multiples of 8): the tensors have `cols` < D columns, the LDS
+// tiles keep the width D.  The 16-byte chunks past the last column are cleared once (nothing else ever writes them: a tile
+// transfer leaves its lanes out), so the padding costs neither memory traffic nor passes over the tensors.  Measured beside
+// zero-padding q, k, v and slicing the results (B=2, 16 heads, D=96, S=777, forward + backward): 163 us with 11 pad, fill and slice
+// launches (47 us of them), 80 us without.
+template <int BYTES>
+__device__ __forceinline__ void clear_lds(unsigned char *smem) {   // followed by a barrier: the fill covers the columns that transfers write
+    for (int i = threadIdx.x * 16; i < BYTES; i += 512 * 16) *(uint4 *)(smem + i) = make_uint4(0, 0, 0, 0);
+    __syncthreads();
 }
 
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 x) {
@@ -569,8 +585,9 @@ __device__ __forceinline__ void collect_shares(unsigned char *smem, int w, int k
 // 64 keys serves 512 query rows: half the LDS reads and half the tile transfers per MFMA.
 // KS = waves that share a 32-row group: each takes its own BN keys of every tile of KS * BN keys, and their partial (reference, row
 // sum, O) are merged through LDS at the end.  For launches with too few query rows to give every CU a block (see FwdPlan).
-template <int D, int RB, int KS>
+template <int D, int RB, int KS, bool PAD>
 __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
+    const int cols = PAD ? p.cols : D;
     constexpr int NW = 8, RG = NW / KS, BM = 32 * RB * RG;   // 8 waves (two per SIMD) share every K / V tile
     constexpr int BN = FwdTile<D, RB, KS>::BN, NB = BN / 32, BNT = BN * KS;   // keys per wave and per tile
     constexpr int CPR = D / 8;   // 16-byte chunks per row
@@ -642,16 +659,17 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
 #pragma unroll
         for (int kb = 0; kb < D / 16; kb++) {
             uint4 x = make_uint4(0, 0, 0, 0);
-            if (row_ok[rb]) x = *(const uint4 *)(qp + kb * 16 + 8 * hh);
+            if (row_ok[rb] && (!PAD || kb * 16 + 8 * hh < cols)) x = *(const uint4 *)(qp + kb * 16 + 8 * hh);
             qreg[rb][kb] = as_bf16x8(x);
         }
         // fused RoPE prologue: q arrives un-rotated and is rotated here, in the registers that hold it as the MFMA operand,
         // by the angles of the row's global position; the rotated row can be stored for the backward
         if ((p.flags & LTR_ROPE_Q) && row_ok[rb]) {
-            const float *fr = p.rope + (long long)(my_pos[rb] - p.rope_pos0) * D + 8 * hh;
+            const float *fr = p.rope + (long long)(my_pos[rb] - p.rope_pos0) * cols + 8 * hh;
             __bf16 *qr = p.q_rot && ks == 0 ? (__bf16 *)p.q_rot + b * p.qrs[0] + (long long)my_row[rb] * p.qrs[1] + h * p.qrs[2] + 8 * hh : nullptr;
 #pragma unroll
             for (int kb = 0; kb < D / 16; kb++) {
+                if (PAD && kb * 16 + 8 * hh >= cols) continue;
                 qreg[rb][kb] = rope_rotate8(qreg[rb][kb], *(const f32x4 *)(fr + 16 * kb), *(const f32x4 *)(fr + 16 * kb + 4));
                 if (qr) *(bf16x8 *)(qr + 16 * kb) = qreg[rb][kb];
             }
@@ -718,7 +736,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
         const int chunk = st_pc ^ lds_swz<D>(row);
         const __bf16 *src = j < NI ? ld_kb + (long long)(key * (int)p.ks[1] + chunk * 8)
                                    : ld_vb + (long long)(key * (int)p.vs[1] + chunk * 8);
-        global_to_lds_b128(src, dst);
+        if (!PAD || chunk * 8 < cols) global_to_lds_b128(src, dst);
     };
     auto gload_begin = [&](int ti) {   // scalar state of the tile whose transfers are issued next
         nx_sk = ld_sk;
@@ -732,6 +750,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     // Merging an empty partial result leaves (O, LSE) as they are: a block that sees no key of this launch's chunks (the
     // early rows of a causal ring step) skips the read-modify-write of its rows altogether.
     if (!have && (p.flags & LTR_MERGE)) continue;
+    if constexpr (PAD) clear_lds<2 * BUF_ELEMS * 2>(smem);
     if (have) {
         gload_begin(t);
 #pragma unroll
@@ -954,7 +973,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
         old[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (merge && wave_row0 + it * ROWS_PER_IT + lane / LPR < Sq_u) {
+        if (merge && wave_row0 + it * ROWS_PER_IT + lane / LPR < Sq_u && (!PAD || col0 + 4 * (lane % LPR) < cols)) {
             if (o_f32) {
                 old[it] = *(const f32x4 *)((const float *)p.o + off0 + it * ROWS_PER_IT * os1);
             } else {
@@ -971,8 +990,8 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     }();
     if (o_f32) {
         float *op = (float *)p.o + off0;
-        wave_tile_rowmajor<CW>(stage, lane, result, w_cur, [&](int row, int, f32x4 val) {
-            if (wave_row0 + row < Sq_u) {
+        wave_tile_rowmajor<CW>(stage, lane, result, w_cur, [&](int row, int col, f32x4 val) {
+            if (wave_row0 + row < Sq_u && (!PAD || col0 + col < cols)) {
                 if (merge) {
                     const float wo = row_w_old[row];
 #pragma unroll
@@ -985,8 +1004,8 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
         });
     } else {
         __bf16 *op = (__bf16 *)p.o + off0;
-        wave_tile_rowmajor<CW>(stage, lane, result, w_cur, [&](int row, int, f32x4 val) {
-            if (wave_row0 + row < Sq_u) {
+        wave_tile_rowmajor<CW>(stage, lane, result, w_cur, [&](int row, int col, f32x4 val) {
+            if (wave_row0 + row < Sq_u && (!PAD || col0 + col < cols)) {
                 if (merge) {
                     const float wo = row_w_old[row];
 #pragma unroll
@@ -1007,11 +1026,15 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
 
 template <int D, int RB>
 __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
-    fwd_bf16_body<D, RB, 1>(p);
+    fwd_bf16_body<D, RB, 1, false>(p);
 }
 template <int D, int KS>
 __global__ __launch_bounds__(512) void fwd_bf16_shares_kernel(const FwdParams p) {
-    fwd_bf16_body<D, 1, KS>(p);
+    fwd_bf16_body<D, 1, KS, false>(p);
+}
+template <int D, int KS>   // head dims below D
+__global__ __launch_bounds__(512) void fwd_bf16_pad_kernel(const FwdParams p) {
+    fwd_bf16_body<D, 1, KS, true>(p);
 }
 
 // ------------------------------------------------------------------------------ forward, fp32
@@ -1399,30 +1422,42 @@ __global__ __launch_bounds__(256) void fwd_f32_mfma_kernel(const FwdParams p) {
 }
 
 // ------------------------------------------------------------------------------ delta
-// 16 lanes per (b, h, row); each lane covers D/16 contiguous elements.
+// 16 lanes per (b, row, h), 8 elements per lane: rows of one sequence index are read head after head, as they lie in memory.
 __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
-    const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
-    const long long rowid = gid >> 4;
-    const int sub = gid & 15;
+    const long long rowid = ((long long)blockIdx.x * 256 + threadIdx.x) >> 4;
+    const int d = 8 * (threadIdx.x & 15);
     const long long nrows = (long long)p.B * p.Hq * p.Sq;
     float acc = 0.f;
+    int i = 0, h = 0, b = 0;
     if (rowid < nrows) {
-        const int i = rowid % p.Sq;
-        const int h = (rowid / p.Sq) % p.Hq;
-        const int b = rowid / ((long long)p.Sq * p.Hq);
-        const long long oo = b * p.os[0] + (long long)i * p.os[1] + h * p.os[2];
-        const long long od = b * p.dos[0] + (long long)i * p.dos[1] + h * p.dos[2];
-        const int per = p.D / 16;
-        for (int e = 0; e < per; e++) {
-            const int d = sub * per + e;
-            const float ov = p.o_f32 ? ((const float *)p.o)[oo + d] : (float)((const __bf16 *)p.o)[oo + d];
-            const float dv = p.do_f32 ? ((const float *)p.d_o)[od + d] : (float)((const __bf16 *)p.d_o)[od + d];
-            acc = fmaf(ov, dv, acc);
+        const unsigned bi = (unsigned)(rowid / p.Hq);   // b * Sq + i: below 2^31 (checked by the host)
+        h = (int)(rowid - (long long)bi * p.Hq);
+        b = (int)(bi / (unsigned)p.Sq);
+        i = (int)(bi - (unsigned)b * (unsigned)p.Sq);
+        if (d < p.D) {
+            const long long oo = b * p.os[0] + (long long)i * p.os[1] + h * p.os[2] + d;
+            const long long od = b * p.dos[0] + (long long)i * p.dos[1] + h * p.dos[2] + d;
+            float ov[8], dv[8];
+            auto load8 = [&](const void *base, long long off, bool f32, float (&v)[8]) {
+                if (!p.vec) {
+                    for (int e = 0; e < 8; e++) v[e] = f32 ? ((const float *)base)[off + e] : (float)((const __bf16 *)base)[off + e];
+                } else if (f32) {
+                    const f32x4 x = *(const f32x4 *)((const float *)base + off), y = *(const f32x4 *)((const float *)base + off + 4);
+                    for (int e = 0; e < 4; e++) v[e] = x[e], v[4 + e] = y[e];
+                } else {
+                    const bf16x8 x = *(const bf16x8 *)((const __bf16 *)base + off);
+                    for (int e = 0; e < 8; e++) v[e] = (float)x[e];
+                }
+            };
+            load8(p.o, oo, p.o_f32, ov);
+            load8(p.d_o, od, p.do_f32, dv);
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc = fmaf(ov[e], dv[e], acc);
         }
     }
 #pragma unroll
     for (int off = 8; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 16);
-    if (rowid < nrows && sub == 0) p.delta[rowid] = acc;
+    if (rowid < nrows && d == 0) p.delta[((long long)b * p.Hq + h) * p.Sq + i] = acc;
 }
 
 __global__ __launch_bounds__(256) void cast_kernel(const float *src, __bf16 *dst, long long n) {
@@ -1509,8 +1544,9 @@ __device__ __forceinline__ void store_partial(float *dst, int lane, const f32x16
         }
 }
 
-template <int D, int KW>
-__global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
+template <int D, int KW, bool PAD>
+__device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
+    const int cols = PAD ? p.cols : D;
     using L = BwdLds<D, KW>;   // KW = 32-key halves per wave
     constexpr int BN = L::BN, BM = L::BM;
     constexpr int CPR = D / 8;
@@ -1567,7 +1603,7 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
             if ((p.flags & LTR_DKDV_BF16) && p.split_log2 == 0 && key_ok[k]) {   // results, not accumulators: these keys get zeros
                 __bf16 *gz = p_role ? (__bf16 *)p.chunk[c].dv + b * p.dvs[0] + (long long)my_key[k] * p.dvs[1] + hkv * p.dvs[2]
                                     : (__bf16 *)p.chunk[c].dk + b * p.dks[0] + (long long)my_key[k] * p.dks[1] + hkv * p.dks[2];
-                for (int d = 8 * hh; d < D; d += 16) *(uint4 *)(gz + d) = make_uint4(0, 0, 0, 0);
+                for (int d = 8 * hh; d < cols; d += 16) *(uint4 *)(gz + d) = make_uint4(0, 0, 0, 0);
             }
             return;
         }
@@ -1585,7 +1621,8 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
             const int ksafe = min(my_key[k], sk - 1);
 #pragma unroll
             for (int kb = 0; kb < D / 16; kb++) {
-                uint4 x = *(const uint4 *)(base + (long long)ksafe * rs + kb * 16 + 8 * hh);
+                uint4 x = make_uint4(0, 0, 0, 0);
+                if (!PAD || kb * 16 + 8 * hh < cols) x = *(const uint4 *)(base + (long long)ksafe * rs + kb * 16 + 8 * hh);
                 if (!key_ok[k]) x = make_uint4(0, 0, 0, 0);
                 kvreg[k][kb] = as_bf16x8(x);
             }
@@ -1706,6 +1743,7 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
                 const unsigned tq = (unsigned)(row0 * (int)p.qs[1]), tdo = (unsigned)(row0 * (int)p.dos[1]);
 #pragma unroll
                 for (int i = 0; i < NI; i++) {
+                    if (PAD && (st_pc ^ lds_swz<D>(RPI * (NI * w + i) + st_row)) * 8 >= cols) continue;
                     global_to_lds_b128(qp_head + (unsigned long long)(tq + offq[i]), Qd + RPI * (NI * w + i) * D * 2);
                     global_to_lds_b128(dop_head + (unsigned long long)(tdo + offdo[i]), dOd + RPI * (NI * w + i) * D * 2);
                 }
@@ -1715,6 +1753,7 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
                     const int row = RPI * (NI * w + i) + st_row;
                     const int grow = min(row0 + row, p.Sq - 1);
                     const int chunk = st_pc ^ lds_swz<D>(row);
+                    if (PAD && chunk * 8 >= cols) continue;
                     global_to_lds_b128(qp_head + (long long)(grow * (int)p.qs[1] + chunk * 8), Qd + RPI * (NI * w + i) * D * 2);
                     global_to_lds_b128(dop_head + (long long)(grow * (int)p.dos[1] + chunk * 8), dOd + RPI * (NI * w + i) * D * 2);
                 }
@@ -1957,6 +1996,7 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
             }
         }
     };
+    if constexpr (PAD) clear_lds<L::P_OFF>(smem);
     run_pass(std::false_type{});
     run_pass(std::true_type{});
 
@@ -1978,8 +2018,8 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
                                (key_base + lane / LPR) * stride + 4 * (lane % LPR);
         if (uniform32(p.flags & LTR_DKDV_BF16)) {   // every query that sees these keys was in this launch: store the result
             __bf16 *gb = (__bf16 *)(p_role ? p.chunk[c].dv : p.chunk[c].dk) + goff;
-            wave_tile_rowmajor<D>(smem + w * WaveStage<D>::BYTES, lane, acc[k], p_role ? 1.f : p.scale, [&](int row, int, f32x4 val) {
-                if (key_base + row < sk_u) {
+            wave_tile_rowmajor<D>(smem + w * WaveStage<D>::BYTES, lane, acc[k], p_role ? 1.f : p.scale, [&](int row, int col, f32x4 val) {
+                if (key_base + row < sk_u && (!PAD || col < cols)) {
                     bf16x4 y;
 #pragma unroll
                     for (int e = 0; e < 4; e++) y[e] = (__bf16)val[e];
@@ -1996,11 +2036,11 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
 #pragma unroll
         for (int it = 0; it < NIT; it++) {
             old[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (key_base + it * ROWS_PER_IT + lane / LPR < sk_u) old[it] = *(const f32x4 *)(gp + it * ROWS_PER_IT * stride);
+            if (key_base + it * ROWS_PER_IT + lane / LPR < sk_u && (!PAD || 4 * (lane % LPR) < cols)) old[it] = *(const f32x4 *)(gp + it * ROWS_PER_IT * stride);
         }
         int it = 0;
-        wave_tile_rowmajor<D>(smem + w * WaveStage<D>::BYTES, lane, acc[k], p_role ? 1.f : p.scale, [&](int row, int, f32x4 val) {
-            if (key_base + row < sk_u) {
+        wave_tile_rowmajor<D>(smem + w * WaveStage<D>::BYTES, lane, acc[k], p_role ? 1.f : p.scale, [&](int row, int col, f32x4 val) {
+            if (key_base + row < sk_u && (!PAD || col < cols)) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) val[e] += old[it][e];
                 *(f32x4 *)gp = val;
@@ -2009,6 +2049,15 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
             it++;
         });
     }
+}
+
+template <int D, int KW>
+__global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
+    bwd_dkdv_body<D, KW, false>(p);
+}
+template <int D>   // head dims below D
+__global__ __launch_bounds__(512) void bwd_dkdv_pad_kernel(const BwdParams p) {
+    bwd_dkdv_body<D, 1, true>(p);
 }
 
 // Sum of the partial dK / dV that the blocks sharing a key tile left in p.part (bf16 and fp32 kernels alike), in the order of
@@ -2071,8 +2120,8 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const BwdParams p)
     unsigned char *const stage = stage_mem + w4 * WaveStage<64>::BYTES;
     float *gp = (is_dv ? p.chunk[c].dv : p.chunk[c].dk) + (out_bf16 ? 0 : off);
     __bf16 *gb = (__bf16 *)(is_dv ? p.chunk[c].dv : p.chunk[c].dk) + (out_bf16 ? off : 0);
-    wave_tile_rowmajor<64>(stage, lane, acc, 1.f, [&](int row, int, f32x4 val) {
-        if (key_base + row < sk) {
+    wave_tile_rowmajor<64>(stage, lane, acc, 1.f, [&](int row, int col, f32x4 val) {
+        if (key_base + row < sk && 64 * half + col < p.cols) {
             if (out_bf16) {
                 bf16x4 y;
 #pragma unroll
@@ -2149,8 +2198,9 @@ __device__ __forceinline__ void lds_tr_gemm_at_rb(const unsigned (&addr)[D / 32]
 }
 
 // RB = 32-row blocks per wave: a lane owns RB query rows, a block 256 * RB / KS; KS = key shares per row group as in the forward
-template <int D, int RB, int KS>
+template <int D, int RB, int KS, bool PAD>
 __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
+    const int cols = PAD ? p.cols : D;
     constexpr int NW = 8, RG = NW / KS, BM = 32 * RB * RG;   // 8 waves (two per SIMD) share every K / V tile
     constexpr int BN = FwdTile<D, 1, KS>::BN, BNT = BN * KS; // keys per wave and per tile
     constexpr int CPR = D / 8;
@@ -2218,6 +2268,10 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
         const __bf16 *dop = (const __bf16 *)p.d_o + b * p.dos[0] + (long long)rsafe * p.dos[1] + h * p.dos[2];
 #pragma unroll
         for (int kb = 0; kb < D / 16; kb++) {
+            if (PAD && kb * 16 + 8 * hh >= cols) {
+                qreg[rb][kb] = doreg[rb][kb] = as_bf16x8(make_uint4(0, 0, 0, 0));
+                continue;
+            }
             qreg[rb][kb] = as_bf16x8(*(const uint4 *)(qp + kb * 16 + 8 * hh));
             doreg[rb][kb] = as_bf16x8(*(const uint4 *)(dop + kb * 16 + 8 * hh));
         }
@@ -2227,6 +2281,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
             float part = 0.f;
 #pragma unroll
             for (int kb = 0; kb < D / 16; kb++) {
+                if (PAD && kb * 16 + 8 * hh >= cols) continue;
                 const bf16x8 ov = as_bf16x8(*(const uint4 *)(op + kb * 16 + 8 * hh));
 #pragma unroll
                 for (int e = 0; e < 8; e++) part += (float)ov[e] * (float)doreg[rb][kb][e];
@@ -2296,6 +2351,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
             const int row = RPI * (NI * w + i) + st_row;
             const int key = min(ti * BNT + row, ld_sk - 1);
             const int chunk = st_pc ^ lds_swz<D>(row);
+            if (PAD && chunk * 8 >= cols) continue;
             global_to_lds_b128(ld_kb + (long long)(key * (int)p.ks[1] + chunk * 8), Kd + RPI * (NI * w + i) * D * 2);
             global_to_lds_b128(ld_vb + (long long)(key * (int)p.vs[1] + chunk * 8), Vd + RPI * (NI * w + i) * D * 2);
         }
@@ -2304,6 +2360,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
     bool have = c < p.n_chunks;
     // a block that sees no key of this launch's chunks adds nothing to an fp32 dQ accumulator: no read-modify-write
     if (!have && !(p.flags & LTR_DQ_BF16)) continue;
+    if constexpr (PAD) clear_lds<2 * BUF_ELEMS * 2>(smem);
     if (have) gload(t, 0);
     tile_barrier();
     // LDS byte addresses of this lane's operands in the K tile of the current buffer (the V tile and the other 32-key
@@ -2420,7 +2477,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
         auto unrotate = [&](int row, int col, f32x4 val) {
             if (!rope) return val;
             const int pos = q_position(wave_row0 + row, split_u, qp0, qp1);
-            return rope_conj4(val, *(const f32x4 *)(rope_tab + (long long)(pos - rope_p0) * D + col0 + col));
+            return rope_conj4(val, *(const f32x4 *)(rope_tab + (long long)(pos - rope_p0) * cols + col0 + col));
         };
         auto &result = [&]() -> f32x16(&)[CW / 32] {
             if constexpr (KS > 1) return own;
@@ -2429,7 +2486,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
         if (uniform32(p.flags & LTR_DQ_BF16)) {   // this call saw every key of these rows: store the result, no accumulator
             __bf16 *dqp = (__bf16 *)p.dq + off0;
             wave_tile_rowmajor<CW>(stage, lane, result, p.scale, [&](int row, int col, f32x4 val) {
-                if (wave_row0 + row < Sq_u) {
+                if (wave_row0 + row < Sq_u && (!PAD || col0 + col < cols)) {
                     val = unrotate(row, col, val);
                     bf16x4 y;
 #pragma unroll
@@ -2445,11 +2502,12 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
 #pragma unroll
             for (int it = 0; it < NIT; it++) {
                 old[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (wave_row0 + it * ROWS_PER_IT + lane / LPR < Sq_u) old[it] = *(const f32x4 *)(dqp + it * ROWS_PER_IT * dqs1);
+                if (wave_row0 + it * ROWS_PER_IT + lane / LPR < Sq_u && (!PAD || col0 + 4 * (lane % LPR) < cols))
+                    old[it] = *(const f32x4 *)(dqp + it * ROWS_PER_IT * dqs1);
             }
             int it = 0;
             wave_tile_rowmajor<CW>(stage, lane, result, p.scale, [&](int row, int col, f32x4 val) {
-                if (wave_row0 + row < Sq_u) {
+                if (wave_row0 + row < Sq_u && (!PAD || col0 + col < cols)) {
                     val = unrotate(row, col, val);
 #pragma unroll
                     for (int e = 0; e < 4; e++) val[e] += old[it][e];
@@ -2465,11 +2523,15 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
 
 template <int D, int RB>
 __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
-    bwd_dq_body<D, RB, 1>(p);
+    bwd_dq_body<D, RB, 1, false>(p);
 }
 template <int D, int KS>
 __global__ __launch_bounds__(512) void bwd_dq_shares_kernel(const BwdParams p) {
-    bwd_dq_body<D, 1, KS>(p);
+    bwd_dq_body<D, 1, KS, false>(p);
+}
+template <int D, int KS>   // head dims below D
+__global__ __launch_bounds__(512) void bwd_dq_pad_kernel(const BwdParams p) {
+    bwd_dq_body<D, 1, KS, true>(p);
 }
 
 // ------------------------------------------------------------------------------ backward, fp32
@@ -3152,6 +3214,20 @@ int enable_large_lds() {
         {(const void *)bwd_dq_f32_mfma_kernel<64, 4>, F32Mfma<64, 4>::LDS},
         {(const void *)bwd_dkdv_f32_mfma_kernel<128>, F32DkdvLds<128>::LDS},
         {(const void *)bwd_dkdv_f32_mfma_kernel<64>, F32DkdvLds<64>::LDS},
+        {(const void *)bwd_dkdv_pad_kernel<128>, BwdLds<128, 1>::TOTAL},
+        {(const void *)fwd_bf16_pad_kernel<128, 1>, fwd_lds_bytes<128>()},
+        {(const void *)fwd_bf16_pad_kernel<128, 2>, shares_lds_bytes<128, 2>()},
+        {(const void *)fwd_bf16_pad_kernel<128, 4>, shares_lds_bytes<128, 4>()},
+        {(const void *)bwd_dq_pad_kernel<128, 1>, dq_lds_bytes<128>()},
+        {(const void *)bwd_dq_pad_kernel<128, 2>, shares_lds_bytes<128, 2>()},
+        {(const void *)bwd_dq_pad_kernel<128, 4>, shares_lds_bytes<128, 4>()},
+        {(const void *)bwd_dkdv_pad_kernel<64>, BwdLds<64, 1>::TOTAL},
+        {(const void *)fwd_bf16_pad_kernel<64, 1>, fwd_lds_bytes<64>()},
+        {(const void *)fwd_bf16_pad_kernel<64, 2>, shares_lds_bytes<64, 2>()},
+        {(const void *)fwd_bf16_pad_kernel<64, 4>, shares_lds_bytes<64, 4>()},
+        {(const void *)bwd_dq_pad_kernel<64, 1>, dq_lds_bytes<64>()},
+        {(const void *)bwd_dq_pad_kernel<64, 2>, shares_lds_bytes<64, 2>()},
+        {(const void *)bwd_dq_pad_kernel<64, 4>, shares_lds_bytes<64, 4>()},
         {(const void *)fwd_bf16_shares_kernel<128, 2>, shares_lds_bytes<128, 2>()},
         {(const void *)fwd_bf16_shares_kernel<128, 4>, shares_lds_bytes<128, 4>()},
         {(const void *)fwd_bf16_shares_kernel<64, 2>, shares_lds_bytes<64, 2>()},
@@ -3176,6 +3252,13 @@ bool strides_ok(const int64_t *s, int elem_bytes) {
     for (int i = 0; i < 3; i++)
         if (s[i] < 0 || (s[i] % per16) != 0) return false;
     return true;
+}
+
+// Width of the kernels that serve head dim D: D itself where they are instantiated, the next width with LTR_HEAD_COLS, 0 = none.
+int head_width(int D, unsigned flags) {
+    if (D == 64 || D == 128) return D;
+    if (!(flags & LTR_HEAD_COLS) || D <= 0 || D > 128 || D % 8) return 0;
+    return D < 64 ? 64 : 128;
 }
 
 int fits_i32(int64_t x) { return x >= 0 && x < (int64_t)0x7fffffff; }
@@ -3334,7 +3417,7 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     if (!wide && !(flags & LTR_FWD_ROWS_256))
         pl.ks = key_shares(D == 128 ? FWD_SHARES_128 : FWD_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
                            n_chunks);
-    if (!wide && !(flags & LTR_FWD_ROWS_256) && D == 64 && pl.ks == 1) {
+    if (!wide && !(flags & (LTR_FWD_ROWS_256 | LTR_HEAD_COLS)) && D == 64 && pl.ks == 1) {
         const int tiles512 = (Sq + 511) / 512;
         const int slots512 = q_tile_slots(tiles512, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, 512, q_split, q_pos0, chunk, n_chunks));
         const long long blocks512 = (long long)slots512 * B * Hq, blocks256 = (long long)((Sq + 255) / 256) * B * Hq;
@@ -3471,7 +3554,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     // a causal mask (unequal blocks), when a block walks many q tiles and there are several rounds of blocks to balance
     // with; the caller can force either size
     bool wide = (flags & LTR_DKDV_KEYS_256) != 0;
-    if (!wide && !(flags & LTR_DKDV_KEYS_128) && D == 64 && !(flags & LTR_NO_DKDV)) {
+    if (!wide && !(flags & LTR_DKDV_KEYS_128) && D == 64 && !(flags & (LTR_NO_DKDV | LTR_HEAD_COLS))) {
         long long blocks256 = 0, blocks128 = 0;
         for (int c = 0; c < n_chunks; c++) {
             blocks256 += (chunk[c].sk + 255) / 256;
@@ -3496,7 +3579,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     if (!wide_q && !(flags & (LTR_DQ_ROWS_256 | LTR_NO_DQ)))
         pl.dq_ks = key_shares(D == 128 ? DQ_SHARES_128 : DQ_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
                               n_chunks);
-    if (!wide_q && !(flags & LTR_DQ_ROWS_256) && D == 64 && !(flags & LTR_NO_DQ) && pl.dq_ks == 1) {
+    if (!wide_q && !(flags & (LTR_DQ_ROWS_256 | LTR_HEAD_COLS)) && D == 64 && !(flags & LTR_NO_DQ) && pl.dq_ks == 1) {
         const int tiles512 = (Sq + 511) / 512;
         const int slots512 = q_tile_slots(tiles512, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, 512, q_split, q_pos0, chunk, n_chunks));
         const long long blocks512 = (long long)slots512 * B * Hq;
@@ -3571,11 +3654,15 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     if (!a || !a->q || !a->o || !a->lse) return LTR_EINVAL;
     if (a->B <= 0 || a->Hq <= 0 || a->Hkv <= 0 || a->Sq <= 0 || a->Hq % a->Hkv) return LTR_EINVAL;
     if (a->n_chunks < 1 || a->n_chunks > LTR_MAX_CHUNKS) return LTR_EINVAL;
-    if (a->flags & ~(LTR_CAUSAL | LTR_MERGE | LTR_ROPE_Q | LTR_FWD_ROWS_256 | LTR_FWD_ROWS_512 | LTR_FWD_F32_SCALAR)) return LTR_EINVAL;
+    if (a->flags & ~(LTR_CAUSAL | LTR_MERGE | LTR_ROPE_Q | LTR_FWD_ROWS_256 | LTR_FWD_ROWS_512 | LTR_FWD_F32_SCALAR | LTR_HEAD_COLS))
+        return LTR_EINVAL;
     if ((a->flags & LTR_FWD_F32_SCALAR) && a->io_dtype != LTR_F32) return LTR_EUNSUP;
     if ((a->flags & LTR_FWD_ROWS_256) && (a->flags & LTR_FWD_ROWS_512)) return LTR_EINVAL;
-    if (a->D != 64 && a->D != 128) return LTR_EUNSUP;
+    const int D = head_width(a->D, a->flags);
+    const bool pad = D != a->D;
+    if (!D) return LTR_EUNSUP;
     if (a->io_dtype != LTR_BF16 && a->io_dtype != LTR_F32) return LTR_EUNSUP;
+    if (pad && a->io_dtype != LTR_BF16) return LTR_EUNSUP;
     if (a->o_dtype != LTR_BF16 && a->o_dtype != LTR_F32) return LTR_EUNSUP;
     if (a->io_dtype == LTR_F32 && a->o_dtype != LTR_F32) return LTR_EUNSUP;
     if (!fits_i32(a->Sq) || a->q_split < 0 || a->q_split > a->Sq) return LTR_EINVAL;
@@ -3639,13 +3726,23 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     p.n_chunks = a->n_chunks;
     hipStream_t st = (hipStream_t)stream;
     if ((a->flags & LTR_FWD_ROWS_512) && (a->D != 64 || a->io_dtype != LTR_BF16)) return LTR_EUNSUP;
-    const FwdPlan pl = plan_fwd(a->D, a->io_dtype == LTR_F32, a->flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks);
+    p.cols = a->D;
+    const FwdPlan pl = plan_fwd(D, a->io_dtype == LTR_F32, pad ? a->flags : a->flags & ~LTR_HEAD_COLS, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks);
     if (pl.blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.n_qtiles = pl.n_qtiles;
     p.n_slots = pl.n_slots;
     if (a->io_dtype == LTR_BF16) {
         rc = enable_large_lds();
         if (rc) return rc;
+        if (pad) {
+            const int i = pl.ks >> 1;
+            const void *const kernels[2][3] = {
+                {(const void *)fwd_bf16_pad_kernel<64, 1>, (const void *)fwd_bf16_pad_kernel<64, 2>, (const void *)fwd_bf16_pad_kernel<64, 4>},
+                {(const void *)fwd_bf16_pad_kernel<128, 1>, (const void *)fwd_bf16_pad_kernel<128, 2>, (const void *)fwd_bf16_pad_kernel<128, 4>}};
+            const int lds[2][3] = {{fwd_lds_bytes<64>(), shares_lds_bytes<64, 2>(), shares_lds_bytes<64, 4>()},
+                                   {fwd_lds_bytes<128>(), shares_lds_bytes<128, 2>(), shares_lds_bytes<128, 4>()}};
+            return launch(kernels[D == 128][i], pl.blocks, 512, lds[D == 128][i], st, p);
+        }
         if (pl.ks == 2)
             return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 2>, pl.blocks, 512, shares_lds_bytes<128, 2>(), st, p)
                                : launch((const void *)fwd_bf16_shares_kernel<64, 2>, pl.blocks, 512, shares_lds_bytes<64, 2>(), st, p);
@@ -3673,8 +3770,8 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
 
 extern "C" int ltr_attn_bwd_delta(const ltr_attn_delta_args *a, void *stream) {
     if (!a || !a->o || !a->d_o || !a->delta) return LTR_EINVAL;
-    if (a->B <= 0 || a->Hq <= 0 || a->Sq <= 0 || !fits_i32(a->Sq)) return LTR_EINVAL;
-    if (a->D != 64 && a->D != 128) return LTR_EUNSUP;
+    if (a->B <= 0 || a->Hq <= 0 || a->Sq <= 0 || !fits_i32(a->Sq) || !fits_i32((int64_t)a->B * a->Sq)) return LTR_EINVAL;
+    if (a->D <= 0 || a->D > 128 || a->D % 8) return LTR_EUNSUP;
     if ((a->o_dtype != LTR_BF16 && a->o_dtype != LTR_F32) || (a->do_dtype != LTR_BF16 && a->do_dtype != LTR_F32))
         return LTR_EUNSUP;
     for (int i = 0; i < 3; i++)
@@ -3695,6 +3792,7 @@ extern "C" int ltr_attn_bwd_delta(const ltr_attn_delta_args *a, void *stream) {
     }
     p.o_f32 = a->o_dtype == LTR_F32;
     p.do_f32 = a->do_dtype == LTR_F32;
+    p.vec = aligned16(a->o) && aligned16(a->d_o) && strides_ok(a->o_stride, p.o_f32 ? 4 : 2) && strides_ok(a->do_stride, p.do_f32 ? 4 : 2);
     const long long nthreads = (long long)p.B * p.Hq * p.Sq * 16;
     const long long nblk = (nthreads + 255) / 256;
     if (nblk > 0x7fffffffLL) return LTR_EINVAL;
@@ -3712,16 +3810,20 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     if (a->B <= 0 || a->Hq <= 0 || a->Hkv <= 0 || a->Sq <= 0 || a->Hq % a->Hkv) return LTR_EINVAL;
     if (a->n_chunks < 1 || a->n_chunks > LTR_MAX_CHUNKS) return LTR_EINVAL;
     if (flags & ~(LTR_CAUSAL | LTR_NO_DQ | LTR_NO_DKDV | LTR_DQ_BF16 | LTR_DELTA_FROM_O | LTR_DKDV_BF16 | LTR_ROPE_DQ | LTR_DKDV_KEYS_128 |
-                  LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR))
+                  LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR | LTR_HEAD_COLS))
         return LTR_EINVAL;
     if ((flags & LTR_BWD_F32_SCALAR) && a->io_dtype != LTR_F32) return LTR_EUNSUP;
     if ((flags & LTR_DKDV_KEYS_128) && (flags & LTR_DKDV_KEYS_256)) return LTR_EINVAL;
     if ((flags & LTR_DQ_ROWS_256) && (flags & LTR_DQ_ROWS_512)) return LTR_EINVAL;
     const bool fused_delta = flags & LTR_DELTA_FROM_O;
     if (fused_delta && (!do_dq || !a->o)) return LTR_EINVAL;
-    if (a->D != 64 && a->D != 128) return LTR_EUNSUP;
+    const int D = head_width(a->D, flags);
+    const bool pad = D != a->D;
+    if (!D) return LTR_EUNSUP;
     if (a->io_dtype != LTR_BF16 && a->io_dtype != LTR_F32) return LTR_EUNSUP;
     const bool f32 = a->io_dtype == LTR_F32;
+    if (pad && f32) return LTR_EUNSUP;
+    if (!pad) flags &= ~LTR_HEAD_COLS;
     if (f32 && (flags & (LTR_DQ_BF16 | LTR_DELTA_FROM_O | LTR_DKDV_BF16 | LTR_ROPE_DQ | LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_512)))
         return LTR_EUNSUP;   // bf16 conveniences and kernels only
     const int gb = (flags & LTR_DKDV_BF16) ? 2 : 4;   // bytes per dK / dV element
@@ -3799,9 +3901,10 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     p.scale = a->scale;
     p.flags = flags;
     p.n_chunks = a->n_chunks;
-    BwdPlan pl = plan_bwd(a->D, f32, flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks, work != nullptr);
+    p.cols = a->D;
+    BwdPlan pl = plan_bwd(D, f32, flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks, work != nullptr);
     if (pl.part_bytes > work_bytes) pl.split = KvSplit{1, 1};
-    const long long kv_grid = pl.kv_blocks * pl.split.n, reduce_grid = pl.kv_blocks * (pl.keys_per_block / 128) * (a->D / 32);
+    const long long kv_grid = pl.kv_blocks * pl.split.n, reduce_grid = pl.kv_blocks * (pl.keys_per_block / 128) * (D / 32);
     if (kv_grid > 0x7fffffffLL || reduce_grid > 0x7fffffffLL || pl.dq_blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.tiles_total = (int)pl.kv_tiles;
     p.split_log2 = __builtin_ctz(pl.split.n);
@@ -3851,7 +3954,15 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     if (rc) return rc;
     // the dQ kernel goes first: with LTR_DELTA_FROM_O it produces the DELTA that the dK/dV kernel reads
     if (do_dq) {
-        if (pl.dq_ks == 2)
+        if (pad) {
+            const int i = pl.dq_ks >> 1;
+            const void *const kernels[2][3] = {
+                {(const void *)bwd_dq_pad_kernel<64, 1>, (const void *)bwd_dq_pad_kernel<64, 2>, (const void *)bwd_dq_pad_kernel<64, 4>},
+                {(const void *)bwd_dq_pad_kernel<128, 1>, (const void *)bwd_dq_pad_kernel<128, 2>, (const void *)bwd_dq_pad_kernel<128, 4>}};
+            const int lds[2][3] = {{dq_lds_bytes<64>(), shares_lds_bytes<64, 2>(), shares_lds_bytes<64, 4>()},
+                                   {dq_lds_bytes<128>(), shares_lds_bytes<128, 2>(), shares_lds_bytes<128, 4>()}};
+            rc = launch(kernels[D == 128][i], pl.dq_blocks, 512, lds[D == 128][i], st, p);
+        } else if (pl.dq_ks == 2)
             rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 2>, pl.dq_blocks, 512, shares_lds_bytes<128, 2>(), st, p)
                              : launch((const void *)bwd_dq_shares_kernel<64, 2>, pl.dq_blocks, 512, shares_lds_bytes<64, 2>(), st, p);
         else if (pl.dq_ks == 4)
@@ -3869,11 +3980,13 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
         // the tail (the sums inside a block do not depend on the table's order).
         if (flags & LTR_CAUSAL)
             std::stable_sort(p.chunk, p.chunk + p.n_chunks, [](const ChunkDev &x, const ChunkDev &y) { return x.pos0 < y.pos0; });
-        if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, kv_grid, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
+        if (pad) rc = D == 128 ? launch((const void *)bwd_dkdv_pad_kernel<128>, kv_grid, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p)
+                               : launch((const void *)bwd_dkdv_pad_kernel<64>, kv_grid, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
+        else if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, kv_grid, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
         else if (pl.wide_kv) rc = launch((const void *)bwd_dkdv_kernel<64, 2>, kv_grid, BwdLds<64, 2>::NT, BwdLds<64, 2>::TOTAL, st, p);
         else rc = launch((const void *)bwd_dkdv_kernel<64, 1>, kv_grid, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
         if (rc || pl.split.n == 1) return rc;
-        rc = a->D == 128 ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
+        rc = D == 128 ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
              : pl.wide_kv ? launch((const void *)bwd_dkdv_reduce_kernel<64, 2>, reduce_grid, 256, 0, st, p)
                           : launch((const void *)bwd_dkdv_reduce_kernel<64, 1>, reduce_grid, 256, 0, st, p);
     }
@@ -3897,7 +4010,8 @@ extern "C" int ltr_attn_bwd_workspace(const ltr_attn_bwd_args *a, int64_t *bytes
     if (!a || !bytes) return LTR_EINVAL;
     *bytes = 0;
     if (a->B <= 0 || a->Hq <= 0 || a->Hkv <= 0 || a->Sq <= 0 || a->Hq % a->Hkv || a->n_chunks < 1 || a->n_chunks > LTR_MAX_CHUNKS) return LTR_EINVAL;
-    if (a->D != 64 && a->D != 128) return LTR_EUNSUP;
+    const int D = head_width(a->D, a->flags);
+    if (!D) return LTR_EUNSUP;
     if (!fits_i32(a->Sq) || a->q_split < 0 || a->q_split > a->Sq) return LTR_EINVAL;
     if (!fits_i32(a->q_pos0[0] + a->Sq) || !fits_i32(a->q_pos0[1] + a->Sq)) return LTR_EINVAL;
     ChunkDev chunk[LTR_MAX_CHUNKS];
@@ -3907,7 +4021,7 @@ extern "C" int ltr_attn_bwd_workspace(const ltr_attn_bwd_args *a, int64_t *bytes
         chunk[c].pos0 = (int)a->chunk[c].pos0;
     }
     const int q_pos0[2] = {(int)a->q_pos0[0], (int)a->q_pos0[1]};
-    *bytes = plan_bwd(a->D, a->io_dtype == LTR_F32, a->flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks, true).part_bytes;
+    *bytes = plan_bwd(D, a->io_dtype == LTR_F32, D != a->D ? a->flags : a->flags & ~LTR_HEAD_COLS, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks, true).part_bytes;
     return LTR_OK;
 }
 

@@ -88,6 +88,7 @@ struct ChunksFunction {
             a.scale = (float)c.scale;
             a.io_dtype = f32 ? LTR_F32 : LTR_BF16;
             a.o_dtype = o_f32 ? LTR_F32 : LTR_BF16;
+            const uint32_t cols = D == 64 || D == 128 ? 0u : LTR_HEAD_COLS;
             if (with_rope) {
                 a.rope_freqs = c.rope.data_ptr<float>();
                 a.rope_len = c.rope.size(0);
@@ -104,7 +105,7 @@ struct ChunksFunction {
                     a.chunk[i].sk = e.rows;
                     a.chunk[i].pos0 = e.pos0;
                 }
-                a.flags = (c.causal ? LTR_CAUSAL : 0u) | (with_rope ? LTR_ROPE_Q : 0u) | (first > 0 ? LTR_MERGE : 0u);
+                a.flags = cols | (c.causal ? LTR_CAUSAL : 0u) | (with_rope ? LTR_ROPE_Q : 0u) | (first > 0 ? LTR_MERGE : 0u);
                 check_rc(ltr_attn_fwd(&a, (void *)c.stream), "ltr_attn_fwd");
                 a.q_rot = nullptr;   // stored by the first launch
             }
@@ -134,6 +135,8 @@ struct ChunksFunction {
         if (d_o.scalar_type() != q.scalar_type()) d_o = d_o.to(q.scalar_type());
         if (d_o.stride(3) != 1) d_o = d_o.contiguous();
         const int64_t B = q.size(0), Sq = q.size(1), Hq = q.size(2), D = q.size(3), Hkv = ks[0].size(2);
+        const uint32_t cols = D == 64 || D == 128 ? 0u : LTR_HEAD_COLS;
+        if (cols && ((d_o.stride(0) | d_o.stride(1) | d_o.stride(2)) % 8 || (uintptr_t)d_o.data_ptr() % 16)) d_o = d_o.clone(at::MemoryFormat::Contiguous);
         // gradients of the K / V tensors: one tensor each when their strides then agree, else slices of one buffer
         std::vector<Tensor> dk(n_t), dv(n_t);
         if (own_acc) {
@@ -226,7 +229,7 @@ struct ChunksFunction {
                 a.chunk[i].pos0 = e.pos0;
             }
             // this node holds every key these rows see and every row of it that sees these keys: the kernels write bf16 results
-            a.flags = (c.causal ? LTR_CAUSAL : 0u) | (direct ? LTR_DQ_BF16 : 0u) | (!f32 && !own_acc ? LTR_DKDV_BF16 : 0u) |
+            a.flags = cols | (c.causal ? LTR_CAUSAL : 0u) | (direct ? LTR_DQ_BF16 : 0u) | (!f32 && !own_acc ? LTR_DKDV_BF16 : 0u) |
                       (delta_from_o && first == 0 ? LTR_DELTA_FROM_O : 0u) | (c.rope.defined() ? LTR_ROPE_DQ : 0u);
             // few key tiles: blocks share them and leave partial sums in a workspace (from torch's caching allocator)
             int64_t part_bytes = 0;
