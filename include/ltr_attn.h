@@ -283,6 +283,25 @@ typedef struct ltr_rope_args {
 int ltr_rope_apply(const ltr_rope_args *args, void *stream);
 
 /*
+ * ltr_copy_strided - a strided view copied into a contiguous buffer: `n_outer` dimensions (outermost first; strides in bytes, any
+ * sign or order) of contiguous runs of run_bytes.  The data movement of the Ulysses exchange (SeqAllToAll,
+ * parallel/parallel_cp.py:49-96: split, all_to_all, cat) when all ranks' tensors lie on one GPU.  Pointers, strides and the run
+ * are multiples of 16 bytes; fewer than 2^31 16-byte vectors in all.  src and dst must not overlap.
+ */
+#define LTR_COPY_DIMS 6
+
+typedef struct ltr_copy_args {
+    const void *src;
+    void *dst;
+    int32_t n_outer;
+    int64_t run_bytes;
+    int64_t size[LTR_COPY_DIMS];
+    int64_t stride_bytes[LTR_COPY_DIMS];
+} ltr_copy_args;
+
+int ltr_copy_strided(const ltr_copy_args *args, void *stream);
+
+/*
  * ltr_attn_plan - which kernels, with which block sizes, ltr_attn_fwd and ltr_attn_bwd would launch for this problem
  * on the CURRENT device (host call: nothing is enqueued and no pointer in args is read; without a device the answer is
  * for 256 compute units).  It has no counterpart in the reference (which leaves the choice of kernel to the library

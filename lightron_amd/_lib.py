@@ -22,7 +22,7 @@ LTR_BWD_F32_SCALAR = 65536
 LTR_HEAD_COLS = 131072
 
 EXPORTS = ("ltr_attn_fwd", "ltr_attn_bwd_delta", "ltr_attn_bwd", "ltr_attn_bwd_ws", "ltr_attn_bwd_workspace", "ltr_attn_bwd_noalloc", "ltr_attn_plan", "ltr_cast_f32_to_bf16",
-           "ltr_rope_apply", "ltr_abi_version", "ltr_strerror")
+           "ltr_rope_apply", "ltr_copy_strided", "ltr_abi_version", "ltr_strerror")
 # the bench-only measurement library (include/ltr_probe.h); not part of the attention path
 PROBE_LIB_PATH = os.path.join(HERE, "csrc", "libltr_probe.so")
 PROBE_EXPORTS = ("ltr_device_info", "ltr_probe_mfma")

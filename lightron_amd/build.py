@@ -10,7 +10,7 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
-SRCS = [os.path.join(HERE, "csrc", f) for f in ("ltr_attn.hip", "ltr_rope.hip")]
+SRCS = [os.path.join(HERE, "csrc", f) for f in ("ltr_attn.hip", "ltr_rope.hip", "ltr_copy.hip")]
 LIB = os.path.join(HERE, "csrc", "libltr_attn.so")
 PROBE_SRCS = [os.path.join(HERE, "csrc", "ltr_probe.hip")]
 PROBE_LIB = os.path.join(HERE, "csrc", "libltr_probe.so")

@@ -343,10 +343,69 @@ std::vector<Tensor> chunks(const Tensor &q, std::vector<Tensor> kv, const std::v
     return ChunksNode::apply(q, at::TensorList(kv), c);
 }
 
+// The exchange of a rank-stacked tensor x [W, *shard]: out[i] = cat_j(split(x[j], scatter)[i], gather) for every rank i at once, as one
+// pass over the data.
+Tensor exchange(const Tensor &x, int64_t scatter, int64_t gather, int64_t W, int64_t stream) {
+    const int64_t nd = x.dim() - 1, chunk = x.size(scatter + 1) / W;
+    std::vector<int64_t> size{W}, stride{chunk * x.stride(scatter + 1)}, out_size{W};
+    for (int64_t i = 0; i < nd; i++) {
+        if (i == gather) size.push_back(W), stride.push_back(x.stride(0));
+        size.push_back(i == scatter ? chunk : x.size(i + 1));
+        stride.push_back(x.stride(i + 1));
+        out_size.push_back((i == scatter ? chunk : x.size(i + 1)) * (i == gather ? W : 1));
+    }
+    // neighbouring dimensions that are one run in memory are one dimension
+    std::vector<int64_t> cs, ct;
+    for (size_t i = 0; i < size.size(); i++) {
+        if (size[i] == 1) continue;
+        if (!cs.empty() && ct.back() == size[i] * stride[i]) cs.back() *= size[i], ct.back() = stride[i];
+        else cs.push_back(size[i]), ct.push_back(stride[i]);
+    }
+    const int64_t e = x.element_size();
+    Tensor out = torch::empty(out_size, x.options());
+    if (x.numel() == 0) return out;
+    ltr_copy_args a{};
+    bool fits = !cs.empty() && ct.back() == 1 && cs.back() * e % 16 == 0 && (int64_t)cs.size() - 1 <= LTR_COPY_DIMS && x.numel() * e / 16 < 0x7fff0000LL &&
+                ((uintptr_t)x.data_ptr() | (uintptr_t)out.data_ptr()) % 16 == 0;
+    for (size_t i = 0; fits && i + 1 < cs.size(); i++) {
+        a.size[i] = cs[i];
+        a.stride_bytes[i] = ct[i] * e;
+        fits = a.stride_bytes[i] % 16 == 0;
+    }
+    if (!fits) return x.as_strided(size, stride).reshape(out_size).contiguous();
+    const c10::DeviceGuard on_x_device(x.device());
+    a.src = x.data_ptr();
+    a.dst = out.data_ptr();
+    a.n_outer = (int32_t)cs.size() - 1;
+    a.run_bytes = cs.back() * e;
+    check_rc(ltr_copy_strided(&a, (void *)stream), "ltr_copy_strided");
+    return out;
+}
+
+struct ExchangeNode : torch::autograd::Function<ExchangeNode> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, int64_t scatter, int64_t gather, int64_t W, int64_t stream) {
+        ctx->saved_data["dims"] = std::vector<int64_t>{scatter, gather, W, stream};
+        return exchange(x, scatter, gather, W, stream);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {   // the exchange with the two dims swapped
+        const auto d = ctx->saved_data["dims"].toIntVector();
+        return {exchange(grads[0], d[1], d[0], d[2], d[3]), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor seq_all_to_all(const Tensor &x, int64_t scatter, int64_t gather, int64_t W, int64_t stream) {
+    const int64_t nd = x.dim() - 1;
+    TORCH_CHECK(x.is_cuda() && nd > 0 && W > 0 && scatter >= 0 && scatter < nd && gather >= 0 && gather < nd && x.size(0) == W && x.size(scatter + 1) % W == 0,
+                "a rank-stacked GPU tensor whose scattered dim divides by the number of ranks");
+    return ExchangeNode::apply(x, scatter, gather, W, stream);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("single_chunk", &single_chunk, "one bf16 KV chunk, forward with a C++ autograd node behind it");
     m.def("chunks", &chunks, "a table of KV chunks, forward with a C++ autograd node behind it");
+    m.def("seq_all_to_all", &seq_all_to_all, "the exchange of a rank-stacked tensor, differentiable");
+    m.def("exchange", [](const Tensor &x, int64_t s, int64_t g, int64_t W, int64_t stream) { return exchange(x, s, g, W, stream); }, "its data movement");
     m.def("abi_version", []() { return ltr_abi_version(); });
 }

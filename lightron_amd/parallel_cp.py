@@ -13,6 +13,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from . import attention
 from .attention import block_attention
 from .layers import rope_one, rope_table
 
@@ -41,6 +42,11 @@ def _world_size(group) -> int:
                               "LocalCPGroup (rank-stacked tensors) instead of a multi-rank ProcessGroup")
 
 
+def _exchange_node(x: torch.Tensor):
+    """The C++ binding when it can move this tensor (a GPU tensor), else None."""
+    return (attention._cpp_node() if attention.USE_CPP_NODE else None) if x.is_cuda else None
+
+
 def _exchange(x: torch.Tensor, scatter_dim: int, gather_dim: int, W: int) -> torch.Tensor:
     """x: [W_src, *shard].  out[i] = cat_j(split(x[j], scatter_dim)[i], gather_dim)
     (parallel_cp.py:65-73 for every rank i at once)."""
@@ -50,6 +56,9 @@ def _exchange(x: torch.Tensor, scatter_dim: int, gather_dim: int, W: int) -> tor
     sd, gd = scatter_dim % nd, gather_dim % nd
     size = x.size(sd + 1)
     assert size % W == 0, f"Input dim {scatter_dim} size {size} not divisible by CP size {W}"   # :61-63
+    node = _exchange_node(x)
+    if node:
+        return node.exchange(x, sd, gd, W, attention._stream_ptr(x.device))      # one pass of ltr_copy_strided
     y = x.unflatten(sd + 1, (W, size // W))      # [W_src, ..., W_dst, chunk, ...]
     y = y.movedim(sd + 1, 0)                     # [W_dst, W_src, *shard with chunk at sd]
     y = y.movedim(1, gd + 1)                     # W_src just before the gather dim
@@ -75,6 +84,12 @@ class SeqAllToAll(torch.autograd.Function):
 
 
 def _all_to_all(input_, scatter_dim, gather_dim, group):
+    W = _world_size(group)
+    nd = input_.dim() - 1
+    if W > 1 and nd > 0 and input_.shape[0] == W and input_.shape[scatter_dim % nd + 1] % W == 0:
+        node = _exchange_node(input_)
+        if node:      # forward and backward as a C++ autograd node
+            return node.seq_all_to_all(input_, scatter_dim % nd, gather_dim % nd, W, attention._stream_ptr(input_.device))
     return SeqAllToAll.apply(input_, scatter_dim, gather_dim, group)
 
 
