@@ -400,11 +400,53 @@ Tensor seq_all_to_all(const Tensor &x, int64_t scatter, int64_t gather, int64_t 
     return ExchangeNode::apply(x, scatter, gather, W, stream);
 }
 
+// RoPE of one [B, S, H, D] tensor (ltr_rope_apply); its gradient is the rotation by the conjugate angles.
+Tensor rope_pass(const Tensor &x0, const Tensor &table, bool conj, int64_t stream) {
+    const Tensor x = x0.stride(3) == 1 ? x0 : x0.contiguous();
+    const c10::DeviceGuard on_x_device(x.device());
+    Tensor out = torch::empty(x.sizes(), x.options());
+    ltr_rope_args a{};
+    a.x = x.data_ptr();
+    a.out = out.data_ptr();
+    a.freqs = table.data_ptr<float>();
+    a.B = (int32_t)x.size(0);
+    a.S = x.size(1);
+    a.H = (int32_t)x.size(2);
+    a.D = (int32_t)x.size(3);
+    strides3(x, a.x_stride);
+    strides3(out, a.out_stride);
+    a.flags = conj ? LTR_ROPE_CONJ : 0u;
+    a.io_dtype = x.scalar_type() == at::kBFloat16 ? LTR_BF16 : LTR_F32;
+    check_rc(ltr_rope_apply(&a, (void *)stream), "ltr_rope_apply");
+    return out;
+}
+
+struct RopeNode : torch::autograd::Function<RopeNode> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &table, int64_t stream) {
+        ctx->save_for_backward({table});
+        ctx->saved_data["stream"] = stream;
+        return rope_pass(x, table, false, stream);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        return {rope_pass(grads[0], ctx->get_saved_variables()[0], true, ctx->saved_data["stream"].toInt()), Tensor(), Tensor()};
+    }
+};
+
+// table: fp32 [S, D/2, 2] (cos, sin) rows of x's sequence indices
+Tensor rope(const Tensor &x, const Tensor &table, int64_t stream) {
+    TORCH_CHECK(x.is_cuda() && x.dim() == 4 && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat), "x must be a bf16 or fp32 [B,S,H,D] GPU tensor");
+    TORCH_CHECK(table.scalar_type() == at::kFloat && table.is_contiguous() && table.dim() == 3 && table.size(0) == x.size(1) && table.size(1) == x.size(3) / 2 &&
+                    table.size(2) == 2 && table.device() == x.device(),
+                "the RoPE table must be a contiguous fp32 [S, D/2, 2] (cos, sin) tensor on x's device");
+    return RopeNode::apply(x, table, stream);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("single_chunk", &single_chunk, "one bf16 KV chunk, forward with a C++ autograd node behind it");
     m.def("chunks", &chunks, "a table of KV chunks, forward with a C++ autograd node behind it");
+    m.def("rope", &rope, "rotary position embedding of one tensor, differentiable");
     m.def("seq_all_to_all", &seq_all_to_all, "the exchange of a rank-stacked tensor, differentiable");
     m.def("exchange", [](const Tensor &x, int64_t s, int64_t g, int64_t W, int64_t stream) { return exchange(x, s, g, W, stream); }, "its data movement");
     m.def("abi_version", []() { return ltr_abi_version(); });

@@ -6,7 +6,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _lib, attention
 
 
 def precompute_freqs_cis(dim: int, end: int, theta: float = 10000.0, device=None) -> torch.Tensor:
@@ -77,6 +77,9 @@ def _rope_gpu(x: torch.Tensor, freqs_cis: torch.Tensor) -> torch.Tensor:
         raise AssertionError("freqs_cis shape %s does not match x shape %s"
                              % (tuple(freqs_cis.shape), (x.shape[1], x.shape[-1] // 2)))
     table = torch.view_as_real(freqs_cis.to(device=x.device, dtype=torch.complex64)).contiguous()
+    node = attention._cpp_node() if attention.USE_CPP_NODE and x.dim() == 4 and not table.requires_grad else None
+    if node:
+        return node.rope(x, table, attention._stream_ptr(x.device))
     return _Rope.apply(x, table)
 
 

@@ -103,9 +103,8 @@ class ContextParallelAttention(nn.Module):
 
     literal=True follows the reference step by step (three seq->head exchanges, RoPE on the
     global sequence, causal attention on [B, S, H/W, D], head->seq exchange).  The default
-    path gives the same result without moving data: each rank's sequence shard is one KV
-    chunk of the kernel's chunk table, all heads are processed in one launch per Q shard, and
-    the two exchanges cancel.
+    path gives the same result without the exchanges, which cancel: the shards are attended as
+    the one sequence they are, all heads in one launch.
     """
 
     def __init__(self, local_attn_module, args, cp_group=None, literal: bool = False, causal: bool = True):
@@ -135,11 +134,11 @@ class ContextParallelAttention(nn.Module):
         S_global = S_local * W
         assert freqs_cis.shape[0] >= S_global, f"freqs_cis too short: {freqs_cis.shape[0]} < S_global {S_global}"
         H, Hkv, D = self.num_heads, self.num_kv_heads, self.head_dim
-        xq = self.local_attn.wq(x).view(W, B, S_local, H, D)
-        xk = self.local_attn.wk(x).view(W, B, S_local, Hkv, D)
-        xv = self.local_attn.wv(x).view(W, B, S_local, Hkv, D)
         fc = freqs_cis[:S_global]
         if self.literal:
+            xq = self.local_attn.wq(x).view(W, B, S_local, H, D)
+            xk = self.local_attn.wk(x).view(W, B, S_local, Hkv, D)
+            xv = self.local_attn.wv(x).view(W, B, S_local, Hkv, D)
             if Hkv % W:
                 raise RuntimeError("literal Ulysses path needs n_kv_heads divisible by the cp size")
             xq = _all_to_all(xq, 2, 1, self.cp_group)            # [W, B, S_global, H/W, D]
@@ -150,24 +149,18 @@ class ContextParallelAttention(nn.Module):
             o, _ = block_attention(qf, [kf], [vf], [0], 0, None, self.causal)
             o = o.view(W, B, S_global, H // W, D)
             o = _all_to_all(o, 1, 2, self.cp_group)              # [W, B, S_local, H, D]
-        else:
-            # RoPE at global positions (:215-219): every K shard is rotated once, in one streaming pass (it is read by
-            # every later q shard); q is rotated inside the attention kernel's prologue, dQ rotated back in the dQ
-            # kernel's epilogue (bf16; fp32 inputs take the streaming pass for q as well)
-            outs = []
-            fused = xq.dtype == torch.bfloat16
-            table = rope_table(fc, xq.device) if fused else None
-            qs, ks = [], []
-            for j in range(W):
-                fj = fc[j * S_local:(j + 1) * S_local]
-                ks.append(rope_one(xk[j], fj))
-                qs.append(xq[j] if fused else rope_one(xq[j], fj))
-            vs = [xv[j] for j in range(W)]
-            pos = [j * S_local for j in range(W)]
-            for j in range(W):
-                n = j + 1 if self.causal else W                  # later shards are fully masked
-                oj, _ = block_attention(qs[j], ks[:n], vs[:n], pos[:n], j * S_local, None, self.causal, q_rope=table)
-                outs.append(oj)
-            o = torch.stack(outs, 0)
-        return self.local_attn.wo(o.flatten(3))
+            return self.local_attn.wo(o.flatten(3))
+        # The shards follow each other in the sequence, so the ranks' work is one attention over all of it: one launch per
+        # kernel instead of one per shard (whose dK / dV autograd would have to add up), and with one batch entry the shards are
+        # that sequence in memory already.  RoPE at global positions (:215-219): K in one streaming pass; q inside the attention
+        # kernel, dQ rotated back in the dQ kernel's epilogue (bf16; fp32 inputs take the streaming pass for q as well)
+        xs = x.transpose(0, 1).reshape(B, S_global, -1)
+        xq = self.local_attn.wq(xs).view(B, S_global, H, D)
+        xk = rope_one(self.local_attn.wk(xs).view(B, S_global, Hkv, D), fc)
+        xv = self.local_attn.wv(xs).view(B, S_global, Hkv, D)
+        fused = xq.dtype == torch.bfloat16
+        o, _ = block_attention(xq if fused else rope_one(xq, fc), [xk], [xv], [0], 0, None, self.causal,
+                               q_rope=rope_table(fc, xq.device) if fused else None)
+        y = self.local_attn.wo(o.reshape(B, S_global, -1))
+        return y.view(B, W, S_local, -1).transpose(0, 1).contiguous()
 
