@@ -598,6 +598,8 @@ def chunk_table_attention(q, ks, vs, entries, q_pos0, q_split, causal, scale, st
     node = _cpp_node() if USE_CPP_NODE else None
     if not node or not q.is_cuda or q.dtype not in _DT or (q.shape[-1] not in (64, 128) and not _native_cols(q, ks, vs, kv_grad_acc)):
         return None
+    if not all(entries[2::4]):      # an empty chunk
+        return None
     out_dtype = out_dtype or q.dtype
     if out_dtype not in _DT or (q.dtype == torch.float32 and out_dtype != torch.float32):
         return None

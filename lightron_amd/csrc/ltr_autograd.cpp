@@ -55,6 +55,26 @@ struct Call : torch::CustomClassHolder {
 
 char *row_ptr(const Tensor &t, int64_t row) { return (char *)t.data_ptr() + row * t.stride(1) * t.element_size(); }
 
+// Saved-tensor hooks may hand a tensor back in another layout than it was saved in; the kernels want whole rows, and one stride
+// triple for all K and one for all V tensors of a table.
+Tensor rows_contiguous(const Tensor &t) {
+    const bool cols = t.size(3) != 64 && t.size(3) != 128 && ((t.stride(0) | t.stride(1) | t.stride(2)) % 8 || (uintptr_t)t.data_ptr() % 16);
+    return (t.numel() == 0 || t.stride(3) == 1) && !cols ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
+std::vector<Tensor> one_layout(const Tensor *t, int64_t n) {
+    std::vector<Tensor> out;
+    bool alike = true;
+    for (int64_t i = 0; i < n; i++) {
+        out.push_back(rows_contiguous(t[i]));
+        alike = alike && same_strides(out[i], out[0]);
+    }
+    if (alike) return out;
+    const Tensor all = at::cat(out, 1);
+    for (int64_t i = 0, row = 0; i < n; row += out[i++].size(1)) out[i] = all.narrow(1, row, out[i].size(1));
+    return out;
+}
+
 // The arithmetic of both nodes below.  kv: the K tensors, then as many V tensors
 struct ChunksFunction {
     static variable_list forward(AutogradContext *ctx, const Tensor &q, at::TensorList kv, const c10::intrusive_ptr<Call> &call) {
@@ -111,7 +131,7 @@ struct ChunksFunction {
             }
         }
         if (o_f32 && !c.out_f32) o = o.to(at::kBFloat16);
-        variable_list saved{with_rope ? q_rot : q, o, lse};
+        variable_list saved{with_rope ? q_rot : q, o, lse, c.rope};
         saved.insert(saved.end(), kv.begin(), kv.end());
         ctx->save_for_backward(std::move(saved));
         ctx->saved_data["call"] = c10::IValue::make_capsule(call);   // with its stream: the engine runs the backward on the forward's
@@ -124,9 +144,10 @@ struct ChunksFunction {
         const auto saved = ctx->get_saved_variables();
         const auto call = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
         const Call &c = *call;
-        const Tensor &q = saved[0], &o = saved[1], &lse = saved[2];
-        const int64_t n_t = ((int64_t)saved.size() - 3) / 2, n = (int64_t)c.entries.size();
-        const Tensor *ks = &saved[3], *vs = ks + n_t;
+        const Tensor q = rows_contiguous(saved[0]), o = rows_contiguous(saved[1]), lse = saved[2].contiguous();
+        const Tensor &rope = saved[3];
+        const int64_t n_t = ((int64_t)saved.size() - 4) / 2, n = (int64_t)c.entries.size();
+        const std::vector<Tensor> ks = one_layout(&saved[4], n_t), vs = one_layout(&saved[4] + n_t, n_t);
         variable_list out(1 + 2 * n_t + 1);
         if (!grads[0].defined()) return out;
         const c10::DeviceGuard on_q_device(q.device());
@@ -213,9 +234,9 @@ struct ChunksFunction {
         a.q_split = c.q_split;
         a.scale = (float)c.scale;
         a.io_dtype = f32 ? LTR_F32 : LTR_BF16;
-        if (c.rope.defined()) {
-            a.rope_freqs = c.rope.data_ptr<float>();
-            a.rope_len = c.rope.size(0);
+        if (rope.defined()) {
+            a.rope_freqs = rope.data_ptr<float>();
+            a.rope_len = rope.size(0);
         }
         for (int64_t first = 0; first < n; first += LTR_MAX_CHUNKS) {
             a.n_chunks = (int32_t)std::min<int64_t>(LTR_MAX_CHUNKS, n - first);
@@ -230,7 +251,7 @@ struct ChunksFunction {
             }
             // this node holds every key these rows see and every row of it that sees these keys: the kernels write bf16 results
             a.flags = cols | (c.causal ? LTR_CAUSAL : 0u) | (direct ? LTR_DQ_BF16 : 0u) | (!f32 && !own_acc ? LTR_DKDV_BF16 : 0u) |
-                      (delta_from_o && first == 0 ? LTR_DELTA_FROM_O : 0u) | (c.rope.defined() ? LTR_ROPE_DQ : 0u);
+                      (delta_from_o && first == 0 ? LTR_DELTA_FROM_O : 0u) | (rope.defined() ? LTR_ROPE_DQ : 0u);
             // few key tiles: blocks share them and leave partial sums in a workspace (from torch's caching allocator)
             int64_t part_bytes = 0;
             check_rc(ltr_attn_bwd_workspace(&a, &part_bytes), "ltr_attn_bwd_workspace");
@@ -389,7 +410,7 @@ struct ExchangeNode : torch::autograd::Function<ExchangeNode> {
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {   // the exchange with the two dims swapped
         const auto d = ctx->saved_data["dims"].toIntVector();
-        return {exchange(grads[0], d[1], d[0], d[2], d[3]), Tensor(), Tensor(), Tensor(), Tensor()};
+        return {ExchangeNode::apply(grads[0], d[1], d[0], d[2], d[3]), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 

@@ -43,8 +43,8 @@ def _world_size(group) -> int:
 
 
 def _exchange_node(x: torch.Tensor):
-    """The C++ binding when it can move this tensor (a GPU tensor), else None."""
-    return (attention._cpp_node() if attention.USE_CPP_NODE else None) if x.is_cuda else None
+    """The C++ binding when it can move this tensor (a GPU tensor whose bytes are its values), else None."""
+    return (attention._cpp_node() if attention.USE_CPP_NODE else None) if x.is_cuda and not (x.is_conj() or x.is_neg()) else None
 
 
 def _exchange(x: torch.Tensor, scatter_dim: int, gather_dim: int, W: int) -> torch.Tensor:
@@ -80,7 +80,7 @@ class SeqAllToAll(torch.autograd.Function):
         W = _world_size(ctx.group)
         if W == 1:
             return grad_output, None, None, None
-        return _exchange(grad_output, ctx.gather_dim, ctx.scatter_dim, W), None, None, None
+        return _all_to_all(grad_output, ctx.gather_dim, ctx.scatter_dim, ctx.group), None, None, None
 
 
 def _all_to_all(input_, scatter_dim, gather_dim, group):
