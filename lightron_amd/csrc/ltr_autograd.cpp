@@ -366,7 +366,8 @@ std::vector<Tensor> chunks(const Tensor &q, std::vector<Tensor> kv, const std::v
 
 // The exchange of a rank-stacked tensor x [W, *shard]: out[i] = cat_j(split(x[j], scatter)[i], gather) for every rank i at once, as one
 // pass over the data.
-Tensor exchange(const Tensor &x, int64_t scatter, int64_t gather, int64_t W, int64_t stream) {
+Tensor exchange(const Tensor &x0, int64_t scatter, int64_t gather, int64_t W, int64_t stream) {
+    const Tensor x = x0.resolve_conj().resolve_neg();   // the bytes that are copied have to be the values (a gradient may come as a conjugated view)
     const int64_t nd = x.dim() - 1, chunk = x.size(scatter + 1) / W;
     std::vector<int64_t> size{W}, stride{chunk * x.stride(scatter + 1)}, out_size{W};
     for (int64_t i = 0; i < nd; i++) {

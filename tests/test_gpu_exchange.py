@@ -37,3 +37,12 @@ def test_exchange_matches_the_oracle(ltr, W, shape, scatter, gather, dtype):
         xo = torch.empty(x.numel() + 1, dtype=dtype, device="cuda")[1:].view(x.shape)
         xo.copy_(x)
         assert torch.equal(ltr._all_to_all(xo, scatter, gather, grp).cpu(), torch.stack(want))
+
+
+def test_gradients_may_be_conjugated_views(ltr):
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(2, 3, 4, 8, generator=g, dtype=torch.complex64).cuda().requires_grad_(True)
+    gy = torch.randn(2, 3, 8, 4, generator=g, dtype=torch.complex64)
+    ltr._all_to_all(x, 2, 1, ltr.LocalCPGroup(2)).backward(gy.cuda().conj())
+    want = torch.stack(orc.seq_all_to_all(list(gy.conj().resolve_conj()), 1, 2))
+    assert torch.equal(x.grad.cpu(), want)
