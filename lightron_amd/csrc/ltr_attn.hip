@@ -3339,13 +3339,27 @@ int q_tile_slots(int n_qtiles, long long blocks_per_tile, bool uneven) {
 //   B=1  8 heads D=128 causal S=4096   99.0 / 128.7   64.8 / 81.3    52.7 / 66.1
 //   B=1  8 heads D=64  causal S=4096   64.9 / 72.8    40.4 / 46.6    34.5 / 40.8
 //   B=1 32 heads D=128 causal S=4096  135.1 / 183.9  158.5 / 204.6  203.2 / 256.8   (256-row blocks fill the device)
+//
+// Under a causal mask two shares may also take their q tiles in pairs (late + early, see q_tile_slots): where 256-row tiles give every
+// CU one block of its own length and the longest decides, 128-row tiles pair to one equal block per CU.  Only for a round that is
+// (nearly) full: with fewer blocks idle CUs cost more than the balance gives.  Kernel us unpaired -> paired, forward / dQ:
+//   B=1 16 heads D=128 S=4096   115 / 128 -> 97 / 123 (256 paired blocks)    B=1 16 heads D=64 S=4096    72 / 86 -> 58 / 70 (256)
+//   B=2 16 heads D=128 S=2048    64 / 86  -> 59 / 74 (256)                   B=4 16 heads D=128 S=1024   39 / 51 -> 40 / 50 (256)
+//   B=1 16 heads D=128 S=3500    79 / 101 -> 83 / 107 (224)                  B=2  8 heads D=128 S=3000   64 / 82 -> 70 / 90 (192)
+//   B=1 12 heads D=64 S=3333     38 / 46  -> 44 / 54 (168)                   B=1 32 heads D=128 S=1237   31 / 39 -> 39 / 50 (160)
+// Four shares in pairs were slower than two at all nine shapes tried.
 struct ShareCost {
     double step_us[3], fixed_us[3];   // per step (one K / V tile) and per block, for 1, 2 and 4 shares
+    double paired_us;                 // per step of two shares in pairs (a block on every CU)
 };
-int key_shares(const ShareCost &cost, int D, bool causal, long long BH, long long kv_heads, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks) {
+struct ShareChoice {
+    int ks;
+    bool paired;
+};
+ShareChoice key_shares(const ShareCost &cost, int D, bool causal, long long BH, long long kv_heads, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks) {
     const int cus = device_cus();
-    if (BH * ((Sq + 255) / 256) >= 4LL * cus) return 1;   // several rounds of 256-row blocks: they balance by themselves
-    int best = 1;
+    if (BH * ((Sq + 255) / 256) >= 4LL * cus) return {1, false};   // several rounds of 256-row blocks: they balance by themselves
+    ShareChoice best{1, false};
     double best_us = 0;
     for (int i = 0; i < 3; i++) {
         const int ks = 1 << i, rows = 256 / ks, keys = ks * (D == 64 ? (ks == 1 ? 128 : 64) : (ks == 4 ? 32 : 64));
@@ -3353,30 +3367,45 @@ int key_shares(const ShareCost &cost, int D, bool causal, long long BH, long lon
         // more than one kv head per XCD and every CU busy: the extra K / V traffic of the shares shows (B=1, 32 kv heads, D=128,
         // S=2048: 57 us with one share, 67 with two; with 8 kv heads 57 and 49)
         const double step_us = cost.step_us[i] * (ks > 1 && BH * n > cus && kv_heads > 8 ? 1.25 : 1.0);
-        double sum = 0, most = 0;
-        for (int t = 0; t < n; t++) {
-            double steps = 0;
+        auto steps = [&](int t) {
+            double sum = 0;
             const int r0 = t * rows, r1 = std::min(Sq, r0 + rows) - 1;
             int hi = r1 < q_split ? q_pos0[0] + r1 : q_pos0[1] + (r1 - q_split);
             if (r0 < q_split && r1 >= q_split) hi = std::max(hi, q_pos0[0] + q_split - 1);
             for (int c = 0; c < n_chunks; c++) {
                 const long long seen = causal ? std::min<long long>(std::max<long long>((long long)hi - chunk[c].pos0 + 1, 0), chunk[c].sk) : chunk[c].sk;
-                steps += (double)((seen + keys - 1) / keys);
+                sum += (double)((seen + keys - 1) / keys);
             }
-            const double us = steps * step_us + cost.fixed_us[i];
+            return sum;
+        };
+        double sum = 0, most = 0;
+        for (int t = 0; t < n; t++) {
+            const double us = steps(t) * step_us + cost.fixed_us[i];
             sum += us;
             most = std::max(most, us);
         }
         const double us = BH * n <= cus ? most : std::max(most, sum * BH / cus + 0.25 * sum / n);
         if (i == 0 || us < 0.97 * best_us) {
             best_us = us;
-            best = ks;
+            best = {ks, false};
+        }
+        const int slots = (n + 1) / 2;
+        if (ks == 2 && causal && BH * slots <= cus && BH * slots * 10 >= cus * 9 && q_tiles_uneven(Sq, rows, q_split, q_pos0, chunk, n_chunks)) {
+            double pair_us = 0;
+            for (int t = 0; t < slots; t++) {
+                const bool two = t < n - 1 - t;
+                pair_us = std::max(pair_us, (steps(t) + (two ? steps(n - 1 - t) : 0)) * cost.paired_us + (two ? 2 : 1) * cost.fixed_us[i]);
+            }
+            if (pair_us < 0.97 * best_us) {
+                best_us = pair_us;
+                best = {ks, true};
+            }
         }
     }
     return best;
 }
-constexpr ShareCost FWD_SHARES_128{{1.45, 1.8, 1.05}, {9.0, 8.0, 10.0}}, FWD_SHARES_64{{1.7, 0.95, 1.0}, {9.0, 8.0, 6.0}};
-constexpr ShareCost DQ_SHARES_128{{1.85, 2.2, 1.4}, {11.0, 10.0, 10.0}}, DQ_SHARES_64{{1.95, 1.15, 1.35}, {10.0, 9.0, 6.0}};
+constexpr ShareCost FWD_SHARES_128{{1.45, 1.8, 1.05}, {9.0, 8.0, 10.0}, 2.2}, FWD_SHARES_64{{1.7, 0.95, 1.0}, {9.0, 8.0, 6.0}, 1.09};
+constexpr ShareCost DQ_SHARES_128{{1.85, 2.2, 1.4}, {11.0, 10.0, 10.0}, 2.7}, DQ_SHARES_64{{1.95, 1.15, 1.35}, {10.0, 9.0, 6.0}, 1.3};
 
 // What a forward launch looks like: rows per block, q tiles, slots (see q_tile_slots), blocks.  One function decides for
 // ltr_attn_fwd and for ltr_attn_plan, so the plan a caller is shown is the launch it gets.
@@ -3414,9 +3443,11 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     // query rows per block: 512 (two 32-row blocks per wave, 64-key tiles) pays at head dim 64 under the conditions of
     // the dQ kernel's 512-row blocks (see plan_bwd)
     bool wide = (flags & LTR_FWD_ROWS_512) != 0;
+    ShareChoice shares{1, false};
     if (!wide && !(flags & LTR_FWD_ROWS_256))
-        pl.ks = key_shares(D == 128 ? FWD_SHARES_128 : FWD_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
-                           n_chunks);
+        shares = key_shares(D == 128 ? FWD_SHARES_128 : FWD_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
+                            n_chunks);
+    pl.ks = shares.ks;
     if (!wide && !(flags & (LTR_FWD_ROWS_256 | LTR_HEAD_COLS)) && D == 64 && pl.ks == 1) {
         const int tiles512 = (Sq + 511) / 512;
         const int slots512 = q_tile_slots(tiles512, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, 512, q_split, q_pos0, chunk, n_chunks));
@@ -3428,8 +3459,9 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.wide = wide;
     if (pl.ks > 1) {
         pl.rows = 256 / pl.ks;
-        pl.n_qtiles = pl.n_slots = (Sq + pl.rows - 1) / pl.rows;
-        pl.blocks = (long long)pl.n_qtiles * B * Hq;
+        pl.n_qtiles = (Sq + pl.rows - 1) / pl.rows;
+        pl.n_slots = shares.paired ? (pl.n_qtiles + 1) / 2 : pl.n_qtiles;
+        pl.blocks = (long long)pl.n_slots * B * Hq;
         return pl;
     }
     pl.rows = wide ? 512 : 256;
@@ -3576,9 +3608,11 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     // query rows per block of the dQ kernel: 512 (two 32-row blocks per wave) pays at head dim 64 when the wider blocks still
     // fill the device, and under a causal mask only on sequences long enough that the diagonal does not dominate
     bool wide_q = (flags & LTR_DQ_ROWS_512) != 0;
+    ShareChoice shares{1, false};
     if (!wide_q && !(flags & (LTR_DQ_ROWS_256 | LTR_NO_DQ)))
-        pl.dq_ks = key_shares(D == 128 ? DQ_SHARES_128 : DQ_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
-                              n_chunks);
+        shares = key_shares(D == 128 ? DQ_SHARES_128 : DQ_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
+                            n_chunks);
+    pl.dq_ks = shares.ks;
     if (!wide_q && !(flags & (LTR_DQ_ROWS_256 | LTR_HEAD_COLS)) && D == 64 && !(flags & LTR_NO_DQ) && pl.dq_ks == 1) {
         const int tiles512 = (Sq + 511) / 512;
         const int slots512 = q_tile_slots(tiles512, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, 512, q_split, q_pos0, chunk, n_chunks));
@@ -3593,7 +3627,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.wide_q = wide_q;
     pl.dq_rows = wide_q ? 512 : 256 / pl.dq_ks;
     pl.dq_qtiles = (Sq + pl.dq_rows - 1) / pl.dq_rows;
-    pl.dq_slots = pl.dq_ks > 1 ? pl.dq_qtiles
+    pl.dq_slots = pl.dq_ks > 1 ? (shares.paired ? (pl.dq_qtiles + 1) / 2 : pl.dq_qtiles)
                                : q_tile_slots(pl.dq_qtiles, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks));
     pl.dq_blocks = (long long)pl.dq_slots * B * Hq;
     return pl;

@@ -60,3 +60,14 @@ def test_key_shares_forward_backward(ltr, D, B, Hq, Hkv, Sq, q_pos, split, chunk
     assert (dq32 - dq_ref).norm() <= 5e-2 * dq_ref.norm()
     # bf16 rounding (2^-8 of the value) and the cancellation of the accumulator's start value (2^-23 of 0.5 + |dQ|)
     assert ((dq16.cpu().float() - dq32).abs() <= dq32.abs() / 256 + 1e-6).all()
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,Sq,q_pos,split,chunks", [
+    (64, 16, 16, 3900, 0, None, [(3900, 0)]),                                           # an odd number of tiles: the middle one alone
+    (128, 16, 16, 3801, 0, None, [(1701, 0), (2100, 1701)]),
+    (64, 16, 16, 3840, (0, 5760), 1920, [(1920, 0), (1920, 5760)]),   # a zig-zag share against its own keys
+])
+def test_key_shares_in_pairs_of_tiles(ltr, D, Hq, Hkv, Sq, q_pos, split, chunks):
+    plan = ltr.attn_plan(1, Hq, Hkv, D, Sq, [n for n, _ in chunks], [p for _, p in chunks], q_pos, split, True)
+    assert plan["fwd"]["paired"] and plan["dq"]["paired"]
+    test_key_shares_forward_backward(ltr, D, 1, Hq, Hkv, Sq, q_pos, split, chunks, True, 2)
