@@ -74,6 +74,9 @@ extern "C" {
                                 run with their columns past D cleared on chip: no padded copies of the tensors.  scale is the caller's
                                 (1/sqrt of the true D); a RoPE table has D/2 pairs per row.  No 512-row / 256-key blocks. */
 
+#define LTR_DQ_F32_RESULT 262144u /* backward, fp32: dq RECEIVES dQ of this call (no accumulation) and delta is computed from the fp32 o by the
+                                    dQ kernel: LTR_DQ_BF16 | LTR_DELTA_FROM_O for fp32.  LTR_EUNSUP with bf16 or LTR_BWD_F32_SCALAR */
+
 /* error codes */
 #define LTR_OK 0
 #define LTR_EINVAL (-1)   /* null pointer, bad size, bad flag */
@@ -203,12 +206,12 @@ typedef struct ltr_attn_bwd_args {
     float scale;
     uint32_t flags;       /* LTR_CAUSAL | LTR_NO_DQ | LTR_NO_DKDV | LTR_DQ_BF16 | LTR_DELTA_FROM_O | LTR_DKDV_BF16 | LTR_ROPE_DQ |
                              LTR_DKDV_KEYS_128 | LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR |
-                             LTR_HEAD_COLS */
+                             LTR_HEAD_COLS | LTR_DQ_F32_RESULT */
     int32_t io_dtype;     /* LTR_BF16 or LTR_F32, of q/k/v/dO (LTR_F32: fp32 kernels on v_mfma_f32_32x32x2_f32 for the 1e-4 cases;
                              LTR_DQ_BF16, LTR_DELTA_FROM_O and LTR_DKDV_BF16 are bf16 only and return LTR_EUNSUP with it) */
     int32_t n_chunks;
     ltr_kv_chunk chunk[LTR_MAX_CHUNKS];
-    const void *o;        /* forward output, bf16, only read with LTR_DELTA_FROM_O */
+    const void *o;        /* forward output, only read with LTR_DELTA_FROM_O (bf16) or LTR_DQ_F32_RESULT (fp32) */
     int64_t o_stride[3];
     /* LTR_ROPE_DQ (bf16 only): q is the ROTATED q (q_rot of a forward with LTR_ROPE_Q); the dQ kernel's epilogue rotates
      * dQ by the conjugate angles of each row's global position before it is stored or accumulated, so dq is the

@@ -111,7 +111,7 @@ struct BwdParams {
     const void *d_o;
     const float *lse;
     float *delta;      // read; written by the dQ kernel with LTR_DELTA_FROM_O
-    const void *o;     // bf16 forward output, read with LTR_DELTA_FROM_O only
+    const void *o;     // forward output, read with LTR_DELTA_FROM_O (bf16) and LTR_DQ_F32_RESULT (fp32) only
     long long os_[3];
     void *dq;          // fp32 accumulator, or bf16 result with LTR_DQ_BF16
     int B, Hq, Hkv, n_rep;
@@ -2740,7 +2740,9 @@ __global__ __launch_bounds__(64) void bwd_dkdv_f32_kernel(const BwdParams p) {
 //   bwd_dq_f32_mfma_kernel<D, KS>   4 waves, a wave owns 32 query rows (lane = row; Q, dO operands in registers) and one of
 //                        KS key shares: S^T = K Q^T and dP^T = V dO^T (accumulators start at -DELTA), dS^T = P (dP - DELTA)
 //                        in registers, dQ^T += K^T dS^T with the accumulator register as the step's operand; the KS partial
-//                        dQ of a row group are summed through LDS; dQ is added to the fp32 accumulator in whole rows.
+//                        dQ of a row group are summed through LDS; dQ is added to the fp32 accumulator in whole rows, or, with
+//                        LTR_DQ_F32_RESULT, stored, and DELTA of the block's rows is computed from O in the prologue and left for the
+//                        dK/dV kernel: no DELTA launch, no fill of dQ (B=2, 8 heads of 64, 256 rows: launches of 3 us each).
 //   bwd_dkdv_f32_mfma_kernel<D>     4 waves, a wave owns 32 keys (lane = key; K, V operands and the dK^T, dV^T accumulators
 //                        in registers: one wave per SIMD), the block loops over the group's query heads and over 32-row
 //                        Q / dO tiles in double-buffered LDS: S = Q K^T, dP = dO V^T (accumulators start at -DELTA of
@@ -2755,7 +2757,7 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p)
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rg = w / KS, ks = w % KS;
-    const bool causal = p.flags & LTR_CAUSAL;
+    const bool causal = p.flags & LTR_CAUSAL, result = p.flags & LTR_DQ_F32_RESULT;
     const int n_qt = (p.Sq + BM - 1) / BM;
     const int idx = blockIdx.x;
     const int qt = n_qt - 1 - idx / (p.B * p.Hq);
@@ -2790,7 +2792,20 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p)
         if (row_ok) {
             const float lse_row = p.lse[((long long)b * p.Hq + h) * p.Sq + my_row];
             lse2 = lse_row == -INFINITY ? INFINITY : lse_row * LTR_LOG2E;
-            dlt = p.delta[((long long)b * p.Hq + h) * p.Sq + my_row];
+            if (!result) dlt = p.delta[((long long)b * p.Hq + h) * p.Sq + my_row];
+        }
+        if (result) {   // the two lanes of a row hold its column groups in turn
+            const float *op = (const float *)p.o + b * p.os_[0] + (long long)rs * p.os_[1] + h * p.os_[2];
+            float part = 0.f;
+#pragma unroll
+            for (int g = 0; g < D / 8; g++) {
+                const f32x4 x = *(const f32x4 *)(op + 8 * g + 4 * hh);
+#pragma unroll
+                for (int j = 0; j < 4; j++) part = fmaf(x[j], doreg[4 * g + j], part);
+            }
+            part = xhalf_sum(part);
+            if (row_ok) dlt = part;
+            if (row_ok && hh == 0 && ks == 0) p.delta[((long long)b * p.Hq + h) * p.Sq + my_row] = part;
         }
     }
     f32x16 dqacc[D / 32], ndlt;
@@ -2837,8 +2852,8 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p)
         }
     };
     bool have = c < p.n_chunks;
-    if (!have) return;              // no visible key: nothing to add to the accumulator (block-uniform)
-    gload(t, 0);
+    if (!have && !result) return;   // no visible key: nothing to add to the accumulator (block-uniform)
+    if (have) gload(t, 0);
     tile_barrier();
     int par = 0;
     while (have) {
@@ -2928,9 +2943,11 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p)
     float *dqp = (float *)p.dq + b * p.dqs[0] + h * p.dqs[2] + (long long)(wave_row0 + lane / LPR) * dqs1 + 4 * (lane % LPR);
     wave_tile_rowmajor<D>(stage, lane, dqacc, p.scale, [&](int row, int, f32x4 val) {
         if (wave_row0 + row < Sq) {
-            const f32x4 old = *(const f32x4 *)dqp;
+            if (!result) {
+                const f32x4 old = *(const f32x4 *)dqp;
 #pragma unroll
-            for (int e = 0; e < 4; e++) val[e] += old[e];
+                for (int e = 0; e < 4; e++) val[e] += old[e];
+            }
             *(f32x4 *)dqp = val;
         }
         dqp += ROWS_PER_IT * dqs1;
@@ -3844,12 +3861,13 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     if (a->B <= 0 || a->Hq <= 0 || a->Hkv <= 0 || a->Sq <= 0 || a->Hq % a->Hkv) return LTR_EINVAL;
     if (a->n_chunks < 1 || a->n_chunks > LTR_MAX_CHUNKS) return LTR_EINVAL;
     if (flags & ~(LTR_CAUSAL | LTR_NO_DQ | LTR_NO_DKDV | LTR_DQ_BF16 | LTR_DELTA_FROM_O | LTR_DKDV_BF16 | LTR_ROPE_DQ | LTR_DKDV_KEYS_128 |
-                  LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR | LTR_HEAD_COLS))
+                  LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR | LTR_HEAD_COLS | LTR_DQ_F32_RESULT))
         return LTR_EINVAL;
     if ((flags & LTR_BWD_F32_SCALAR) && a->io_dtype != LTR_F32) return LTR_EUNSUP;
+    if ((flags & LTR_DQ_F32_RESULT) && (a->io_dtype != LTR_F32 || (flags & LTR_BWD_F32_SCALAR))) return LTR_EUNSUP;
     if ((flags & LTR_DKDV_KEYS_128) && (flags & LTR_DKDV_KEYS_256)) return LTR_EINVAL;
     if ((flags & LTR_DQ_ROWS_256) && (flags & LTR_DQ_ROWS_512)) return LTR_EINVAL;
-    const bool fused_delta = flags & LTR_DELTA_FROM_O;
+    const bool fused_delta = flags & (LTR_DELTA_FROM_O | LTR_DQ_F32_RESULT);
     if (fused_delta && (!do_dq || !a->o)) return LTR_EINVAL;
     const int D = head_width(a->D, flags);
     const bool pad = D != a->D;
@@ -3871,8 +3889,8 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     for (int i = 0; i < 3; i++)
         if (a->dq_stride[i] < 0) return LTR_EINVAL;
     if (do_dq && !strides_ok(a->dq_stride, (flags & LTR_DQ_BF16) ? 2 : 4)) return LTR_EALIGN;
-    if (fused_delta && (!aligned16(a->o) || !strides_ok(a->o_stride, 2))) return LTR_EALIGN;
-    if (fused_delta && (a->Sq + 64) * a->o_stride[1] >= 0x7fffffffLL) return LTR_EUNSUP;
+    if (fused_delta && (!aligned16(a->o) || !strides_ok(a->o_stride, eb))) return LTR_EALIGN;
+    if (fused_delta && !f32 && (a->Sq + 64) * a->o_stride[1] >= 0x7fffffffLL) return LTR_EUNSUP;
     if ((a->Sq + 63) / 64 > BwdLds<128, 1>::MAX_QTILES) return LTR_EUNSUP;       // q tile lists live in LDS
     if ((a->Sq + 64) * a->q_stride[1] >= 0x7fffffffLL || (a->Sq + 64) * a->do_stride[1] >= 0x7fffffffLL) return LTR_EUNSUP;
     BwdParams p;

@@ -188,9 +188,12 @@ struct ChunksFunction {
                 for (int64_t t = 0; t < n_t; t++) dk[t].zero_(), dv[t].zero_();
             return out;
         }
-        // one launch sees every chunk: dQ is written as bf16 by the kernel; otherwise it accumulates in fp32
-        const bool direct = !f32 && n <= LTR_MAX_CHUNKS, delta_from_o = !f32 && o.scalar_type() == at::kBFloat16;
-        Tensor dq = direct ? torch::empty({B, Sq, Hq, D}, q.options()) : torch::zeros({B, Sq, Hq, D}, q.options().dtype(at::kFloat));
+        // one launch sees every chunk: dQ is written by the kernel; otherwise it accumulates in fp32
+        const bool direct = !f32 && n <= LTR_MAX_CHUNKS;
+        const bool direct32 = f32 && n <= LTR_MAX_CHUNKS && o.scalar_type() == at::kFloat && (o.stride(0) | o.stride(1) | o.stride(2)) % 4 == 0 &&
+                              (uintptr_t)o.data_ptr() % 16 == 0;
+        const bool delta_from_o = direct32 || (!f32 && o.scalar_type() == at::kBFloat16);
+        Tensor dq = direct || direct32 ? torch::empty({B, Sq, Hq, D}, q.options()) : torch::zeros({B, Sq, Hq, D}, q.options().dtype(at::kFloat));
         Tensor delta = torch::empty({B, Hq, Sq}, lse.options());   // with delta_from_o a workspace: filled by the dQ kernel
         if (!delta_from_o) {
             ltr_attn_delta_args d{};
@@ -251,7 +254,7 @@ struct ChunksFunction {
             }
             // this node holds every key these rows see and every row of it that sees these keys: the kernels write bf16 results
             a.flags = cols | (c.causal ? LTR_CAUSAL : 0u) | (direct ? LTR_DQ_BF16 : 0u) | (!f32 && !own_acc ? LTR_DKDV_BF16 : 0u) |
-                      (delta_from_o && first == 0 ? LTR_DELTA_FROM_O : 0u) | (rope.defined() ? LTR_ROPE_DQ : 0u);
+                      (direct32 ? LTR_DQ_F32_RESULT : delta_from_o && first == 0 ? LTR_DELTA_FROM_O : 0u) | (rope.defined() ? LTR_ROPE_DQ : 0u);
             // few key tiles: blocks share them and leave partial sums in a workspace (from torch's caching allocator)
             int64_t part_bytes = 0;
             check_rc(ltr_attn_bwd_workspace(&a, &part_bytes), "ltr_attn_bwd_workspace");
