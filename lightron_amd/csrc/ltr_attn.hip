@@ -124,6 +124,8 @@ struct BwdParams {
     unsigned flags;
     int n_chunks;
     int tiles_total;  // key tiles over all chunks
+    int tiles_seen;   // those that have blocks in the dK/dV kernel: all of them, or (shared tiles, causal mask) those a query sees
+    int q_last;       // largest position that counts as a query's for that: see seen_tiles
     int split_log2;   // log2 of the blocks that share one key tile of the dK/dV kernel (0: a block owns its keys alone), see KvSplit
     int share_log2;   // log2 of those that share out the q tiles of a head; the others share out the group's q heads,
     int n_reps;       // of which a block walks this many
@@ -1544,6 +1546,14 @@ __device__ __forceinline__ void store_partial(float *dst, int lane, const f32x16
         }
 }
 
+// Key tiles of a chunk that have blocks: those up to position q_last.  Blocks that share a tile leave partial sums, so a tile that no
+// query sees gets neither blocks nor a place in the workspace (the reduction kernel alone visits it); q_last is the largest
+// int where every tile has its one block.
+__host__ __device__ __forceinline__ int seen_tiles(int sk, int pos0, int q_last, int keys) {
+    const long long seen = (long long)q_last - pos0 + 1;
+    return seen <= 0 ? 0 : ((int)(seen < sk ? seen : sk) + keys - 1) / keys;
+}
+
 template <int D, int KW, bool PAD>
 __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
     const int cols = PAD ? p.cols : D;
@@ -1565,7 +1575,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
     int idx = blockIdx.x, pair, rest;
     const int P = p.B * p.Hkv;
     if ((P & 7) == 0) {
-        const int xcd = idx & 7, j = idx >> 3, n = p.tiles_total << p.split_log2;
+        const int xcd = idx & 7, j = idx >> 3, n = p.tiles_seen << p.split_log2;
         pair = (j / n) * 8 + xcd;
         rest = j % n;
     } else {
@@ -1578,7 +1588,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
     int c = 0, kt = tile;
     for (; c < p.n_chunks; c++) {
-        int n = (p.chunk[c].sk + BN - 1) / BN;
+        const int n = seen_tiles(p.chunk[c].sk, p.chunk[c].pos0, p.q_last, BN);
         if (kt < n) break;
         kt -= n;
     }
@@ -1600,7 +1610,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
         q_pos_range(0, (int)p.Sq - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], q_lo, q_hi);
         if (q_hi < tile_kpos_lo) {
             for (int k = 0; k < KW; k++)
-            if ((p.flags & LTR_DKDV_BF16) && p.split_log2 == 0 && key_ok[k]) {   // results, not accumulators: these keys get zeros
+            if ((p.flags & LTR_DKDV_BF16) && key_ok[k]) {   // results, not accumulators: these keys get zeros
                 __bf16 *gz = p_role ? (__bf16 *)p.chunk[c].dv + b * p.dvs[0] + (long long)my_key[k] * p.dvs[1] + hkv * p.dvs[2]
                                     : (__bf16 *)p.chunk[c].dk + b * p.dks[0] + (long long)my_key[k] * p.dks[1] + hkv * p.dks[2];
                 for (int d = 8 * hh; d < cols; d += 16) *(uint4 *)(gz + d) = make_uint4(0, 0, 0, 0);
@@ -2001,7 +2011,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
     run_pass(std::true_type{});
 
     if (p.split_log2) {   // a share of the keys' gradients: stored as it lies in registers, summed by the reduction kernel
-        float *const part = p.part + (((((long long)pair * p.tiles_total + tile) << p.split_log2) + split) * 8 + w) * (KW * 32 * D);
+        float *const part = p.part + (((((long long)pair * p.tiles_seen + tile) << p.split_log2) + split) * 8 + w) * (KW * 32 * D);
         const float mul = p_role ? 1.f : p.scale;
 #pragma unroll
         for (int k = 0; k < KW; k++) store_partial<D>(part + k * 32 * D, lane, acc[k], mul);
@@ -2083,21 +2093,17 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const BwdParams p)
     const int half = item % (D / 64), k = (item / (D / 64)) % KW, slot = item / (D / 64 * KW);
     const bool is_dv = slot < 4;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
-    int c = 0, kt = tile;
+    int c = 0, kt = tile, first = 0;   // first: tiles with partials in the chunks before
     for (; c < p.n_chunks; c++) {
         const int n = (p.chunk[c].sk + BN - 1) / BN;
         if (kt < n) break;
         kt -= n;
+        first += seen_tiles(p.chunk[c].sk, p.chunk[c].pos0, p.q_last, BN);
     }
     if (c >= p.n_chunks) return;
     const int sk = p.chunk[c].sk, key_base = kt * BN + (slot & 3) * 32 * KW + 32 * k;
     const bool out_bf16 = (p.flags & LTR_DKDV_BF16) != 0;
-    bool seen = true;
-    if (p.flags & LTR_CAUSAL) {   // a tile that no query sees: its blocks left nothing
-        int q_lo, q_hi;
-        q_pos_range(0, p.Sq - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], q_lo, q_hi);
-        seen = q_hi >= p.chunk[c].pos0 + kt * BN;
-    }
+    const bool seen = kt < seen_tiles(sk, p.chunk[c].pos0, p.q_last, BN);   // else: a tile without blocks, nothing but zeros to store
     if (key_base >= sk || (!seen && !out_bf16)) return;
     f32x16 acc[2];
 #pragma unroll
@@ -2105,7 +2111,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const BwdParams p)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
     if (seen) {
-        const float *src = p.part + ((((long long)pair * p.tiles_total + tile) << p.split_log2) * 8 + slot) * (KW * 32 * D) + k * 32 * D + half * 2048;
+        const float *src = p.part + ((((long long)pair * p.tiles_seen + first + kt) << p.split_log2) * 8 + slot) * (KW * 32 * D) + k * 32 * D + half * 2048;
         for (int s = 0; s < 1 << p.split_log2; s++, src += 8 * KW * 32 * D)
 #pragma unroll
             for (int i = 0; i < 8; i++) {
@@ -2978,7 +2984,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_f32_mfma_kernel(const BwdParams 
     const int split = rest & (step - 1), tile = rest >> p.split_log2;
     int c = 0, kt = tile;
     for (; c < p.n_chunks; c++) {
-        const int n = (p.chunk[c].sk + BN - 1) / BN;
+        const int n = seen_tiles(p.chunk[c].sk, p.chunk[c].pos0, p.q_last, BN);
         if (kt < n) break;
         kt -= n;
     }
@@ -3132,7 +3138,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_f32_mfma_kernel(const BwdParams 
         it = nxt;
     }
     if (p.split_log2) {   // a share of the keys' gradients, summed by the reduction kernel
-        float *const part = p.part + (((((long long)pair * p.tiles_total + tile) << p.split_log2) + split) * 8 + w) * (32 * D);
+        float *const part = p.part + (((((long long)pair * p.tiles_seen + tile) << p.split_log2) + split) * 8 + w) * (32 * D);
         store_partial<D>(part, lane, dvacc, 1.f);
         store_partial<D>(part + 4 * 32 * D, lane, dkacc, p.scale);
         return;
@@ -3499,7 +3505,10 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
 // fp32, 4/16 heads, D=128, S=700: 870, 445, 233, 128, 83 (n=16).
 struct KvSplit {
     int n, reps;      // blocks per key tile; how many of them share out the q heads (the largest power of two that divides both)
+    int q_last;       // n > 1: the tiles that have blocks, see seen_tiles
+    long long tiles;  // and how many of them there are for one (batch, kv head)
 };
+constexpr double MAX_PART_BYTES = 512e6;   // of partial sums
 struct KvSplitCost {
     int rows;                        // q rows per step
     double step_us, fixed;           // time of a step; a block's fixed part in steps
@@ -3514,19 +3523,20 @@ KvSplit kv_split(const KvSplitCost &cost, int D, int keys, bool causal, int B, i
                    std::min<long long>(std::max<long long>(q_pos0[1] + (long long)(Sq - q_split) - kpos, 0), Sq - q_split);
         return (rows + cost.rows - 1) / cost.rows;
     };
-    const long long q_last = std::max(q_split > 0 ? q_pos0[0] + (long long)q_split - 1 : -1,
-                                      Sq > q_split ? q_pos0[1] + (long long)(Sq - q_split) - 1 : -1);
+    int q_last = 0x7fffffff;
+    if (causal)
+        q_last = std::max(q_split > 0 ? q_pos0[0] + q_split - 1 : (int)0x80000000, Sq > q_split ? q_pos0[1] + (Sq - q_split) - 1 : (int)0x80000000);
     long long tiles = 0, longest = 0;
     double total = 0;
     for (int c = 0; c < n_chunks; c++) {
-        const long long seen = causal ? std::min<long long>(chunk[c].sk, q_last - chunk[c].pos0 + 1) : chunk[c].sk;
-        if (seen <= 0) continue;
-        const long long n = (seen + keys - 1) / keys, first = steps_at(chunk[c].pos0), last = steps_at(chunk[c].pos0 + (n - 1) * keys);
+        const long long n = seen_tiles(chunk[c].sk, chunk[c].pos0, q_last, keys);
+        if (n == 0) continue;
+        const long long first = steps_at(chunk[c].pos0), last = steps_at(chunk[c].pos0 + (n - 1) * keys);
         tiles += n;
         total += 0.5 * n * (first + last);
         longest = std::max(longest, first);
     }
-    KvSplit best{1, 1};
+    KvSplit best{1, 1, q_last, tiles};
     if (tiles == 0) return best;
     const double cus = device_cus(), blocks = (double)tiles * B * Hkv, avg = total / tiles * n_rep, most = (double)longest * n_rep;
     double best_us = 0;
@@ -3536,7 +3546,7 @@ KvSplit kv_split(const KvSplitCost &cost, int D, int keys, bool causal, int B, i
         const double bytes = blocks * n * keys * D * 8.0;
         double us = launch * cost.step_us;
         if (n > 1) us += 2.0 + 2.0 * bytes / cost.part_bytes_per_us;   // 2 us: the reduction's launch
-        if (n == 1 || (us < best_us && bytes <= 512e6)) {
+        if (n == 1 || (us < best_us && bytes <= MAX_PART_BYTES)) {
             best_us = us;
             best.n = n;
         }
@@ -3563,13 +3573,13 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
                  int n_chunks, bool may_split = false) {
     BwdPlan pl;
     pl.f32_ks = 0;
-    pl.split = KvSplit{1, 1};
+    pl.split = KvSplit{1, 1, 0x7fffffff, 0};
     pl.part_bytes = 0;
     pl.dq_ks = 1;
     may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
     auto split_keys = [&](const KvSplitCost &cost) {
         if (may_split) pl.split = kv_split(cost, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks);
-        if (pl.split.n > 1) pl.part_bytes = (int64_t)pl.kv_blocks * pl.split.n * pl.keys_per_block * D * 2 * 4;
+        if (pl.split.n > 1) pl.part_bytes = (int64_t)pl.split.tiles * B * Hkv * pl.split.n * pl.keys_per_block * D * 2 * 4;
     };
     if (f32) {
         pl.wide_kv = pl.wide_q = false;
@@ -3955,10 +3965,13 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     p.n_chunks = a->n_chunks;
     p.cols = a->D;
     BwdPlan pl = plan_bwd(D, f32, flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks, work != nullptr);
-    if (pl.part_bytes > work_bytes) pl.split = KvSplit{1, 1};
-    const long long kv_grid = pl.kv_blocks * pl.split.n, reduce_grid = pl.kv_blocks * (pl.keys_per_block / 128) * (D / 32);
+    if (pl.part_bytes > work_bytes) pl.split.n = pl.split.reps = 1;
+    p.q_last = pl.split.n > 1 ? pl.split.q_last : 0x7fffffff;
+    const long long tiles_seen = pl.split.n > 1 ? pl.split.tiles : pl.kv_tiles;
+    const long long kv_grid = tiles_seen * p.B * p.Hkv * pl.split.n, reduce_grid = pl.kv_blocks * (pl.keys_per_block / 128) * (D / 32);
     if (kv_grid > 0x7fffffffLL || reduce_grid > 0x7fffffffLL || pl.dq_blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.tiles_total = (int)pl.kv_tiles;
+    p.tiles_seen = (int)tiles_seen;
     p.split_log2 = __builtin_ctz(pl.split.n);
     p.share_log2 = __builtin_ctz(pl.split.n / pl.split.reps);
     p.n_reps = p.n_rep / pl.split.reps;

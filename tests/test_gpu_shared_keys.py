@@ -70,3 +70,10 @@ def test_shared_key_tiles(ltr, D, Hq, Hkv, Sq, q_pos, split, chunks, causal, dty
     for got, r in zip((dk, dv), ref[3:5]):
         got = got.cpu().float() - (0.25 if f32 else 0.0)
         assert (got - r).norm() <= (1e-4 if f32 else 5e-2) * r.norm()
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,dtype", [(128, 6, 2, torch.bfloat16), (64, 8, 1, torch.bfloat16), (64, 4, 1, torch.float32)])
+def test_masked_tiles_between_shared_ones(ltr, D, Hq, Hkv, dtype):
+    """Chunks and tails of chunks that no row sees lie before and between the visible ones of the table: they have no partial sums,
+    and the visible tiles' partials are numbered without them."""
+    test_shared_key_tiles(ltr, D, Hq, Hkv, 300, (40, 700), 130, [(300, 2000), (128, 0), (140, 3000), (520, 500), (77, 1500), (64, 128)], True, dtype, None)
