@@ -17,6 +17,8 @@ from . import attention
 from .attention import block_attention
 from .layers import rope_one, rope_table
 
+_CUS = 256               # of an MI355X
+_MAX_BWD_ROWS = 4096 * 64    # q rows of one backward launch: its lists of 64-row q tiles hold 4096
 
 class LocalCPGroup:
     """Stand-in for the cp ProcessGroup: `world_size` ranks emulated by one process."""
@@ -104,7 +106,8 @@ class ContextParallelAttention(nn.Module):
     literal=True follows the reference step by step (three seq->head exchanges, RoPE on the
     global sequence, causal attention on [B, S, H/W, D], head->seq exchange).  The default
     path gives the same result without the exchanges, which cancel: the shards are attended as
-    the one sequence they are, all heads in one launch.
+    the one sequence they are, all heads in one launch, or each
+    against the shards as the kernel's chunk table (_one_sequence).
     """
 
     def __init__(self, local_attn_module, args, cp_group=None, literal: bool = False, causal: bool = True):
@@ -150,10 +153,12 @@ class ContextParallelAttention(nn.Module):
             o = o.view(W, B, S_global, H // W, D)
             o = _all_to_all(o, 1, 2, self.cp_group)              # [W, B, S_local, H, D]
             return self.local_attn.wo(o.flatten(3))
+        if not self._one_sequence(x, S_global):
+            return self._per_shard(x, fc)
         # The shards follow each other in the sequence, so the ranks' work is one attention over all of it: one launch per
-        # kernel instead of one per shard (whose dK / dV autograd would have to add up), and with one batch entry the shards are
-        # that sequence in memory already.  RoPE at global positions (:215-219): K in one streaming pass; q inside the attention
-        # kernel, dQ rotated back in the dQ kernel's epilogue (bf16; fp32 inputs take the streaming pass for q as well)
+        # kernel instead of one per shard (whose dK / dV autograd would have to add up).  RoPE at global positions (:215-219): K
+        # in one streaming pass; q inside the attention kernel, dQ rotated back in the dQ kernel's epilogue (bf16; fp32 inputs
+        # take the streaming pass for q as well)
         xs = x.transpose(0, 1).reshape(B, S_global, -1)
         xq = self.local_attn.wq(xs).view(B, S_global, H, D)
         xk = rope_one(self.local_attn.wk(xs).view(B, S_global, Hkv, D), fc)
@@ -164,3 +169,50 @@ class ContextParallelAttention(nn.Module):
         y = self.local_attn.wo(o.reshape(B, S_global, -1))
         return y.view(B, W, S_local, -1).transpose(0, 1).contiguous()
 
+    def _one_sequence(self, x, S_global) -> bool:
+        """Whether the shards are attended as one sequence, or one launch per shard against the shards as KV chunks.
+
+        With one batch entry the shards are that sequence in memory already.  With more, joining them and splitting the result
+        are two passes over the activations where per-shard launches pay one (their outputs are stacked).  In training the
+        fewer launches and the dK / dV that need no adding up always pay for it (0.48 - 1.00 of the per-shard time at 244 shapes of
+        2 and 4 ranks, batch 1 - 16, 37 - 2048 tokens per rank, 12 - 32 heads; 0.78 - 1.00 from 5 ms on).  Forward
+        only, they pay while the extra launches cost more than the pass, 12 us each at 4 TB/s, or leave CUs idle.  us,
+        sequence / per shard:
+            W=2 B=8  16 heads D=128 1024 tokens per rank   688 / 657     W=4 B=16 16 heads D=64 (4 kv)  128      132 / 186
+            W=2 B=8  16 heads D=64 (4 kv) 1024             254 / 234     W=4 B=4  32 heads D=64         128      129 / 185
+            W=2 B=8  12 heads D=64 2048 (idle CUs)         566 / 606     W=2 B=2  16 heads D=64 (4 kv) 2048      185 / 196
+        A sequence longer than the backward's q tile lists, or whose rows lie further apart than the kernels' 32-bit tile
+        offsets reach, is attended shard by shard."""
+        W, B = x.shape[0], x.shape[1]
+        attn = self.local_attn
+        trained = torch.is_grad_enabled() and (x.requires_grad or any(not isinstance(m, nn.Module) or any(p.requires_grad for p in m.parameters())
+                                                                       for m in (attn.wq, attn.wk, attn.wv, attn.wo)))
+        if (S_global + 64) * max(self.num_heads, self.num_kv_heads) * self.head_dim >= 0x7fffffff or (trained and S_global > _MAX_BWD_ROWS):
+            return False
+        if B == 1 or trained:
+            return True
+
+        def fill(rows):     # of the CUs, by blocks of 256 rows (under a causal mask a late one and an early one together)
+            blocks = B * self.num_heads * -(-rows // 256)
+            blocks = -(-blocks // 2) if self.causal and blocks > _CUS else max(blocks, _CUS)
+            return blocks / (-(-blocks // _CUS) * _CUS)
+
+        activation = B * S_global * self.num_heads * self.head_dim * x.element_size()
+        return 2 * activation < 48e6 * (W - 1) or fill(S_global // W) < fill(S_global)
+
+    def _per_shard(self, x, fc):
+        W, B, S_local, _ = x.shape
+        H, Hkv, D = self.num_heads, self.num_kv_heads, self.head_dim
+        xq = self.local_attn.wq(x).view(W, B, S_local, H, D)
+        xk = self.local_attn.wk(x).view(W, B, S_local, Hkv, D)
+        xv = self.local_attn.wv(x).view(W, B, S_local, Hkv, D)
+        fused = xq.dtype == torch.bfloat16
+        table = rope_table(fc, xq.device) if fused else None
+        rows = [fc[j * S_local:(j + 1) * S_local] for j in range(W)]
+        qs = [xq[j] if fused else rope_one(xq[j], rows[j]) for j in range(W)]
+        ks = [rope_one(xk[j], rows[j]) for j in range(W)]       # every K shard once: it is read by every later q shard
+        vs, pos, outs = list(xv.unbind(0)), [j * S_local for j in range(W)], []
+        for j in range(W):
+            n = j + 1 if self.causal else W                     # later shards are fully masked
+            outs.append(block_attention(qs[j], ks[:n], vs[:n], pos[:n], pos[j], None, self.causal, q_rope=table)[0])
+        return self.local_attn.wo(torch.stack(outs, 0).flatten(3))
