@@ -132,7 +132,9 @@ typedef struct ltr_attn_fwd_args {
      * MFMA operand, by the angles of its GLOBAL position; no separate pass over q.  rope_freqs: the table of
      * precompute_freqs_cis as interleaved fp32 (cos, sin), [rope_len][D/2][2], row 0 = position rope_pos0; it must
      * cover every position of the local rows.  The rotated row has the bits ltr_rope_apply would have written.
-     * q_rot (optional, bf16, own strides): receives the rotated q, which is what ltr_attn_bwd takes as q.
+     * q_rot (optional, bf16, own strides): receives the rotated q, which is what ltr_attn_bwd takes as q.  It may be q
+     * itself with q's strides (rotated in place; a later call of the same q must then come without LTR_ROPE_Q), but must not
+     * overlap it otherwise.
      * K is NOT rotated here: a K row is read by every q block that sees it, so its rotation belongs before the
      * attention (one ltr_rope_apply per K tensor), not inside it. */
     const float *rope_freqs;

@@ -3440,7 +3440,7 @@ struct FwdPlan {
     long long blocks;
 };
 FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
-                 int n_chunks) {
+                 int n_chunks, bool may_share = true) {
     FwdPlan pl;
     pl.f32_ks = 0;
     pl.ks = 1;
@@ -3467,7 +3467,7 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     // the dQ kernel's 512-row blocks (see plan_bwd)
     bool wide = (flags & LTR_FWD_ROWS_512) != 0;
     ShareChoice shares{1, false};
-    if (!wide && !(flags & LTR_FWD_ROWS_256))
+    if (!wide && !(flags & LTR_FWD_ROWS_256) && may_share)
         shares = key_shares(D == 128 ? FWD_SHARES_128 : FWD_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
                             n_chunks);
     pl.ks = shares.ks;
@@ -3788,7 +3788,9 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     hipStream_t st = (hipStream_t)stream;
     if ((a->flags & LTR_FWD_ROWS_512) && (a->D != 64 || a->io_dtype != LTR_BF16)) return LTR_EUNSUP;
     p.cols = a->D;
-    const FwdPlan pl = plan_fwd(D, a->io_dtype == LTR_F32, pad ? a->flags : a->flags & ~LTR_HEAD_COLS, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks);
+    const FwdPlan pl = plan_fwd(D, a->io_dtype == LTR_F32, pad ? a->flags : a->flags & ~LTR_HEAD_COLS, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks,
+                                // q rotated in place: a row is read and written by one wave only without key shares
+                                !p.q_rot || p.q_rot != p.q);
     if (pl.blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.n_qtiles = pl.n_qtiles;
     p.n_slots = pl.n_slots;
