@@ -1424,12 +1424,13 @@ __global__ __launch_bounds__(256) void fwd_f32_mfma_kernel(const FwdParams p) {
 }
 
 // ------------------------------------------------------------------------------ delta
-// 16 lanes per (b, row, h), 8 elements per lane: rows of one sequence index are read head after head, as they lie in memory.
+// 16 lanes per (b, row, h), 8 elements per lane in two sums of four: rows of one sequence index are read head after head, as they
+// lie in memory.
 __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
     const long long rowid = ((long long)blockIdx.x * 256 + threadIdx.x) >> 4;
     const int d = 8 * (threadIdx.x & 15);
     const long long nrows = (long long)p.B * p.Hq * p.Sq;
-    float acc = 0.f;
+    float acc = 0.f, acc_hi = 0.f;
     int i = 0, h = 0, b = 0;
     if (rowid < nrows) {
         const unsigned bi = (unsigned)(rowid / p.Hq);   // b * Sq + i: below 2^31 (checked by the host)
@@ -1454,7 +1455,8 @@ __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
             load8(p.o, oo, p.o_f32, ov);
             load8(p.d_o, od, p.do_f32, dv);
 #pragma unroll
-            for (int e = 0; e < 8; e++) acc = fmaf(ov[e], dv[e], acc);
+            for (int e = 0; e < 4; e++) acc = fmaf(ov[e], dv[e], acc), acc_hi = fmaf(ov[4 + e], dv[4 + e], acc_hi);
+            acc += acc_hi;
         }
     }
 #pragma unroll
@@ -2800,16 +2802,18 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p)
             lse2 = lse_row == -INFINITY ? INFINITY : lse_row * LTR_LOG2E;
             if (!result) dlt = p.delta[((long long)b * p.Hq + h) * p.Sq + my_row];
         }
-        if (result) {   // the two lanes of a row hold its column groups in turn
+        if (result) {   // the two lanes of a row hold its column groups in turn: 16 sums of D / 16 terms in all, as in delta_kernel
             const float *op = (const float *)p.o + b * p.os_[0] + (long long)rs * p.os_[1] + h * p.os_[2];
-            float part = 0.f;
+            float sum[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) sum[i] = 0.f;
 #pragma unroll
             for (int g = 0; g < D / 8; g++) {
                 const f32x4 x = *(const f32x4 *)(op + 8 * g + 4 * hh);
 #pragma unroll
-                for (int j = 0; j < 4; j++) part = fmaf(x[j], doreg[4 * g + j], part);
+                for (int j = 0; j < 4; j++) sum[(g & 1) * 4 + j] = fmaf(x[j], doreg[4 * g + j], sum[(g & 1) * 4 + j]);
             }
-            part = xhalf_sum(part);
+            const float part = xhalf_sum(((sum[0] + sum[1]) + (sum[2] + sum[3])) + ((sum[4] + sum[5]) + (sum[6] + sum[7])));
             if (row_ok) dlt = part;
             if (row_ok && hh == 0 && ks == 0) p.delta[((long long)b * p.Hq + h) * p.Sq + my_row] = part;
         }
