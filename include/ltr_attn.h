@@ -312,8 +312,11 @@ int ltr_copy_strided(const ltr_copy_args *args, void *stream);
  * for 256 compute units).  It has no counterpart in the reference (which leaves the choice of kernel to the library
  * behind F.scaled_dot_product_attention, model/model.py:193); it is for benchmarks and profiles that must name the kernel
  * they measured, and for tests of the size hints.  The sizes, strides' owner shapes, positions, chunk lengths, dtype and
- * flags of args are read; flags may also carry the forward's hints (LTR_FWD_ROWS_256 / LTR_FWD_ROWS_512 / LTR_FWD_F32_SCALAR).  The library's
- * launches and this answer come from one function, so they cannot drift apart.  Kernel names are those a profiler shows.
+ * flags of args are read; flags may also carry the forward's hints (LTR_FWD_ROWS_256 / LTR_FWD_ROWS_512 / LTR_FWD_F32_SCALAR) and
+ * LTR_HEAD_COLS.  The library's launches and this answer come from one function, so they cannot drift apart (a forward that
+ * rotates q in place, see q_rot, takes one wave per row group where the plan may name key shares).  Kernel names are those a
+ * profiler shows.  ltr_attn_plan_ws is the plan of ltr_attn_fwd and of ltr_attn_bwd_ws with a workspace of workspace_bytes: dkdv_blocks
+ * then counts the blocks that share key tiles, and the kernel that sums their partial results is named beside them.
  */
 typedef struct ltr_attn_plan_t {
     int32_t compute_units;   /* CUs the choices were made for */
@@ -327,6 +330,15 @@ typedef struct ltr_attn_plan_t {
 } ltr_attn_plan_t;
 
 int ltr_attn_plan(const ltr_attn_bwd_args *args, ltr_attn_plan_t *out);
+
+typedef struct ltr_attn_plan_ws_t {
+    ltr_attn_plan_t plan;
+    int32_t blocks_per_tile;  /* dK/dV blocks that share a key tile; 1: none do, and no reduction runs */
+    int64_t reduce_blocks;
+    char reduce_kernel[48];   /* empty without a reduction */
+} ltr_attn_plan_ws_t;
+
+int ltr_attn_plan_ws(const ltr_attn_bwd_args *args, int64_t workspace_bytes, ltr_attn_plan_ws_t *out);
 
 int ltr_abi_version(void);
 const char *ltr_strerror(int code);

@@ -22,7 +22,7 @@ LTR_BWD_F32_SCALAR = 65536
 LTR_HEAD_COLS = 131072
 LTR_DQ_F32_RESULT = 262144
 
-EXPORTS = ("ltr_attn_fwd", "ltr_attn_bwd_delta", "ltr_attn_bwd", "ltr_attn_bwd_ws", "ltr_attn_bwd_workspace", "ltr_attn_bwd_noalloc", "ltr_attn_plan", "ltr_cast_f32_to_bf16",
+EXPORTS = ("ltr_attn_fwd", "ltr_attn_bwd_delta", "ltr_attn_bwd", "ltr_attn_bwd_ws", "ltr_attn_bwd_workspace", "ltr_attn_bwd_noalloc", "ltr_attn_plan", "ltr_attn_plan_ws", "ltr_cast_f32_to_bf16",
            "ltr_rope_apply", "ltr_copy_strided", "ltr_abi_version", "ltr_strerror")
 # the bench-only measurement library (include/ltr_probe.h); not part of the attention path
 PROBE_LIB_PATH = os.path.join(HERE, "csrc", "libltr_probe.so")
@@ -94,6 +94,10 @@ class AttnPlan(ctypes.Structure):
                 ("fwd_kernel", ctypes.c_char * 48), ("dq_kernel", ctypes.c_char * 48), ("dkdv_kernel", ctypes.c_char * 48)]
 
 
+class AttnPlanWs(ctypes.Structure):
+    _fields_ = [("plan", AttnPlan), ("blocks_per_tile", ctypes.c_int32), ("reduce_blocks", ctypes.c_int64), ("reduce_kernel", ctypes.c_char * 48)]
+
+
 LTR_PROBE_MIN_WORKSPACE = 8192 + 65536
 
 _lib = None
@@ -128,6 +132,8 @@ def load():
     lib.ltr_rope_apply.restype = ctypes.c_int
     lib.ltr_attn_plan.argtypes = [ctypes.POINTER(BwdArgs), ctypes.POINTER(AttnPlan)]
     lib.ltr_attn_plan.restype = ctypes.c_int
+    lib.ltr_attn_plan_ws.argtypes = [ctypes.POINTER(BwdArgs), ctypes.c_int64, ctypes.POINTER(AttnPlanWs)]
+    lib.ltr_attn_plan_ws.restype = ctypes.c_int
     lib.ltr_abi_version.argtypes = []
     lib.ltr_abi_version.restype = ctypes.c_int
     lib.ltr_strerror.argtypes = [ctypes.c_int]

@@ -316,16 +316,20 @@ def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_a
 
 def attn_plan(B: int, Hq: int, Hkv: int, D: int, Sq: int, chunk_lens: Sequence[int], k_pos0: Sequence[int], q_pos0=0,
               q_split: Optional[int] = None, causal: bool = False, dtype: torch.dtype = torch.bfloat16, fwd_rows=None,
-              dq_rows=None, dkdv_keys=None, f32_scalar: bool = False) -> dict:
+              dq_rows=None, dkdv_keys=None, f32_scalar: bool = False, share_keys: bool = False) -> dict:
     """Which kernels the library would launch for this problem on the current device (ltr_attn_plan: a host call, no
     tensors needed; at most 32 chunks = one launch): block sizes, block counts and the kernels' names as a profiler
-    shows them.  fwd_rows / dq_rows / dkdv_keys force a size like the arguments of attn_fwd / attn_bwd_accumulate."""
+    shows them.  fwd_rows / dq_rows / dkdv_keys force a size like the arguments of attn_fwd / attn_bwd_accumulate.
+    share_keys: the backward gets the workspace it asks for, as in block_attention's backward: "dkdv" then also names the
+    blocks that share a key tile and, where any do, the kernel that sums their partial dK / dV."""
     lib = _lib.load()
     a = _lib.BwdArgs()
     a.B, a.Hq, a.Hkv, a.D, a.Sq, a.n_chunks = B, Hq, Hkv, D, Sq, len(chunk_lens)
     a.q_pos0, a.q_split = _qpos(q_pos0, Sq, q_split)
     a.io_dtype = _DT[dtype]
     a.flags = (_lib.LTR_CAUSAL if causal else 0) | ((_lib.LTR_FWD_F32_SCALAR | _lib.LTR_BWD_F32_SCALAR) if f32_scalar else 0)
+    if D not in (64, 128) and dtype == torch.bfloat16:
+        a.flags |= _lib.LTR_HEAD_COLS
     for val, lo, hi, name in ((fwd_rows, _lib.LTR_FWD_ROWS_256, _lib.LTR_FWD_ROWS_512, "fwd_rows"),
                               (dq_rows, _lib.LTR_DQ_ROWS_256, _lib.LTR_DQ_ROWS_512, "dq_rows"),
                               (dkdv_keys, _lib.LTR_DKDV_KEYS_128, _lib.LTR_DKDV_KEYS_256, "dkdv_keys")):
@@ -336,12 +340,18 @@ def attn_plan(B: int, Hq: int, Hkv: int, D: int, Sq: int, chunk_lens: Sequence[i
             a.flags |= lo if val == sizes[0] else hi
     for i, (sk, p0) in enumerate(zip(chunk_lens, k_pos0)):
         a.chunk[i].sk, a.chunk[i].pos0 = int(sk), int(p0)
-    out = _lib.AttnPlan()
-    _lib.check(lib.ltr_attn_plan(ctypes.byref(a), ctypes.byref(out)), "ltr_attn_plan")
-    return {"compute_units": out.compute_units,
+    ws, need = _lib.AttnPlanWs(), ctypes.c_int64(0)
+    if share_keys:
+        _lib.check(lib.ltr_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(need)), "ltr_attn_bwd_workspace")
+    _lib.check(lib.ltr_attn_plan_ws(ctypes.byref(a), need, ctypes.byref(ws)), "ltr_attn_plan")
+    out = ws.plan
+    plan = {"compute_units": out.compute_units,
             "fwd": {"kernel": out.fwd_kernel.decode(), "rows": out.fwd_rows, "paired": bool(out.fwd_paired), "blocks": out.fwd_blocks},
             "dq": {"kernel": out.dq_kernel.decode(), "rows": out.dq_rows, "paired": bool(out.dq_paired), "blocks": out.dq_blocks},
             "dkdv": {"kernel": out.dkdv_kernel.decode(), "keys": out.dkdv_keys, "blocks": out.dkdv_blocks}}
+    if share_keys:
+        plan["dkdv"].update(blocks_per_tile=ws.blocks_per_tile, reduce_kernel=ws.reduce_kernel.decode(), reduce_blocks=ws.reduce_blocks)
+    return plan
 
 
 def cast_to_bf16(src: torch.Tensor) -> torch.Tensor:

@@ -3663,6 +3663,8 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.dq_blocks = (long long)pl.dq_slots * B * Hq;
     return pl;
 }
+// blocks of bwd_dkdv_reduce_kernel: four waves each, one per 64 columns of a 32-key slice of dK or dV
+long long reduce_blocks(const BwdPlan &pl, int D) { return pl.kv_blocks * (pl.keys_per_block / 128) * (D / 32); }
 
 // every position of the local rows lies inside the rows [pos0, pos0 + len) of a RoPE table
 bool rope_table_covers(const int64_t *q_pos0, int64_t q_split, int64_t Sq, int64_t pos0, int64_t len) {
@@ -3974,7 +3976,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     if (pl.part_bytes > work_bytes) pl.split.n = pl.split.reps = 1;
     p.q_last = pl.split.n > 1 ? pl.split.q_last : 0x7fffffff;
     const long long tiles_seen = pl.split.n > 1 ? pl.split.tiles : pl.kv_tiles;
-    const long long kv_grid = tiles_seen * p.B * p.Hkv * pl.split.n, reduce_grid = pl.kv_blocks * (pl.keys_per_block / 128) * (D / 32);
+    const long long kv_grid = tiles_seen * p.B * p.Hkv * pl.split.n, reduce_grid = reduce_blocks(pl, D);
     if (kv_grid > 0x7fffffffLL || reduce_grid > 0x7fffffffLL || pl.dq_blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.tiles_total = (int)pl.kv_tiles;
     p.tiles_seen = (int)tiles_seen;
@@ -4096,20 +4098,23 @@ extern "C" int ltr_attn_bwd_workspace(const ltr_attn_bwd_args *a, int64_t *bytes
     return LTR_OK;
 }
 
-// Host-only: nothing is enqueued, no pointer is read.
-extern "C" int ltr_attn_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out) {
-    if (!a || !out) return LTR_EINVAL;
+namespace {
+// ltr_attn_plan and ltr_attn_plan_ws; ws: the plan of ltr_attn_bwd_ws with a workspace of that many bytes, or nullptr
+int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work_bytes, ltr_attn_plan_ws_t *ws) {
     if (a->B <= 0 || a->Hq <= 0 || a->Hkv <= 0 || a->Sq <= 0 || a->Hq % a->Hkv) return LTR_EINVAL;
     if (a->n_chunks < 1 || a->n_chunks > LTR_MAX_CHUNKS) return LTR_EINVAL;
-    if (a->D != 64 && a->D != 128) return LTR_EUNSUP;
+    const int D = head_width(a->D, a->flags);
+    const bool pad = D != a->D;
+    if (!D) return LTR_EUNSUP;
     if (a->io_dtype != LTR_BF16 && a->io_dtype != LTR_F32) return LTR_EUNSUP;
     if (!fits_i32(a->Sq) || a->q_split < 0 || a->q_split > a->Sq) return LTR_EINVAL;
     if (!fits_i32(a->q_pos0[0] + a->Sq) || !fits_i32(a->q_pos0[1] + a->Sq)) return LTR_EINVAL;
-    const unsigned flags = a->flags;
+    const unsigned flags = pad ? a->flags : a->flags & ~LTR_HEAD_COLS;
     if ((flags & LTR_DKDV_KEYS_128) && (flags & LTR_DKDV_KEYS_256)) return LTR_EINVAL;
     if ((flags & LTR_DQ_ROWS_256) && (flags & LTR_DQ_ROWS_512)) return LTR_EINVAL;
     if ((flags & LTR_FWD_ROWS_256) && (flags & LTR_FWD_ROWS_512)) return LTR_EINVAL;
     const bool f32 = a->io_dtype == LTR_F32;
+    if (pad && f32) return LTR_EUNSUP;
     if ((flags & (LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_512 | LTR_FWD_ROWS_512)) && (a->D != 64 || f32)) return LTR_EUNSUP;
     if ((flags & (LTR_FWD_F32_SCALAR | LTR_BWD_F32_SCALAR)) && !f32) return LTR_EUNSUP;
     ChunkDev chunk[LTR_MAX_CHUNKS];
@@ -4122,8 +4127,9 @@ extern "C" int ltr_attn_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out) {
         chunk[c].pos0 = (int)ch.pos0;
     }
     const int q_pos0[2] = {(int)a->q_pos0[0], (int)a->q_pos0[1]};
-    const FwdPlan f = plan_fwd(a->D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks);
-    const BwdPlan b = plan_bwd(a->D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks);
+    const FwdPlan f = plan_fwd(D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks);
+    const BwdPlan b = plan_bwd(D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks, work_bytes > 0);
+    const bool shared = b.split.n > 1 && b.part_bytes <= work_bytes;
     out->compute_units = device_cus();
     out->fwd_rows = f.rows;
     out->fwd_paired = f.n_slots != f.n_qtiles;
@@ -4132,25 +4138,43 @@ extern "C" int ltr_attn_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out) {
     out->dq_paired = b.dq_slots != b.dq_qtiles;
     out->dq_blocks = b.dq_blocks;
     out->dkdv_keys = b.keys_per_block;
-    out->dkdv_blocks = b.kv_blocks;
+    out->dkdv_blocks = shared ? b.split.tiles * a->B * a->Hkv * b.split.n : b.kv_blocks;
     if (f32) {
-        if (f.f32_ks) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_f32_mfma_kernel<%d, %d>", a->D, f.f32_ks);
-        else snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_f32_kernel<%d>", a->D);
+        if (f.f32_ks) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_f32_mfma_kernel<%d, %d>", D, f.f32_ks);
+        else snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_f32_kernel<%d>", D);
         if (b.f32_ks) {
-            snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_f32_mfma_kernel<%d, %d>", a->D, b.f32_ks);
-            snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_f32_mfma_kernel<%d>", a->D);
+            snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_f32_mfma_kernel<%d, %d>", D, b.f32_ks);
+            snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_f32_mfma_kernel<%d>", D);
         } else {
-            snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_f32_kernel<%d>", a->D);
-            snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_f32_kernel<%d, *>", a->D);
+            snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_f32_kernel<%d>", D);
+            snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_f32_kernel<%d, *>", D);
         }
+    } else if (pad) {
+        snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_pad_kernel<%d, %d>", D, f.ks);
+        snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_pad_kernel<%d, %d>", D, b.dq_ks);
+        snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_pad_kernel<%d>", D);
     } else {
-        if (f.ks > 1) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_shares_kernel<%d, %d>", a->D, f.ks);
-        else snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_kernel<%d, %d>", a->D, f.wide ? 2 : 1);
-        if (b.dq_ks > 1) snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_shares_kernel<%d, %d>", a->D, b.dq_ks);
-        else snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_kernel<%d, %d>", a->D, b.wide_q ? 2 : 1);
-        snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", a->D, b.wide_kv ? 2 : 1);
+        if (f.ks > 1) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_shares_kernel<%d, %d>", D, f.ks);
+        else snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_kernel<%d, %d>", D, f.wide ? 2 : 1);
+        if (b.dq_ks > 1) snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_shares_kernel<%d, %d>", D, b.dq_ks);
+        else snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_kernel<%d, %d>", D, b.wide_q ? 2 : 1);
+        snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);
+    }
+    if (ws) {
+        ws->blocks_per_tile = shared ? b.split.n : 1;
+        ws->reduce_blocks = shared ? reduce_blocks(b, D) : 0;
+        ws->reduce_kernel[0] = 0;
+        if (shared) snprintf(ws->reduce_kernel, sizeof(ws->reduce_kernel), "bwd_dkdv_reduce_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);
     }
     return LTR_OK;
+}
+}  // namespace
+
+// Host-only: nothing is enqueued, no pointer is read.
+extern "C" int ltr_attn_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out) { return a && out ? describe_plan(a, out, 0, nullptr) : LTR_EINVAL; }
+
+extern "C" int ltr_attn_plan_ws(const ltr_attn_bwd_args *a, int64_t workspace_bytes, ltr_attn_plan_ws_t *out) {
+    return a && out && workspace_bytes >= 0 ? describe_plan(a, &out->plan, workspace_bytes, out) : LTR_EINVAL;
 }
 
 extern "C" int ltr_attn_bwd_noalloc(const ltr_attn_bwd_args *a, void *stream) {
