@@ -39,6 +39,8 @@
 extern "C" {
 #endif
 
+/* Counts changes that break a caller.  Additions do not raise it: a library of the same version that is older than a caller's header
+ * lacks the entry points it does not know, and answers LTR_EINVAL to flags it does not know. */
 #define LTR_ABI_VERSION 8
 #define LTR_MAX_CHUNKS 32
 

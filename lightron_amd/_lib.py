@@ -114,6 +114,9 @@ def load():
             "lightron_amd: %s is missing - build it with `python -m lightron_amd.build` "
             "(there is no CPU or PyTorch fallback)" % LIB_PATH)
     lib = ctypes.CDLL(LIB_PATH)
+    missing = [f for f in EXPORTS if not hasattr(lib, f)]
+    if missing:         # same ABI version, but built before these were added
+        raise RuntimeError("lightron_amd: %s has no %s - build it again with `python -m lightron_amd.build`" % (LIB_PATH, ", ".join(missing)))
     lib.ltr_attn_fwd.argtypes = [ctypes.POINTER(FwdArgs), ctypes.c_void_p]
     lib.ltr_attn_fwd.restype = ctypes.c_int
     lib.ltr_attn_bwd_delta.argtypes = [ctypes.POINTER(DeltaArgs), ctypes.c_void_p]

@@ -570,7 +570,8 @@ class SingleChunkAttentionFunction(torch.autograd.Function):
 
 # A call has two host sides over the same C-ABI calls: a C++ autograd node (_ltr_node.so, built by lightron_amd.build: arguments are
 # filled and the backward runs on the autograd thread without the interpreter) and the Python Functions above.  The C++ node is
-# used when it has been built for this ABI version and the library is the in-tree one.
+# used when it has been built for this ABI version, with all of these entry points, and the library is the in-tree one.
+_NODE_CALLS = ("single_chunk", "chunks", "rope", "seq_all_to_all", "exchange")
 USE_CPP_NODE = True
 _node = None
 
@@ -582,7 +583,8 @@ def _cpp_node():
         if not os.environ.get("LTR_ATTN_LIB"):        # the node is linked against the in-tree library
             try:
                 from . import _ltr_node
-                if _ltr_node.abi_version() == _lib.LTR_ABI_VERSION:
+                # the version counts the C ABI; a node built before an entry point was added has the same
+                if _ltr_node.abi_version() == _lib.LTR_ABI_VERSION and all(hasattr(_ltr_node, f) for f in _NODE_CALLS):
                     _node = _ltr_node
             except (ImportError, OSError):       # not built, or built against another torch: the Python node serves
                 pass
