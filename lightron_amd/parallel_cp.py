@@ -17,6 +17,7 @@ from . import attention
 from .attention import block_attention
 from .layers import rope_one, rope_table
 
+_PLAIN = (torch.Tensor, nn.Parameter)
 _CUS = 256               # of an MI355X
 _MAX_BWD_ROWS = 4096 * 64    # q rows of one backward launch: its lists of 64-row q tiles hold 4096
 
@@ -45,8 +46,13 @@ def _world_size(group) -> int:
 
 
 def _exchange_node(x: torch.Tensor):
-    """The C++ binding when it can move this tensor (a GPU tensor whose bytes are its values), else None."""
-    return (attention._cpp_node() if attention.USE_CPP_NODE else None) if x.is_cuda and not (x.is_conj() or x.is_neg()) else None
+    """The C++ binding when it can move this tensor (a plain GPU tensor whose bytes are its values), else None: under tracing, a
+    dispatch mode or a tensor subclass the exchange is the torch ops below, which those see."""
+    if not x.is_cuda or x.is_conj() or x.is_neg() or type(x) not in _PLAIN or not attention.USE_CPP_NODE:
+        return None
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack():
+        return None
+    return attention._cpp_node()
 
 
 def _exchange(x: torch.Tensor, scatter_dim: int, gather_dim: int, W: int) -> torch.Tensor:
