@@ -34,19 +34,27 @@ class RingKVGrads:
         self._buf = torch.zeros(end, dtype=torch.float32, device=tensors[0].device if tensors else None)
         acc = self._views(self._buf)
         self.dk, self.dv = acc[:len(self.kv)], acc[len(self.kv):]
+        self._acc = acc
+
+    def _whole(self):
+        """The buffer while dk / dv are still its slices; None once a caller has put tensors of its own in their place."""
+        acc = [*self.dk, *self.dv]
+        return self._buf if len(acc) == len(self._acc) and all(a is b for a, b in zip(acc, self._acc)) else None
 
     def _views(self, buf):
         tensors = [k for k, _ in self.kv] + [v for _, v in self.kv]
         return [buf[a:a + t.numel()].view(t.shape) for a, t in zip(self._cuts, tensors)]
 
     def zero_(self):
-        self._buf.zero_()
+        for t in self.dk + self.dv if self._whole() is None else [self._buf]:
+            t.zero_()
 
     def finalize(self, assign: bool = True):
         """[(dK, dV)] per rank in the chunks' dtype; with assign=True also added to k.grad / v.grad of leaf tensors."""
         from .attention import cast_to_bf16
         out = []
-        grads = self._views(cast_to_bf16(self._buf)) if all(t.dtype == torch.bfloat16 for kv in self.kv for t in kv) else self.dk + self.dv
+        whole = self._whole() if all(t.dtype == torch.bfloat16 for kv in self.kv for t in kv) else None
+        grads = self._views(cast_to_bf16(whole)) if whole is not None else [*self.dk, *self.dv]
         for (k, v), dk, dv in zip(self.kv, grads[:len(self.kv)], grads[len(self.kv):]):
             gk, gv = dk.to(k.dtype), dv.to(v.dtype)
             if assign:
