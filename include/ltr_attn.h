@@ -157,7 +157,7 @@ typedef struct ltr_attn_delta_args {
     const void *o;
     const void *d_o;
     float *delta;       /* [B, Hq, Sq] */
-    int32_t B, Hq, D;
+    int32_t B, Hq, D;   /* D: a multiple of 8 up to 128 */
     int64_t Sq;
     int64_t o_stride[3];
     int64_t do_stride[3];

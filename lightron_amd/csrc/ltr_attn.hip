@@ -144,6 +144,7 @@ struct DeltaParams {
     long long os[3], dos[3];
     int o_f32, do_f32;
     int vec;           // rows start 16-byte aligned: 16-byte loads
+    int rows32;        // B * Sq < 2^31
 };
 
 __device__ __forceinline__ int q_position(int row, int split, int p0, int p1) {
@@ -1433,10 +1434,15 @@ __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
     float acc = 0.f, acc_hi = 0.f;
     int i = 0, h = 0, b = 0;
     if (rowid < nrows) {
-        const unsigned bi = (unsigned)(rowid / p.Hq);   // b * Sq + i: below 2^31 (checked by the host)
-        h = (int)(rowid - (long long)bi * p.Hq);
-        b = (int)(bi / (unsigned)p.Sq);
-        i = (int)(bi - (unsigned)b * (unsigned)p.Sq);
+        const long long bi = rowid / p.Hq;   // b * Sq + i
+        h = (int)(rowid - bi * p.Hq);
+        if (p.rows32) {   // the usual case spares the 64-bit division
+            b = (int)((unsigned)bi / (unsigned)p.Sq);
+            i = (int)((unsigned)bi - (unsigned)b * (unsigned)p.Sq);
+        } else {
+            b = (int)(bi / p.Sq);
+            i = (int)(bi - (long long)b * p.Sq);
+        }
         if (d < p.D) {
             const long long oo = b * p.os[0] + (long long)i * p.os[1] + h * p.os[2] + d;
             const long long od = b * p.dos[0] + (long long)i * p.dos[1] + h * p.dos[2] + d;
@@ -3839,7 +3845,7 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
 
 extern "C" int ltr_attn_bwd_delta(const ltr_attn_delta_args *a, void *stream) {
     if (!a || !a->o || !a->d_o || !a->delta) return LTR_EINVAL;
-    if (a->B <= 0 || a->Hq <= 0 || a->Sq <= 0 || !fits_i32(a->Sq) || !fits_i32((int64_t)a->B * a->Sq)) return LTR_EINVAL;
+    if (a->B <= 0 || a->Hq <= 0 || a->Sq <= 0 || !fits_i32(a->Sq)) return LTR_EINVAL;
     if (a->D <= 0 || a->D > 128 || a->D % 8) return LTR_EUNSUP;
     if ((a->o_dtype != LTR_BF16 && a->o_dtype != LTR_F32) || (a->do_dtype != LTR_BF16 && a->do_dtype != LTR_F32))
         return LTR_EUNSUP;
@@ -3861,6 +3867,7 @@ extern "C" int ltr_attn_bwd_delta(const ltr_attn_delta_args *a, void *stream) {
     }
     p.o_f32 = a->o_dtype == LTR_F32;
     p.do_f32 = a->do_dtype == LTR_F32;
+    p.rows32 = fits_i32((int64_t)a->B * a->Sq);
     p.vec = aligned16(a->o) && aligned16(a->d_o) && strides_ok(a->o_stride, p.o_f32 ? 4 : 2) && strides_ok(a->do_stride, p.do_f32 ? 4 : 2);
     const long long nthreads = (long long)p.B * p.Hq * p.Sq * 16;
     const long long nblk = (nthreads + 255) / 256;
