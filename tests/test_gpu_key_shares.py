@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
     (128, 1, 8, 2, 512, 0, None, [(512, 0)], True, 4),
     (128, 1, 4, 4, 33, 100, None, [(31, 0), (97, 31), (64, 90)], True, 2),            # chunks shorter than a tile of all shares
     (128, 1, 4, 2, 200, (40, 1300), 130, [(128, 0), (933, 500), (256, 4000)], True, 4), # two segments, rows that see no key, a chunk no row sees
-    (64, 8, 12, 4, 200, 0, None, [(520, 0)], False, 2),    
+    (64, 8, 12, 4, 200, 0, None, [(520, 0)], False, 2),
     (64, 1, 8, 1, 100, 0, None, [(300, 50)], True, 4),                                # the first rows see no key
     (64, 1, 4, 2, 65, 0, None, [(65, 0), (1, 65)], False, 4),
 ])
@@ -57,7 +57,15 @@ def test_key_shares_forward_backward(ltr, D, B, Hq, Hkv, Sq, q_pos, split, chunk
     assert (delta.cpu() - (do.float() * o.cpu().float()).sum(-1).transpose(1, 2)).abs().max() < 1e-3 * D
     ltr.attn_bwd_accumulate(qd, dod, lse, delta, cut(kd), cut(vd), pos, dq32, sink, sink, q_pos, split, causal, do_dkdv=False)
     dq32 = dq32.cpu() - 0.5
-    assert (dq32 - dq_ref).norm() <= 5e-2 * dq_ref.norm()
+    assert (dq32 - dq_ref).norm() <= 1e-2 * dq_ref.norm()       # 2.0e-3 .. 3.1e-3: P, dS and the inputs' products in bf16
+    # one key lost or taken twice at a border of shares or chunks would hide in that: against the kernels that share nothing.  dQ: the
+    # same bf16 P and dS, summed in another order; O: P rounded against another reference (2^-9 of each term, on both sides)
+    of, lf = ltr.attn_fwd(qd, cut(kd), cut(vd), pos, q_pos, split, causal, out_dtype=torch.float32)
+    o1, l1 = ltr.attn_fwd(qd, cut(kd), cut(vd), pos, q_pos, split, causal, out_dtype=torch.float32, fwd_rows=256)
+    assert (of - o1).norm() <= 4e-3 * o1.norm() and (lf.cpu()[fin] - l1.cpu()[fin]).abs().max() <= 2e-4
+    dq1 = torch.zeros(q.shape, dtype=torch.float32, device="cuda")
+    ltr.attn_bwd_accumulate(qd, dod, lse, delta, cut(kd), cut(vd), pos, dq1, sink, sink, q_pos, split, causal, do_dkdv=False, dq_rows=256)
+    assert (dq32 - dq1.cpu()).norm() <= 1e-5 * dq1.cpu().norm()
     # bf16 rounding (2^-8 of the value) and the cancellation of the accumulator's start value (2^-23 of 0.5 + |dQ|)
     assert ((dq16.cpu().float() - dq32).abs() <= dq32.abs() / 256 + 1e-6).all()
 
