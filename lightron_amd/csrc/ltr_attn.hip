@@ -3609,8 +3609,9 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         pl.kv_tiles = 0;
         for (int c = 0; c < n_chunks; c++) pl.kv_tiles += (chunk[c].sk + pl.keys_per_block - 1) / pl.keys_per_block;
         pl.kv_blocks = pl.kv_tiles * B * Hkv;
-        // at any length: the shares' shorter sums, added up, are nearer to fp64 than one serial sum (4 q heads on one kv head,
-        // D=128, causal, dK relative to its norm, whole -> shared): 1024 rows 1.3e-6 -> 5.3e-7, 6766 rows 3.1e-6 -> 9.6e-7
+        // fp32 sums of more than 4096 rows keep their one serial order: its rounding reaches 1e-4 of single elements (measured at
+        // 27064 rows), and a sum in another order differs from it by as much
+        may_split = may_split && (long long)(Hq / Hkv) * Sq <= 4096;
         split_keys(D == 128 ? KvSplitCost{32, 9.0, 2.0, 6e6} : KvSplitCost{32, 4.5, 1.5, 6e6});
         pl.dq_qtiles = pl.dq_slots = (Sq + pl.dq_rows - 1) / pl.dq_rows;
         pl.dq_blocks = (long long)pl.dq_qtiles * B * Hq;
