@@ -3609,8 +3609,11 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         pl.kv_tiles = 0;
         for (int c = 0; c < n_chunks; c++) pl.kv_tiles += (chunk[c].sk + pl.keys_per_block - 1) / pl.keys_per_block;
         pl.kv_blocks = pl.kv_tiles * B * Hkv;
-        // fp32 sums of more than 4096 rows keep their one serial order: its rounding reaches 1e-4 of single elements (measured at
-        // 27064 rows), and a sum in another order differs from it by as much
+        // fp32 sums of more than 4096 rows keep their one serial order, and with it their rounding: shared sums are nearer to fp64
+        // (4 q heads on one kv head, D=128, causal, error of dK relative to its norm, whole / shared: 4096 rows 1.3e-6 / 5.3e-7, 27064 rows
+        // 3.1e-6 / 9.6e-7; largest single error in units of the rms 4e-5 / 1e-5 and 2.5e-4 / 5e-5) and faster (8513 / 1081 us at
+        // 27064), but they would move single elements by the whole sum's error, which from about here on exceeds 1e-4 of them:
+        // the tolerance to which results of this path are to stay the same
         may_split = may_split && (long long)(Hq / Hkv) * Sq <= 4096;
         split_keys(D == 128 ? KvSplitCost{32, 9.0, 2.0, 6e6} : KvSplitCost{32, 4.5, 1.5, 6e6});
         pl.dq_qtiles = pl.dq_slots = (Sq + pl.dq_rows - 1) / pl.dq_rows;

@@ -77,3 +77,31 @@ def test_masked_tiles_between_shared_ones(ltr, D, Hq, Hkv, dtype):
     """Chunks and tails of chunks that no row sees lie before and between the visible ones of the table: they have no partial sums,
     and the visible tiles' partials are numbered without them."""
     test_shared_key_tiles(ltr, D, Hq, Hkv, 300, (40, 700), 130, [(300, 2000), (128, 0), (140, 3000), (520, 500), (77, 1500), (64, 128)], True, dtype, None)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,S,causal", [(128, 4, 1, 1000, True), (64, 4, 2, 2000, False)])
+def test_shared_fp32_sums_are_no_further_from_fp64(ltr, D, Hq, Hkv, S, causal):
+    """fp32 sums of up to 4096 rows: several shorter ones added up have the smaller rounding error."""
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, do = (torch.randn(1, S, Hq, D, device="cuda", generator=g) for _ in range(2))
+    k, v = (torch.randn(1, S, Hkv, D, device="cuda", generator=g) for _ in range(2))
+    plan = ltr.attn_plan(1, Hq, Hkv, D, S, [S], [0], causal=causal, dtype=torch.float32, share_keys=True)["dkdv"]
+    assert plan["blocks_per_tile"] > 1 and plan["reduce_blocks"] > 0
+    o, lse = ltr.attn_fwd(q, [k], [v], [0], causal=causal)
+    delta = ltr.attn_delta(o, do)
+    want = [torch.zeros(k.shape, dtype=torch.float64, device="cuda") for _ in range(2)]
+    for h in range(Hq):
+        qh, doh, kh, vh = (t[0, :, i].double() for t, i in ((q, h), (do, h), (k, h * Hkv // Hq), (v, h * Hkv // Hq)))
+        s = qh @ kh.T * D ** -0.5
+        p = (s.masked_fill(~torch.ones(S, S, dtype=torch.bool, device="cuda").tril(), -torch.inf) if causal else s).softmax(-1)
+        ds = p * (doh @ vh.T - (doh * (p @ vh)).sum(-1, keepdim=True)) * D ** -0.5
+        want[0][0, :, h * Hkv // Hq] += ds.T @ qh
+        want[1][0, :, h * Hkv // Hq] += p.T @ doh
+    err = []
+    for share in (False, True):
+        got = [torch.zeros_like(k) for _ in range(2)]
+        ltr.attn_bwd_accumulate(q, do, lse, delta, [k], [v], [0], torch.zeros_like(q), got[:1], got[1:], 0, None, causal, share_keys=share)
+        err.append([((x.double() - w).norm() / w.norm()).item() for x, w in zip(got, want)])
+    assert all(shared <= whole for whole, shared in zip(*err)) and max(err[1]) < 2e-6
+    rows = 4097 * Hkv // Hq + 1          # and one row more than the rule takes: the whole sum
+    assert ltr.attn_plan(1, Hq, Hkv, D, rows, [rows], [0], causal=causal, dtype=torch.float32, share_keys=True)["dkdv"]["blocks_per_tile"] == 1
