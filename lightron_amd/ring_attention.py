@@ -10,6 +10,7 @@ build has no collectives.
 """
 from __future__ import annotations
 
+import operator
 from typing import List, Optional, Sequence, Tuple
 
 import torch
@@ -38,8 +39,8 @@ class RingKVGrads:
 
     def _whole(self):
         """The buffer while dk / dv are still its slices; None once a caller has put tensors of its own in their place."""
-        acc = [*self.dk, *self.dv]
-        return self._buf if len(acc) == len(self._acc) and all(a is b for a, b in zip(acc, self._acc)) else None
+        same = len(self.dk) + len(self.dv) == len(self._acc) and all(map(operator.is_, (*self.dk, *self.dv), self._acc))
+        return self._buf if same else None
 
     def _views(self, buf):
         tensors = [k for k, _ in self.kv] + [v for _, v in self.kv]
