@@ -84,6 +84,19 @@ struct ChunkDev {
     int pos0;
 };
 
+// Division by a number that the host knows, of n < 2^31.
+struct Div {
+    int d;
+    unsigned mul, shift;
+    __device__ __forceinline__ int of(int n) const { return (int)(((unsigned long long)(unsigned)n * mul) >> shift); }
+};
+struct BlockMap {   // see block_item
+    int group;              // (batch, kv head) pairs of an XCD whose blocks are handed out together; 0: the pairs do not divide among the XCDs
+    int last_group;         // the group of last_pairs pairs
+    Div inner, group_items; // blocks per item; items per group
+    Div pairs, last_pairs;  // pairs per group (group = 0: all pairs)
+};
+
 struct FwdParams {
     const void *q;
     void *o;
@@ -92,6 +105,7 @@ struct FwdParams {
     int cols;              // head dim of the tensors (the kernel's own width, or less: PAD kernels)
     int Sq, n_qtiles;
     int n_slots;           // q tiles are handed out in slots: n_qtiles of one tile, or (n_qtiles + 1) / 2 of two (see q_tile_slots)
+    BlockMap map;
     long long qs[3], os[3], ks[3], vs[3];
     int q_pos0[2];
     int q_split;
@@ -131,6 +145,7 @@ struct BwdParams {
     int n_reps;       // of which a block walks this many
     float *part;      // n_split > 1: the blocks' partial dK / dV, summed by bwd_dkdv_reduce_kernel
     int n_slots;      // slots of 256-row q tiles of the dQ kernel (see q_tile_slots)
+    BlockMap q_map, kv_map;   // of the dQ and the dK/dV kernel
     const float *rope;     // LTR_ROPE_DQ: (cos, sin) rows, cols floats per position, row 0 = position rope_pos0
     int rope_pos0;
     ChunkDev chunk[LTR_MAX_CHUNKS];
@@ -161,6 +176,33 @@ __device__ __forceinline__ void q_pos_range(int r0, int r1, int split, int p0, i
         lo = min(lo, min(c, d));
         hi = max(hi, max(c, d));
     }
+}
+
+// Block id -> (pair = batch x kv head, item = q tile slot or key tile of the pair, sub = one of the `inner` blocks of an item).
+// Consecutive block ids go to the 8 XCDs round-robin.  All blocks of a pair run on one XCD and next to each other in time, so the
+// blocks that are resident together stream the same K / V (or Q / dO) through that XCD's L2; the inner blocks of an item follow each
+// other.  The items of `group` pairs of an XCD are handed out item by item (the first of every pair, the second of every pair, ...):
+// items come longest first, so blocks of unequal length end together (see pair_group).
+// The divisions are multiplications prepared by the host: four of the device's own cost a block 0.3 us.
+struct BlockItem {
+    int pair, item, sub;
+};
+__device__ __forceinline__ BlockItem block_item(const BlockMap &m) {
+    BlockItem r;
+    const int idx = blockIdx.x;
+    if (m.group) {
+        const int j = idx >> 3, i = m.inner.of(j), g = m.group_items.of(i), in_group = i - g * m.group_items.d;
+        const bool last = g == m.last_group;
+        r.sub = j - i * m.inner.d;
+        r.item = last ? m.last_pairs.of(in_group) : m.pairs.of(in_group);
+        r.pair = (g * m.group + in_group - r.item * (last ? m.last_pairs.d : m.pairs.d)) * 8 + (idx & 7);
+    } else {   // pairs that do not divide among the XCDs: pair after pair, then the next block of each
+        const int rest = m.pairs.of(idx);
+        r.pair = idx - rest * m.pairs.d;
+        r.item = m.inner.of(rest);
+        r.sub = rest - r.item * m.inner.d;
+    }
+    return r;
 }
 
 // both halves of the wave end up with combine(x[l], x[l ^ 32])
@@ -605,21 +647,9 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     const int rg = w / KS, ks = w % KS;      // row group and key share of the wave
     const bool causal = p.flags & LTR_CAUSAL;
 
-    // block -> (batch, kv head, q head of the group, q tile).  Consecutive block ids go to
-    // the 8 XCDs round-robin; all q tiles / q heads of one (batch, kv head) run on one XCD and
-    // next to each other in time, so the blocks that are resident together stream the same K/V
-    // through that XCD's L2.  Late (heavier under a causal mask) q tiles first.
-    int idx = blockIdx.x, pair, rest;
-    const int P = p.B * p.Hkv;
-    if ((P & 7) == 0) {
-        int xcd = idx & 7, j = idx >> 3, nr = p.n_slots * p.n_rep;
-        pair = (j / nr) * 8 + xcd;
-        rest = j % nr;
-    } else {
-        pair = idx % P;
-        rest = idx / P;
-    }
-    const int rep = rest % p.n_rep, slot = rest / p.n_rep;
+    // block -> (batch, kv head, q head of the group, q tile); late (heavier under a causal mask) q tiles first
+    const BlockItem item = block_item(p.map);
+    const int pair = item.pair, rep = item.sub, slot = item.item;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv, h = hkv * p.n_rep + rep;
     // A slot is one q tile (late, heavier tiles first) or, when the host paired them, a late tile and its early
     // counterpart: under a causal mask every block then has the same amount of work.
@@ -1579,20 +1609,10 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
     const int l32 = lane & 31, hh = lane >> 5;
     const bool causal = p.flags & LTR_CAUSAL;
 
-    // block -> (batch, kv head, chunk, key tile); same XCD grouping as the forward
-    int idx = blockIdx.x, pair, rest;
-    const int P = p.B * p.Hkv;
-    if ((P & 7) == 0) {
-        const int xcd = idx & 7, j = idx >> 3, n = p.tiles_seen << p.split_log2;
-        pair = (j / n) * 8 + xcd;
-        rest = j % n;
-    } else {
-        pair = idx % P;
-        rest = idx / P;
-    }
-    // blocks that share a key tile follow each other: each takes n_reps of the q heads and, of a head's visible q tiles, every
-    // 2^share_log2-th
-    const int split = rest & ((1 << p.split_log2) - 1), tile = rest >> p.split_log2;
+    // block -> (batch, kv head, chunk, key tile); same XCD grouping as the forward.  Blocks that share a key tile follow each
+    // other: each takes n_reps of the q heads and, of a head's visible q tiles, every 2^share_log2-th
+    const BlockItem item = block_item(p.kv_map);
+    const int pair = item.pair, split = item.sub, tile = item.item;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
     int c = 0, kt = tile;
     for (; c < p.n_chunks; c++) {
@@ -2229,18 +2249,9 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
     const int rg = w / KS, ks = w % KS;      // row group and key share of the wave
     const bool causal = p.flags & LTR_CAUSAL;
 
-    int idx = blockIdx.x, pair, rest;
-    const int P = p.B * p.Hkv;
-    if ((P & 7) == 0) {
-        int xcd = idx & 7, j = idx >> 3, nr = p.n_slots * p.n_rep;
-        pair = (j / nr) * 8 + xcd;
-        rest = j % nr;
-    } else {
-        pair = idx % P;
-        rest = idx / P;
-    }
+    const BlockItem item = block_item(p.q_map);
+    const int pair = item.pair, rep = item.sub, slot = item.item;
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int rep = rest % p.n_rep, slot = rest / p.n_rep;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv, h = hkv * p.n_rep + rep;
     // one q tile per block (late tiles first) or a late tile and its early counterpart (see q_tile_slots)
     const bool paired = p.n_slots != n_qt;
@@ -3348,6 +3359,19 @@ bool q_tiles_uneven(int Sq, int rows, int q_split, const int *q_pos0, const Chun
     return std::min(first, last) * 4 < std::max(first, last) * 3;
 }
 
+// The same for the key tiles of the dK/dV kernel: the rows that see the first and the last tile's first key.
+bool key_tiles_uneven(int Sq, int keys, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks) {
+    long long lo = 0x7fffffff, hi = 0;
+    for (int c = 0; c < n_chunks; c++)
+        for (const int kpos : {chunk[c].pos0, chunk[c].pos0 + (chunk[c].sk - 1) / keys * keys}) {
+            const long long rows = std::min<long long>(std::max<long long>(q_pos0[0] + (long long)q_split - kpos, 0), q_split) +
+                                   std::min<long long>(std::max<long long>(q_pos0[1] + (long long)(Sq - q_split) - kpos, 0), Sq - q_split);
+            lo = std::min(lo, rows);
+            hi = std::max(hi, rows);
+        }
+    return lo * 4 < hi * 3;
+}
+
 // Slots of q tiles handed to the blocks of the forward and dQ kernels.  Under a causal mask a tile's work grows with its
 // rows' positions; pairing tile t with tile n - 1 - t in one block gives every block the same work (no long blocks left
 // over at the end of the launch) and halves the number of blocks to start.  Only done when the tiles do differ (see
@@ -3360,6 +3384,42 @@ int q_tile_slots(int n_qtiles, long long blocks_per_tile, bool uneven) {
     const int n_slots = (n_qtiles + 1) / 2;
     const long long n = n_slots * blocks_per_tile, rounds = (n + cus - 1) / cus;
     return n * 10 >= rounds * cus * 9 ? n_slots : n_qtiles;
+}
+
+// How many (batch, kv head) pairs of an XCD hand out their blocks together, longest first across them (block_item).  Pair after pair, every
+// pair ends with its short blocks and the next one begins with long ones: the launch ends with long blocks running alone.  All
+// pairs together, more K / V (or Q / dO) is in use than an L2 holds.  A group is taken as large as two rounds of the blocks that an XCD runs
+// at once (`slots`), and equal blocks are left pair after pair.  Kernel us, one pair / 4 pairs / all pairs at a time:
+//   dK/dV      B=8  8 kv heads of 32 D=128 causal S=1000   206 / 151 / 154 (8 pairs per XCD)    B=4 16 heads D=128 S=1024   67 / 50 / 51 (8)
+//   dK/dV      B=8 32 heads D=128 causal S=2048   685 / 636 / 696 (32)     the same, S=512    94 / 75 / 80 (32)
+//   dQ         B=4 12 heads D=64  causal S=2048    69 / 58 / 52 (6)        forward            58 / 48 / 42
+//   dK/dV      B=4 32 heads D=128 S=8192 causal  4087 / 4069 / 4453 (16)   no mask          7473 / 7607 / 8515
+int pair_group(long long pairs, long long blocks_per_pair, int slots, bool uneven) {
+    if (!uneven || pairs % 8) return 1;
+    const long long n = pairs / 8, want = std::max(1LL, (2LL * slots + blocks_per_pair - 1) / blocks_per_pair), groups = std::max(1LL, (n + want / 2) / want);
+    return (int)((n + groups - 1) / groups);
+}
+
+Div make_div(long long d) {   // exact for n < 2^31: mul = 2^shift / d rounded up, off by less than d <= 2^(shift - 31)
+    const int lg = 63 - __builtin_clzll((unsigned long long)d);
+    Div r;
+    r.d = (int)d;
+    const bool pow2 = (d & (d - 1)) == 0;
+    r.shift = 31 + lg + (pow2 ? 0 : 1);
+    r.mul = (unsigned)(((1ull << r.shift) + (unsigned long long)d - 1) / (unsigned long long)d);
+    return r;
+}
+// pairs x items x inner < 2^31 blocks; see block_item
+BlockMap block_map(long long pairs, long long items, long long inner, int group) {
+    BlockMap m;
+    m.group = pairs % 8 ? 0 : group;
+    const long long n = m.group ? pairs / 8 : pairs, per = m.group ? group : pairs;
+    m.last_group = (int)((n - 1) / per);
+    m.inner = make_div(std::max(1LL, inner));
+    m.group_items = make_div(std::max(1LL, items * per));
+    m.pairs = make_div(per);
+    m.last_pairs = make_div(n - (n - 1) / per * per);
+    return m;
 }
 
 // Waves that share a row group's keys in the bf16 forward and dQ kernels.  Blocks of 256 rows leave CUs idle when a launch has few
@@ -3446,7 +3506,7 @@ struct FwdPlan {
     bool wide;          // 512-row blocks (two 32-row blocks per wave, head dim 64)
     int ks;             // bf16: key shares per row group (1, or 2 / 4 with blocks of 256 / ks rows; see key_shares)
     int f32_ks;         // fp32: 0 = scalar kernel, else the key shares per row group of fwd_f32_mfma_kernel
-    int rows, n_qtiles, n_slots;
+    int rows, n_qtiles, n_slots, group;
     long long blocks;
 };
 FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
@@ -3454,6 +3514,7 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     FwdPlan pl;
     pl.f32_ks = 0;
     pl.ks = 1;
+    pl.group = 1;
     if (f32) {
         pl.wide = false;
         if (flags & LTR_FWD_F32_SCALAR) {
@@ -3473,6 +3534,10 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         return pl;
     }
     const bool causal_ = (flags & LTR_CAUSAL) != 0;
+    auto group_of = [&]() {   // paired tiles are equal blocks
+        const bool uneven = causal_ && pl.n_slots == pl.n_qtiles && q_tiles_uneven(Sq, pl.rows, q_split, q_pos0, chunk, n_chunks);
+        return pair_group((long long)B * Hkv, (long long)pl.n_slots * (Hq / Hkv), device_cus() / 8, uneven);
+    };
     // query rows per block: 512 (two 32-row blocks per wave, 64-key tiles) pays at head dim 64 under the conditions of
     // the dQ kernel's 512-row blocks (see plan_bwd)
     bool wide = (flags & LTR_FWD_ROWS_512) != 0;
@@ -3495,12 +3560,14 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         pl.n_qtiles = (Sq + pl.rows - 1) / pl.rows;
         pl.n_slots = shares.paired ? (pl.n_qtiles + 1) / 2 : pl.n_qtiles;
         pl.blocks = (long long)pl.n_slots * B * Hq;
+        pl.group = group_of();
         return pl;
     }
     pl.rows = wide ? 512 : 256;
     pl.n_qtiles = (Sq + pl.rows - 1) / pl.rows;
     pl.n_slots = q_tile_slots(pl.n_qtiles, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, pl.rows, q_split, q_pos0, chunk, n_chunks));
     pl.blocks = (long long)pl.n_slots * B * Hq;
+    pl.group = group_of();
     return pl;
 }
 
@@ -3577,6 +3644,7 @@ struct BwdPlan {
     bool wide_q;        // dQ kernel: 512 rows per block
     int dq_ks;          // bf16 dQ kernel: key shares per row group, as in the forward
     int dq_rows, dq_qtiles, dq_slots;
+    int dq_group, kv_group;   // see pair_group
     long long dq_blocks;
 };
 BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
@@ -3586,6 +3654,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.split = KvSplit{1, 1, 0x7fffffff, 0};
     pl.part_bytes = 0;
     pl.dq_ks = 1;
+    pl.dq_group = pl.kv_group = 1;
     may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
     auto split_keys = [&](const KvSplitCost &cost) {
         if (may_split) pl.split = kv_split(cost, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks);
@@ -3670,6 +3739,12 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.dq_slots = pl.dq_ks > 1 ? (shares.paired ? (pl.dq_qtiles + 1) / 2 : pl.dq_qtiles)
                                : q_tile_slots(pl.dq_qtiles, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks));
     pl.dq_blocks = (long long)pl.dq_slots * B * Hq;
+    const long long pairs = (long long)B * Hkv;
+    const int slots = device_cus() / 8;
+    pl.dq_group = pair_group(pairs, (long long)pl.dq_slots * (Hq / Hkv), slots,
+                             causal_ && pl.dq_slots == pl.dq_qtiles && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks));
+    pl.kv_group = pair_group(pairs, (pl.split.n > 1 ? pl.split.tiles : pl.kv_tiles) * pl.split.n, slots,
+                             causal_ && key_tiles_uneven(Sq, pl.keys_per_block, q_split, q_pos0, chunk, n_chunks));
     return pl;
 }
 // blocks of bwd_dkdv_reduce_kernel: four waves each, one per 64 columns of a 32-key slice of dK or dV
@@ -3809,6 +3884,7 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     if (pl.blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.n_qtiles = pl.n_qtiles;
     p.n_slots = pl.n_slots;
+    if (a->io_dtype == LTR_BF16) p.map = block_map((long long)p.B * p.Hkv, pl.n_slots, p.n_rep, pl.group);
     if (a->io_dtype == LTR_BF16) {
         rc = enable_large_lds();
         if (rc) return rc;
@@ -3995,6 +4071,8 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     p.n_reps = p.n_rep / pl.split.reps;
     p.part = (float *)work;
     p.n_slots = pl.dq_slots;
+    if (!f32) p.q_map = block_map((long long)p.B * p.Hkv, pl.dq_slots, p.n_rep, pl.dq_group);
+    if (!f32) p.kv_map = block_map((long long)p.B * p.Hkv, tiles_seen, pl.split.n, pl.kv_group);
     hipStream_t st = (hipStream_t)stream;
     if (f32 && pl.f32_ks) {   // fp32 on the matrix pipe
         rc = enable_large_lds();
