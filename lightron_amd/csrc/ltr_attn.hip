@@ -30,7 +30,8 @@
 //                        bwd_dkdv_kernel<64, 2>: two 32-key halves per wave (256 keys per block): every Q / dO operand
 //                        read from LDS feeds two MFMAs, and a block's transfers and per-step costs are spread over
 //                        twice the matrix work.  The registers allow it at head dim 64 only; chosen by the host
-//                        when the blocks are long and still many (or forced with LTR_DKDV_KEYS_256).
+//                        for long equal blocks without masked tiles (or forced with LTR_DKDV_KEYS_256).
+//   bwd_dkdv_keywave_kernel<64>  head dim 64: a wave does both halves of the work of its 32 keys, four waves per block, two blocks per CU.
 //   bwd_dkdv_reduce_kernel<D, KW>  sums the partial dK / dV of blocks that share a key tile (see KvSplit).
 //   bwd_dq_kernel<D, RB> forward-shaped: a block owns 256 * RB query rows, loops over K/V tiles
 //                        (same direct-to-LDS tiles as the forward), recomputes S and dP and
@@ -440,6 +441,8 @@ __device__ __forceinline__ void lds_tr_gemm(const __bf16 *T, int row0, int lane,
 // XOR each per tile, instead of rebuilding every address from pointer + swizzle before each read.
 typedef __attribute__((address_space(3))) const bf16x8 *lds_bf16x8_ptr;
 typedef __attribute__((address_space(3))) i16x4 *lds_i16x4_ptr;
+typedef __attribute__((address_space(3))) const f32x4 *lds_f32x4_ptr;
+typedef __attribute__((address_space(3))) const i32x4 *lds_i32x4_ptr;
 
 template <int D>
 __device__ __forceinline__ void lds_gemm_pair_at(const unsigned (&addr)[D / 16], int imm_a, int imm_b,
@@ -1592,6 +1595,93 @@ __host__ __device__ __forceinline__ int seen_tiles(int sk, int pos0, int q_last,
     return seen <= 0 ? 0 : ((int)(seen < sk ? seen : sk) + keys - 1) / keys;
 }
 
+// The q tiles (BM rows) of a dK/dV block, listed once per block by one wave (ballot compaction: the order, and with it the rounding of
+// the accumulation, is fixed), so that the main loops carry no classification arithmetic.  A tile's class depends on its rows
+// only: 0 = no row sees any key of the block (skipped); 1 = every (row, key) pair is visible (list 0); 2 = needs the mask
+// (diagonal, tails: list 1).  kpos_lo, kpos_hi: positions of the block's first and last key; split: which of the blocks that share the
+// keys this is.
+template <int BM, int MAX_QTILES>
+__device__ __forceinline__ void list_q_tiles(const BwdParams &p, int lane, int split, int kpos_lo, int kpos_hi, bool key_tail,
+                                             unsigned short *tlist, int *tcount) {
+    const bool causal = p.flags & LTR_CAUSAL;
+    auto tile_class = [&](int qt) {
+        const int row0 = qt * BM;
+        const bool edge = key_tail || row0 + BM > p.Sq;
+        if (!causal) return edge ? 2 : 1;
+        int lo, hi;
+        q_pos_range(row0, min(row0 + BM, p.Sq) - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], lo, hi);
+        if (hi < kpos_lo) return 0;
+        return (edge || kpos_hi > lo) ? 2 : 1;
+    };
+    // a block that shares its keys lists every n_share-th visible tile, counted from its own offset
+    const int n_share = 1 << p.share_log2;
+    int n1 = 0, n2 = 0;
+    int skip = split & (n_share - 1);   // visible tiles to pass over before the next one of this block
+    for (int base = 0; base < p.n_qtiles; base += 64) {
+        const int qt = base + lane;
+        int cls = qt < p.n_qtiles ? tile_class(qt) : 0;
+        if (n_share > 1) {
+            const unsigned long long vis = __builtin_amdgcn_ballot_w64(cls != 0);
+            const int rank = __builtin_popcountll(vis & ((1ull << lane) - 1ull)), n = __builtin_popcountll(vis);
+            if (((rank - skip) & (n_share - 1)) != 0 || rank < skip) cls = 0;
+            skip = (skip - n) & (n_share - 1);
+        }
+        const unsigned long long m1 = __builtin_amdgcn_ballot_w64(cls == 1), m2 = __builtin_amdgcn_ballot_w64(cls == 2);
+        const unsigned long long below = (1ull << lane) - 1ull;
+        if (cls == 1) tlist[n1 + __builtin_popcountll(m1 & below)] = (unsigned short)qt;
+        if (cls == 2) tlist[MAX_QTILES + n2 + __builtin_popcountll(m2 & below)] = (unsigned short)qt;
+        n1 += __builtin_popcountll(m1);
+        n2 += __builtin_popcountll(m2);
+    }
+    if (lane == 0) {
+        tcount[0] = n1;
+        tcount[1] = n2;
+    }
+}
+
+// A wave's dK^T or dV^T tile of 32 keys (times mul) through its LDS staging area: stored as bf16 rows (LTR_DKDV_BF16: every query that
+// sees these keys was in this launch) or added to the fp32 accumulator in whole rows.  base + off: key 0, column 0.
+template <int D, bool PAD>
+__device__ __forceinline__ void write_key_rows(unsigned char *stage, int lane, const f32x16 (&acc)[D / 32], float mul, bool as_bf16,
+                                               void *base, long long off, long long row_stride, int first_key, int n_keys, int cols) {
+    constexpr int LPR = D / 4, ROWS_PER_IT = 64 / LPR;      // see wave_tile_rowmajor
+    const long long stride = uniform64(row_stride);
+    const int key_base = uniform32(first_key), sk = uniform32(n_keys);
+    const long long goff = off + (key_base + lane / LPR) * stride + 4 * (lane % LPR);
+    if (as_bf16) {
+        __bf16 *gb = (__bf16 *)base + goff;
+        wave_tile_rowmajor<D>(stage, lane, acc, mul, [&](int row, int col, f32x4 val) {
+            if (key_base + row < sk && (!PAD || col < cols)) {
+                bf16x4 y;
+#pragma unroll
+                for (int e = 0; e < 4; e++) y[e] = (__bf16)val[e];
+                *(bf16x4 *)gb = y;
+            }
+            gb += ROWS_PER_IT * stride;
+        });
+        return;
+    }
+    float *gp = (float *)base + goff;
+    // all reads of the accumulator first (independent loads in flight together), then the adds and the writes
+    constexpr int NIT = 32 / ROWS_PER_IT;
+    f32x4 old[NIT];
+#pragma unroll
+    for (int it = 0; it < NIT; it++) {
+        old[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (key_base + it * ROWS_PER_IT + lane / LPR < sk && (!PAD || 4 * (lane % LPR) < cols)) old[it] = *(const f32x4 *)(gp + it * ROWS_PER_IT * stride);
+    }
+    int it = 0;
+    wave_tile_rowmajor<D>(stage, lane, acc, mul, [&](int row, int col, f32x4 val) {
+        if (key_base + row < sk && (!PAD || col < cols)) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) val[e] += old[it][e];
+            *(f32x4 *)gp = val;
+        }
+        gp += ROWS_PER_IT * stride;
+        it++;
+    });
+}
+
 template <int D, int KW, bool PAD>
 __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
     const int cols = PAD ? p.cols : D;
@@ -1677,48 +1767,9 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
         for (int i = 0; i < D / 32; i++) acc[k][i] = zero16;
     const float c2 = p.scale * LTR_LOG2E;
 
-    // A tile's class depends on its rows only: 0 = no row sees any key of the block (skipped);
-    // 1 = every (row, key) pair is visible; 2 = needs the mask (diagonal, tails).
-    auto tile_class = [&](int qt) {
-        const int row0 = qt * BM;
-        const bool edge = key_tail || row0 + BM > p.Sq;
-        if (!causal) return edge ? 2 : 1;
-        int lo, hi;
-        q_pos_range(row0, min(row0 + BM, p.Sq) - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], lo, hi);
-        if (hi < tile_kpos_lo) return 0;
-        return (edge || tile_kpos_hi > lo) ? 2 : 1;
-    };
-
-    // The q tiles of each class are listed once per block (wave 0, ballot compaction: the order, and with it
-    // the rounding of the accumulation, is fixed), so the main loops carry no classification arithmetic.
     unsigned short *const tlist = (unsigned short *)(smem + L::LIST_OFF);     // [2][MAX_QTILES]
     int *const tcount = (int *)(smem + L::LIST_OFF + 2 * L::MAX_QTILES * 2);
-    if (w == 0) {
-        // a block that shares its keys lists every n_share-th visible tile, counted from its own offset
-        const int n_share = 1 << p.share_log2;
-        int n1 = 0, n2 = 0;
-        int skip = split & (n_share - 1);   // visible tiles to pass over before the next one of this block
-        for (int base = 0; base < p.n_qtiles; base += 64) {
-            const int qt = base + lane;
-            int cls = qt < p.n_qtiles ? tile_class(qt) : 0;
-            if (n_share > 1) {
-                const unsigned long long vis = __builtin_amdgcn_ballot_w64(cls != 0);
-                const int rank = __builtin_popcountll(vis & ((1ull << lane) - 1ull)), n = __builtin_popcountll(vis);
-                if (((rank - skip) & (n_share - 1)) != 0 || rank < skip) cls = 0;
-                skip = (skip - n) & (n_share - 1);
-            }
-            const unsigned long long m1 = __builtin_amdgcn_ballot_w64(cls == 1), m2 = __builtin_amdgcn_ballot_w64(cls == 2);
-            const unsigned long long below = (1ull << lane) - 1ull;
-            if (cls == 1) tlist[n1 + __builtin_popcountll(m1 & below)] = (unsigned short)qt;
-            if (cls == 2) tlist[L::MAX_QTILES + n2 + __builtin_popcountll(m2 & below)] = (unsigned short)qt;
-            n1 += __builtin_popcountll(m1);
-            n2 += __builtin_popcountll(m2);
-        }
-        if (lane == 0) {
-            tcount[0] = n1;
-            tcount[1] = n2;
-        }
-    }
+    if (w == 0) list_q_tiles<BM, L::MAX_QTILES>(p, lane, split, tile_kpos_lo, tile_kpos_hi, key_tail, tlist, tcount);
     __syncthreads();
 
     const int st_row = lane / CPR, st_pc = lane % CPR;   // this lane's place inside a 1 KB LDS-direct load
@@ -2045,48 +2096,13 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
         for (int k = 0; k < KW; k++) store_partial<D>(part + k * 32 * D, lane, acc[k], mul);
         return;
     }
-    // dV^T (P wave) / dK^T (dS wave) tile of the wave's 32 keys: added to the fp32 accumulators in whole rows, through the
-    // wave's LDS staging area (every wave is past the last barrier: tiles, slots and lists are no longer read)
+    // dV^T (P wave) / dK^T (dS wave); every wave is past the last barrier: tiles, slots and lists are no longer read
 #pragma unroll
-    for (int k = 0; k < KW; k++) {
-        constexpr int LPR = D / 4, ROWS_PER_IT = 64 / LPR;      // see wave_tile_rowmajor
-        const long long stride = uniform64(p_role ? p.dvs[1] : p.dks[1]);
-        const int key_base = uniform32(key0 + slice * 32 * KW + 32 * k), sk_u = uniform32(sk);
-        const long long goff = (p_role ? b * p.dvs[0] + hkv * p.dvs[2] : b * p.dks[0] + hkv * p.dks[2]) +
-                               (key_base + lane / LPR) * stride + 4 * (lane % LPR);
-        if (uniform32(p.flags & LTR_DKDV_BF16)) {   // every query that sees these keys was in this launch: store the result
-            __bf16 *gb = (__bf16 *)(p_role ? p.chunk[c].dv : p.chunk[c].dk) + goff;
-            wave_tile_rowmajor<D>(smem + w * WaveStage<D>::BYTES, lane, acc[k], p_role ? 1.f : p.scale, [&](int row, int col, f32x4 val) {
-                if (key_base + row < sk_u && (!PAD || col < cols)) {
-                    bf16x4 y;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) y[e] = (__bf16)val[e];
-                    *(bf16x4 *)gb = y;
-                }
-                gb += ROWS_PER_IT * stride;
-            });
-            continue;
-        }
-        float *gp = (p_role ? p.chunk[c].dv : p.chunk[c].dk) + goff;
-        // all reads of the accumulator first (independent loads in flight together), then the adds and the writes
-        constexpr int NIT = 32 / ROWS_PER_IT;
-        f32x4 old[NIT];
-#pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            old[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (key_base + it * ROWS_PER_IT + lane / LPR < sk_u && (!PAD || 4 * (lane % LPR) < cols)) old[it] = *(const f32x4 *)(gp + it * ROWS_PER_IT * stride);
-        }
-        int it = 0;
-        wave_tile_rowmajor<D>(smem + w * WaveStage<D>::BYTES, lane, acc[k], p_role ? 1.f : p.scale, [&](int row, int col, f32x4 val) {
-            if (key_base + row < sk_u && (!PAD || col < cols)) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) val[e] += old[it][e];
-                *(f32x4 *)gp = val;
-            }
-            gp += ROWS_PER_IT * stride;
-            it++;
-        });
-    }
+    for (int k = 0; k < KW; k++)
+        write_key_rows<D, PAD>(smem + w * WaveStage<D>::BYTES, lane, acc[k], p_role ? 1.f : p.scale, uniform32(p.flags & LTR_DKDV_BF16),
+                               p_role ? p.chunk[c].dv : p.chunk[c].dk,
+                               p_role ? b * p.dvs[0] + hkv * p.dvs[2] : b * p.dks[0] + hkv * p.dks[2], p_role ? p.dvs[1] : p.dks[1],
+                               key0 + slice * 32 * KW + 32 * k, sk, cols);
 }
 
 template <int D, int KW>
@@ -2096,6 +2112,285 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
 template <int D>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_dkdv_pad_kernel(const BwdParams p) {
     bwd_dkdv_body<D, 1, true>(p);
+}
+
+// dK/dV at head dim 64, one wave per 32-key slice: K and V operands (32 registers) and both accumulators (64) fit one wave, so nothing is
+// handed over between waves, a block of four waves owns 128 keys in 51 KB of LDS, and two blocks share a CU: one's start, end and barriers run
+// under the other's matrix work, which is what bounds bwd_dkdv_kernel<64, 1> on short rows of blocks (16 x 12 heads, causal S=1024:
+// 115 us there, 97 here, 82 with the blocks longest first; 32 x 4 heads S=4096: 680 -> 579; the same sums in the same order, bit for
+// bit).  Bound: matrix and vector pipe taking turns, 1.06 PFLOP/s without a mask at S=4096.  Three blocks per CU would need 168 registers:
+// 21 and more spill, 83 -> 88 us.  Every (row, key) sub-tile of 32 x 32: S and dP in two alternating chains, P and dS in registers,
+// dV^T += dO^T P, dK^T += Q^T dS.
+template <int D>
+struct KeyWaveLds {
+    static constexpr int NW = 4, BN = 32 * NW, BM = 64, NT = 64 * NW;
+    static constexpr int TILE = BM * D;                                  // elements; rows unpadded, chunks swizzled
+    static constexpr int BUF_BYTES = 2 * TILE * 2 + 3 * BM * 4;          // Q, dO, -LSE/scale, -DELTA, row positions (masked tiles)
+    static constexpr int MAX_QTILES = BwdLds<D, 1>::MAX_QTILES;
+    static constexpr int LIST_OFF = 2 * BUF_BYTES;
+    static constexpr int TOTAL = LIST_OFF + 2 * MAX_QTILES * 2 + 16;     // two tile lists (ushort) + counts
+    static_assert(TOTAL >= NW * WaveStage<D>::BYTES, "the epilogue's staging areas reuse this memory");
+    static_assert(2 * TOTAL <= 160 * 1024, "two blocks per CU");
+};
+template <int D>
+__global__ __launch_bounds__(256, 2) void bwd_dkdv_keywave_kernel(const BwdParams p) {
+    using L = KeyWaveLds<D>;
+    constexpr int BN = L::BN, BM = L::BM;
+    constexpr int CPR = D / 8;
+    constexpr int RPI = 64 / CPR;            // rows filled by one wave-wide LDS-direct load (1 KB)
+    constexpr int NI = BM / (RPI * L::NW);   // such loads per wave, per tensor and per tile
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool causal = p.flags & LTR_CAUSAL;
+    // block -> (batch, kv head, chunk, key tile), shares of a key tile: as in bwd_dkdv_body
+    const BlockItem item = block_item(p.kv_map);
+    const int pair = item.pair, split = item.sub, tile = item.item;
+    const int b = pair / p.Hkv, hkv = pair % p.Hkv;
+    int c = 0, kt = tile;
+    for (; c < p.n_chunks; c++) {
+        const int n = seen_tiles(p.chunk[c].sk, p.chunk[c].pos0, p.q_last, BN);
+        if (kt < n) break;
+        kt -= n;
+    }
+    if (c >= p.n_chunks) return;
+    const int sk = p.chunk[c].sk, pos0 = p.chunk[c].pos0;
+    const int key0 = kt * BN, my_key = key0 + 32 * w + l32;
+    const bool key_ok = my_key < sk;
+    const int kpos = key_ok ? pos0 + my_key : BWD_KPOS_NONE;
+    const int tile_kpos_lo = pos0 + key0, w_kpos_lo = tile_kpos_lo + 32 * w;
+    const int tile_kpos_hi = pos0 + min(key0 + BN, sk) - 1;
+    if (causal) {   // no query of this launch sees the block: nothing to add; results are zero
+        int q_lo, q_hi;
+        q_pos_range(0, (int)p.Sq - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], q_lo, q_hi);
+        if (q_hi < tile_kpos_lo) {
+            if ((p.flags & LTR_DKDV_BF16) && key_ok) {
+                __bf16 *gv = (__bf16 *)p.chunk[c].dv + b * p.dvs[0] + (long long)my_key * p.dvs[1] + hkv * p.dvs[2];
+                __bf16 *gk = (__bf16 *)p.chunk[c].dk + b * p.dks[0] + (long long)my_key * p.dks[1] + hkv * p.dks[2];
+                for (int d = 8 * hh; d < D; d += 16) *(uint4 *)(gv + d) = *(uint4 *)(gk + d) = make_uint4(0, 0, 0, 0);
+            }
+            return;
+        }
+    }
+
+    // resident B operands: the lane's K and V row, d = 16*kb + 8*hh .. +7
+    bf16x8 kreg[D / 16], vreg[D / 16];
+    {
+        const int ksafe = min(my_key, sk - 1);
+        const __bf16 *kp = (const __bf16 *)p.chunk[c].k + b * p.ks[0] + (long long)ksafe * p.ks[1] + hkv * p.ks[2];
+        const __bf16 *vp = (const __bf16 *)p.chunk[c].v + b * p.vs[0] + (long long)ksafe * p.vs[1] + hkv * p.vs[2];
+#pragma unroll
+        for (int kb = 0; kb < D / 16; kb++) {
+            uint4 x = *(const uint4 *)(kp + kb * 16 + 8 * hh), y = *(const uint4 *)(vp + kb * 16 + 8 * hh);
+            if (!key_ok) x = y = make_uint4(0, 0, 0, 0);
+            kreg[kb] = as_bf16x8(x);
+            vreg[kb] = as_bf16x8(y);
+        }
+    }
+    f32x16 dkacc[D / 32], dvacc[D / 32];
+#pragma unroll
+    for (int i = 0; i < D / 32; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) dkacc[i][r] = dvacc[i][r] = 0.f;
+    const float c2 = p.scale * LTR_LOG2E;
+
+    unsigned short *const tlist = (unsigned short *)(smem + L::LIST_OFF);     // [2][MAX_QTILES]
+    int *const tcount = (int *)(smem + L::LIST_OFF + 2 * L::MAX_QTILES * 2);
+    if (w == 0) list_q_tiles<BM, L::MAX_QTILES>(p, lane, split, tile_kpos_lo, tile_kpos_hi, key0 + BN > sk, tlist, tcount);
+    __syncthreads();
+
+    // tile transfers and the rows' scalars: see bwd_dkdv_body
+    const int st_row = lane / CPR, st_pc = lane % CPR;
+    unsigned offq[NI], offdo[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int row = RPI * (NI * w + i) + st_row;
+        const int chunk = st_pc ^ lds_swz<D>(row);
+        offq[i] = (unsigned)(row * (int)p.qs[1] + chunk * 8);
+        offdo[i] = (unsigned)(row * (int)p.dos[1] + chunk * 8);
+    }
+    const __bf16 *qp_head = nullptr, *dop_head = nullptr;
+    const float *sp_head = nullptr;   // LSE (wave 0) or DELTA - BM (wave 1) of the head's rows, indexed by row0 + tid
+    const int h_first = hkv * p.n_rep + (split >> p.share_log2) * p.n_reps;   // first of the n_reps q heads this block walks
+    auto set_head = [&](int rep) __attribute__((always_inline)) {
+        const int h = h_first + rep;
+        qp_head = (const __bf16 *)p.q + b * p.qs[0] + h * p.qs[2];
+        dop_head = (const __bf16 *)p.d_o + b * p.dos[0] + h * p.dos[2];
+        const long long so = ((long long)b * p.Hq + h) * p.Sq;
+        sp_head = w == 0 ? p.lse + so : p.delta + so - BM;
+    };
+    const float st_mul = tid < BM ? -1.f / p.scale : -1.f;   // threads 0..63 stage -LSE/scale, 64..127 -DELTA, 128..191 positions
+    float sld = 0.f;      // raw LSE / DELTA value in flight
+    bool sld_ok = true;
+    int sld_row0 = 0;     // first row of the tile in flight
+    // LDS byte addresses of this lane's operands in the first buffer's Q tile and of its scalars; all else is an immediate
+    unsigned pa[D / 16], ta[D / 32][2];
+    const unsigned lds0 = lds_address(smem), sa = lds0 + 16 * hh;
+    {
+        const int sw = lds_swz<D>(l32) ^ hh;        // rows l32 + 32 n share the swizzle word of row l32
+#pragma unroll
+        for (int kb = 0; kb < D / 16; kb++) pa[kb] = lds0 + ((l32 * D + (((2 * kb) ^ sw) << 3)) << 1);
+        const int li = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int j = 0; j < D / 32; j++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int col = j * 32 + ((g & 1) << 4) + ((li & 3) << 2), row = 4 * (g >> 1) + (li >> 2) + 8 * e;
+                ta[j][e] = lds0 + ((lds_swz_off<D>(row, col >> 3) + (col & 7)) << 1);
+            }
+    }
+
+    auto run_pass = [&](auto mask_tag) {   // unmasked tiles, then masked ones
+        constexpr bool MASK = decltype(mask_tag)::value;
+        constexpr int list_of = MASK ? 1 : 0;
+        const int cnt = __builtin_amdgcn_readfirstlane(tcount[list_of]);
+        const unsigned short *const list = tlist + list_of * L::MAX_QTILES;
+        int li_ = -1;
+        unsigned short pre = list[0];   // the next call's entry, read one call ahead
+        auto advance = [&](int &rep, int &qt) {   // next tile of this class after (rep, qt); false when done
+            if (++li_ >= cnt) {
+                li_ = 0;
+                if (++rep >= p.n_reps) return false;
+                set_head(rep);
+            }
+            qt = __builtin_amdgcn_readfirstlane((int)pre);
+            pre = list[li_ + 1 < cnt ? li_ + 1 : 0];
+            return true;
+        };
+        auto gload = [&](int qt, int buf) {
+            const int row0 = qt * BM;
+            sld_row0 = row0;
+            const unsigned Qd = lds0 + buf * L::BUF_BYTES, dOd = Qd + L::TILE * 2;
+            if (!MASK) {
+                const unsigned tq = (unsigned)(row0 * (int)p.qs[1]), tdo = (unsigned)(row0 * (int)p.dos[1]);
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    global_to_lds_b128(qp_head + (unsigned long long)(tq + offq[i]), Qd + RPI * (NI * w + i) * D * 2);
+                    global_to_lds_b128(dop_head + (unsigned long long)(tdo + offdo[i]), dOd + RPI * (NI * w + i) * D * 2);
+                }
+            } else {   // rows past the end repeat the last row (they are masked)
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    const int row = RPI * (NI * w + i) + st_row;
+                    const int grow = min(row0 + row, p.Sq - 1);
+                    const int chunk = st_pc ^ lds_swz<D>(row);
+                    global_to_lds_b128(qp_head + (long long)(grow * (int)p.qs[1] + chunk * 8), Qd + RPI * (NI * w + i) * D * 2);
+                    global_to_lds_b128(dop_head + (long long)(grow * (int)p.dos[1] + chunk * 8), dOd + RPI * (NI * w + i) * D * 2);
+                }
+            }
+            if (tid < 2 * BM) {
+                const float *sp = sp_head + row0;
+                if (!MASK) {
+                    sld = sp[tid];
+                } else {
+                    const int r = tid < BM ? tid : tid - BM;
+                    sld_ok = row0 + r < p.Sq;
+                    sld = sp[sld_ok ? tid : (tid < BM ? 0 : BM)];
+                }
+            }
+        };
+        auto lds_store = [&](int buf) {   // the scalars of the tile that gload fetched last
+            float *st = (float *)(smem + buf * L::BUF_BYTES) + L::TILE;
+            if (tid < 2 * BM) {
+                float x = sld * st_mul;
+                if (MASK) x = sld_ok ? x : (tid < BM ? -INFINITY : 0.f);
+                st[tid] = x;
+            } else if (MASK && tid < 3 * BM) {
+                const int row = sld_row0 + tid - 2 * BM;
+                ((int *)st)[tid] = row >= p.Sq ? BWD_QPOS_NONE
+                                   : causal ? q_position(row, p.q_split, p.q_pos0[0], p.q_pos0[1]) : BWD_QPOS_ALL;
+            }
+        };
+        if (cnt == 0) return;
+        int rep = 0, qt = 0;
+        set_head(0);
+        advance(rep, qt);
+        __syncthreads();   // the previous pass has finished reading LDS
+        gload(qt, 0);
+        lds_store(0);
+        tile_barrier();
+        // one barrier per tile: tile t+1 streams into the other buffer, whose readers all passed the previous barrier
+        bool more = true;
+        auto step = [&](auto buf_tag) {
+            constexpr int buf = decltype(buf_tag)::value;
+            const int row0 = sld_row0;
+            more = advance(rep, qt);
+            if (more) gload(qt, buf ^ 1);
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                if (MASK && causal) {   // no row of the sub-tile sees a key of this wave
+                    const int r0 = row0 + 32 * half;
+                    if (r0 >= p.Sq) continue;
+                    int lo, hi;
+                    q_pos_range(r0, min(r0 + 32, p.Sq) - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], lo, hi);
+                    if (hi < w_kpos_lo) continue;
+                }
+                constexpr int Q0 = buf * L::BUF_BYTES, DO0 = Q0 + L::TILE * 2;
+                const int rows = 32 * half, at = DO0 + L::TILE * 2 + rows * 4;
+                // both accumulators start at their rows' scalars (register r <-> row 8*(r/4) + 4*hh + r%4)
+                f32x16 s, dp;
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const f32x4 a = *(lds_f32x4_ptr)(uintptr_t)(sa + at + 32 * g), d4 = *(lds_f32x4_ptr)(uintptr_t)(sa + at + BM * 4 + 32 * g);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        s[4 * g + e] = a[e];
+                        dp[4 * g + e] = d4[e];
+                    }
+                }
+                __builtin_amdgcn_s_setprio(1);
+                lds_gemm_pair_at<D>(pa, Q0 + rows * D * 2, DO0 + rows * D * 2, kreg, vreg, s, dp);
+                __builtin_amdgcn_s_setprio(0);
+                PackedTile pt, ds;
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    int qpos[4] = {0, 0, 0, 0};
+                    if (MASK) {
+                        const i32x4 q4 = *(lds_i32x4_ptr)(uintptr_t)(sa + at + 2 * BM * 4 + 32 * g);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) qpos[e] = q4[e];
+                    }
+#pragma unroll
+                    for (int j = 2 * g; j < 2 * g + 2; j++) {
+                        float p0 = __builtin_amdgcn_exp2f(s[2 * j] * c2), p1 = __builtin_amdgcn_exp2f(s[2 * j + 1] * c2);
+                        if (MASK) {
+                            p0 = kpos <= qpos[2 * (j & 1)] ? p0 : 0.f;
+                            p1 = kpos <= qpos[2 * (j & 1) + 1] ? p1 : 0.f;
+                        }
+                        pt.u[j] = pack2_bf16(p0, p1);
+                        ds.u[j] = bwd_ds_pair(pt.u[j], dp, j);
+                    }
+                }
+                const bf16x8 pb[2] = {operand_of(pt, 0), operand_of(pt, 1)}, db[2] = {operand_of(ds, 0), operand_of(ds, 1)};
+                __builtin_amdgcn_s_setprio(1);
+                lds_tr_gemm_at<D, 2>(ta, DO0 + rows * D * 2, pb, dvacc);
+                lds_tr_gemm_at<D, 2>(ta, Q0 + rows * D * 2, db, dkacc);
+                __builtin_amdgcn_s_setprio(0);
+            }
+            if (more) lds_store(buf ^ 1);
+            tile_barrier();
+        };
+        for (;;) {
+            step(std::integral_constant<int, 0>{});
+            if (!more) break;
+            step(std::integral_constant<int, 1>{});
+            if (!more) break;
+        }
+    };
+    run_pass(std::false_type{});
+    run_pass(std::true_type{});
+
+    if (p.split_log2) {   // a share of the keys' gradients, in the layout of bwd_dkdv_body's partials
+        float *const part = p.part + (((((long long)pair * p.tiles_seen + tile) << p.split_log2) + split) * 8 + w) * (32 * D);
+        store_partial<D>(part, lane, dvacc, 1.f);
+        store_partial<D>(part + 4 * 32 * D, lane, dkacc, p.scale);
+        return;
+    }
+    unsigned char *const stage = smem + w * WaveStage<D>::BYTES;   // every wave is past the last barrier
+    const bool as_bf16 = uniform32(p.flags & LTR_DKDV_BF16);
+    write_key_rows<D, false>(stage, lane, dvacc, 1.f, as_bf16, p.chunk[c].dv, b * p.dvs[0] + hkv * p.dvs[2], p.dvs[1], key0 + 32 * w, sk, D);
+    write_key_rows<D, false>(stage, lane, dkacc, p.scale, as_bf16, p.chunk[c].dk, b * p.dks[0] + hkv * p.dks[2], p.dks[1], key0 + 32 * w, sk, D);
 }
 
 // Sum of the partial dK / dV that the blocks sharing a key tile left in p.part (bf16 and fp32 kernels alike), in the order of
@@ -3240,6 +3535,7 @@ int enable_large_lds() {
         {(const void *)bwd_dkdv_kernel<128, 1>, BwdLds<128, 1>::TOTAL},
         {(const void *)bwd_dkdv_kernel<64, 1>, BwdLds<64, 1>::TOTAL},
         {(const void *)bwd_dkdv_kernel<64, 2>, BwdLds<64, 2>::TOTAL},
+        {(const void *)bwd_dkdv_keywave_kernel<64>, KeyWaveLds<64>::TOTAL},
         {(const void *)fwd_bf16_kernel<128, 1>, fwd_lds_bytes<128>()},
         {(const void *)fwd_bf16_kernel<64, 1>, fwd_lds_bytes<64>()},
         {(const void *)fwd_bf16_kernel<64, 2>, fwd_lds_bytes<64, 2>()},
@@ -3584,14 +3880,18 @@ struct KvSplit {
     int n, reps;      // blocks per key tile; how many of them share out the q heads (the largest power of two that divides both)
     int q_last;       // n > 1: the tiles that have blocks, see seen_tiles
     long long tiles;  // and how many of them there are for one (batch, kv head)
+    double us;        // the launch by the model below
 };
 constexpr double MAX_PART_BYTES = 512e6;   // of partial sums
 struct KvSplitCost {
-    int rows;                        // q rows per step
-    double step_us, fixed;           // time of a step; a block's fixed part in steps
-    double part_bytes_per_us;        // rate at which partials move (each is written and read)
+    int rows;                           // q rows per step
+    double alone_us, alone_fixed_us;    // a block that has its CU to itself: per step, and its fixed part
+    double step_us, fixed_us;           // what a block costs its CU when there are enough of them
+    double tail;                        // of an average block, at the end of such a launch
+    double reduce_us;                   // the reduction's launch
+    double part_bytes_per_us;           // rate at which partials move (each is written and read)
 };
-KvSplit kv_split(const KvSplitCost &cost, int D, int keys, bool causal, int B, int Hkv, int n_rep, int Sq, int q_split, const int *q_pos0,
+KvSplit kv_split(const KvSplitCost &cost, int max_n, int D, int keys, bool causal, int B, int Hkv, int n_rep, int Sq, int q_split, const int *q_pos0,
                  const ChunkDev *chunk, int n_chunks) {
     auto steps_at = [&](long long kpos) -> long long {   // steps of one q head that see the key at position kpos
         long long rows = Sq;
@@ -3613,18 +3913,16 @@ KvSplit kv_split(const KvSplitCost &cost, int D, int keys, bool causal, int B, i
         total += 0.5 * n * (first + last);
         longest = std::max(longest, first);
     }
-    KvSplit best{1, 1, q_last, tiles};
+    KvSplit best{1, 1, q_last, tiles, 0};
     if (tiles == 0) return best;
     const double cus = device_cus(), blocks = (double)tiles * B * Hkv, avg = total / tiles * n_rep, most = (double)longest * n_rep;
-    double best_us = 0;
-    for (int n = 1; n <= 32 && n <= most; n *= 2) {
-        const double one = avg / n + cost.fixed, max_one = (double)(((long long)most + n - 1) / n) + cost.fixed;
-        const double launch = std::max(max_one, blocks * n * one / cus + 0.25 * one);
+    for (int n = 1; n <= max_n && n <= std::max(most, 1.0); n *= 2) {
+        const double one = avg / n * cost.step_us + cost.fixed_us, longest_us = (double)(((long long)most + n - 1) / n) * cost.alone_us + cost.alone_fixed_us;
         const double bytes = blocks * n * keys * D * 8.0;
-        double us = launch * cost.step_us;
-        if (n > 1) us += 2.0 + 2.0 * bytes / cost.part_bytes_per_us;   // 2 us: the reduction's launch
-        if (n == 1 || (us < best_us && bytes <= MAX_PART_BYTES)) {
-            best_us = us;
+        double us = std::max(longest_us, blocks * n * one / cus + cost.tail * one);
+        if (n > 1) us += cost.reduce_us + 2.0 * bytes / cost.part_bytes_per_us;
+        if (n == 1 || (us < best.us && bytes <= MAX_PART_BYTES)) {
+            best.us = us;
             best.n = n;
         }
     }
@@ -3636,6 +3934,7 @@ KvSplit kv_split(const KvSplitCost &cost, int D, int keys, bool causal, int B, i
 struct BwdPlan {
     int f32_ks;         // fp32: 0 = scalar kernels, else the key shares per row group of bwd_dq_f32_mfma_kernel
     bool wide_kv;       // dK/dV kernel: 256 keys per block (two 32-key halves per wave, head dim 64)
+    bool key_waves;     // dK/dV kernel: bwd_dkdv_keywave_kernel (head dim 64)
     int keys_per_block;
     long long kv_tiles; // key blocks over all chunks of one (batch, kv head)
     long long kv_blocks;
@@ -3651,13 +3950,16 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
                  int n_chunks, bool may_split = false) {
     BwdPlan pl;
     pl.f32_ks = 0;
-    pl.split = KvSplit{1, 1, 0x7fffffff, 0};
+    pl.split = KvSplit{1, 1, 0x7fffffff, 0, 0};
     pl.part_bytes = 0;
     pl.dq_ks = 1;
     pl.dq_group = pl.kv_group = 1;
     may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
+    pl.key_waves = false;
     auto split_keys = [&](const KvSplitCost &cost) {
-        if (may_split) pl.split = kv_split(cost, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks);
+        pl.split = kv_split(cost, may_split ? 32 : 1, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks);
+    };
+    auto size_parts = [&]() {
         if (pl.split.n > 1) pl.part_bytes = (int64_t)pl.split.tiles * B * Hkv * pl.split.n * pl.keys_per_block * D * 2 * 4;
     };
     if (f32) {
@@ -3684,36 +3986,49 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         // 27064), but they would move single elements by the whole sum's error, which from about here on exceeds 1e-4 of them:
         // the tolerance to which results of this path are to stay the same
         may_split = may_split && (long long)(Hq / Hkv) * Sq <= 4096;
-        split_keys(D == 128 ? KvSplitCost{32, 9.0, 2.0, 6e6} : KvSplitCost{32, 4.5, 1.5, 6e6});
+        split_keys(D == 128 ? KvSplitCost{32, 9.0, 18.0, 9.0, 18.0, 0.25, 2.0, 6e6} : KvSplitCost{32, 4.5, 6.75, 4.5, 6.75, 0.25, 2.0, 6e6});
+        size_parts();
         pl.dq_qtiles = pl.dq_slots = (Sq + pl.dq_rows - 1) / pl.dq_rows;
         pl.dq_blocks = (long long)pl.dq_qtiles * B * Hq;
         return pl;
     }
     const bool causal_ = (flags & LTR_CAUSAL) != 0;
-    // keys per block of the dK/dV kernel: 256 (two 32-key halves per wave, about 12 % less time per key) pays at head dim 64
-    // when the wider blocks fill the device's CUs about as evenly as the 128-key blocks do (equal blocks, no mask), or, under
-    // a causal mask (unequal blocks), when a block walks many q tiles and there are several rounds of blocks to balance
-    // with; the caller can force either size
+    // keys per block of the dK/dV kernel: 256 (two 32-key halves per wave) pays at head dim 64 for long equal blocks without any masked
+    // tile, against bwd_dkdv_keywave_kernel (us, 256 keys / one wave per 32 keys, no mask): 128 heads S=4096 1000 / 1060, 128 heads S=2048 263 / 276,
+    // 192 heads S=1024 116 / 115; with tails 160 heads S=1231 562 / 443 (its masked pass spills), causal 30 heads S=2571 315 / 235
     bool wide = (flags & LTR_DKDV_KEYS_256) != 0;
     if (!wide && !(flags & LTR_DKDV_KEYS_128) && D == 64 && !(flags & (LTR_NO_DKDV | LTR_HEAD_COLS))) {
         long long blocks256 = 0, blocks128 = 0;
+        bool tails = Sq % 64 != 0;
         for (int c = 0; c < n_chunks; c++) {
             blocks256 += (chunk[c].sk + 255) / 256;
             blocks128 += (chunk[c].sk + 127) / 128;
+            tails = tails || chunk[c].sk % 256 != 0;
         }
         blocks256 *= (long long)B * Hkv;
         blocks128 *= (long long)B * Hkv;
-        const long long q_tiles = (long long)(Hq / Hkv) * ((Sq + 63) / 64);
+        const long long q_tiles = (long long)(Hq / Hkv) * (Sq / 64);
         const int cus = device_cus();
-        if (causal_) wide = q_tiles >= 96 && blocks256 >= 4LL * cus;
-        else wide = q_tiles >= 16 && cu_fill(blocks256, cus) * 1.12 >= cu_fill(blocks128, cus);
+        wide = !causal_ && !tails && q_tiles >= 32 && cu_fill(blocks256, cus) * 1.12 >= cu_fill(blocks128, cus);
     }
     pl.wide_kv = wide;
     pl.keys_per_block = wide ? BwdLds<64, 2>::BN : BwdLds<64, 1>::BN;
     pl.kv_tiles = 0;
     for (int c = 0; c < n_chunks; c++) pl.kv_tiles += (chunk[c].sk + pl.keys_per_block - 1) / pl.keys_per_block;
     pl.kv_blocks = pl.kv_tiles * B * Hkv;
-    split_keys(D == 128 ? KvSplitCost{64, 1.4, 8.0, 8e6} : KvSplitCost{64, wide ? 1.9 : 1.0, wide ? 6.0 : 8.0, 6e6});
+    if (D == 128 || (flags & LTR_HEAD_COLS) || wide) {
+        split_keys(D == 128 ? KvSplitCost{64, 1.4, 11.2, 1.4, 11.2, 0.25, 2.0, 8e6}
+                            : wide ? KvSplitCost{64, 1.9, 11.4, 1.9, 11.4, 0.25, 2.0, 6e6} : KvSplitCost{64, 1.0, 8.0, 1.0, 8.0, 0.25, 2.0, 6e6});
+    } else {
+        // head dim 64: one wave per 32 keys (two blocks per CU) or two (one block).  A block alone on its CU is faster with eight
+        // waves, a CU is faster with two blocks of four.  Constants fitted to 195 launches each (60 shapes, n = 1 .. 32; rms 7 %)
+        split_keys(KvSplitCost{64, 1.43, 6.7, 0.82, 3.4, 1.35, 3.5, 19e6});
+        const KvSplit one_wave = pl.split;
+        split_keys(KvSplitCost{64, 1.14, 7.0, 1.01, 5.8, 0.6, 4.0, 17e6});
+        pl.key_waves = one_wave.us < 0.96 * pl.split.us;
+        if (pl.key_waves) pl.split = one_wave;
+    }
+    size_parts();
     // query rows per block of the dQ kernel: 512 (two 32-row blocks per wave) pays at head dim 64 when the wider blocks still
     // fill the device, and under a causal mask only on sequences long enough that the diagonal does not dominate
     bool wide_q = (flags & LTR_DQ_ROWS_512) != 0;
@@ -3743,7 +4058,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     const int slots = device_cus() / 8;
     pl.dq_group = pair_group(pairs, (long long)pl.dq_slots * (Hq / Hkv), slots,
                              causal_ && pl.dq_slots == pl.dq_qtiles && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks));
-    pl.kv_group = pair_group(pairs, (pl.split.n > 1 ? pl.split.tiles : pl.kv_tiles) * pl.split.n, slots,
+    pl.kv_group = pair_group(pairs, (pl.split.n > 1 ? pl.split.tiles : pl.kv_tiles) * pl.split.n, pl.key_waves ? 2 * slots : slots,
                              causal_ && key_tiles_uneven(Sq, pl.keys_per_block, q_split, q_pos0, chunk, n_chunks));
     return pl;
 }
@@ -4145,6 +4460,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
                                : launch((const void *)bwd_dkdv_pad_kernel<64>, kv_grid, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
         else if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, kv_grid, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
         else if (pl.wide_kv) rc = launch((const void *)bwd_dkdv_kernel<64, 2>, kv_grid, BwdLds<64, 2>::NT, BwdLds<64, 2>::TOTAL, st, p);
+        else if (pl.key_waves) rc = launch((const void *)bwd_dkdv_keywave_kernel<64>, kv_grid, KeyWaveLds<64>::NT, KeyWaveLds<64>::TOTAL, st, p);
         else rc = launch((const void *)bwd_dkdv_kernel<64, 1>, kv_grid, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
         if (rc || pl.split.n == 1) return rc;
         rc = D == 128 ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
@@ -4246,7 +4562,8 @@ int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work
         else snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_kernel<%d, %d>", D, f.wide ? 2 : 1);
         if (b.dq_ks > 1) snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_shares_kernel<%d, %d>", D, b.dq_ks);
         else snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_kernel<%d, %d>", D, b.wide_q ? 2 : 1);
-        snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);
+        if (b.key_waves) snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_keywave_kernel<%d>", D);
+        else snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);
     }
     if (ws) {
         ws->blocks_per_tile = shared ? b.split.n : 1;

@@ -1,0 +1,55 @@
+"""bwd_dkdv_keywave_kernel (head dim 64, one wave per 32 keys), which launches with many key tiles take: against the dense oracle, at
+the edges of its tiles (128 keys per block, 32 per wave, 64 rows per step in two halves)."""
+import pytest
+import torch
+
+from oracle import ring_attention_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,q_pos,split,chunks,causal,share", [
+    (24, 16, 16, 140, 0, None, [(140, 0)], True, False),                                   # a wave with 12 keys, a row tile with 12 rows
+    (20, 16, 16, 97, (40, 300), 33, [(31, 0), (130, 31), (64, 500)], True, False),         # two segments; keys of a chunk no row sees
+    (20, 16, 16, 65, 0, None, [(129, 0)], False, False),                                   # one row and one key past a tile
+    (40, 8, 8, 256, 0, None, [(256, 0)], True, False),                                     # nothing past a tile
+    (36, 8, 8, 1, 200, None, [(1, 0), (300, 1)], True, False),                             # a single row
+    (3, 32, 8, 294, 0, None, [(294, 0)], True, True),                                      # shared key tiles, four q heads per kv head
+])
+def test_key_waves(ltr, B, Hq, Hkv, Sq, q_pos, split, chunks, causal, share):
+    D, total = 64, sum(n for n, _ in chunks)
+    plan = ltr.attn_plan(B, Hq, Hkv, D, Sq, [n for n, _ in chunks], [p for _, p in chunks], q_pos, split, causal, share_keys=share)
+    assert plan["dkdv"]["kernel"] == "bwd_dkdv_keywave_kernel<64>" and plan["dkdv"]["keys"] == 128
+    assert plan["dkdv"].get("blocks_per_tile", 1) == (4 if share else 1)
+    g = torch.Generator().manual_seed(Sq)
+    mk = lambda s, h: torch.randn(B, s, h, D, generator=g).to(torch.bfloat16)
+    q, do, k, v = mk(Sq, Hq), mk(Sq, Hq), mk(total, Hkv), mk(total, Hkv)
+    at = [sum(n for n, _ in chunks[:i]) for i in range(len(chunks))]
+    cut = lambda t: [t[:, a:a + n] for a, (n, _) in zip(at, chunks)]
+    pos = [p for _, p in chunks]
+    qp = q_pos if isinstance(q_pos, tuple) else (q_pos, q_pos)
+    rows = torch.arange(Sq)
+    qpos = rows + qp[0] if split is None else torch.where(rows < split, rows + qp[0], rows - split + qp[1])
+    kpos = torch.cat([torch.arange(p, p + n) for n, p in chunks])
+    _, _, _, dk_ref, dv_ref = orc.dense_attention_grads(q.float(), k.float(), v.float(), do.float(), qpos, kpos, causal, dtype=torch.float32)
+    qd, kd, vd, dod = q.cuda(), k.cuda(), v.cuda(), do.cuda()
+    o, lse = ltr.attn_fwd(qd, cut(kd), cut(vd), pos, q_pos, split, causal)
+    delta = ltr.attn_delta(o, dod)
+
+    def grads(dtype, start):
+        dk, dv = (torch.full(k.shape, start, dtype=dtype, device="cuda") for _ in range(2))
+        dq = torch.zeros(q.shape, dtype=torch.float32, device="cuda")
+        ltr.attn_bwd_accumulate(qd, dod, lse, delta, cut(kd), cut(vd), pos, dq, cut(dk), cut(dv), q_pos, split, causal, do_dq=False, share_keys=share)
+        return dk.cpu().float() - (start if dtype == torch.float32 else 0), dv.cpu().float() - (start if dtype == torch.float32 else 0)
+
+    acc, res = grads(torch.float32, 0.5), grads(torch.bfloat16, 7.0)
+    for x, y, ref in zip(acc, res, (dk_ref, dv_ref)):
+        seen = ref.flatten(2).norm(dim=2) > 0
+        assert (x - ref).norm() <= 1e-2 * ref.norm()        # 2e-3 .. 3.1e-3: P, dS and the inputs' products in bf16
+        # a row or key lost at a border is the whole of a few entries: by groups of 32 keys as well
+        for first in range(0, total, 32):
+            a, b = x[:, first:first + 32], ref[:, first:first + 32]
+            assert (a - b).norm() <= 3e-2 * b.norm() + 1e-5, first
+        assert (x[~seen].abs() < 1e-6).all() and (y[~seen] == 0).all()
+        # bf16 rounding (2^-8 of the value) and the cancellation of the accumulator's start value (2^-23 of 0.5 + |x|)
+        assert ((y - x).abs() <= x.abs() / 256 + 1e-6).all()
