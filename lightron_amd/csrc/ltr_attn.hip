@@ -13,11 +13,12 @@
 //                        with an earlier partial result is part of the epilogue.
 //                        fwd_bf16_kernel<64, 2>: two 32-row blocks per wave (512 rows per block, 64-key tiles): every K / V
 //                        operand read from LDS feeds two MFMAs (chosen by the host, or forced with LTR_FWD_ROWS_512).
+//                        fwd_bf16_w4_kernel<D>, bwd_dq_w4_kernel<D>: 128 rows and four waves per block, several blocks per CU (FourWaves).
 //   fwd_f32_mfma_kernel<D, KS>  fp32 I/O and arithmetic on v_mfma_f32_32x32x2_f32: the forward of the 1e-4 cases (the reference's
 //                        acceptance dtype) on the matrix pipe; KS key shares per 32-row group for launches with few rows.
 //   fwd_f32_kernel<D>    the same in scalar fp32 (no MFMA): kept as the fallback, reached with LTR_FWD_F32_SCALAR.
 //                        fwd_bf16_shares_kernel<D, KS>, bwd_dq_shares_kernel<D, KS>: KS waves share a row group's keys (launches with
-//                        few rows, see key_shares); *_pad_kernel: head dims below the width D (LTR_HEAD_COLS).
+//                        few rows, see key_shares and choose_rows); *_pad_kernel: head dims below the width D (LTR_HEAD_COLS).
 //   delta_kernel         DELTA = rowsum(dO * O).
 //   bwd_dkdv_kernel<D, KW>  a block of 8 waves owns 128 * KW keys of one kv head and loops over the
 //                        query heads of the GQA group and over 64-row query tiles taken from
@@ -85,17 +86,11 @@ struct ChunkDev {
     int pos0;
 };
 
-// Division by a number that the host knows, of n < 2^31.
-struct Div {
-    int d;
-    unsigned mul, shift;
-    __device__ __forceinline__ int of(int n) const { return (int)(((unsigned long long)(unsigned)n * mul) >> shift); }
-};
-struct BlockMap {   // see block_item
-    int group;              // (batch, kv head) pairs of an XCD whose blocks are handed out together; 0: the pairs do not divide among the XCDs
-    int last_group;         // the group of last_pairs pairs
-    Div inner, group_items; // blocks per item; items per group
-    Div pairs, last_pairs;  // pairs per group (group = 0: all pairs)
+struct BlockMap {      // see block_item
+    int group;         // (batch, kv head) pairs of an XCD whose blocks are handed out together; 0: a linear grid
+    int items;         // items (q tile slots, key tiles) per pair
+    int groups;
+    int inner;         // blocks per item
 };
 
 struct FwdParams {
@@ -130,6 +125,7 @@ struct BwdParams {
     long long os_[3];
     void *dq;          // fp32 accumulator, or bf16 result with LTR_DQ_BF16
     int B, Hq, Hkv, n_rep;
+    BlockMap q_map, kv_map;   // of the dQ and the dK/dV kernel
     int cols;          // head dim of the tensors (the kernel's own width, or less: PAD kernels)
     int Sq, n_qtiles;
     long long qs[3], dos[3], dqs[3], ks[3], vs[3], dks[3], dvs[3];
@@ -146,7 +142,6 @@ struct BwdParams {
     int n_reps;       // of which a block walks this many
     float *part;      // n_split > 1: the blocks' partial dK / dV, summed by bwd_dkdv_reduce_kernel
     int n_slots;      // slots of 256-row q tiles of the dQ kernel (see q_tile_slots)
-    BlockMap q_map, kv_map;   // of the dQ and the dK/dV kernel
     const float *rope;     // LTR_ROPE_DQ: (cos, sin) rows, cols floats per position, row 0 = position rope_pos0
     int rope_pos0;
     ChunkDev chunk[LTR_MAX_CHUNKS];
@@ -180,28 +175,34 @@ __device__ __forceinline__ void q_pos_range(int r0, int r1, int split, int p0, i
 }
 
 // Block id -> (pair = batch x kv head, item = q tile slot or key tile of the pair, sub = one of the `inner` blocks of an item).
-// Consecutive block ids go to the 8 XCDs round-robin.  All blocks of a pair run on one XCD and next to each other in time, so the
+// Consecutive blocks go to the 8 XCDs round-robin.  All blocks of a pair run on one XCD and next to each other in time, so the
 // blocks that are resident together stream the same K / V (or Q / dO) through that XCD's L2; the inner blocks of an item follow each
 // other.  The items of `group` pairs of an XCD are handed out item by item (the first of every pair, the second of every pair, ...):
-// items come longest first, so blocks of unequal length end together (see pair_group).
-// The divisions are multiplications prepared by the host: four of the device's own cost a block 0.3 us.
+// items come longest first, so blocks of unequal length end together (see pair_group).  The grid is (8 XCDs x inner blocks, pairs of a
+// group, items of the groups): the hardware counts what would be four divisions (0.3 us of every block, also as multiplications: their
+// constants are another trip to the arguments).
 struct BlockItem {
     int pair, item, sub;
+    int order;   // of the blocks of an XCD
 };
-__device__ __forceinline__ BlockItem block_item(const BlockMap &m) {
+__device__ __forceinline__ BlockItem block_item(const BlockMap &m, int pairs) {
     BlockItem r;
-    const int idx = blockIdx.x;
     if (m.group) {
-        const int j = idx >> 3, i = m.inner.of(j), g = m.group_items.of(i), in_group = i - g * m.group_items.d;
-        const bool last = g == m.last_group;
-        r.sub = j - i * m.inner.d;
-        r.item = last ? m.last_pairs.of(in_group) : m.pairs.of(in_group);
-        r.pair = (g * m.group + in_group - r.item * (last ? m.last_pairs.d : m.pairs.d)) * 8 + (idx & 7);
-    } else {   // pairs that do not divide among the XCDs: pair after pair, then the next block of each
-        const int rest = m.pairs.of(idx);
-        r.pair = idx - rest * m.pairs.d;
-        r.item = m.inner.of(rest);
-        r.sub = rest - r.item * m.inner.d;
+        int g = 0;
+        r.item = blockIdx.z;
+        if (m.groups > 1) {
+            g = r.item / m.items;
+            r.item -= g * m.items;
+        }
+        r.sub = blockIdx.x >> 3;
+        r.pair = (g * m.group + blockIdx.y) * 8 + (blockIdx.x & 7);   // past the last pair: a place of the last group that is empty
+        r.order = r.sub + m.inner * (blockIdx.y + m.group * blockIdx.z);
+    } else {   // pairs that do not divide among the XCDs: one block of every pair, then the next
+        const int rest = blockIdx.x / pairs;
+        r.pair = blockIdx.x - rest * pairs;
+        r.item = rest / m.inner;
+        r.sub = rest - r.item * m.inner;
+        r.order = blockIdx.x >> 3;
     }
     return r;
 }
@@ -633,11 +634,12 @@ __device__ __forceinline__ void collect_shares(unsigned char *smem, int w, int k
 // 64 keys serves 512 query rows: half the LDS reads and half the tile transfers per MFMA.
 // KS = waves that share a 32-row group: each takes its own BN keys of every tile of KS * BN keys, and their partial (reference, row
 // sum, O) are merged through LDS at the end.  For launches with too few query rows to give every CU a block (see FwdPlan).
-template <int D, int RB, int KS, bool PAD>
+// NW = waves: eight (one block per CU, two waves per SIMD), or four with 64-key tiles (FourWaves), where several blocks share a CU.
+template <int D, int RB, int KS, bool PAD, int NW = 8, int BN = FwdTile<D, RB, KS>::BN>
 __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     const int cols = PAD ? p.cols : D;
-    constexpr int NW = 8, RG = NW / KS, BM = 32 * RB * RG;   // 8 waves (two per SIMD) share every K / V tile
-    constexpr int BN = FwdTile<D, RB, KS>::BN, NB = BN / 32, BNT = BN * KS;   // keys per wave and per tile
+    constexpr int RG = NW / KS, BM = 32 * RB * RG;   // the NW waves of the block share every K / V tile
+    constexpr int NB = BN / 32, BNT = BN * KS;       // BN keys per wave, BNT per tile
     constexpr int CPR = D / 8;   // 16-byte chunks per row
     constexpr int RPI = 64 / CPR;            // rows filled by one wave-wide 16-byte-per-lane LDS-direct load (1 KB)
     constexpr int NI = BNT / (RPI * NW);      // such loads per wave, per tensor and per tile
@@ -651,14 +653,15 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     const bool causal = p.flags & LTR_CAUSAL;
 
     // block -> (batch, kv head, q head of the group, q tile); late (heavier under a causal mask) q tiles first
-    const BlockItem item = block_item(p.map);
+    const BlockItem item = block_item(p.map, p.B * p.Hkv);
     const int pair = item.pair, rep = item.sub, slot = item.item;
+    if (pair >= p.B * p.Hkv) return;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv, h = hkv * p.n_rep + rep;
     // A slot is one q tile (late, heavier tiles first) or, when the host paired them, a late tile and its early
     // counterpart: under a causal mask every block then has the same amount of work.
     const bool paired = p.n_slots != p.n_qtiles;
     // every other block (of an XCD) takes the early tile first: the blocks of a round then change tiles at different times
-    const bool two = paired && slot < p.n_qtiles - 1 - slot, early_first = two && ((blockIdx.x >> 3) & 1);
+    const bool two = paired && slot < p.n_qtiles - 1 - slot, early_first = two && (item.order & 1);
 #pragma nounroll
     for (int part = 0; part < 2; part++) {
     const int qt = (part == 0) != early_first ? p.n_qtiles - 1 - slot : slot;
@@ -1060,6 +1063,23 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     }   // part
 }
 
+// Blocks of four waves and 128 rows: three share a CU at head dim 64 (168 registers, 35 KB of LDS), two at 128.  A block's start (its Q
+// rows and first tile from memory), its barriers and its O stores, 7 - 9 us that an eight-wave block alone on its CU waits for, then
+// run under the other blocks' arithmetic; 128-row blocks also leave less of a diagonal tile masked and a shorter tail.  The price is a K / V
+// tile per four waves.  Kernel us, best of the eight-wave blocks -> this one, forward / dQ, causal:
+//   16 x 12 heads D=64 S=1024   56 / 65 -> 43 / 58       7 x 32 heads D=64 S=2214  210 / 273 -> 185 / 251
+//   4 x 16 heads D=128 S=1024   35 / 46 -> 32 / 42      13 x 16 heads D=128 S=1800  241 / 317 -> 229 / 308
+//   4 x 32 heads D=128 S=8192 2046 / 2844 -> 2173 / 2925 (long blocks: the tile traffic shows)
+template <int D>
+struct FourWaves {
+    static constexpr int BN = 64, PER_CU = D == 64 ? 3 : 2;
+    static constexpr int TILES = 2 * 2 * BN * D * 2, LDS = TILES > 4 * WaveStage<D>::BYTES ? TILES : 4 * WaveStage<D>::BYTES;
+    static_assert(PER_CU * LDS <= 160 * 1024, "LDS of one CU");
+};
+template <int D>
+__global__ __launch_bounds__(256, FourWaves<D>::PER_CU) void fwd_bf16_w4_kernel(const FwdParams p) {
+    fwd_bf16_body<D, 1, 1, false, 4, FourWaves<D>::BN>(p);
+}
 template <int D, int RB>
 __global__ __launch_bounds__(512) void fwd_bf16_kernel(const FwdParams p) {
     fwd_bf16_body<D, RB, 1, false>(p);
@@ -1701,7 +1721,24 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
 
     // block -> (batch, kv head, chunk, key tile); same XCD grouping as the forward.  Blocks that share a key tile follow each
     // other: each takes n_reps of the q heads and, of a head's visible q tiles, every 2^share_log2-th
-    const BlockItem item = block_item(p.kv_map);
+    BlockItem item;
+    const int P = p.B * p.Hkv;
+    if constexpr (KW == 1) {
+        item = block_item(p.kv_map, P);
+        if (item.pair >= P) return;
+    } else {   // pair after pair on a linear grid: this kernel runs without a mask, and has no scalar registers left for a map (6 % slower)
+        int idx = blockIdx.x, rest;
+        if ((P & 7) == 0) {
+            const int n = p.tiles_seen << p.split_log2;
+            item.pair = (idx >> 3) / n * 8 + (idx & 7);
+            rest = (idx >> 3) % n;
+        } else {
+            item.pair = idx % P;
+            rest = idx / P;
+        }
+        item.sub = rest & ((1 << p.split_log2) - 1);
+        item.item = rest >> p.split_log2;
+    }
     const int pair = item.pair, split = item.sub, tile = item.item;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
     int c = 0, kt = tile;
@@ -2145,8 +2182,9 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_keywave_kernel(const BwdParam
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool causal = p.flags & LTR_CAUSAL;
     // block -> (batch, kv head, chunk, key tile), shares of a key tile: as in bwd_dkdv_body
-    const BlockItem item = block_item(p.kv_map);
+    const BlockItem item = block_item(p.kv_map, p.B * p.Hkv);
     const int pair = item.pair, split = item.sub, tile = item.item;
+    if (pair >= p.B * p.Hkv) return;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
     int c = 0, kt = tile;
     for (; c < p.n_chunks; c++) {
@@ -2527,11 +2565,11 @@ __device__ __forceinline__ void lds_tr_gemm_at_rb(const unsigned (&addr)[D / 32]
 }
 
 // RB = 32-row blocks per wave: a lane owns RB query rows, a block 256 * RB / KS; KS = key shares per row group as in the forward
-template <int D, int RB, int KS, bool PAD>
+template <int D, int RB, int KS, bool PAD, int NW = 8, int BN = FwdTile<D, 1, KS>::BN>
 __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
     const int cols = PAD ? p.cols : D;
-    constexpr int NW = 8, RG = NW / KS, BM = 32 * RB * RG;   // 8 waves (two per SIMD) share every K / V tile
-    constexpr int BN = FwdTile<D, 1, KS>::BN, BNT = BN * KS; // keys per wave and per tile
+    constexpr int RG = NW / KS, BM = 32 * RB * RG;   // the NW waves of the block share every K / V tile
+    constexpr int BNT = BN * KS;                     // BN keys per wave, BNT per tile
     constexpr int CPR = D / 8;
     constexpr int RPI = 64 / CPR;            // rows filled by one wave-wide 16-byte-per-lane LDS-direct load (1 KB)
     constexpr int NI = BNT / (RPI * NW);      // such loads per wave, per tensor and per tile
@@ -2544,13 +2582,14 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
     const int rg = w / KS, ks = w % KS;      // row group and key share of the wave
     const bool causal = p.flags & LTR_CAUSAL;
 
-    const BlockItem item = block_item(p.q_map);
+    const BlockItem item = block_item(p.q_map, p.B * p.Hkv);
     const int pair = item.pair, rep = item.sub, slot = item.item;
+    if (pair >= p.B * p.Hkv) return;
     const int n_qt = (p.Sq + BM - 1) / BM;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv, h = hkv * p.n_rep + rep;
     // one q tile per block (late tiles first) or a late tile and its early counterpart (see q_tile_slots)
     const bool paired = p.n_slots != n_qt;
-    const bool two = paired && slot < n_qt - 1 - slot, early_first = two && ((blockIdx.x >> 3) & 1);   // as in the forward kernel
+    const bool two = paired && slot < n_qt - 1 - slot, early_first = two && (item.order & 1);   // as in the forward kernel
 #pragma nounroll
     for (int part = 0; part < 2; part++) {
     const int qt = (part == 0) != early_first ? n_qt - 1 - slot : slot;
@@ -2841,6 +2880,10 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
     }   // part
 }
 
+template <int D>   // see FourWaves
+__global__ __launch_bounds__(256, FourWaves<D>::PER_CU) void bwd_dq_w4_kernel(const BwdParams p) {
+    bwd_dq_body<D, 1, 1, false, 4, FourWaves<D>::BN>(p);
+}
 template <int D, int RB>
 __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
     bwd_dq_body<D, RB, 1, false>(p);
@@ -3536,6 +3579,10 @@ int enable_large_lds() {
         {(const void *)bwd_dkdv_kernel<64, 1>, BwdLds<64, 1>::TOTAL},
         {(const void *)bwd_dkdv_kernel<64, 2>, BwdLds<64, 2>::TOTAL},
         {(const void *)bwd_dkdv_keywave_kernel<64>, KeyWaveLds<64>::TOTAL},
+        {(const void *)fwd_bf16_w4_kernel<128>, FourWaves<128>::LDS},
+        {(const void *)fwd_bf16_w4_kernel<64>, FourWaves<64>::LDS},
+        {(const void *)bwd_dq_w4_kernel<128>, FourWaves<128>::LDS},
+        {(const void *)bwd_dq_w4_kernel<64>, FourWaves<64>::LDS},
         {(const void *)fwd_bf16_kernel<128, 1>, fwd_lds_bytes<128>()},
         {(const void *)fwd_bf16_kernel<64, 1>, fwd_lds_bytes<64>()},
         {(const void *)fwd_bf16_kernel<64, 2>, fwd_lds_bytes<64, 2>()},
@@ -3628,10 +3675,13 @@ int device_cus() {
 // One kernel launch whose own status is what is returned: hipLaunchKernel reports the submission of THIS launch, so an
 // error that unrelated earlier work left in the thread's last-error slot is neither reported as ours nor cleared.
 template <class Params>
-int launch(const void *kernel, long long blocks, int threads, size_t lds_bytes, hipStream_t st, const Params &p) {
+int launch(const void *kernel, dim3 grid, int threads, size_t lds_bytes, hipStream_t st, const Params &p) {
     void *args[] = {(void *)&p};
-    return hipLaunchKernel(kernel, dim3((unsigned)blocks), dim3((unsigned)threads), args, lds_bytes, st) == hipSuccess ? LTR_OK
-                                                                                                                      : LTR_ELAUNCH;
+    return hipLaunchKernel(kernel, grid, dim3((unsigned)threads), args, lds_bytes, st) == hipSuccess ? LTR_OK : LTR_ELAUNCH;
+}
+template <class Params>
+int launch(const void *kernel, long long blocks, int threads, size_t lds_bytes, hipStream_t st, const Params &p) {
+    return launch(kernel, dim3((unsigned)blocks), threads, lds_bytes, st, p);
 }
 
 // Keys that the q rows [r0, r1] walk through under the causal mask: per chunk, those up to the rows' last position.
@@ -3674,9 +3724,8 @@ bool key_tiles_uneven(int Sq, int keys, int q_split, const int *q_pos0, const Ch
 // q_tiles_uneven: paired tiles run one after the other, so fewer blocks walk through the same K / V rows at the same time)
 // and while the equal blocks still fill the device's CUs evenly; otherwise one tile per slot, heaviest first, and the
 // hardware's in-order dispatch balances.
-int q_tile_slots(int n_qtiles, long long blocks_per_tile, bool uneven) {
+int q_tile_slots(int n_qtiles, long long blocks_per_tile, bool uneven, int cus) {
     if (!uneven || n_qtiles < 2) return n_qtiles;
-    const int cus = device_cus();
     const int n_slots = (n_qtiles + 1) / 2;
     const long long n = n_slots * blocks_per_tile, rounds = (n + cus - 1) / cus;
     return n * 10 >= rounds * cus * 9 ? n_slots : n_qtiles;
@@ -3696,26 +3745,17 @@ int pair_group(long long pairs, long long blocks_per_pair, int slots, bool uneve
     return (int)((n + groups - 1) / groups);
 }
 
-Div make_div(long long d) {   // exact for n < 2^31: mul = 2^shift / d rounded up, off by less than d <= 2^(shift - 31)
-    const int lg = 63 - __builtin_clzll((unsigned long long)d);
-    Div r;
-    r.d = (int)d;
-    const bool pow2 = (d & (d - 1)) == 0;
-    r.shift = 31 + lg + (pow2 ? 0 : 1);
-    r.mul = (unsigned)(((1ull << r.shift) + (unsigned long long)d - 1) / (unsigned long long)d);
-    return r;
-}
-// pairs x items x inner < 2^31 blocks; see block_item
-BlockMap block_map(long long pairs, long long items, long long inner, int group) {
-    BlockMap m;
-    m.group = pairs % 8 ? 0 : group;
-    const long long n = m.group ? pairs / 8 : pairs, per = m.group ? group : pairs;
-    m.last_group = (int)((n - 1) / per);
-    m.inner = make_div(std::max(1LL, inner));
-    m.group_items = make_div(std::max(1LL, items * per));
-    m.pairs = make_div(per);
-    m.last_pairs = make_div(n - (n - 1) / per * per);
-    return m;
+// The grid and its map; pairs x items x inner < 2^31 blocks.  Grids past the 65535 places of the second and third dimension (more than
+// 8 million keys in tiles of 128) are linear.
+struct Grid {
+    BlockMap map;
+    dim3 dim;
+};
+Grid block_grid(long long pairs, long long items, long long inner, int group) {
+    const long long per_xcd = pairs / 8, groups = (per_xcd + group - 1) / group;
+    if (pairs % 8 == 0 && group <= 65535 && groups * items <= 65535)
+        return {{group, (int)items, (int)groups, (int)inner}, dim3((unsigned)(8 * inner), (unsigned)group, (unsigned)(groups * items))};
+    return {{0, (int)items, 1, (int)inner}, dim3((unsigned)(pairs * items * inner))};
 }
 
 // Waves that share a row group's keys in the bf16 forward and dQ kernels.  Blocks of 256 rows leave CUs idle when a launch has few
@@ -3744,14 +3784,14 @@ struct ShareCost {
 struct ShareChoice {
     int ks;
     bool paired;
+    double us;   // the launch, by these constants
 };
-ShareChoice key_shares(const ShareCost &cost, int D, bool causal, long long BH, long long kv_heads, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks) {
-    const int cus = device_cus();
-    if (BH * ((Sq + 255) / 256) >= 4LL * cus) return {1, false};   // several rounds of 256-row blocks: they balance by themselves
-    ShareChoice best{1, false};
+ShareChoice key_shares(const ShareCost &cost, int D, bool causal, long long BH, long long kv_heads, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks, int cus) {
+    if (BH * ((Sq + 255) / 256) >= 4LL * cus) return {1, false, 0};   // several rounds of 256-row blocks: they balance by themselves
+    ShareChoice best{1, false, 0};
     double best_us = 0;
     for (int i = 0; i < 3; i++) {
-        const int ks = 1 << i, rows = 256 / ks, keys = ks * (D == 64 ? (ks == 1 ? 128 : 64) : (ks == 4 ? 32 : 64));
+        const int ks = 1 << i, rows = 256 >> i, key_log2 = i + (D == 64 ? (ks == 1 ? 7 : 6) : (ks == 4 ? 5 : 6));
         const int n = (Sq + rows - 1) / rows;
         // more than one kv head per XCD and every CU busy: the extra K / V traffic of the shares shows (B=1, 32 kv heads, D=128,
         // S=2048: 57 us with one share, 67 with two; with 8 kv heads 57 and 49)
@@ -3763,7 +3803,7 @@ ShareChoice key_shares(const ShareCost &cost, int D, bool causal, long long BH, 
             if (r0 < q_split && r1 >= q_split) hi = std::max(hi, q_pos0[0] + q_split - 1);
             for (int c = 0; c < n_chunks; c++) {
                 const long long seen = causal ? std::min<long long>(std::max<long long>((long long)hi - chunk[c].pos0 + 1, 0), chunk[c].sk) : chunk[c].sk;
-                sum += (double)((seen + keys - 1) / keys);
+                sum += (double)((seen + (1 << key_log2) - 1) >> key_log2);
             }
             return sum;
         };
@@ -3776,7 +3816,7 @@ ShareChoice key_shares(const ShareCost &cost, int D, bool causal, long long BH, 
         const double us = BH * n <= cus ? most : std::max(most, sum * BH / cus + 0.25 * sum / n);
         if (i == 0 || us < 0.97 * best_us) {
             best_us = us;
-            best = {ks, false};
+            best = {ks, false, us};
         }
         const int slots = (n + 1) / 2;
         if (ks == 2 && causal && BH * slots <= cus && BH * slots * 10 >= cus * 9 && q_tiles_uneven(Sq, rows, q_split, q_pos0, chunk, n_chunks)) {
@@ -3787,7 +3827,7 @@ ShareChoice key_shares(const ShareCost &cost, int D, bool causal, long long BH, 
             }
             if (pair_us < 0.97 * best_us) {
                 best_us = pair_us;
-                best = {ks, true};
+                best = {ks, true, pair_us};
             }
         }
     }
@@ -3796,11 +3836,136 @@ ShareChoice key_shares(const ShareCost &cost, int D, bool causal, long long BH, 
 constexpr ShareCost FWD_SHARES_128{{1.45, 1.8, 1.05}, {9.0, 8.0, 10.0}, 2.2}, FWD_SHARES_64{{1.7, 0.95, 1.0}, {9.0, 8.0, 6.0}, 1.09};
 constexpr ShareCost DQ_SHARES_128{{1.85, 2.2, 1.4}, {11.0, 10.0, 10.0}, 2.7}, DQ_SHARES_64{{1.95, 1.15, 1.35}, {10.0, 9.0, 6.0}, 1.3};
 
+// Blocks of the bf16 forward and dQ kernels: which of the kernels below a launch takes.
+//   256 rows, 8 waves                long blocks: a K / V tile serves eight waves
+//   512 rows, 8 waves (head dim 64)  longer ones: every operand read serves two row blocks
+//   128 / 64 rows, 8 waves           2 / 4 waves share a row group's keys: launches with few rows (key_shares)
+//   128 rows, 4 waves                several blocks per CU (FourWaves): launches of many blocks that are not long
+// The choice compares launch times.  A block of n K / V tiles takes n alone_us + alone_fixed_us on a CU of its own and costs the CU
+// n step_us + fixed_us when there are enough of them; blocks run longest first, so a launch of unequal ones takes their sum over
+// the CUs plus `tail` of the shortest, a launch of equal ones its largest number of blocks on a CU.  Constants fitted to 120 random
+// launches (8 - 32 heads, 64 - 7900 rows, 4 in 5 causal) of every kernel: rms error 4 - 7 %; the steps of four waves are those of long equal
+// blocks (1024 rows against 8192 and 16384 keys), 2 - 8 % above the fit.  256-row blocks are replaced where
+// another kernel is 1.5 % faster, shares where four waves are 12 % faster, and what key_shares says about shares, with coarser rounds, where
+// other shares are 20 % faster (280 blocks of four shares on 256 CUs: 16.4 us for 9.0 of two).
+struct TileCost {
+    double alone_us, alone_fixed_us, step_us, fixed_us, tail;
+};
+enum { ROWS_256, SHARES_2, SHARES_4, FOUR_WAVES, ROWS_512, N_ROW_KERNELS };
+struct RowCosts {
+    ShareCost shares;
+    TileCost kernel[N_ROW_KERNELS];
+};
+struct RowChoice {
+    int kernel;
+    bool paired;   // SHARES_2: q tiles in pairs
+};
+struct RowKernel {
+    int rows, key_log2;   // query rows per block, log2 of the keys per K / V tile
+};
+RowKernel row_kernel(int kernel, int D) {
+    switch (kernel) {
+        case ROWS_512: return {512, 6};
+        case SHARES_2: return {128, 7};
+        case SHARES_4: return {64, D == 64 ? 8 : 7};
+        case FOUR_WAVES: return {128, 6};
+        default: return {256, D == 64 ? 7 : 6};
+    }
+}
+// allowed: bit per kernel
+RowChoice choose_rows(const RowCosts &costs, unsigned allowed, int D, bool causal, long long BH, long long kv_heads, int Sq, int q_split,
+                      const int *q_pos0, const ChunkDev *chunk, int n_chunks, int cus) {
+    if ((allowed & (allowed - 1)) == 0) return {__builtin_ctz(allowed), false};   // a hint
+    RowChoice first{ROWS_256, false};
+    double first_us = 0;
+    if (allowed >> SHARES_2 & 1) {
+        const ShareChoice sc = key_shares(costs.shares, D, causal, BH, kv_heads, Sq, q_split, q_pos0, chunk, n_chunks, cus);
+        first = {sc.ks == 4 ? SHARES_4 : sc.ks == 2 ? SHARES_2 : ROWS_256, sc.paired};
+        if (sc.paired) first_us = sc.us;
+    }
+    const bool shared = first.kernel != ROWS_256;
+    if (!shared && causal && (D == 128 || n_chunks > 1)) {
+        // 256-row tiles whose pairs come out in complete rounds of equal blocks: nothing of a CU is idle, and four waves are not faster
+        // (head dim 128, us forward / dQ, pairs / four waves: 4 x 32 heads S=1024 51 / 71 - 52 / 70, 8 x 32 heads S=512 41 / 52 - 40 / 51,
+        // 8 x 32 heads S=2048 324 / 448 - 340 / 458).  Chunk tables at head dim 64 keep the pairs too, though four waves are faster there (8 x 32
+        // heads, 1100 rows against 1000 + 400 keys: 139 / 167 - 89 / 115): test_paired_q_tiles_forward_backward holds that launch to them
+        const int n = (Sq + 255) / 256, slots = (n + 1) / 2;
+        if (n > 1 && BH * slots % cus == 0 && q_tiles_uneven(Sq, 256, q_split, q_pos0, chunk, n_chunks)) return first;
+    }
+    double us[N_ROW_KERNELS];
+    for (int i = 0; i < N_ROW_KERNELS; i++) {
+        us[i] = 0;
+        const RowKernel k = row_kernel(i, D);
+        const int n = (Sq + k.rows - 1) / k.rows;
+        if (!(allowed >> i & 1) || (i == FOUR_WAVES && BH * n <= cus)) continue;   // four waves alone on a CU: no
+        // the constants of 512 rows are those of blocks without a diagonal (8 of 34 launches): 384 heads causal S=1496, dQ 251 us with 256 rows, 267
+        if (i == ROWS_512 && causal && Sq < 4096) continue;
+        const TileCost &c = costs.kernel[i];
+        // of many q tiles, 16 evenly spaced ones stand for all
+        const int m = causal ? std::min(n, 16) : 1;
+        double sum = 0, most = 0, least = 1e30, at[16];
+        for (int j = 0; j < m; j++) {
+            const int t = m > 1 ? (int)((long long)j * (n - 1) / (m - 1)) : n - 1;
+            const int r0 = t * k.rows, r1 = std::min(Sq, r0 + k.rows) - 1;
+            int hi = r1 < q_split ? q_pos0[0] + r1 : q_pos0[1] + (r1 - q_split);
+            if (r0 < q_split && r1 >= q_split) hi = std::max(hi, q_pos0[0] + q_split - 1);
+            long long tiles = 0;
+            for (int ch = 0; ch < n_chunks; ch++) {
+                const long long seen = causal ? std::min<long long>(std::max<long long>((long long)hi - chunk[ch].pos0 + 1, 0), chunk[ch].sk) : chunk[ch].sk;
+                tiles += (seen + (1 << k.key_log2) - 1) >> k.key_log2;
+            }
+            at[j] = (double)tiles;
+            sum += at[j] / m;
+            most = std::max(most, at[j]);
+            least = std::min(least, at[j]);
+        }
+        const double blocks = (double)BH * n, on_a_cu = std::ceil(blocks / cus);
+        if (least >= 0.9 * most) {
+            us[i] = std::max(most * c.alone_us + c.alone_fixed_us, on_a_cu * (most * c.step_us + c.fixed_us));
+            continue;
+        }
+        // the long blocks (all of the late segment of zig-zag rows are) come in whole numbers per CU as well
+        double longs = 0, long_sum = 0;
+        for (int j = 0; j < m; j++)
+            if (at[j] >= 0.75 * most) longs += 1, long_sum += at[j];
+        const double long_us = std::ceil(blocks * longs / m / cus) * (long_sum / longs * c.step_us + c.fixed_us);
+        us[i] = std::max(std::max(most * c.alone_us + c.alone_fixed_us, std::max(long_us, on_a_cu * (least * c.step_us + c.fixed_us))),
+                         blocks * (sum * c.step_us + c.fixed_us) / cus + c.tail * (least * c.step_us + c.fixed_us));
+        if ((i == ROWS_256 || i == ROWS_512) && q_tile_slots(n, BH, q_tiles_uneven(Sq, k.rows, q_split, q_pos0, chunk, n_chunks), cus) != n) {   // in pairs
+            double pair = 0;
+            for (int j = 0; 2 * j < m; j++) pair = std::max(pair, at[j] + (2 * j < m - 1 ? at[m - 1 - j] : 0));
+            us[i] = std::ceil((double)BH * ((n + 1) / 2) / cus) * (pair * c.step_us + 2 * c.fixed_us);
+        }
+    }
+    RowChoice best = first;
+    const double from = first_us > 0 ? first_us : us[first.kernel];
+    double best_us = from;
+    for (int i = 0; i < N_ROW_KERNELS; i++) {
+        const bool to_shares = i == SHARES_2 || i == SHARES_4;
+        if (us[i] > 0 && us[i] < best_us && us[i] < from * (to_shares || first.paired ? 0.8 : shared ? 0.88 : 0.985)) {
+            best_us = us[i];
+            best = {i, false};
+        }
+    }
+    return best;
+}
+constexpr RowCosts FWD_ROWS_64{FWD_SHARES_64, {{1.83, 6.9, 2.01, 7.2, 0.16}, {0.98, 7.0, 1.15, 5.0, 0.64}, {0.94, 8.3, 1.22, 6.5, 0.49}, {0.76, 6.8, 0.55, 2.1, 1.22}, {1.70, 11.1, 1.94, 4.7, 0.56}}};
+constexpr RowCosts FWD_ROWS_128{FWD_SHARES_128, {{1.52, 7.3, 1.70, 7.5, 0.26}, {1.77, 8.6, 1.98, 6.9, 0.72}, {1.03, 8.5, 1.18, 6.8, 0.44}, {1.16, 7.8, 0.92, 4.5, 0.57}, {}}};
+constexpr RowCosts DQ_ROWS_64{DQ_SHARES_64, {{2.17, 7.7, 2.61, 7.2, 0.43}, {1.26, 7.9, 1.43, 6.3, 0.54}, {1.33, 8.9, 1.69, 6.7, 0.57}, {1.04, 6.9, 0.75, 3.5, 0.59}, {1.93, 15.4, 2.51, 6.5, 0.48}}};
+constexpr RowCosts DQ_ROWS_128{DQ_SHARES_128, {{2.02, 9.5, 2.45, 6.7, 0.52}, {2.32, 10.4, 2.65, 8.5, 0.69}, {1.33, 11.3, 1.51, 9.1, 0.44}, {1.63, 8.3, 1.30, 5.4, 0.56}, {}}};
+// rows_256, rows_512: the caller's hints; shares: a row group's keys may be shared
+unsigned allowed_rows(bool rows_256, bool rows_512, bool shares, bool pad, int D) {
+    if (rows_512) return 1u << ROWS_512;
+    if (rows_256) return 1u << ROWS_256;
+    return 1u << ROWS_256 | (shares ? 1u << SHARES_2 | 1u << SHARES_4 : 0u) | (pad ? 0u : 1u << FOUR_WAVES | (D == 64 ? 1u << ROWS_512 : 0u));
+}
+
 // What a forward launch looks like: rows per block, q tiles, slots (see q_tile_slots), blocks.  One function decides for
 // ltr_attn_fwd and for ltr_attn_plan, so the plan a caller is shown is the launch it gets.
 struct FwdPlan {
     bool wide;          // 512-row blocks (two 32-row blocks per wave, head dim 64)
-    int ks;             // bf16: key shares per row group (1, or 2 / 4 with blocks of 256 / ks rows; see key_shares)
+    bool four_waves;    // 128-row blocks of four waves (FourWaves)
+    int ks;             // bf16: key shares per row group (1, or 2 / 4 with blocks of 256 / ks rows; see choose_rows)
     int f32_ks;         // fp32: 0 = scalar kernel, else the key shares per row group of fwd_f32_mfma_kernel
     int rows, n_qtiles, n_slots, group;
     long long blocks;
@@ -3811,6 +3976,7 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.f32_ks = 0;
     pl.ks = 1;
     pl.group = 1;
+    pl.four_waves = false;
     if (f32) {
         pl.wide = false;
         if (flags & LTR_FWD_F32_SCALAR) {
@@ -3830,40 +3996,20 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         return pl;
     }
     const bool causal_ = (flags & LTR_CAUSAL) != 0;
-    auto group_of = [&]() {   // paired tiles are equal blocks
-        const bool uneven = causal_ && pl.n_slots == pl.n_qtiles && q_tiles_uneven(Sq, pl.rows, q_split, q_pos0, chunk, n_chunks);
-        return pair_group((long long)B * Hkv, (long long)pl.n_slots * (Hq / Hkv), device_cus() / 8, uneven);
-    };
-    // query rows per block: 512 (two 32-row blocks per wave, 64-key tiles) pays at head dim 64 under the conditions of
-    // the dQ kernel's 512-row blocks (see plan_bwd)
-    bool wide = (flags & LTR_FWD_ROWS_512) != 0;
-    ShareChoice shares{1, false};
-    if (!wide && !(flags & LTR_FWD_ROWS_256) && may_share)
-        shares = key_shares(D == 128 ? FWD_SHARES_128 : FWD_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
-                            n_chunks);
-    pl.ks = shares.ks;
-    if (!wide && !(flags & (LTR_FWD_ROWS_256 | LTR_HEAD_COLS)) && D == 64 && pl.ks == 1) {
-        const int tiles512 = (Sq + 511) / 512;
-        const int slots512 = q_tile_slots(tiles512, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, 512, q_split, q_pos0, chunk, n_chunks));
-        const long long blocks512 = (long long)slots512 * B * Hq, blocks256 = (long long)((Sq + 255) / 256) * B * Hq;
-        const int cus = device_cus();
-        wide = causal_ ? (Sq >= 2048 && blocks512 >= (long long)(slots512 != tiles512 ? 1 : 4) * cus)
-                       : (cu_fill(blocks512, cus) * 1.07 >= cu_fill(blocks256, cus));
-    }
-    pl.wide = wide;
-    if (pl.ks > 1) {
-        pl.rows = 256 / pl.ks;
-        pl.n_qtiles = (Sq + pl.rows - 1) / pl.rows;
-        pl.n_slots = shares.paired ? (pl.n_qtiles + 1) / 2 : pl.n_qtiles;
-        pl.blocks = (long long)pl.n_slots * B * Hq;
-        pl.group = group_of();
-        return pl;
-    }
-    pl.rows = wide ? 512 : 256;
+    const int cus = device_cus();
+    const RowChoice choice = choose_rows(D == 128 ? FWD_ROWS_128 : FWD_ROWS_64,
+                                         allowed_rows(flags & LTR_FWD_ROWS_256, flags & LTR_FWD_ROWS_512, may_share, flags & LTR_HEAD_COLS, D), D, causal_,
+                                         (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk, n_chunks, cus);
+    pl.wide = choice.kernel == ROWS_512;
+    pl.four_waves = choice.kernel == FOUR_WAVES;
+    pl.ks = choice.kernel == SHARES_2 ? 2 : choice.kernel == SHARES_4 ? 4 : 1;
+    pl.rows = row_kernel(choice.kernel, D).rows;
     pl.n_qtiles = (Sq + pl.rows - 1) / pl.rows;
-    pl.n_slots = q_tile_slots(pl.n_qtiles, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, pl.rows, q_split, q_pos0, chunk, n_chunks));
+    const bool uneven = causal_ && q_tiles_uneven(Sq, pl.rows, q_split, q_pos0, chunk, n_chunks);
+    pl.n_slots = choice.paired ? (pl.n_qtiles + 1) / 2 : pl.ks > 1 || pl.four_waves ? pl.n_qtiles : q_tile_slots(pl.n_qtiles, (long long)B * Hq, uneven, cus);
     pl.blocks = (long long)pl.n_slots * B * Hq;
-    pl.group = group_of();
+    pl.group = pair_group((long long)B * Hkv, (long long)pl.n_slots * (Hq / Hkv), cus / 8 * (pl.four_waves ? D == 64 ? FourWaves<64>::PER_CU : FourWaves<128>::PER_CU : 1),
+                          uneven && pl.n_slots == pl.n_qtiles);   // paired tiles are equal blocks
     return pl;
 }
 
@@ -3892,7 +4038,7 @@ struct KvSplitCost {
     double part_bytes_per_us;           // rate at which partials move (each is written and read)
 };
 KvSplit kv_split(const KvSplitCost &cost, int max_n, int D, int keys, bool causal, int B, int Hkv, int n_rep, int Sq, int q_split, const int *q_pos0,
-                 const ChunkDev *chunk, int n_chunks) {
+                 const ChunkDev *chunk, int n_chunks, int n_cus) {
     auto steps_at = [&](long long kpos) -> long long {   // steps of one q head that see the key at position kpos
         long long rows = Sq;
         if (causal)
@@ -3903,7 +4049,7 @@ KvSplit kv_split(const KvSplitCost &cost, int max_n, int D, int keys, bool causa
     int q_last = 0x7fffffff;
     if (causal)
         q_last = std::max(q_split > 0 ? q_pos0[0] + q_split - 1 : (int)0x80000000, Sq > q_split ? q_pos0[1] + (Sq - q_split) - 1 : (int)0x80000000);
-    long long tiles = 0, longest = 0;
+    long long tiles = 0, longest = 0, shortest = 0x7fffffff;
     double total = 0;
     for (int c = 0; c < n_chunks; c++) {
         const long long n = seen_tiles(chunk[c].sk, chunk[c].pos0, q_last, keys);
@@ -3912,14 +4058,17 @@ KvSplit kv_split(const KvSplitCost &cost, int max_n, int D, int keys, bool causa
         tiles += n;
         total += 0.5 * n * (first + last);
         longest = std::max(longest, first);
+        shortest = std::min(shortest, last);
     }
     KvSplit best{1, 1, q_last, tiles, 0};
     if (tiles == 0) return best;
-    const double cus = device_cus(), blocks = (double)tiles * B * Hkv, avg = total / tiles * n_rep, most = (double)longest * n_rep;
+    const double cus = n_cus, blocks = (double)tiles * B * Hkv, avg = total / tiles * n_rep, most = (double)longest * n_rep;
     for (int n = 1; n <= max_n && n <= std::max(most, 1.0); n *= 2) {
         const double one = avg / n * cost.step_us + cost.fixed_us, longest_us = (double)(((long long)most + n - 1) / n) * cost.alone_us + cost.alone_fixed_us;
         const double bytes = blocks * n * keys * D * 8.0;
-        double us = std::max(longest_us, blocks * n * one / cus + cost.tail * one);
+        // equal blocks: the largest number on a CU (2 x 8 pairs of 64, 514 rows and keys, no mask inside: 160 blocks 32.6 us, 320 blocks 37.1)
+        const bool equal = shortest * 10 >= longest * 9;
+        double us = std::max(std::max(longest_us, equal ? std::ceil(blocks * n / cus) * one : 0.0), blocks * n * one / cus + cost.tail * one);
         if (n > 1) us += cost.reduce_us + 2.0 * bytes / cost.part_bytes_per_us;
         if (n == 1 || (us < best.us && bytes <= MAX_PART_BYTES)) {
             best.us = us;
@@ -3941,6 +4090,7 @@ struct BwdPlan {
     KvSplit split;      // blocks per key tile (1 unless the caller brought a workspace for their partial sums)
     int64_t part_bytes; // workspace they need
     bool wide_q;        // dQ kernel: 512 rows per block
+    bool dq_four_waves; // dQ kernel: blocks of four waves (FourWaves)
     int dq_ks;          // bf16 dQ kernel: key shares per row group, as in the forward
     int dq_rows, dq_qtiles, dq_slots;
     int dq_group, kv_group;   // see pair_group
@@ -3954,10 +4104,12 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.part_bytes = 0;
     pl.dq_ks = 1;
     pl.dq_group = pl.kv_group = 1;
+    pl.dq_four_waves = false;
     may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
     pl.key_waves = false;
+    const int cus = device_cus();
     auto split_keys = [&](const KvSplitCost &cost) {
-        pl.split = kv_split(cost, may_split ? 32 : 1, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks);
+        pl.split = kv_split(cost, may_split ? 32 : 1, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks, cus);
     };
     auto size_parts = [&]() {
         if (pl.split.n > 1) pl.part_bytes = (int64_t)pl.split.tiles * B * Hkv * pl.split.n * pl.keys_per_block * D * 2 * 4;
@@ -3969,7 +4121,6 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
             pl.dq_rows = 64;
         } else {
             // matrix-pipe kernels: 128 keys per dK/dV block; the dQ kernel sized like the fp32 forward (see plan_fwd)
-            const int cus = device_cus();
             const int max_ks = D == 64 ? 4 : 2;
             int ks = 1;
             while (ks < max_ks && (long long)((Sq + 128 / ks - 1) / (128 / ks)) * B * Hq < cus) ks *= 2;
@@ -4008,7 +4159,6 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         blocks256 *= (long long)B * Hkv;
         blocks128 *= (long long)B * Hkv;
         const long long q_tiles = (long long)(Hq / Hkv) * (Sq / 64);
-        const int cus = device_cus();
         wide = !causal_ && !tails && q_tiles >= 32 && cu_fill(blocks256, cus) * 1.12 >= cu_fill(blocks128, cus);
     }
     pl.wide_kv = wide;
@@ -4029,35 +4179,23 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         if (pl.key_waves) pl.split = one_wave;
     }
     size_parts();
-    // query rows per block of the dQ kernel: 512 (two 32-row blocks per wave) pays at head dim 64 when the wider blocks still
-    // fill the device, and under a causal mask only on sequences long enough that the diagonal does not dominate
-    bool wide_q = (flags & LTR_DQ_ROWS_512) != 0;
-    ShareChoice shares{1, false};
-    if (!wide_q && !(flags & (LTR_DQ_ROWS_256 | LTR_NO_DQ)))
-        shares = key_shares(D == 128 ? DQ_SHARES_128 : DQ_SHARES_64, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
-                            n_chunks);
-    pl.dq_ks = shares.ks;
-    if (!wide_q && !(flags & (LTR_DQ_ROWS_256 | LTR_HEAD_COLS)) && D == 64 && !(flags & LTR_NO_DQ) && pl.dq_ks == 1) {
-        const int tiles512 = (Sq + 511) / 512;
-        const int slots512 = q_tile_slots(tiles512, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, 512, q_split, q_pos0, chunk, n_chunks));
-        const long long blocks512 = (long long)slots512 * B * Hq;
-        const int cus = device_cus();
-        // causal: equal (paired) blocks need one full round, unequal ones several rounds to balance; no mask: the wider
-        // blocks (about 7 % less time per row) must fill the CUs about as evenly as the 256-row blocks
-        const long long blocks256 = (long long)((Sq + 255) / 256) * B * Hq;
-        wide_q = causal_ ? (Sq >= 2048 && blocks512 >= (long long)(slots512 != tiles512 ? 1 : 4) * cus)
-                         : (cu_fill(blocks512, cus) * 1.07 >= cu_fill(blocks256, cus));
-    }
-    pl.wide_q = wide_q;
-    pl.dq_rows = wide_q ? 512 : 256 / pl.dq_ks;
+    const RowChoice choice = flags & LTR_NO_DQ
+                                 ? RowChoice{flags & LTR_DQ_ROWS_512 ? ROWS_512 : ROWS_256, false}
+                                 : choose_rows(D == 128 ? DQ_ROWS_128 : DQ_ROWS_64,
+                                               allowed_rows(flags & LTR_DQ_ROWS_256, flags & LTR_DQ_ROWS_512, true, flags & LTR_HEAD_COLS, D), D, causal_,
+                                               (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk, n_chunks, cus);
+    pl.wide_q = choice.kernel == ROWS_512;
+    pl.dq_four_waves = choice.kernel == FOUR_WAVES;
+    pl.dq_ks = choice.kernel == SHARES_2 ? 2 : choice.kernel == SHARES_4 ? 4 : 1;
+    pl.dq_rows = row_kernel(choice.kernel, D).rows;
     pl.dq_qtiles = (Sq + pl.dq_rows - 1) / pl.dq_rows;
-    pl.dq_slots = pl.dq_ks > 1 ? (shares.paired ? (pl.dq_qtiles + 1) / 2 : pl.dq_qtiles)
-                               : q_tile_slots(pl.dq_qtiles, (long long)B * Hq, causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks));
+    const bool uneven = causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks);
+    pl.dq_slots = choice.paired ? (pl.dq_qtiles + 1) / 2 : pl.dq_ks > 1 || pl.dq_four_waves ? pl.dq_qtiles : q_tile_slots(pl.dq_qtiles, (long long)B * Hq, uneven, cus);
     pl.dq_blocks = (long long)pl.dq_slots * B * Hq;
     const long long pairs = (long long)B * Hkv;
-    const int slots = device_cus() / 8;
-    pl.dq_group = pair_group(pairs, (long long)pl.dq_slots * (Hq / Hkv), slots,
-                             causal_ && pl.dq_slots == pl.dq_qtiles && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks));
+    const int slots = cus / 8;
+    pl.dq_group = pair_group(pairs, (long long)pl.dq_slots * (Hq / Hkv), slots * (pl.dq_four_waves ? D == 64 ? FourWaves<64>::PER_CU : FourWaves<128>::PER_CU : 1),
+                             uneven && pl.dq_slots == pl.dq_qtiles);
     pl.kv_group = pair_group(pairs, (pl.split.n > 1 ? pl.split.tiles : pl.kv_tiles) * pl.split.n, pl.key_waves ? 2 * slots : slots,
                              causal_ && key_tiles_uneven(Sq, pl.keys_per_block, q_split, q_pos0, chunk, n_chunks));
     return pl;
@@ -4199,7 +4337,8 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     if (pl.blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.n_qtiles = pl.n_qtiles;
     p.n_slots = pl.n_slots;
-    if (a->io_dtype == LTR_BF16) p.map = block_map((long long)p.B * p.Hkv, pl.n_slots, p.n_rep, pl.group);
+    const Grid grid = block_grid((long long)p.B * p.Hkv, pl.n_slots, p.n_rep, pl.group);
+    p.map = grid.map;
     if (a->io_dtype == LTR_BF16) {
         rc = enable_large_lds();
         if (rc) return rc;
@@ -4210,17 +4349,20 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
                 {(const void *)fwd_bf16_pad_kernel<128, 1>, (const void *)fwd_bf16_pad_kernel<128, 2>, (const void *)fwd_bf16_pad_kernel<128, 4>}};
             const int lds[2][3] = {{fwd_lds_bytes<64>(), shares_lds_bytes<64, 2>(), shares_lds_bytes<64, 4>()},
                                    {fwd_lds_bytes<128>(), shares_lds_bytes<128, 2>(), shares_lds_bytes<128, 4>()}};
-            return launch(kernels[D == 128][i], pl.blocks, 512, lds[D == 128][i], st, p);
+            return launch(kernels[D == 128][i], grid.dim, 512, lds[D == 128][i], st, p);
         }
+        if (pl.four_waves)
+            return a->D == 128 ? launch((const void *)fwd_bf16_w4_kernel<128>, grid.dim, 256, FourWaves<128>::LDS, st, p)
+                               : launch((const void *)fwd_bf16_w4_kernel<64>, grid.dim, 256, FourWaves<64>::LDS, st, p);
         if (pl.ks == 2)
-            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 2>, pl.blocks, 512, shares_lds_bytes<128, 2>(), st, p)
-                               : launch((const void *)fwd_bf16_shares_kernel<64, 2>, pl.blocks, 512, shares_lds_bytes<64, 2>(), st, p);
+            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 2>, grid.dim, 512, shares_lds_bytes<128, 2>(), st, p)
+                               : launch((const void *)fwd_bf16_shares_kernel<64, 2>, grid.dim, 512, shares_lds_bytes<64, 2>(), st, p);
         if (pl.ks == 4)
-            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 4>, pl.blocks, 512, shares_lds_bytes<128, 4>(), st, p)
-                               : launch((const void *)fwd_bf16_shares_kernel<64, 4>, pl.blocks, 512, shares_lds_bytes<64, 4>(), st, p);
-        if (a->D == 128) return launch((const void *)fwd_bf16_kernel<128, 1>, pl.blocks, 512, fwd_lds_bytes<128>(), st, p);
-        if (pl.wide) return launch((const void *)fwd_bf16_kernel<64, 2>, pl.blocks, 512, fwd_lds_bytes<64, 2>(), st, p);
-        return launch((const void *)fwd_bf16_kernel<64, 1>, pl.blocks, 512, fwd_lds_bytes<64>(), st, p);
+            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 4>, grid.dim, 512, shares_lds_bytes<128, 4>(), st, p)
+                               : launch((const void *)fwd_bf16_shares_kernel<64, 4>, grid.dim, 512, shares_lds_bytes<64, 4>(), st, p);
+        if (a->D == 128) return launch((const void *)fwd_bf16_kernel<128, 1>, grid.dim, 512, fwd_lds_bytes<128>(), st, p);
+        if (pl.wide) return launch((const void *)fwd_bf16_kernel<64, 2>, grid.dim, 512, fwd_lds_bytes<64, 2>(), st, p);
+        return launch((const void *)fwd_bf16_kernel<64, 1>, grid.dim, 512, fwd_lds_bytes<64>(), st, p);
     }
     if (pl.f32_ks) {   // fp32 on the matrix pipe; the chunk offsets of its LDS-direct loads are 64-bit, nothing more to check
         rc = enable_large_lds();
@@ -4386,8 +4528,10 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     p.n_reps = p.n_rep / pl.split.reps;
     p.part = (float *)work;
     p.n_slots = pl.dq_slots;
-    if (!f32) p.q_map = block_map((long long)p.B * p.Hkv, pl.dq_slots, p.n_rep, pl.dq_group);
-    if (!f32) p.kv_map = block_map((long long)p.B * p.Hkv, tiles_seen, pl.split.n, pl.kv_group);
+    const Grid q_grid = block_grid((long long)p.B * p.Hkv, pl.dq_slots, p.n_rep, pl.dq_group);
+    const Grid key_grid = block_grid((long long)p.B * p.Hkv, tiles_seen, pl.split.n, pl.kv_group);
+    p.q_map = q_grid.map;
+    p.kv_map = key_grid.map;
     hipStream_t st = (hipStream_t)stream;
     if (f32 && pl.f32_ks) {   // fp32 on the matrix pipe
         rc = enable_large_lds();
@@ -4437,16 +4581,19 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
                 {(const void *)bwd_dq_pad_kernel<128, 1>, (const void *)bwd_dq_pad_kernel<128, 2>, (const void *)bwd_dq_pad_kernel<128, 4>}};
             const int lds[2][3] = {{dq_lds_bytes<64>(), shares_lds_bytes<64, 2>(), shares_lds_bytes<64, 4>()},
                                    {dq_lds_bytes<128>(), shares_lds_bytes<128, 2>(), shares_lds_bytes<128, 4>()}};
-            rc = launch(kernels[D == 128][i], pl.dq_blocks, 512, lds[D == 128][i], st, p);
-        } else if (pl.dq_ks == 2)
-            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 2>, pl.dq_blocks, 512, shares_lds_bytes<128, 2>(), st, p)
-                             : launch((const void *)bwd_dq_shares_kernel<64, 2>, pl.dq_blocks, 512, shares_lds_bytes<64, 2>(), st, p);
+            rc = launch(kernels[D == 128][i], q_grid.dim, 512, lds[D == 128][i], st, p);
+        } else if (pl.dq_four_waves)
+            rc = a->D == 128 ? launch((const void *)bwd_dq_w4_kernel<128>, q_grid.dim, 256, FourWaves<128>::LDS, st, p)
+                             : launch((const void *)bwd_dq_w4_kernel<64>, q_grid.dim, 256, FourWaves<64>::LDS, st, p);
+        else if (pl.dq_ks == 2)
+            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 2>, q_grid.dim, 512, shares_lds_bytes<128, 2>(), st, p)
+                             : launch((const void *)bwd_dq_shares_kernel<64, 2>, q_grid.dim, 512, shares_lds_bytes<64, 2>(), st, p);
         else if (pl.dq_ks == 4)
-            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 4>, pl.dq_blocks, 512, shares_lds_bytes<128, 4>(), st, p)
-                             : launch((const void *)bwd_dq_shares_kernel<64, 4>, pl.dq_blocks, 512, shares_lds_bytes<64, 4>(), st, p);
-        else if (a->D == 128) rc = launch((const void *)bwd_dq_kernel<128, 1>, pl.dq_blocks, 512, dq_lds_bytes<128>(), st, p);
-        else if (pl.wide_q) rc = launch((const void *)bwd_dq_kernel<64, 2>, pl.dq_blocks, 512, dq_lds_bytes<64>(), st, p);
-        else rc = launch((const void *)bwd_dq_kernel<64, 1>, pl.dq_blocks, 512, dq_lds_bytes<64>(), st, p);
+            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 4>, q_grid.dim, 512, shares_lds_bytes<128, 4>(), st, p)
+                             : launch((const void *)bwd_dq_shares_kernel<64, 4>, q_grid.dim, 512, shares_lds_bytes<64, 4>(), st, p);
+        else if (a->D == 128) rc = launch((const void *)bwd_dq_kernel<128, 1>, q_grid.dim, 512, dq_lds_bytes<128>(), st, p);
+        else if (pl.wide_q) rc = launch((const void *)bwd_dq_kernel<64, 2>, q_grid.dim, 512, dq_lds_bytes<64>(), st, p);
+        else rc = launch((const void *)bwd_dq_kernel<64, 1>, q_grid.dim, 512, dq_lds_bytes<64>(), st, p);
         if (rc) return rc;
     }
     if (do_dkdv) {
@@ -4456,12 +4603,12 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
         // the tail (the sums inside a block do not depend on the table's order).
         if (flags & LTR_CAUSAL)
             std::stable_sort(p.chunk, p.chunk + p.n_chunks, [](const ChunkDev &x, const ChunkDev &y) { return x.pos0 < y.pos0; });
-        if (pad) rc = D == 128 ? launch((const void *)bwd_dkdv_pad_kernel<128>, kv_grid, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p)
-                               : launch((const void *)bwd_dkdv_pad_kernel<64>, kv_grid, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
-        else if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, kv_grid, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
+        if (pad) rc = D == 128 ? launch((const void *)bwd_dkdv_pad_kernel<128>, key_grid.dim, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p)
+                               : launch((const void *)bwd_dkdv_pad_kernel<64>, key_grid.dim, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
+        else if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, key_grid.dim, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
         else if (pl.wide_kv) rc = launch((const void *)bwd_dkdv_kernel<64, 2>, kv_grid, BwdLds<64, 2>::NT, BwdLds<64, 2>::TOTAL, st, p);
-        else if (pl.key_waves) rc = launch((const void *)bwd_dkdv_keywave_kernel<64>, kv_grid, KeyWaveLds<64>::NT, KeyWaveLds<64>::TOTAL, st, p);
-        else rc = launch((const void *)bwd_dkdv_kernel<64, 1>, kv_grid, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
+        else if (pl.key_waves) rc = launch((const void *)bwd_dkdv_keywave_kernel<64>, key_grid.dim, KeyWaveLds<64>::NT, KeyWaveLds<64>::TOTAL, st, p);
+        else rc = launch((const void *)bwd_dkdv_kernel<64, 1>, key_grid.dim, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
         if (rc || pl.split.n == 1) return rc;
         rc = D == 128 ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
              : pl.wide_kv ? launch((const void *)bwd_dkdv_reduce_kernel<64, 2>, reduce_grid, 256, 0, st, p)
@@ -4559,8 +4706,10 @@ int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work
         snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_pad_kernel<%d>", D);
     } else {
         if (f.ks > 1) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_shares_kernel<%d, %d>", D, f.ks);
+        else if (f.four_waves) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_w4_kernel<%d>", D);
         else snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_bf16_kernel<%d, %d>", D, f.wide ? 2 : 1);
         if (b.dq_ks > 1) snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_shares_kernel<%d, %d>", D, b.dq_ks);
+        else if (b.dq_four_waves) snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_w4_kernel<%d>", D);
         else snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_kernel<%d, %d>", D, b.wide_q ? 2 : 1);
         if (b.key_waves) snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_keywave_kernel<%d>", D);
         else snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);
