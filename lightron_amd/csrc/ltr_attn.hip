@@ -15,7 +15,8 @@
 //                        operand read from LDS feeds two MFMAs (chosen by the host, or forced with LTR_FWD_ROWS_512).
 //                        fwd_bf16_w4_kernel<D>, bwd_dq_w4_kernel<D>: 128 rows and four waves per block, several blocks per CU (FourWaves).
 //   fwd_f32_mfma_kernel<D, KS>  fp32 I/O and arithmetic on v_mfma_f32_32x32x2_f32: the forward of the 1e-4 cases (the reference's
-//                        acceptance dtype) on the matrix pipe; KS key shares per 32-row group for launches with few rows.
+//                        acceptance dtype) on the matrix pipe; KS key shares per 32-row group for launches with few rows,
+//                        <64, 4, 16> groups of 16 rows for those with the fewest (F32Rows16; bwd_dq_f32_mfma_kernel likewise).
 //   fwd_f32_kernel<D>    the same in scalar fp32 (no MFMA): kept as the fallback, reached with LTR_FWD_F32_SCALAR.
 //                        fwd_bf16_shares_kernel<D, KS>, bwd_dq_shares_kernel<D, KS>: KS waves share a row group's keys (launches with
 //                        few rows, see key_shares and choose_rows); *_pad_kernel: head dims below the width D (LTR_HEAD_COLS).
@@ -1227,7 +1228,7 @@ struct F32Mfma {
     static_assert(LDS <= 160 * 1024, "LDS of one CU");
 };
 
-template <int D, int KS>
+template <int D, int KS, int GROUP = 32>   // GROUP: rows of a row group; 16: see F32Rows16
 __global__ __launch_bounds__(256) void fwd_f32_mfma_kernel(const FwdParams p) {
     using L = F32Mfma<D, KS>;
     constexpr int NW = L::NW, RG = L::RG, BM = L::BM, BN = L::BN, TILE = L::TILE;
@@ -1475,6 +1476,254 @@ __global__ __launch_bounds__(256) void fwd_f32_mfma_kernel(const FwdParams p) {
         }
         op += ROWS_PER_IT * os1;
     });
+}
+
+
+// Four key shares per row group (head dim 64), for launches with the fewest rows: groups of 16 rows on v_mfma_f32_16x16x4_f32 (the rate of
+// 32x32x2), so that a launch has twice the blocks of 32-row groups: 2 x 8 heads of 256 rows give every CU one instead of every other.
+// A wave's 32 keys of a step are two sub-tiles whose chains alternate.  Operand layout (lane l, i = l % 16, g = l / 16): A[i][g], B[g][i],
+// C[4g + r][i] for accumulator register r.  As in the 32-row kernels both contractions choose their order: step 4s + j of S^T contracts d = 16s + 4g + j (K: one 128-bit read for four steps), step r of O^T / dQ^T the keys 4g + r of a
+// sub-tile, whose P^T / dS^T is the accumulator register r as it is.  f32_swz serves both reads (rows 4 apart land 4 chunks apart).
+// Each wave ends up with 16 of the 64 columns of all shares and writes 16 bytes per lane.  Bound by the wave's chain of MFMAs
+// and its LDS reads (one block per CU).  Kernel us, 32 -> 16 rows, forward and dQ, 2 x 8 heads of 256 rows against 256, 768, 1024 keys:
+// 10.8 -> 7.5, 22.0 -> 14.6, 27.7 -> 18.1 and 15.0 -> 9.4, 29.9 -> 18.7, 37.3 -> 23.3; one head of 8 rows and 64 keys 7.1 -> 5.0, 9.2 -> 6.2.
+struct F32Rows16 {
+    static constexpr int D = 64, KS = 4, BM = 16;
+    static constexpr int PART = 16 * 64 * 4;             // one wave's D x 16 partial result
+    static constexpr int PART_OFF = 4 * 32 * 4;          // after the waves' references and sums (forward)
+    static constexpr int BYTES = PART_OFF + KS * PART;
+    static_assert(BYTES <= F32Mfma<D, KS>::LDS, "reuses the tile buffers");
+};
+__device__ __forceinline__ float quarter_max(float x) {   // over the four lanes of a row (16 apart)
+    const unsigned u = __float_as_uint(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return xhalf_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+__device__ __forceinline__ float quarter_sum(float x) {
+    const unsigned u = __float_as_uint(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return xhalf_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+// The row-group operand Q (or dO) of lane (row i, g): reg[4s + j] = X[row][16s + 4g + j]
+__device__ __forceinline__ void rows16_operand(const float *row, int g, float (&reg)[16]) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const f32x4 x = *(const f32x4 *)(row + 16 * s + 4 * g);
+#pragma unroll
+        for (int j = 0; j < 4; j++) reg[4 * s + j] = x[j];
+    }
+}
+// acc[kb] += (rows 16 kb .. of the 32-row tile T) x reg^T, both sub-tiles' chains in turn
+__device__ __forceinline__ void rows16_scores(const float *T, int i, int g, const float (&reg)[16], f32x4 (&acc)[2]) {
+    const int sw = f32_swz(i);   // rows 16 apart share it
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const f32x4 a = *(const f32x4 *)(T + i * 64 + (((4 * s + g) ^ sw) << 2)), b = *(const f32x4 *)(T + (16 + i) * 64 + (((4 * s + g) ^ sw) << 2));
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], reg[4 * s + j], acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j], reg[4 * s + j], acc[1], 0, 0, 0);
+        }
+    }
+}
+// out[db] += T^T x w over the 32 keys: w[kb][r] belongs to key 16 kb + 4g + r of the lane's row
+__device__ __forceinline__ void rows16_weighted(const float *T, int i, int g, const f32x4 (&w)[2], f32x4 (&out)[4]) {
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int key = 16 * kb + 4 * g + r, sw = f32_swz(key);
+            const float *row = T + key * 64 + (i & 3);
+#pragma unroll
+            for (int db = 0; db < 4; db++)
+                out[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(row[((4 * db + (i >> 2)) ^ sw) << 2], w[kb][r], out[db], 0, 0, 0);
+        }
+}
+// Wave ks collects columns 16 ks .. +15 of all shares (times their factors): lane (row i, g) gets columns 16 ks + 4g .. +3.  The tile
+// buffers are no longer read.
+__device__ __forceinline__ f32x4 rows16_collect(unsigned char *smem, int ks, int lane, const f32x4 (&part)[4], float mul) {
+    float *const parts = (float *)(smem + F32Rows16::PART_OFF);
+#pragma unroll
+    for (int db = 0; db < 4; db++) {
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = part[db][e] * mul;
+        *(f32x4 *)(parts + ((ks * 4 + db) * 64 + lane) * 4) = x;
+    }
+    __syncthreads();
+    f32x4 own = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const f32x4 x = *(const f32x4 *)(parts + ((k * 4 + ks) * 64 + lane) * 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) own[e] += x[e];
+    }
+    return own;
+}
+
+template <>
+__global__ __launch_bounds__(256) void fwd_f32_mfma_kernel<64, 4, 16>(const FwdParams p) {   // see F32Rows16
+    using L = F32Mfma<64, 4>;
+    constexpr int D = 64, BM = F32Rows16::BM, BN = L::BN, TILE = L::TILE;
+    constexpr int CPR = D / 4, RPI = 64 / CPR, NI = BN / (RPI * L::NW);
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool causal = p.flags & LTR_CAUSAL;
+    const int qt = p.n_qtiles - 1 - blockIdx.x / (p.B * p.Hq);     // late (heavier under a causal mask) q tiles first
+    const int bh = blockIdx.x % (p.B * p.Hq);
+    const int b = bh / p.Hq, h = bh % p.Hq, hkv = h / p.n_rep;
+    const int row0 = qt * BM, my_row = row0 + i;
+    const bool row_ok = my_row < p.Sq;
+    const int my_pos = q_position(my_row, p.q_split, p.q_pos0[0], p.q_pos0[1]);
+    int blk_lo, blk_hi;
+    q_pos_range(row0, min(row0 + BM, p.Sq) - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], blk_lo, blk_hi);
+
+    float qreg[16];
+    rows16_operand((const float *)p.q + b * p.qs[0] + (long long)min(my_row, p.Sq - 1) * p.qs[1] + h * p.qs[2], g, qreg);
+    f32x4 oacc[4];
+#pragma unroll
+    for (int db = 0; db < 4; db++) oacc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;   // exp2 domain; l_run: this lane's quarter of the keys
+    const float c2 = p.scale * LTR_LOG2E;
+
+    // step iterator and tile transfers: as in the kernels of 32-row groups
+    int c = -1, t = 0, nt = 0;
+    int ld_sk = 0, ld_pos0 = 0;
+    const float *ld_kb = nullptr, *ld_vb = nullptr;
+    auto settle = [&]() {
+        while (c < p.n_chunks && t >= nt) {
+            c++;
+            t = 0;
+            if (c < p.n_chunks) {
+                ld_sk = p.chunk[c].sk;
+                ld_pos0 = p.chunk[c].pos0;
+                ld_kb = (const float *)p.chunk[c].k + b * p.ks[0] + hkv * p.ks[2];
+                ld_vb = (const float *)p.chunk[c].v + b * p.vs[0] + hkv * p.vs[2];
+                const int nvis = causal ? max(0, min(ld_sk, blk_hi - ld_pos0 + 1)) : ld_sk;
+                nt = (nvis + BN - 1) / BN;
+            }
+        }
+    };
+    settle();
+    const int st_row = lane / CPR, st_pc = lane % CPR;
+    int nx_sk = 0, nx_pos0 = 0, nx_key0 = 0;
+    auto gload = [&](int ti, int buf) {
+        nx_sk = ld_sk;
+        nx_pos0 = ld_pos0;
+        nx_key0 = ti * BN;
+        const unsigned Kd = lds_address(smem) + buf * L::BUF_BYTES, Vd = Kd + TILE * 4;
+#pragma unroll
+        for (int n = 0; n < NI; n++) {
+            const int row = RPI * (NI * ks + n) + st_row;
+            const int key = min(ti * BN + row, ld_sk - 1);       // rows past the end repeat the last row; they are masked
+            const int chunk = st_pc ^ f32_swz(row);
+            global_to_lds_b128(ld_kb + ((long long)key * p.ks[1] + chunk * 4), Kd + RPI * (NI * ks + n) * D * 4);
+            global_to_lds_b128(ld_vb + ((long long)key * p.vs[1] + chunk * 4), Vd + RPI * (NI * ks + n) * D * 4);
+        }
+    };
+    bool have = c < p.n_chunks;
+    if (!have && (p.flags & LTR_MERGE)) return;   // merging an empty partial result changes nothing (block-uniform)
+    if (have) gload(t, 0);
+    tile_barrier();
+    int par = 0;
+    while (have) {
+        const int sk = nx_sk, pos0 = nx_pos0, key0 = nx_key0 + 32 * ks;   // this wave's 32 keys of the step
+        const float *Ks = (const float *)(smem + par * L::BUF_BYTES) + 32 * ks * D, *Vs = Ks + TILE;
+        t++;
+        settle();
+        const bool have_next = c < p.n_chunks;
+        if (have_next) gload(t, par ^ 1);
+        // nothing to add: the sub-tile starts past the chunk's end, or every row precedes its first key
+        if (key0 < sk && (!causal || pos0 + key0 <= blk_hi)) {
+            f32x4 s[2];
+            s[0] = s[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            rows16_scores(Ks, i, g, qreg, s);
+            const bool need_mask = (key0 + 32 > sk) || (causal && (pos0 + key0 + 31 > blk_lo));
+            float mx = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float tv = s[kb][r] * c2;
+                    if (need_mask) {
+                        const int key = key0 + 16 * kb + 4 * g + r;
+                        const bool vis = key < sk && (!causal || pos0 + key <= my_pos);
+                        tv = vis ? tv : -INFINITY;
+                    }
+                    s[kb][r] = tv;
+                    mx = fmaxf(mx, tv);
+                }
+            mx = quarter_max(mx);
+            const float m_new = fmaxf(m_run, mx);
+            const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);   // m_run = -inf: 0 (nothing accumulated yet)
+            float l_tile = 0.f;
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    s[kb][r] = __builtin_amdgcn_exp2f(s[kb][r] - m_use);
+                    l_tile += s[kb][r];
+                }
+            l_run = l_run * alpha + l_tile;
+            m_run = m_new;
+#pragma unroll
+            for (int db = 0; db < 4; db++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) oacc[db][r] *= alpha;
+            rows16_weighted(Vs, i, g, s, oacc);
+        }
+        tile_barrier();
+        par ^= 1;
+        have = have_next;
+    }
+
+    // the shares agree on a reference, scale to it and exchange columns
+    float *const ml = (float *)smem + ks * 32;   // [wave][16 references | 16 sums]
+    const float l_own = quarter_sum(l_run);
+    float *lse_p = p.lse + ((long long)b * p.Hq + h) * p.Sq + my_row;
+    float lse_old = 0.f;
+    if ((p.flags & LTR_MERGE) && row_ok) lse_old = *lse_p;   // before any wave writes it
+    if (g == 0) {
+        ml[i] = m_run;
+        ml[16 + i] = l_own;
+    }
+    __syncthreads();
+    float m_all = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < 4; k++) m_all = fmaxf(m_all, ml[(k - ks) * 32 + i]);
+    const float m_ref = m_all == -INFINITY ? 0.f : m_all;
+    float l_tot = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) l_tot += ml[(k - ks) * 32 + 16 + i] * __builtin_amdgcn_exp2f(ml[(k - ks) * 32 + i] - m_ref);
+    const f32x4 own = rows16_collect(smem, ks, lane, oacc, __builtin_amdgcn_exp2f(m_run - m_ref));
+    float lse_new = (l_tot > 0.f) ? m_all * LTR_LN2 + logf(l_tot) : -INFINITY;
+    float w_cur = (l_tot > 0.f) ? 1.f / l_tot : 0.f, w_old = 0.f;
+    if ((p.flags & LTR_MERGE) && row_ok) {
+        const float mxl = fmaxf(lse_old, lse_new);
+        if (mxl == -INFINITY) {
+            w_cur = 0.f;
+        } else {
+            const float e_old = expf(lse_old - mxl), e_new = expf(lse_new - mxl);
+            const float tot = e_old + e_new;
+            w_old = e_old / tot;
+            w_cur *= e_new / tot;
+            lse_new = mxl + logf(tot);
+        }
+    }
+    if (!row_ok) return;
+    if (ks == 0 && g == 0) *lse_p = lse_new;
+    float *op = (float *)p.o + b * p.os[0] + h * p.os[2] + (long long)my_row * p.os[1] + 16 * ks + 4 * g;
+    f32x4 val;
+#pragma unroll
+    for (int e = 0; e < 4; e++) val[e] = own[e] * w_cur;
+    if (p.flags & LTR_MERGE) {
+        const f32x4 old = *(const f32x4 *)op;
+#pragma unroll
+        for (int e = 0; e < 4; e++) val[e] += old[e] * w_old;
+    }
+    *(f32x4 *)op = val;
 }
 
 // ------------------------------------------------------------------------------ delta
@@ -3110,7 +3359,7 @@ __global__ __launch_bounds__(64) void bwd_dkdv_f32_kernel(const BwdParams p) {
 //                        in registers: one wave per SIMD), the block loops over the group's query heads and over 32-row
 //                        Q / dO tiles in double-buffered LDS: S = Q K^T, dP = dO V^T (accumulators start at -DELTA of
 //                        their rows), P and dS in registers, dV^T += dO^T P, dK^T += Q^T dS.
-template <int D, int KS>
+template <int D, int KS, int GROUP = 32>
 __global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p) {
     using L = F32Mfma<D, KS>;
     constexpr int NW = L::NW, RG = L::RG, BM = L::BM, BN = L::BN, TILE = L::TILE;
@@ -3317,6 +3566,140 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p)
         }
         dqp += ROWS_PER_IT * dqs1;
     });
+}
+
+template <>
+__global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel<64, 4, 16>(const BwdParams p) {   // see F32Rows16
+    using L = F32Mfma<64, 4>;
+    constexpr int D = 64, BM = F32Rows16::BM, BN = L::BN, TILE = L::TILE;
+    constexpr int CPR = D / 4, RPI = 64 / CPR, NI = BN / (RPI * L::NW);
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool causal = p.flags & LTR_CAUSAL, result = p.flags & LTR_DQ_F32_RESULT;
+    const int n_qt = (p.Sq + BM - 1) / BM;
+    const int qt = n_qt - 1 - blockIdx.x / (p.B * p.Hq);
+    const int bh = blockIdx.x % (p.B * p.Hq);
+    const int b = bh / p.Hq, h = bh % p.Hq, hkv = h / p.n_rep;
+    const int row0 = qt * BM, my_row = row0 + i;
+    const bool row_ok = my_row < p.Sq;
+    const int my_pos = q_position(my_row, p.q_split, p.q_pos0[0], p.q_pos0[1]);
+    int blk_lo, blk_hi;
+    q_pos_range(row0, min(row0 + BM, p.Sq) - 1, p.q_split, p.q_pos0[0], p.q_pos0[1], blk_lo, blk_hi);
+    float qreg[16], doreg[16];
+    float lse2 = INFINITY, dlt = 0.f;   // +inf: P = exp2(s - inf) = 0 for rows past the end and rows that saw no key
+    {
+        const int rs = min(my_row, p.Sq - 1);
+        const long long so = ((long long)b * p.Hq + h) * p.Sq + my_row;
+        rows16_operand((const float *)p.q + b * p.qs[0] + (long long)rs * p.qs[1] + h * p.qs[2], g, qreg);
+        rows16_operand((const float *)p.d_o + b * p.dos[0] + (long long)rs * p.dos[1] + h * p.dos[2], g, doreg);
+        if (row_ok) {
+            const float lse_row = p.lse[so];
+            lse2 = lse_row == -INFINITY ? INFINITY : lse_row * LTR_LOG2E;
+            if (!result) dlt = p.delta[so];
+        }
+        if (result) {   // the four lanes of a row: 16 sums of D / 16 terms in all, as in delta_kernel
+            float oreg[16], sum[4];
+            rows16_operand((const float *)p.o + b * p.os_[0] + (long long)rs * p.os_[1] + h * p.os_[2], g, oreg);
+#pragma unroll
+            for (int j = 0; j < 4; j++) sum[j] = 0.f;
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) sum[j] = fmaf(oreg[4 * s + j], doreg[4 * s + j], sum[j]);
+            const float part = quarter_sum((sum[0] + sum[1]) + (sum[2] + sum[3]));
+            if (row_ok) dlt = part;
+            if (row_ok && g == 0 && ks == 0) p.delta[so] = part;
+        }
+    }
+    f32x4 dqacc[4];
+#pragma unroll
+    for (int db = 0; db < 4; db++) dqacc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float c2 = p.scale * LTR_LOG2E;
+
+    int c = -1, t = 0, nt = 0;
+    int ld_sk = 0, ld_pos0 = 0;
+    const float *ld_kb = nullptr, *ld_vb = nullptr;
+    auto settle = [&]() {
+        while (c < p.n_chunks && t >= nt) {
+            c++;
+            t = 0;
+            if (c < p.n_chunks) {
+                ld_sk = p.chunk[c].sk;
+                ld_pos0 = p.chunk[c].pos0;
+                ld_kb = (const float *)p.chunk[c].k + b * p.ks[0] + hkv * p.ks[2];
+                ld_vb = (const float *)p.chunk[c].v + b * p.vs[0] + hkv * p.vs[2];
+                const int nvis = causal ? max(0, min(ld_sk, blk_hi - ld_pos0 + 1)) : ld_sk;
+                nt = (nvis + BN - 1) / BN;
+            }
+        }
+    };
+    settle();
+    const int st_row = lane / CPR, st_pc = lane % CPR;
+    int nx_sk = 0, nx_pos0 = 0, nx_key0 = 0;
+    auto gload = [&](int ti, int buf) {
+        nx_sk = ld_sk;
+        nx_pos0 = ld_pos0;
+        nx_key0 = ti * BN;
+        const unsigned Kd = lds_address(smem) + buf * L::BUF_BYTES, Vd = Kd + TILE * 4;
+#pragma unroll
+        for (int n = 0; n < NI; n++) {
+            const int row = RPI * (NI * ks + n) + st_row;
+            const int key = min(ti * BN + row, ld_sk - 1);
+            const int chunk = st_pc ^ f32_swz(row);
+            global_to_lds_b128(ld_kb + ((long long)key * p.ks[1] + chunk * 4), Kd + RPI * (NI * ks + n) * D * 4);
+            global_to_lds_b128(ld_vb + ((long long)key * p.vs[1] + chunk * 4), Vd + RPI * (NI * ks + n) * D * 4);
+        }
+    };
+    bool have = c < p.n_chunks;
+    if (!have && !result) return;   // no visible key: nothing to add to the accumulator (block-uniform)
+    if (have) gload(t, 0);
+    tile_barrier();
+    int par = 0;
+    while (have) {
+        const int sk = nx_sk, pos0 = nx_pos0, key0 = nx_key0 + 32 * ks;
+        const float *Ks = (const float *)(smem + par * L::BUF_BYTES) + 32 * ks * D, *Vs = Ks + TILE;
+        t++;
+        settle();
+        const bool have_next = c < p.n_chunks;
+        if (have_next) gload(t, par ^ 1);
+        if (key0 < sk && (!causal || pos0 + key0 <= blk_hi)) {
+            f32x4 s[2], dp[2];
+            s[0] = s[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            dp[0] = dp[1] = f32x4{-dlt, -dlt, -dlt, -dlt};
+            rows16_scores(Ks, i, g, qreg, s);
+            rows16_scores(Vs, i, g, doreg, dp);
+            const bool need_mask = (key0 + 32 > sk) || (causal && (pos0 + key0 + 31 > blk_lo));
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float pv = __builtin_amdgcn_exp2f(s[kb][r] * c2 - lse2);
+                    if (need_mask) {
+                        const int key = key0 + 16 * kb + 4 * g + r;
+                        const bool vis = key < sk && row_ok && (!causal || pos0 + key <= my_pos);
+                        pv = vis ? pv : 0.f;
+                    }
+                    s[kb][r] = pv * dp[kb][r];
+                }
+            rows16_weighted(Ks, i, g, s, dqacc);
+        }
+        tile_barrier();
+        par ^= 1;
+        have = have_next;
+    }
+    const f32x4 own = rows16_collect(smem, ks, lane, dqacc, 1.f);
+    if (!row_ok) return;
+    float *dqp = (float *)p.dq + b * p.dqs[0] + h * p.dqs[2] + (long long)my_row * p.dqs[1] + 16 * ks + 4 * g;
+    f32x4 val;
+#pragma unroll
+    for (int e = 0; e < 4; e++) val[e] = own[e] * p.scale;
+    if (!result) {
+        const f32x4 old = *(const f32x4 *)dqp;
+#pragma unroll
+        for (int e = 0; e < 4; e++) val[e] += old[e];
+    }
+    *(f32x4 *)dqp = val;
 }
 
 template <int D>
@@ -3594,11 +3977,13 @@ int enable_large_lds() {
         {(const void *)fwd_f32_mfma_kernel<64, 1>, F32Mfma<64, 1>::LDS},
         {(const void *)fwd_f32_mfma_kernel<64, 2>, F32Mfma<64, 2>::LDS},
         {(const void *)fwd_f32_mfma_kernel<64, 4>, F32Mfma<64, 4>::LDS},
+        {(const void *)fwd_f32_mfma_kernel<64, 4, 16>, F32Mfma<64, 4>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<128, 1>, F32Mfma<128, 1>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<128, 2>, F32Mfma<128, 2>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<64, 1>, F32Mfma<64, 1>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<64, 2>, F32Mfma<64, 2>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<64, 4>, F32Mfma<64, 4>::LDS},
+        {(const void *)bwd_dq_f32_mfma_kernel<64, 4, 16>, F32Mfma<64, 4>::LDS},
         {(const void *)bwd_dkdv_f32_mfma_kernel<128>, F32DkdvLds<128>::LDS},
         {(const void *)bwd_dkdv_f32_mfma_kernel<64>, F32DkdvLds<64>::LDS},
         {(const void *)bwd_dkdv_pad_kernel<128>, BwdLds<128, 1>::TOTAL},
@@ -3970,6 +4355,19 @@ struct FwdPlan {
     int rows, n_qtiles, n_slots, group;
     long long blocks;
 };
+// Rows per block and key shares of the fp32 forward and dQ kernels: 128 rows, or fewer and the keys split over 2 / 4 waves of a row group
+// when the launch has too few rows to give every CU a block (4 key shares need the LDS that only head dim 64 leaves); with 4 shares groups
+// of 16 rows where the launch still fits the chip in one round.  Kernel us with 32 and 16 rows, 1024 keys at head dim 64, forward / dQ:
+// 256 blocks of 16 rows 27.7 / 37.3 and 18.1 / 23.3; 336 blocks, a second round, 27.7 / 37.0 and 34.4 / 44.8; 864 blocks 53.7 / 72.7 and
+// 67.0 / 87.8.
+int f32_rows(int D, long long pairs, int Sq, int cus, int &ks) {
+    const int max_ks = D == 64 ? 4 : 2;
+    auto blocks = [&](int rows) { return (long long)((Sq + rows - 1) / rows) * pairs; };
+    ks = 1;
+    while (ks < max_ks && blocks(128 / ks) < cus) ks *= 2;
+    return ks == F32Rows16::KS && blocks(F32Rows16::BM) <= cus ? F32Rows16::BM : 128 / ks;
+}
+
 FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
                  int n_chunks, bool may_share = true) {
     FwdPlan pl;
@@ -3982,14 +4380,8 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
         if (flags & LTR_FWD_F32_SCALAR) {
             pl.rows = 64;
         } else {
-            // matrix-pipe kernel: 128 rows per block, or fewer rows and the keys split over 2 / 4 waves of a row group when
-            // the launch has too few rows to give every CU a block (4 key shares need the LDS that only head dim 64 leaves)
-            const int cus = device_cus();
-            const int max_ks = D == 64 ? 4 : 2;
-            int ks = 1;
-            while (ks < max_ks && (long long)((Sq + 128 / ks - 1) / (128 / ks)) * B * Hq < cus) ks *= 2;
-            pl.f32_ks = ks;
-            pl.rows = 128 / ks;
+            // matrix-pipe kernel
+            pl.rows = f32_rows(D, (long long)B * Hq, Sq, device_cus(), pl.f32_ks);
         }
         pl.n_qtiles = pl.n_slots = (Sq + pl.rows - 1) / pl.rows;
         pl.blocks = (long long)pl.n_qtiles * B * Hq;
@@ -4121,12 +4513,8 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
             pl.dq_rows = 64;
         } else {
             // matrix-pipe kernels: 128 keys per dK/dV block; the dQ kernel sized like the fp32 forward (see plan_fwd)
-            const int max_ks = D == 64 ? 4 : 2;
-            int ks = 1;
-            while (ks < max_ks && (long long)((Sq + 128 / ks - 1) / (128 / ks)) * B * Hq < cus) ks *= 2;
-            pl.f32_ks = ks;
             pl.keys_per_block = 128;
-            pl.dq_rows = 128 / ks;
+            pl.dq_rows = f32_rows(D, (long long)B * Hq, Sq, cus, pl.f32_ks);
         }
         pl.kv_tiles = 0;
         for (int c = 0; c < n_chunks; c++) pl.kv_tiles += (chunk[c].sk + pl.keys_per_block - 1) / pl.keys_per_block;
@@ -4373,7 +4761,7 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
         }
         if (pl.f32_ks == 1) return launch((const void *)fwd_f32_mfma_kernel<64, 1>, pl.blocks, 256, F32Mfma<64, 1>::LDS, st, p);
         if (pl.f32_ks == 2) return launch((const void *)fwd_f32_mfma_kernel<64, 2>, pl.blocks, 256, F32Mfma<64, 2>::LDS, st, p);
-        return launch((const void *)fwd_f32_mfma_kernel<64, 4>, pl.blocks, 256, F32Mfma<64, 4>::LDS, st, p);
+        return launch(pl.rows == F32Rows16::BM ? (const void *)fwd_f32_mfma_kernel<64, 4, 16> : (const void *)fwd_f32_mfma_kernel<64, 4>, pl.blocks, 256, F32Mfma<64, 4>::LDS, st, p);
     }
     if (a->D == 128) return launch((const void *)fwd_f32_kernel<128>, pl.blocks, 64, 0, st, p);
     return launch((const void *)fwd_f32_kernel<64>, pl.blocks, 64, 0, st, p);
@@ -4543,7 +4931,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
             else
                 rc = pl.f32_ks == 1   ? launch((const void *)bwd_dq_f32_mfma_kernel<64, 1>, pl.dq_blocks, 256, F32Mfma<64, 1>::LDS, st, p)
                      : pl.f32_ks == 2 ? launch((const void *)bwd_dq_f32_mfma_kernel<64, 2>, pl.dq_blocks, 256, F32Mfma<64, 2>::LDS, st, p)
-                                      : launch((const void *)bwd_dq_f32_mfma_kernel<64, 4>, pl.dq_blocks, 256, F32Mfma<64, 4>::LDS, st, p);
+                                      : launch(pl.dq_rows == F32Rows16::BM ? (const void *)bwd_dq_f32_mfma_kernel<64, 4, 16> : (const void *)bwd_dq_f32_mfma_kernel<64, 4>, pl.dq_blocks, 256, F32Mfma<64, 4>::LDS, st, p);
             if (rc) return rc;
         }
         if (do_dkdv) {
