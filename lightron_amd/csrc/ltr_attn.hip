@@ -4319,7 +4319,10 @@ RowChoice choose_rows(const RowCosts &costs, unsigned allowed, int D, bool causa
         if ((i == ROWS_256 || i == ROWS_512) && q_tile_slots(n, BH, q_tiles_uneven(Sq, k.rows, q_split, q_pos0, chunk, n_chunks), cus) != n) {   // in pairs
             double pair = 0;
             for (int j = 0; 2 * j < m; j++) pair = std::max(pair, at[j] + (2 * j < m - 1 ? at[m - 1 - j] : 0));
-            us[i] = std::ceil((double)BH * ((n + 1) / 2) / cus) * (pair * c.step_us + 2 * c.fixed_us);
+            // the middle one of an odd number is a block by itself, of half the work: it can fill half a round (384 heads, 13 tiles of 512 rows:
+            // 9.75 pairs per CU; taken for 11 whole rounds the launch went to 256 rows, dQ 3007 us for 2900)
+            const double halves = n % 2 ? std::ceil((double)BH * n / cus) : 2 * std::ceil((double)BH * (n / 2) / cus);
+            us[i] = halves / 2 * (pair * c.step_us + 2 * c.fixed_us);
         }
     }
     RowChoice best = first;
