@@ -4304,6 +4304,9 @@ RowChoice choose_rows(const RowCosts &costs, unsigned allowed, int D, bool causa
             most = std::max(most, at[j]);
             least = std::min(least, at[j]);
         }
+        // head dim 128: past 8192 keys the tile traffic of four waves outweighs the fixed cost they hide (4 x 32 heads S=8192 forward / dQ
+        // 2046 / 2844 us with eight, 2173 / 2925 with four; zig-zag share of 32768 tokens, 32 heads, dQ 1295 / 1360)
+        if (i == FOUR_WAVES && D == 128 && most * (1 << k.key_log2) > 8192) continue;
         const double blocks = (double)BH * n, on_a_cu = std::ceil(blocks / cus);
         if (least >= 0.9 * most) {
             us[i] = std::max(most * c.alone_us + c.alone_fixed_us, on_a_cu * (most * c.step_us + c.fixed_us));
