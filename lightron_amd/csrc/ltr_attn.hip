@@ -15,8 +15,9 @@
 //                        operand read from LDS feeds two MFMAs (chosen by the host, or forced with LTR_FWD_ROWS_512).
 //                        fwd_bf16_w4_kernel<D>, bwd_dq_w4_kernel<D>: 128 rows and four waves per block, several blocks per CU (FourWaves).
 //   fwd_f32_mfma_kernel<D, KS>  fp32 I/O and arithmetic on v_mfma_f32_32x32x2_f32: the forward of the 1e-4 cases (the reference's
-//                        acceptance dtype) on the matrix pipe; KS key shares per 32-row group for launches with few rows,
-//                        <64, 4, 16> groups of 16 rows for those with the fewest (F32Rows16; bwd_dq_f32_mfma_kernel likewise).
+//                        acceptance dtype) on the matrix pipe; KS key shares per 32-row group for launches with few rows, <64, 4> of 16-row
+//                        groups for those with the fewest (F32Rows16) and fwd_f32_rows32_kernel<64, 4> where their blocks pass one round;
+//                        bwd_dq_f32_mfma_kernel, bwd_dq_f32_rows32_kernel likewise.
 //   fwd_f32_kernel<D>    the same in scalar fp32 (no MFMA): kept as the fallback, reached with LTR_FWD_F32_SCALAR.
 //                        fwd_bf16_shares_kernel<D, KS>, bwd_dq_shares_kernel<D, KS>: KS waves share a row group's keys (launches with
 //                        few rows, see key_shares and choose_rows); *_pad_kernel: head dims below the width D (LTR_HEAD_COLS).
@@ -1228,8 +1229,8 @@ struct F32Mfma {
     static_assert(LDS <= 160 * 1024, "LDS of one CU");
 };
 
-template <int D, int KS, int GROUP = 32>   // GROUP: rows of a row group; 16: see F32Rows16
-__global__ __launch_bounds__(256) void fwd_f32_mfma_kernel(const FwdParams p) {
+template <int D, int KS>
+__device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
     using L = F32Mfma<D, KS>;
     constexpr int NW = L::NW, RG = L::RG, BM = L::BM, BN = L::BN, TILE = L::TILE;
     constexpr int CPR = D / 4;               // 16-byte chunks per row
@@ -1561,8 +1562,16 @@ __device__ __forceinline__ f32x4 rows16_collect(unsigned char *smem, int ks, int
     return own;
 }
 
+template <int D, int KS>   // one key share at head dim 64: 36 KB of LDS; three blocks per CU (168 registers)
+__global__ __launch_bounds__(256, D == 64 && KS == 1 ? 3 : 1) void fwd_f32_mfma_kernel(const FwdParams p) {
+    fwd_f32_body<D, KS>(p);
+}
+template <int D, int KS>
+__global__ __launch_bounds__(256) void fwd_f32_rows32_kernel(const FwdParams p) {
+    fwd_f32_body<D, KS>(p);
+}
 template <>
-__global__ __launch_bounds__(256) void fwd_f32_mfma_kernel<64, 4, 16>(const FwdParams p) {   // see F32Rows16
+__global__ __launch_bounds__(256) void fwd_f32_mfma_kernel<64, 4>(const FwdParams p) {   // see F32Rows16
     using L = F32Mfma<64, 4>;
     constexpr int D = 64, BM = F32Rows16::BM, BN = L::BN, TILE = L::TILE;
     constexpr int CPR = D / 4, RPI = 64 / CPR, NI = BN / (RPI * L::NW);
@@ -3359,8 +3368,8 @@ __global__ __launch_bounds__(64) void bwd_dkdv_f32_kernel(const BwdParams p) {
 //                        in registers: one wave per SIMD), the block loops over the group's query heads and over 32-row
 //                        Q / dO tiles in double-buffered LDS: S = Q K^T, dP = dO V^T (accumulators start at -DELTA of
 //                        their rows), P and dS in registers, dV^T += dO^T P, dK^T += Q^T dS.
-template <int D, int KS, int GROUP = 32>
-__global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p) {
+template <int D, int KS>
+__device__ __forceinline__ void bwd_dq_f32_body(const BwdParams &p) {
     using L = F32Mfma<D, KS>;
     constexpr int NW = L::NW, RG = L::RG, BM = L::BM, BN = L::BN, TILE = L::TILE;
     constexpr int CPR = D / 4, RPI = 64 / CPR, NI = BN / (RPI * NW);
@@ -3568,8 +3577,16 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p)
     });
 }
 
+template <int D, int KS>
+__global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel(const BwdParams p) {
+    bwd_dq_f32_body<D, KS>(p);
+}
+template <int D, int KS>
+__global__ __launch_bounds__(256) void bwd_dq_f32_rows32_kernel(const BwdParams p) {
+    bwd_dq_f32_body<D, KS>(p);
+}
 template <>
-__global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel<64, 4, 16>(const BwdParams p) {   // see F32Rows16
+__global__ __launch_bounds__(256) void bwd_dq_f32_mfma_kernel<64, 4>(const BwdParams p) {   // see F32Rows16
     using L = F32Mfma<64, 4>;
     constexpr int D = 64, BM = F32Rows16::BM, BN = L::BN, TILE = L::TILE;
     constexpr int CPR = D / 4, RPI = 64 / CPR, NI = BN / (RPI * L::NW);
@@ -3977,13 +3994,13 @@ int enable_large_lds() {
         {(const void *)fwd_f32_mfma_kernel<64, 1>, F32Mfma<64, 1>::LDS},
         {(const void *)fwd_f32_mfma_kernel<64, 2>, F32Mfma<64, 2>::LDS},
         {(const void *)fwd_f32_mfma_kernel<64, 4>, F32Mfma<64, 4>::LDS},
-        {(const void *)fwd_f32_mfma_kernel<64, 4, 16>, F32Mfma<64, 4>::LDS},
+        {(const void *)fwd_f32_rows32_kernel<64, 4>, F32Mfma<64, 4>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<128, 1>, F32Mfma<128, 1>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<128, 2>, F32Mfma<128, 2>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<64, 1>, F32Mfma<64, 1>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<64, 2>, F32Mfma<64, 2>::LDS},
         {(const void *)bwd_dq_f32_mfma_kernel<64, 4>, F32Mfma<64, 4>::LDS},
-        {(const void *)bwd_dq_f32_mfma_kernel<64, 4, 16>, F32Mfma<64, 4>::LDS},
+        {(const void *)bwd_dq_f32_rows32_kernel<64, 4>, F32Mfma<64, 4>::LDS},
         {(const void *)bwd_dkdv_f32_mfma_kernel<128>, F32DkdvLds<128>::LDS},
         {(const void *)bwd_dkdv_f32_mfma_kernel<64>, F32DkdvLds<64>::LDS},
         {(const void *)bwd_dkdv_pad_kernel<128>, BwdLds<128, 1>::TOTAL},
@@ -4373,6 +4390,26 @@ int f32_rows(int D, long long pairs, int Sq, int cus, int &ks) {
     while (ks < max_ks && blocks(128 / ks) < cus) ks *= 2;
     return ks == F32Rows16::KS && blocks(F32Rows16::BM) <= cus ? F32Rows16::BM : 128 / ks;
 }
+// The kernels of these choices, for the launches and for the plans: a plan's name is that of the kernel a launch takes.
+struct F32Kernel {
+    const void *fn;
+    const char *name;
+    int lds;
+};
+#define LTR_KERNEL(...) (const void *)__VA_ARGS__, #__VA_ARGS__
+F32Kernel f32_fwd_kernel(int D, int ks, int rows) {
+    if (D == 128) return ks == 1 ? F32Kernel{LTR_KERNEL(fwd_f32_mfma_kernel<128, 1>), F32Mfma<128, 1>::LDS} : F32Kernel{LTR_KERNEL(fwd_f32_mfma_kernel<128, 2>), F32Mfma<128, 2>::LDS};
+    if (ks == 1) return {LTR_KERNEL(fwd_f32_mfma_kernel<64, 1>), F32Mfma<64, 1>::LDS};
+    if (ks == 2) return {LTR_KERNEL(fwd_f32_mfma_kernel<64, 2>), F32Mfma<64, 2>::LDS};
+    return rows == F32Rows16::BM ? F32Kernel{LTR_KERNEL(fwd_f32_mfma_kernel<64, 4>), F32Mfma<64, 4>::LDS} : F32Kernel{LTR_KERNEL(fwd_f32_rows32_kernel<64, 4>), F32Mfma<64, 4>::LDS};
+}
+F32Kernel f32_dq_kernel(int D, int ks, int rows) {
+    if (D == 128) return ks == 1 ? F32Kernel{LTR_KERNEL(bwd_dq_f32_mfma_kernel<128, 1>), F32Mfma<128, 1>::LDS} : F32Kernel{LTR_KERNEL(bwd_dq_f32_mfma_kernel<128, 2>), F32Mfma<128, 2>::LDS};
+    if (ks == 1) return {LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 1>), F32Mfma<64, 1>::LDS};
+    if (ks == 2) return {LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 2>), F32Mfma<64, 2>::LDS};
+    return rows == F32Rows16::BM ? F32Kernel{LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 4>), F32Mfma<64, 4>::LDS} : F32Kernel{LTR_KERNEL(bwd_dq_f32_rows32_kernel<64, 4>), F32Mfma<64, 4>::LDS};
+}
+#undef LTR_KERNEL
 
 FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
                  int n_chunks, bool may_share = true) {
@@ -4761,13 +4798,8 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     if (pl.f32_ks) {   // fp32 on the matrix pipe; the chunk offsets of its LDS-direct loads are 64-bit, nothing more to check
         rc = enable_large_lds();
         if (rc) return rc;
-        if (a->D == 128) {
-            if (pl.f32_ks == 1) return launch((const void *)fwd_f32_mfma_kernel<128, 1>, pl.blocks, 256, F32Mfma<128, 1>::LDS, st, p);
-            return launch((const void *)fwd_f32_mfma_kernel<128, 2>, pl.blocks, 256, F32Mfma<128, 2>::LDS, st, p);
-        }
-        if (pl.f32_ks == 1) return launch((const void *)fwd_f32_mfma_kernel<64, 1>, pl.blocks, 256, F32Mfma<64, 1>::LDS, st, p);
-        if (pl.f32_ks == 2) return launch((const void *)fwd_f32_mfma_kernel<64, 2>, pl.blocks, 256, F32Mfma<64, 2>::LDS, st, p);
-        return launch(pl.rows == F32Rows16::BM ? (const void *)fwd_f32_mfma_kernel<64, 4, 16> : (const void *)fwd_f32_mfma_kernel<64, 4>, pl.blocks, 256, F32Mfma<64, 4>::LDS, st, p);
+        const F32Kernel k = f32_fwd_kernel(a->D, pl.f32_ks, pl.rows);
+        return launch(k.fn, pl.blocks, 256, k.lds, st, p);
     }
     if (a->D == 128) return launch((const void *)fwd_f32_kernel<128>, pl.blocks, 64, 0, st, p);
     return launch((const void *)fwd_f32_kernel<64>, pl.blocks, 64, 0, st, p);
@@ -4931,13 +4963,8 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
         rc = enable_large_lds();
         if (rc) return rc;
         if (do_dq) {
-            if (a->D == 128)
-                rc = pl.f32_ks == 1 ? launch((const void *)bwd_dq_f32_mfma_kernel<128, 1>, pl.dq_blocks, 256, F32Mfma<128, 1>::LDS, st, p)
-                                    : launch((const void *)bwd_dq_f32_mfma_kernel<128, 2>, pl.dq_blocks, 256, F32Mfma<128, 2>::LDS, st, p);
-            else
-                rc = pl.f32_ks == 1   ? launch((const void *)bwd_dq_f32_mfma_kernel<64, 1>, pl.dq_blocks, 256, F32Mfma<64, 1>::LDS, st, p)
-                     : pl.f32_ks == 2 ? launch((const void *)bwd_dq_f32_mfma_kernel<64, 2>, pl.dq_blocks, 256, F32Mfma<64, 2>::LDS, st, p)
-                                      : launch(pl.dq_rows == F32Rows16::BM ? (const void *)bwd_dq_f32_mfma_kernel<64, 4, 16> : (const void *)bwd_dq_f32_mfma_kernel<64, 4>, pl.dq_blocks, 256, F32Mfma<64, 4>::LDS, st, p);
+            const F32Kernel k = f32_dq_kernel(a->D, pl.f32_ks, pl.dq_rows);
+            rc = launch(k.fn, pl.dq_blocks, 256, k.lds, st, p);
             if (rc) return rc;
         }
         if (do_dkdv) {
@@ -5085,10 +5112,10 @@ int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work
     out->dkdv_keys = b.keys_per_block;
     out->dkdv_blocks = shared ? b.split.tiles * a->B * a->Hkv * b.split.n : b.kv_blocks;
     if (f32) {
-        if (f.f32_ks) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_f32_mfma_kernel<%d, %d>", D, f.f32_ks);
+        if (f.f32_ks) snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "%s", f32_fwd_kernel(D, f.f32_ks, f.rows).name);
         else snprintf(out->fwd_kernel, sizeof(out->fwd_kernel), "fwd_f32_kernel<%d>", D);
         if (b.f32_ks) {
-            snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_f32_mfma_kernel<%d, %d>", D, b.f32_ks);
+            snprintf(out->dq_kernel, sizeof(out->dq_kernel), "%s", f32_dq_kernel(D, b.f32_ks, b.dq_rows).name);
             snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_f32_mfma_kernel<%d>", D);
         } else {
             snprintf(out->dq_kernel, sizeof(out->dq_kernel), "bwd_dq_f32_kernel<%d>", D);

@@ -1,4 +1,4 @@
-"""fwd_f32_mfma_kernel<64, 4, 16> / bwd_dq_f32_mfma_kernel<64, 4, 16> (groups of 16 rows, the keys of a step shared by four waves of 32),
+"""fwd_f32_mfma_kernel<64, 4> / bwd_dq_f32_mfma_kernel<64, 4> (groups of 16 rows, the keys of a step shared by four waves of 32),
 which fp32 launches of the fewest rows take: against the dense oracle in 64 bits at the edges of their tiles."""
 import pytest
 import torch
@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
 def test_rows16(ltr, B, Hq, Hkv, Sq, q_pos, split, chunks, causal):
     D, pos, lens = 64, [p for _, p in chunks], [n for n, _ in chunks]
     plan = ltr.attn_plan(B, Hq, Hkv, D, Sq, lens, pos, q_pos, split, causal, dtype=torch.float32)
+    assert plan["fwd"]["kernel"] == "fwd_f32_mfma_kernel<64, 4>" and plan["dq"]["kernel"] == "bwd_dq_f32_mfma_kernel<64, 4>"
     assert plan["fwd"]["rows"] == 16 and plan["dq"]["rows"] == 16 and plan["fwd"]["blocks"] == B * Hq * ((Sq + 15) // 16)
     total, at = sum(lens), [sum(lens[:i]) for i in range(len(lens))]
     g = torch.Generator().manual_seed(Sq)

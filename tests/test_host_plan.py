@@ -1,5 +1,9 @@
 """CPU tests of the launch plans: head dims that run in the next width's kernels, and key tiles shared with a workspace."""
 import ctypes
+import random
+import re
+import shutil
+import subprocess
 
 import pytest
 import torch
@@ -66,3 +70,39 @@ def test_shared_key_tiles_are_in_the_plan(dtype, width):
 def test_plan_of_a_problem_that_shares_nothing():
     d = la.attn_plan(8, 32, 32, 128, 2048, [2048], [0], causal=True, share_keys=True)["dkdv"]
     assert d["blocks_per_tile"] == 1 and d["reduce_kernel"] == "" and d["reduce_blocks"] == 0
+
+
+def _kernels_of_the_library():
+    """Demangled names of the kernels compiled into the library, as a profiler shows them."""
+    out = subprocess.run(["nm", "-C", la._lib.LIB_PATH], capture_output=True, text=True, check=True).stdout
+    return set(re.findall(r"(?:\(anonymous namespace\)::|\s)(\w+_kernel<[^()]*>)\(", out.replace("__device_stub__", "")))
+
+
+@pytest.mark.skipif(shutil.which("nm") is None, reason="no nm")
+def test_every_plan_names_kernels_that_exist():
+    names = _kernels_of_the_library()
+    assert "bwd_dkdv_reduce_kernel<64, 1>" in names
+    rng = random.Random(5)
+    seen = set()
+    for _ in range(400):
+        D = rng.choice([40, 64, 64, 96, 128, 128])
+        dtype = rng.choice([torch.bfloat16, torch.float32]) if D in (64, 128) else torch.bfloat16
+        Hkv, rep, B, Sq = rng.choice([1, 4, 8, 12, 16]), rng.choice([1, 2, 4]), rng.choice([1, 2, 5, 8, 32]), rng.choice([1, 16, 100, 256, 777, 1024, 2048, 4096])
+        lens = rng.choice([[Sq], [128, 300], [2048] * 4])
+        plan = la.attn_plan(B, Hkv * rep, Hkv, D, Sq, lens, [sum(lens[:i]) for i in range(len(lens))], 0, None, rng.random() < 0.7, dtype=dtype, share_keys=rng.random() < 0.5)
+        for k in (plan["fwd"]["kernel"], plan["dq"]["kernel"], plan["dkdv"]["kernel"], plan["dkdv"].get("reduce_kernel", "")):
+            assert k == "" or k in names, k
+            seen.add(k)
+    for part in ("w4", "shares", "pad", "keywave", "f32_mfma_kernel<64, 4>", "f32_rows32_kernel<64, 4>", "f32_mfma_kernel<128, 2>", "reduce"):
+        assert any(part in k for k in seen), part
+
+
+@pytest.mark.parametrize("pairs,Sq,kernel,rows", [
+    (16, 256, "f32_mfma_kernel<64, 4>", 16), (16, 257, "f32_rows32_kernel<64, 4>", 32), (1, 4096, "f32_mfma_kernel<64, 4>", 16),
+    (1, 4097, "f32_rows32_kernel<64, 4>", 32), (64, 512, "f32_mfma_kernel<64, 1>", 128), (33, 512, "f32_mfma_kernel<64, 2>", 64),
+])
+def test_fp32_rows_and_names_belong_together(pairs, Sq, kernel, rows):
+    """Groups of 16 rows and of 32 rows with four key shares are different kernels: a name stands for one of them."""
+    plan = la.attn_plan(1, pairs, pairs, 64, Sq, [64], [0], 0, None, True, dtype=torch.float32)
+    assert plan["compute_units"] != 256 or (plan["fwd"]["kernel"], plan["fwd"]["rows"]) == ("fwd_" + kernel, rows)
+    assert plan["compute_units"] != 256 or (plan["dq"]["kernel"], plan["dq"]["rows"]) == ("bwd_dq_" + kernel, rows)
