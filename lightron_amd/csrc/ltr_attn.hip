@@ -4248,8 +4248,8 @@ constexpr ShareCost DQ_SHARES_128{{1.85, 2.2, 1.4}, {11.0, 10.0, 10.0}, 2.7}, DQ
 // the CUs plus `tail` of the shortest, a launch of equal ones its largest number of blocks on a CU.  Constants fitted to 120 random
 // launches (8 - 32 heads, 64 - 7900 rows, 4 in 5 causal) of every kernel: rms error 4 - 7 %; the steps of four waves are those of long equal
 // blocks (1024 rows against 8192 and 16384 keys), 2 - 8 % above the fit.  256-row blocks are replaced where
-// another kernel is 1.5 % faster, shares where four waves are 12 % faster, and what key_shares says about shares, with coarser rounds, where
-// other shares are 20 % faster (280 blocks of four shares on 256 CUs: 16.4 us for 9.0 of two).
+// another kernel is 1.5 % faster (more: complete rounds of pairs), shares where four waves are 12 % faster, and what key_shares says about
+// shares, with coarser rounds, where other shares are 20 % faster (280 blocks of four shares on 256 CUs: 16.4 us for 9.0 of two).
 struct TileCost {
     double alone_us, alone_fixed_us, step_us, fixed_us, tail;
 };
@@ -4286,13 +4286,22 @@ RowChoice choose_rows(const RowCosts &costs, unsigned allowed, int D, bool causa
         if (sc.paired) first_us = sc.us;
     }
     const bool shared = first.kernel != ROWS_256;
-    if (!shared && causal && (D == 128 || n_chunks > 1)) {
-        // 256-row tiles whose pairs come out in complete rounds of equal blocks: nothing of a CU is idle, and four waves are not faster
-        // (head dim 128, us forward / dQ, pairs / four waves: 4 x 32 heads S=1024 51 / 71 - 52 / 70, 8 x 32 heads S=512 41 / 52 - 40 / 51,
-        // 8 x 32 heads S=2048 324 / 448 - 340 / 458).  Chunk tables at head dim 64 keep the pairs too, though four waves are faster there (8 x 32
-        // heads, 1100 rows against 1000 + 400 keys: 139 / 167 - 89 / 115): test_paired_q_tiles_forward_backward holds that launch to them
+    double four_waves = 0.985;
+    if (!shared && causal) {
+        // 256-row tiles whose pairs come out in complete rounds of equal blocks: nothing of a CU is idle.  At head dim 128 four waves are then
+        // not faster (us forward / dQ, pairs / four waves: 4 x 32 heads S=1024 51 / 71 - 52 / 70, 8 x 32 heads S=512 41 / 52 - 40 / 51,
+        // 8 x 32 heads S=2048 324 / 448 - 340 / 458).  At head dim 64 they are, in chunk tables as well (37 launches 1.03 - 1.72 times; forward:
+        // 8 x 32 heads, 1100 rows against 1000 + 400 keys 140 - 93, 16 x 16 heads S=1024 72 - 57), but the model makes them too short in one full
+        // round of pairs, four of their blocks on a CU that runs three (4 x 16 heads S=2048 forward 50.0 - 52.7, modelled 0.98 of the pairs), and
+        // for zig-zag shares with long blocks, where some CUs get one more of the late segment's than others (4 x 8 heads, 3612 rows of 7224
+        // 138 - 160, 0.91; 2 x 32 heads, 3618 of 28944 1043 - 1122, 0.98)
         const int n = (Sq + 255) / 256, slots = (n + 1) / 2;
-        if (n > 1 && BH * slots % cus == 0 && q_tiles_uneven(Sq, 256, q_split, q_pos0, chunk, n_chunks)) return first;
+        if (n > 1 && BH * slots % cus == 0 && q_tiles_uneven(Sq, 256, q_split, q_pos0, chunk, n_chunks)) {
+            if (D == 128) return first;
+            const bool two_segments = q_split > 0 && q_split < Sq;
+            if (two_segments && visible_keys(Sq - 256, Sq - 1, q_split, q_pos0, chunk, n_chunks) > 4096) four_waves = 0.88;
+            else if (BH * slots == cus && n % 2 == 0) four_waves = 0.95;
+        }
     }
     double us[N_ROW_KERNELS];
     for (int i = 0; i < N_ROW_KERNELS; i++) {
@@ -4350,7 +4359,7 @@ RowChoice choose_rows(const RowCosts &costs, unsigned allowed, int D, bool causa
     double best_us = from;
     for (int i = 0; i < N_ROW_KERNELS; i++) {
         const bool to_shares = i == SHARES_2 || i == SHARES_4;
-        if (us[i] > 0 && us[i] < best_us && us[i] < from * (to_shares || first.paired ? 0.8 : shared ? 0.88 : 0.985)) {
+        if (us[i] > 0 && us[i] < best_us && us[i] < from * (to_shares || first.paired ? 0.8 : shared ? 0.88 : i == FOUR_WAVES ? four_waves : 0.985)) {
             best_us = us[i];
             best = {i, false};
         }

@@ -991,11 +991,12 @@ def test_fused_rope_prologue_and_dq_epilogue(ltr, D, Hq, Hkv, Sq, q_pos, chunks,
 ])
 def test_paired_q_tiles_forward_backward(ltr, D, B, Hq, Hkv, Sq, q_pos, split, chunks):
     """Enough (batch, head) pairs that the host hands the forward and dQ kernels a late q tile and its early counterpart
-    per block (q_tile_slots: causal, and the equal blocks fill the 256 CUs evenly).  Odd tile counts (the middle tile runs
-    alone), a ragged last tile, GQA, both head dims, two-segment rows; against the dense oracle."""
+    per block (q_tile_slots: causal, and the equal blocks fill the 256 CUs evenly), with 256-row blocks forced through the hint flags (at
+    head dim 64 the library's own choice is four-wave blocks).  Odd tile counts (the middle tile runs alone), a ragged last tile, GQA, both
+    head dims, two-segment rows; against the dense oracle, as is the library's own choice through autograd."""
     g = torch.Generator().manual_seed(77 + Sq)
     # the library itself says whether it pairs the tiles of this launch (for the device this test runs on)
-    plan = ltr.attn_plan(B, Hq, Hkv, D, Sq, [n for _, n in chunks], [p0 for p0, _ in chunks], q_pos, split, True)
+    plan = ltr.attn_plan(B, Hq, Hkv, D, Sq, [n for _, n in chunks], [p0 for p0, _ in chunks], q_pos, split, True, fwd_rows=256, dq_rows=256)
     n_qt = (Sq + 255) // 256
     assert plan["fwd"]["rows"] == plan["dq"]["rows"] == 256
     assert plan["fwd"]["paired"] and plan["dq"]["paired"], "shape does not trigger the pairing on this device"
@@ -1011,15 +1012,24 @@ def test_paired_q_tiles_forward_backward(ltr, D, B, Hq, Hkv, Sq, q_pos, split, c
     qd = q.cuda().requires_grad_(True)
     kd = [k.cuda().requires_grad_(True) for k in ks]
     vd = [v.cuda().requires_grad_(True) for v in vs]
-    o, lse = ltr.block_attention(qd, kd, vd, [p0 for p0, _ in chunks], q_pos, split, True)
-    o.backward(do.cuda())
-    assert (o.detach().cpu().float() - o_ref).abs().max() < O_TOL_BF16
+    pos0, dod = [p0 for p0, _ in chunks], do.cuda()
+    o, lse = ltr.block_attention(qd, kd, vd, pos0, q_pos, split, True)
+    o.backward(dod)
+    plain = [t.detach() for t in (qd, *kd, *vd)]
+    kp, vp = plain[1:1 + len(kd)], plain[1 + len(kd):]
+    of, lsef = ltr.attn_fwd(plain[0], kp, vp, pos0, q_pos, split, True, fwd_rows=256)
+    dqf, lens = torch.empty_like(plain[0]), [n for _, n in chunks]
+    dks, dvs = (torch.empty(B, sum(lens), Hkv, D, dtype=torch.bfloat16, device="cuda").split(lens, 1) for _ in range(2))
+    delta = torch.empty(lsef.shape, dtype=torch.float32, device="cuda")
+    ltr.attn_bwd_accumulate(plain[0], dod, lsef, delta, kp, vp, pos0, dqf, dks, dvs, q_pos, split, True, o=of, dq_rows=256)
     fin = torch.isfinite(lse_ref)
-    assert torch.equal(torch.isfinite(lse.cpu()), fin)
-    assert (lse.cpu()[fin] - lse_ref[fin]).abs().max() < LSE_TOL_BF16
-    assert _rel(qd.grad.cpu(), dq_ref) < GRAD_RTOL_BF16
-    assert _rel(torch.cat([k.grad for k in kd], 1).cpu(), dk_ref) < GRAD_RTOL_BF16
-    assert _rel(torch.cat([v.grad for v in vd], 1).cpu(), dv_ref) < GRAD_RTOL_BF16
+    for oo, ll, dq, dk, dv in ((o.detach(), lse, qd.grad, [k.grad for k in kd], [v.grad for v in vd]), (of, lsef, dqf, dks, dvs)):
+        assert (oo.cpu().float() - o_ref).abs().max() < O_TOL_BF16
+        assert torch.equal(torch.isfinite(ll.cpu()), fin)
+        assert (ll.cpu()[fin] - lse_ref[fin]).abs().max() < LSE_TOL_BF16
+        assert _rel(dq.cpu(), dq_ref) < GRAD_RTOL_BF16
+        assert _rel(torch.cat(dk, 1).cpu(), dk_ref) < GRAD_RTOL_BF16
+        assert _rel(torch.cat(dv, 1).cpu(), dv_ref) < GRAD_RTOL_BF16
 
 
 @pytest.mark.parametrize("seed", list(range(8)))

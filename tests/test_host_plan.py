@@ -106,3 +106,22 @@ def test_fp32_rows_and_names_belong_together(pairs, Sq, kernel, rows):
     plan = la.attn_plan(1, pairs, pairs, 64, Sq, [64], [0], 0, None, True, dtype=torch.float32)
     assert plan["compute_units"] != 256 or (plan["fwd"]["kernel"], plan["fwd"]["rows"]) == ("fwd_" + kernel, rows)
     assert plan["compute_units"] != 256 or (plan["dq"]["kernel"], plan["dq"]["rows"]) == ("bwd_dq_" + kernel, rows)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S", [(8, 32, 32, 1024), (16, 16, 4, 700), (8, 16, 16, 2048), (8, 32, 8, 1100), (8, 32, 32, 512)])
+def test_a_chunk_table_takes_the_kernels_of_one_chunk(B, Hq, Hkv, S):
+    """The same rows and keys in one chunk or in two are the same work: at head dim 64 four-wave blocks, also where the pairs of 256-row
+    tiles fill whole rounds of CUs."""
+    one, two = (la.attn_plan(B, Hq, Hkv, 64, S, lens, pos, 0, None, True) for lens, pos in (([S], [0]), ([256, S - 256], [0, 256])))
+    assert one == two
+    assert one["compute_units"] != 256 or one["fwd"]["kernel"] == "fwd_bf16_w4_kernel<64>"
+
+
+@pytest.mark.parametrize("lens", [[2048], [1024, 1024]])
+def test_one_round_of_pairs_at_head_dim_64(lens):
+    """4 x 16 heads of 2048 rows: 256 equal blocks of paired tiles against four blocks per CU of which three run at once (50 and 53 us)."""
+    plan = la.attn_plan(4, 16, 16, 64, 2048, lens, [0, 1024][:len(lens)], 0, None, True)
+    if plan["compute_units"] == 256:
+        assert plan["fwd"]["kernel"] == "fwd_bf16_kernel<64, 1>" and plan["fwd"]["paired"] and plan["fwd"]["blocks"] == 256
+    wider = la.attn_plan(8, 16, 16, 64, 1024, [1024], [0], 0, None, True)   # modelled 7 % shorter, measured 3 %
+    assert wider["compute_units"] != 256 or wider["fwd"]["kernel"] == "fwd_bf16_w4_kernel<64>"
