@@ -4334,6 +4334,14 @@ RowChoice choose_rows(const RowCosts &costs, unsigned allowed, int D, bool causa
         // 2046 / 2844 us with eight, 2173 / 2925 with four; zig-zag share of 32768 tokens, 32 heads, dQ 1295 / 1360)
         if (i == FOUR_WAVES && D == 128 && most * (1 << k.key_log2) > 8192) continue;
         const double blocks = (double)BH * n, on_a_cu = std::ceil(blocks / cus);
+        // one round of the shares that key_shares chose ends with its longest block.  With a tail on top, 8 x 16 heads of 128 with 200 rows went
+        // from 256 blocks of two shares to 128 of 256 rows (forward / dQ 12.1 / 14.5 us - 16.1 / 19.4), 84 of 18000 launches likewise (1.08 - 1.35
+        // times).  At head dim 64 key_shares takes four shares for two too early, which the tail mends (8 x 8 heads, 216 rows of a zig-zag
+        // share 12.8 / 14.3 - 11.3 / 13.1)
+        if (D == 128 && shared && i == first.kernel && blocks <= cus) {
+            us[i] = std::max(most * c.alone_us + c.alone_fixed_us, most * c.step_us + c.fixed_us);
+            continue;
+        }
         if (least >= 0.9 * most) {
             us[i] = std::max(most * c.alone_us + c.alone_fixed_us, on_a_cu * (most * c.step_us + c.fixed_us));
             continue;

@@ -125,3 +125,11 @@ def test_one_round_of_pairs_at_head_dim_64(lens):
         assert plan["fwd"]["kernel"] == "fwd_bf16_kernel<64, 1>" and plan["fwd"]["paired"] and plan["fwd"]["blocks"] == 256
     wider = la.attn_plan(8, 16, 16, 64, 1024, [1024], [0], 0, None, True)   # modelled 7 % shorter, measured 3 %
     assert wider["compute_units"] != 256 or wider["fwd"]["kernel"] == "fwd_bf16_w4_kernel<64>"
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S", [(8, 16, 4, 135), (8, 16, 4, 200), (4, 32, 32, 164), (8, 16, 16, 252)])
+def test_one_round_of_shares_stays(B, Hq, Hkv, S):
+    """256 blocks of 128 rows against 128 blocks of 256 (12 and 16 us): every CU has a block."""
+    plan = la.attn_plan(B, Hq, Hkv, 128, S, [S], [0], 0, None, True)
+    if plan["compute_units"] == 256:
+        assert plan["fwd"]["kernel"] == "fwd_bf16_shares_kernel<128, 2>" and plan["dq"]["kernel"] == "bwd_dq_shares_kernel<128, 2>"
