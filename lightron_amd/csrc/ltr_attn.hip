@@ -65,6 +65,7 @@
 #include <atomic>
 #include <algorithm>
 #include "ltr_attn.h"
+#include "ltr_blocks.h"
 
 namespace {
 
@@ -86,13 +87,6 @@ struct ChunkDev {
     float *dv;
     int sk;
     int pos0;
-};
-
-struct BlockMap {      // see block_item
-    int group;         // (batch, kv head) pairs of an XCD whose blocks are handed out together; 0: a linear grid
-    int items;         // items (q tile slots, key tiles) per pair
-    int groups;
-    int inner;         // blocks per item
 };
 
 struct FwdParams {
@@ -176,38 +170,7 @@ __device__ __forceinline__ void q_pos_range(int r0, int r1, int split, int p0, i
     }
 }
 
-// Block id -> (pair = batch x kv head, item = q tile slot or key tile of the pair, sub = one of the `inner` blocks of an item).
-// Consecutive blocks go to the 8 XCDs round-robin.  All blocks of a pair run on one XCD and next to each other in time, so the
-// blocks that are resident together stream the same K / V (or Q / dO) through that XCD's L2; the inner blocks of an item follow each
-// other.  The items of `group` pairs of an XCD are handed out item by item (the first of every pair, the second of every pair, ...):
-// items come longest first, so blocks of unequal length end together (see pair_group).  The grid is (8 XCDs x inner blocks, pairs of a
-// group, items of the groups): the hardware counts what would be four divisions (0.3 us of every block, also as multiplications: their
-// constants are another trip to the arguments).
-struct BlockItem {
-    int pair, item, sub;
-    int order;   // of the blocks of an XCD
-};
-__device__ __forceinline__ BlockItem block_item(const BlockMap &m, int pairs) {
-    BlockItem r;
-    if (m.group) {
-        int g = 0;
-        r.item = blockIdx.z;
-        if (m.groups > 1) {
-            g = r.item / m.items;
-            r.item -= g * m.items;
-        }
-        r.sub = blockIdx.x >> 3;
-        r.pair = (g * m.group + blockIdx.y) * 8 + (blockIdx.x & 7);   // past the last pair: a place of the last group that is empty
-        r.order = r.sub + m.inner * (blockIdx.y + m.group * blockIdx.z);
-    } else {   // pairs that do not divide among the XCDs: one block of every pair, then the next
-        const int rest = blockIdx.x / pairs;
-        r.pair = blockIdx.x - rest * pairs;
-        r.item = rest / m.inner;
-        r.sub = rest - r.item * m.inner;
-        r.order = blockIdx.x >> 3;
-    }
-    return r;
-}
+__device__ __forceinline__ BlockItem block_item(const BlockMap &m, int pairs) { return block_item_at(m, pairs, blockIdx.x, blockIdx.y, blockIdx.z); }
 
 // both halves of the wave end up with combine(x[l], x[l ^ 32])
 __device__ __forceinline__ float xhalf_max(float x) {
@@ -4076,6 +4039,7 @@ int device_cus() {
 
 // One kernel launch whose own status is what is returned: hipLaunchKernel reports the submission of THIS launch, so an
 // error that unrelated earlier work left in the thread's last-error slot is neither reported as ours nor cleared.
+dim3 dims(const BlockGrid &g) { return dim3(g.x, g.y, g.z); }
 template <class Params>
 int launch(const void *kernel, dim3 grid, int threads, size_t lds_bytes, hipStream_t st, const Params &p) {
     void *args[] = {(void *)&p};
@@ -4131,33 +4095,6 @@ int q_tile_slots(int n_qtiles, long long blocks_per_tile, bool uneven, int cus) 
     const int n_slots = (n_qtiles + 1) / 2;
     const long long n = n_slots * blocks_per_tile, rounds = (n + cus - 1) / cus;
     return n * 10 >= rounds * cus * 9 ? n_slots : n_qtiles;
-}
-
-// How many (batch, kv head) pairs of an XCD hand out their blocks together, longest first across them (block_item).  Pair after pair, every
-// pair ends with its short blocks and the next one begins with long ones: the launch ends with long blocks running alone.  All
-// pairs together, more K / V (or Q / dO) is in use than an L2 holds.  A group is taken as large as two rounds of the blocks that an XCD runs
-// at once (`slots`), and equal blocks are left pair after pair.  Kernel us, one pair / 4 pairs / all pairs at a time:
-//   dK/dV      B=8  8 kv heads of 32 D=128 causal S=1000   206 / 151 / 154 (8 pairs per XCD)    B=4 16 heads D=128 S=1024   67 / 50 / 51 (8)
-//   dK/dV      B=8 32 heads D=128 causal S=2048   685 / 636 / 696 (32)     the same, S=512    94 / 75 / 80 (32)
-//   dQ         B=4 12 heads D=64  causal S=2048    69 / 58 / 52 (6)        forward            58 / 48 / 42
-//   dK/dV      B=4 32 heads D=128 S=8192 causal  4087 / 4069 / 4453 (16)   no mask          7473 / 7607 / 8515
-int pair_group(long long pairs, long long blocks_per_pair, int slots, bool uneven) {
-    if (!uneven || pairs % 8) return 1;
-    const long long n = pairs / 8, want = std::max(1LL, (2LL * slots + blocks_per_pair - 1) / blocks_per_pair), groups = std::max(1LL, (n + want / 2) / want);
-    return (int)((n + groups - 1) / groups);
-}
-
-// The grid and its map; pairs x items x inner < 2^31 blocks.  Grids past the 65535 places of the second and third dimension (more than
-// 8 million keys in tiles of 128) are linear.
-struct Grid {
-    BlockMap map;
-    dim3 dim;
-};
-Grid block_grid(long long pairs, long long items, long long inner, int group) {
-    const long long per_xcd = pairs / 8, groups = (per_xcd + group - 1) / group;
-    if (pairs % 8 == 0 && group <= 65535 && groups * items <= 65535)
-        return {{group, (int)items, (int)groups, (int)inner}, dim3((unsigned)(8 * inner), (unsigned)group, (unsigned)(groups * items))};
-    return {{0, (int)items, 1, (int)inner}, dim3((unsigned)(pairs * items * inner))};
 }
 
 // Waves that share a row group's keys in the bf16 forward and dQ kernels.  Blocks of 256 rows leave CUs idle when a launch has few
@@ -4785,7 +4722,7 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     if (pl.blocks > 0x7fffffffLL) return LTR_EINVAL;
     p.n_qtiles = pl.n_qtiles;
     p.n_slots = pl.n_slots;
-    const Grid grid = block_grid((long long)p.B * p.Hkv, pl.n_slots, p.n_rep, pl.group);
+    const BlockGrid grid = block_grid((long long)p.B * p.Hkv, pl.n_slots, p.n_rep, pl.group);
     p.map = grid.map;
     if (a->io_dtype == LTR_BF16) {
         rc = enable_large_lds();
@@ -4797,20 +4734,20 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
                 {(const void *)fwd_bf16_pad_kernel<128, 1>, (const void *)fwd_bf16_pad_kernel<128, 2>, (const void *)fwd_bf16_pad_kernel<128, 4>}};
             const int lds[2][3] = {{fwd_lds_bytes<64>(), shares_lds_bytes<64, 2>(), shares_lds_bytes<64, 4>()},
                                    {fwd_lds_bytes<128>(), shares_lds_bytes<128, 2>(), shares_lds_bytes<128, 4>()}};
-            return launch(kernels[D == 128][i], grid.dim, 512, lds[D == 128][i], st, p);
+            return launch(kernels[D == 128][i], dims(grid), 512, lds[D == 128][i], st, p);
         }
         if (pl.four_waves)
-            return a->D == 128 ? launch((const void *)fwd_bf16_w4_kernel<128>, grid.dim, 256, FourWaves<128>::LDS, st, p)
-                               : launch((const void *)fwd_bf16_w4_kernel<64>, grid.dim, 256, FourWaves<64>::LDS, st, p);
+            return a->D == 128 ? launch((const void *)fwd_bf16_w4_kernel<128>, dims(grid), 256, FourWaves<128>::LDS, st, p)
+                               : launch((const void *)fwd_bf16_w4_kernel<64>, dims(grid), 256, FourWaves<64>::LDS, st, p);
         if (pl.ks == 2)
-            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 2>, grid.dim, 512, shares_lds_bytes<128, 2>(), st, p)
-                               : launch((const void *)fwd_bf16_shares_kernel<64, 2>, grid.dim, 512, shares_lds_bytes<64, 2>(), st, p);
+            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 2>, dims(grid), 512, shares_lds_bytes<128, 2>(), st, p)
+                               : launch((const void *)fwd_bf16_shares_kernel<64, 2>, dims(grid), 512, shares_lds_bytes<64, 2>(), st, p);
         if (pl.ks == 4)
-            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 4>, grid.dim, 512, shares_lds_bytes<128, 4>(), st, p)
-                               : launch((const void *)fwd_bf16_shares_kernel<64, 4>, grid.dim, 512, shares_lds_bytes<64, 4>(), st, p);
-        if (a->D == 128) return launch((const void *)fwd_bf16_kernel<128, 1>, grid.dim, 512, fwd_lds_bytes<128>(), st, p);
-        if (pl.wide) return launch((const void *)fwd_bf16_kernel<64, 2>, grid.dim, 512, fwd_lds_bytes<64, 2>(), st, p);
-        return launch((const void *)fwd_bf16_kernel<64, 1>, grid.dim, 512, fwd_lds_bytes<64>(), st, p);
+            return a->D == 128 ? launch((const void *)fwd_bf16_shares_kernel<128, 4>, dims(grid), 512, shares_lds_bytes<128, 4>(), st, p)
+                               : launch((const void *)fwd_bf16_shares_kernel<64, 4>, dims(grid), 512, shares_lds_bytes<64, 4>(), st, p);
+        if (a->D == 128) return launch((const void *)fwd_bf16_kernel<128, 1>, dims(grid), 512, fwd_lds_bytes<128>(), st, p);
+        if (pl.wide) return launch((const void *)fwd_bf16_kernel<64, 2>, dims(grid), 512, fwd_lds_bytes<64, 2>(), st, p);
+        return launch((const void *)fwd_bf16_kernel<64, 1>, dims(grid), 512, fwd_lds_bytes<64>(), st, p);
     }
     if (pl.f32_ks) {   // fp32 on the matrix pipe; the chunk offsets of its LDS-direct loads are 64-bit, nothing more to check
         rc = enable_large_lds();
@@ -4971,8 +4908,8 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     p.n_reps = p.n_rep / pl.split.reps;
     p.part = (float *)work;
     p.n_slots = pl.dq_slots;
-    const Grid q_grid = block_grid((long long)p.B * p.Hkv, pl.dq_slots, p.n_rep, pl.dq_group);
-    const Grid key_grid = block_grid((long long)p.B * p.Hkv, tiles_seen, pl.split.n, pl.kv_group);
+    const BlockGrid q_grid = block_grid((long long)p.B * p.Hkv, pl.dq_slots, p.n_rep, pl.dq_group);
+    const BlockGrid key_grid = block_grid((long long)p.B * p.Hkv, tiles_seen, pl.split.n, pl.kv_group);
     p.q_map = q_grid.map;
     p.kv_map = key_grid.map;
     hipStream_t st = (hipStream_t)stream;
@@ -5019,19 +4956,19 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
                 {(const void *)bwd_dq_pad_kernel<128, 1>, (const void *)bwd_dq_pad_kernel<128, 2>, (const void *)bwd_dq_pad_kernel<128, 4>}};
             const int lds[2][3] = {{dq_lds_bytes<64>(), shares_lds_bytes<64, 2>(), shares_lds_bytes<64, 4>()},
                                    {dq_lds_bytes<128>(), shares_lds_bytes<128, 2>(), shares_lds_bytes<128, 4>()}};
-            rc = launch(kernels[D == 128][i], q_grid.dim, 512, lds[D == 128][i], st, p);
+            rc = launch(kernels[D == 128][i], dims(q_grid), 512, lds[D == 128][i], st, p);
         } else if (pl.dq_four_waves)
-            rc = a->D == 128 ? launch((const void *)bwd_dq_w4_kernel<128>, q_grid.dim, 256, FourWaves<128>::LDS, st, p)
-                             : launch((const void *)bwd_dq_w4_kernel<64>, q_grid.dim, 256, FourWaves<64>::LDS, st, p);
+            rc = a->D == 128 ? launch((const void *)bwd_dq_w4_kernel<128>, dims(q_grid), 256, FourWaves<128>::LDS, st, p)
+                             : launch((const void *)bwd_dq_w4_kernel<64>, dims(q_grid), 256, FourWaves<64>::LDS, st, p);
         else if (pl.dq_ks == 2)
-            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 2>, q_grid.dim, 512, shares_lds_bytes<128, 2>(), st, p)
-                             : launch((const void *)bwd_dq_shares_kernel<64, 2>, q_grid.dim, 512, shares_lds_bytes<64, 2>(), st, p);
+            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 2>, dims(q_grid), 512, shares_lds_bytes<128, 2>(), st, p)
+                             : launch((const void *)bwd_dq_shares_kernel<64, 2>, dims(q_grid), 512, shares_lds_bytes<64, 2>(), st, p);
         else if (pl.dq_ks == 4)
-            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 4>, q_grid.dim, 512, shares_lds_bytes<128, 4>(), st, p)
-                             : launch((const void *)bwd_dq_shares_kernel<64, 4>, q_grid.dim, 512, shares_lds_bytes<64, 4>(), st, p);
-        else if (a->D == 128) rc = launch((const void *)bwd_dq_kernel<128, 1>, q_grid.dim, 512, dq_lds_bytes<128>(), st, p);
-        else if (pl.wide_q) rc = launch((const void *)bwd_dq_kernel<64, 2>, q_grid.dim, 512, dq_lds_bytes<64>(), st, p);
-        else rc = launch((const void *)bwd_dq_kernel<64, 1>, q_grid.dim, 512, dq_lds_bytes<64>(), st, p);
+            rc = a->D == 128 ? launch((const void *)bwd_dq_shares_kernel<128, 4>, dims(q_grid), 512, shares_lds_bytes<128, 4>(), st, p)
+                             : launch((const void *)bwd_dq_shares_kernel<64, 4>, dims(q_grid), 512, shares_lds_bytes<64, 4>(), st, p);
+        else if (a->D == 128) rc = launch((const void *)bwd_dq_kernel<128, 1>, dims(q_grid), 512, dq_lds_bytes<128>(), st, p);
+        else if (pl.wide_q) rc = launch((const void *)bwd_dq_kernel<64, 2>, dims(q_grid), 512, dq_lds_bytes<64>(), st, p);
+        else rc = launch((const void *)bwd_dq_kernel<64, 1>, dims(q_grid), 512, dq_lds_bytes<64>(), st, p);
         if (rc) return rc;
     }
     if (do_dkdv) {
@@ -5041,12 +4978,12 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
         // the tail (the sums inside a block do not depend on the table's order).
         if (flags & LTR_CAUSAL)
             std::stable_sort(p.chunk, p.chunk + p.n_chunks, [](const ChunkDev &x, const ChunkDev &y) { return x.pos0 < y.pos0; });
-        if (pad) rc = D == 128 ? launch((const void *)bwd_dkdv_pad_kernel<128>, key_grid.dim, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p)
-                               : launch((const void *)bwd_dkdv_pad_kernel<64>, key_grid.dim, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
-        else if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, key_grid.dim, BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
+        if (pad) rc = D == 128 ? launch((const void *)bwd_dkdv_pad_kernel<128>, dims(key_grid), BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p)
+                               : launch((const void *)bwd_dkdv_pad_kernel<64>, dims(key_grid), BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
+        else if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, dims(key_grid), BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
         else if (pl.wide_kv) rc = launch((const void *)bwd_dkdv_kernel<64, 2>, kv_grid, BwdLds<64, 2>::NT, BwdLds<64, 2>::TOTAL, st, p);
-        else if (pl.key_waves) rc = launch((const void *)bwd_dkdv_keywave_kernel<64>, key_grid.dim, KeyWaveLds<64>::NT, KeyWaveLds<64>::TOTAL, st, p);
-        else rc = launch((const void *)bwd_dkdv_kernel<64, 1>, key_grid.dim, BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
+        else if (pl.key_waves) rc = launch((const void *)bwd_dkdv_keywave_kernel<64>, dims(key_grid), KeyWaveLds<64>::NT, KeyWaveLds<64>::TOTAL, st, p);
+        else rc = launch((const void *)bwd_dkdv_kernel<64, 1>, dims(key_grid), BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
         if (rc || pl.split.n == 1) return rc;
         rc = D == 128 ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
              : pl.wide_kv ? launch((const void *)bwd_dkdv_reduce_kernel<64, 2>, reduce_grid, 256, 0, st, p)

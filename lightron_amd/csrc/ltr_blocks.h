@@ -1,0 +1,84 @@
+// Which (batch, kv head) pair, which of its tiles and which of the blocks of that tile a block of the bf16 kernels works on: the grid that the
+// host launches (block_grid, pair_group) and the arithmetic that undoes it (block_item_at).  Plain C++, so that it can be checked on a CPU.
+#pragma once
+#include <algorithm>
+
+#ifdef __HIP__
+#define LTR_HOST_DEVICE __host__ __device__ __forceinline__
+#else
+#define LTR_HOST_DEVICE inline
+#endif
+
+struct BlockMap {      // see block_item_at
+    int group;         // (batch, kv head) pairs of an XCD whose blocks are handed out together; 0: a linear grid
+    int items;         // items (q tile slots, key tiles) per pair
+    int groups;
+    int inner;         // blocks per item
+};
+
+// Block (x, y, z) -> (pair = batch x kv head, item = q tile slot or key tile of the pair, sub = one of the `inner` blocks of an item).
+// Consecutive blocks go to the 8 XCDs round-robin.  All blocks of a pair run on one XCD and next to each other in time, so the
+// blocks that are resident together stream the same K / V (or Q / dO) through that XCD's L2; the inner blocks of an item follow each
+// other.  The items of `group` pairs of an XCD are handed out item by item (the first of every pair, the second of every pair, ...):
+// items come longest first, so blocks of unequal length end together (see pair_group).  The grid is (8 XCDs x inner blocks, pairs of a
+// group, items of the groups): the hardware counts what would be four divisions (0.3 us of every block, also as multiplications: their
+// constants are another trip to the arguments).
+struct BlockItem {
+    int pair, item, sub;
+    int order;   // of the blocks of an XCD
+};
+LTR_HOST_DEVICE BlockItem block_item_at(const BlockMap &m, int pairs, unsigned x, unsigned y, unsigned z) {
+    BlockItem r;
+    if (m.group) {
+        int g = 0;
+        r.item = z;
+        if (m.groups > 1) {
+            g = r.item / m.items;
+            r.item -= g * m.items;
+        }
+        r.sub = x >> 3;
+        r.pair = (g * m.group + y) * 8 + (x & 7);   // past the last pair: a place of the last group that is empty
+        r.order = r.sub + m.inner * (y + m.group * z);
+    } else {   // pairs that do not divide among the XCDs: one block of every pair, then the next
+        const int rest = x / pairs;
+        r.pair = x - rest * pairs;
+        r.item = rest / m.inner;
+        r.sub = rest - r.item * m.inner;
+        r.order = x >> 3;
+    }
+    return r;
+}
+
+// How many (batch, kv head) pairs of an XCD hand out their blocks together, longest first across them (block_item_at).  Pair after pair, every
+// pair ends with its short blocks and the next one begins with long ones: the launch ends with long blocks running alone.  All
+// pairs together, more K / V (or Q / dO) is in use than an L2 holds.  A group is taken as large as two rounds of the blocks that an XCD runs
+// at once (`slots`), and equal blocks are left pair after pair.  Kernel us, one pair / 4 pairs / all pairs at a time:
+//   dK/dV      B=8  8 kv heads of 32 D=128 causal S=1000   206 / 151 / 154 (8 pairs per XCD)    B=4 16 heads D=128 S=1024   67 / 50 / 51 (8)
+//   dK/dV      B=8 32 heads D=128 causal S=2048   685 / 636 / 696 (32)     the same, S=512    94 / 75 / 80 (32)
+//   dQ         B=4 12 heads D=64  causal S=2048    69 / 58 / 52 (6)        forward            58 / 48 / 42
+//   dK/dV      B=4 32 heads D=128 S=8192 causal  4087 / 4069 / 4453 (16)   no mask          7473 / 7607 / 8515
+inline int pair_group(long long pairs, long long blocks_per_pair, int slots, bool uneven) {
+    if (!uneven || pairs % 8) return 1;
+    const long long n = pairs / 8, want = std::max(1LL, (2LL * slots + blocks_per_pair - 1) / blocks_per_pair), groups = std::max(1LL, (n + want / 2) / want);
+    return (int)((n + groups - 1) / groups);
+}
+
+// The grid and its map; pairs x items x inner < 2^31 blocks.  The second and third dimension end at 65535: more items of groups than that
+// (1024 pairs of 65536 keys in tiles of 128, 131072 pairs of 512) take larger groups, a pair with more items (8 million keys) a linear grid.
+// dK/dV without a mask, all pairs block by block as the linear grid has them / groups of two, ms:
+//   4096 x 32 heads S=512  D=64 27.0 / 24.2  D=128 52.8 / 48.4      32 x 32 heads D=128, 512 rows against 65600 keys 52.4 / 44.9
+constexpr int GRID_YZ_MAX = 65535;
+struct BlockGrid {
+    BlockMap map;
+    unsigned x, y, z;
+};
+inline BlockGrid block_grid(long long pairs, long long items, long long inner, long long group) {
+    const long long per_xcd = pairs / 8;
+    if (pairs % 8 == 0 && items > 0 && items <= GRID_YZ_MAX) {
+        const long long most = GRID_YZ_MAX / items;   // groups
+        group = std::max(group, (per_xcd + most - 1) / most);
+        const long long groups = (per_xcd + group - 1) / group;
+        if (group <= GRID_YZ_MAX) return {{(int)group, (int)items, (int)groups, (int)inner}, (unsigned)(8 * inner), (unsigned)group, (unsigned)(groups * items)};
+    }
+    return {{0, (int)items, 1, (int)inner}, (unsigned)(pairs * items * inner), 1, 1};
+}

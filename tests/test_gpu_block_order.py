@@ -53,3 +53,29 @@ def test_every_block_runs_once(ltr, D, B, Hq, Hkv, S):
             a, b = tiles(x)[:, first:first + 64], tiles(r)[:, first:first + 64]
             err = (a - b).flatten(1).norm(dim=1) / b.flatten(1).norm(dim=1).clamp_min(1e-3)
             assert err.max() < 2e-2, (name, first, err.max().item())
+
+
+@pytest.mark.parametrize("B,H", [(65536, 8), (65537, 8)])   # no empty place in the last group; one per XCD
+def test_more_pairs_than_places_of_the_grid(ltr, B, H):
+    """65536 pairs per XCD: one more than the grid's third dimension holds.  Two rows and keys, against the closed form."""
+    g = torch.Generator(device="cuda").manual_seed(B)
+    q, k, v, do = (torch.randn(B, 2, H, 64, generator=g, device="cuda").to(torch.bfloat16) for _ in range(4))
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    o, lse = ltr.block_attention(q, [k], [v], [0], causal=True)
+    o.backward(do)
+    qf, kf, vf, df = (t.detach().float() for t in (q, k, v, do))
+    s = torch.stack([(qf[:, 1] * kf[:, j]).sum(-1) for j in range(2)], -1) / 8         # row 1: [B, H, 2]; row 0 sees key 0 alone
+    p = torch.softmax(s, -1)
+    o1 = p[..., :1] * vf[:, 0] + p[..., 1:] * vf[:, 1]
+    dp = torch.stack([(df[:, 1] * vf[:, j]).sum(-1) for j in range(2)], -1)
+    ds = p * (dp - (p * dp).sum(-1, keepdim=True)) / 8
+    ref = {"o": torch.stack([vf[:, 0], o1], 1), "dq": torch.stack([torch.zeros_like(o1), ds[..., :1] * kf[:, 0] + ds[..., 1:] * kf[:, 1]], 1),
+           "dk": torch.stack([ds[..., j:j + 1] * qf[:, 1] for j in range(2)], 1),
+           "dv": torch.stack([df[:, 0] + p[..., :1] * df[:, 1], p[..., 1:] * df[:, 1]], 1)}
+    assert (lse[:, :, 1] - torch.logsumexp(s, -1)).abs().max() < 2e-2
+    # bf16 operands and results: 3e-3 of a row's norm, 2e-2 with the largest of a million rows.  dS = P (dO . v - DELTA) besides has DELTA from
+    # the bf16 O: 64 products of order 1 rounded to 2^-9 each, 0.016 rms and 0.1 at six sigma, times |k| / 8 of at most 1.5 (dQ; dK alike).
+    # A block left out or run twice is the whole of a row, of norm 3 .. 10
+    for name, got in (("o", o.detach()), ("dq", q.grad), ("dk", k.grad), ("dv", v.grad)):
+        err, norm = (got.float() - ref[name]).flatten(2).norm(dim=2) / H ** 0.5, ref[name].flatten(2).norm(dim=2) / H ** 0.5
+        assert (err <= 2e-2 * norm + 0.15).all(), (name, (err - 2e-2 * norm).max().item())
