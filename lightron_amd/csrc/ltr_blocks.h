@@ -57,10 +57,19 @@ LTR_HOST_DEVICE BlockItem block_item_at(const BlockMap &m, int pairs, unsigned x
 //   dK/dV      B=8 32 heads D=128 causal S=2048   685 / 636 / 696 (32)     the same, S=512    94 / 75 / 80 (32)
 //   dQ         B=4 12 heads D=64  causal S=2048    69 / 58 / 52 (6)        forward            58 / 48 / 42
 //   dK/dV      B=4 32 heads D=128 S=8192 causal  4087 / 4069 / 4453 (16)   no mask          7473 / 7607 / 8515
+// A small last group, of less than 1.4 rounds and 0.7 of the others, ends the launch with its own long blocks alone: larger groups are
+// taken instead.  Kernel us with the small one / without:
+//   dK/dV      B=2 12 heads D=96  causal S=4730   322 / 255 (2+1 pairs, 3)       B=13 8 heads D=96 S=3464   753 / 652 (4+4+4+1, 5+5+3)
+//   dK/dV      B=10 8 kv heads of 32 D=64 S=7950  6293 / 5344 (4+4+2, 5+5)        B=8  8 kv heads of 32 D=128, 1306 of 2612 keys  309 / 262 (3+3+2, 4+4)
+//   forward    B=5 16 heads D=64  causal S=6284   529 / 465 (4+4+2, 5+5)
 inline int pair_group(long long pairs, long long blocks_per_pair, int slots, bool uneven) {
     if (!uneven || pairs % 8) return 1;
-    const long long n = pairs / 8, want = std::max(1LL, (2LL * slots + blocks_per_pair - 1) / blocks_per_pair), groups = std::max(1LL, (n + want / 2) / want);
-    return (int)((n + groups - 1) / groups);
+    const long long n = pairs / 8, want = std::max(1LL, (2LL * slots + blocks_per_pair - 1) / blocks_per_pair);
+    for (long long groups = (n + want / 2) / want; groups > 1; groups--) {
+        const long long group = (n + groups - 1) / groups, last = n - (n - 1) / group * group;
+        if (last * 10 >= want * 7 || last * 10 >= group * 7) return (int)group;
+    }
+    return (int)n;
 }
 
 // The grid and its map; pairs x items x inner < 2^31 blocks.  The second and third dimension end at 65535: more items of groups than that

@@ -85,3 +85,20 @@ def test_limits_of_the_grid(blocks, pairs, items, inner, group, used):
     out = blocks(pairs, items, inner, group)
     assert out[4] == "ok" and out[0] == str(used), out
     assert int(out[5]) <= (used or pairs // 8)
+
+
+@pytest.mark.parametrize("per_xcd,per_pair,slots,group", [
+    (3, 46, 32, 3), (5, 40, 32, 3), (10, 24, 32, 5), (13, 28, 32, 5), (8, 22, 32, 4), (10, 63, 64, 5),       # not 2+1, 2+2+1, 4+4+2, 4+4+4+1, 3+3+2
+    (33, 3, 32, 17), (60, 3, 32, 20), (15, 12, 32, 5), (6, 20, 32, 3), (28, 6, 32, 10), (7, 18, 32, 4), (9, 12, 32, 5),   # 1.3 - 1.9 rounds stay
+    (1, 10, 32, 1), (8, 8, 32, 8), (24, 8, 32, 8), (32, 16, 32, 4), (16, 64, 32, 1), (16, 200, 32, 1), (4, 12, 96, 4),
+])
+def test_groups_of_pairs(blocks, per_xcd, per_pair, slots, group):
+    assert blocks(8 * per_xcd, per_pair, slots, "group")[0] == str(group)
+
+
+def test_the_last_group_is_not_a_small_one(blocks):
+    """It would end the launch with its own long blocks alone."""
+    for per_xcd in (1, 2, 3, 5, 6, 7, 8, 10, 11, 13, 16, 24, 32, 60):
+        for per_pair, slots in ((8, 32), (18, 32), (24, 32), (30, 64), (46, 32), (12, 96), (64, 32), (200, 32)):
+            group, last = (int(x) for x in blocks(8 * per_xcd, per_pair, slots, "group"))
+            assert group == per_xcd or last * per_pair >= 1.4 * slots or last >= 0.7 * group, (per_xcd, per_pair, slots, group, last)
