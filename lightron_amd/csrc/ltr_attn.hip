@@ -4585,6 +4585,16 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
                              causal_ && key_tiles_uneven(Sq, pl.keys_per_block, q_split, q_pos0, chunk, n_chunks));
     return pl;
 }
+// The plan with a workspace of that many bytes: shared key tiles if their partial sums fit, else the launch without a workspace (whose kernel
+// and block order are other ones than those chosen for sharing).
+BwdPlan plan_bwd_ws(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks,
+                    int64_t work_bytes) {
+    if (work_bytes > 0) {
+        const BwdPlan pl = plan_bwd(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, true);
+        if (pl.part_bytes <= work_bytes) return pl;
+    }
+    return plan_bwd(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks);
+}
 // blocks of bwd_dkdv_reduce_kernel: four waves each, one per 64 columns of a 32-key slice of dK or dV
 long long reduce_blocks(const BwdPlan &pl, int D) { return pl.kv_blocks * (pl.keys_per_block / 128) * (D / 32); }
 
@@ -4895,8 +4905,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     p.flags = flags;
     p.n_chunks = a->n_chunks;
     p.cols = a->D;
-    BwdPlan pl = plan_bwd(D, f32, flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks, work != nullptr);
-    if (pl.part_bytes > work_bytes) pl.split.n = pl.split.reps = 1;
+    const BwdPlan pl = plan_bwd_ws(D, f32, flags, p.B, p.Hq, p.Hkv, p.Sq, p.q_split, p.q_pos0, p.chunk, p.n_chunks, work ? work_bytes : 0);
     p.q_last = pl.split.n > 1 ? pl.split.q_last : 0x7fffffff;
     const long long tiles_seen = pl.split.n > 1 ? pl.split.tiles : pl.kv_tiles;
     const long long kv_grid = tiles_seen * p.B * p.Hkv * pl.split.n, reduce_grid = reduce_blocks(pl, D);
@@ -5054,8 +5063,8 @@ int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work
     }
     const int q_pos0[2] = {(int)a->q_pos0[0], (int)a->q_pos0[1]};
     const FwdPlan f = plan_fwd(D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks);
-    const BwdPlan b = plan_bwd(D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks, work_bytes > 0);
-    const bool shared = b.split.n > 1 && b.part_bytes <= work_bytes;
+    const BwdPlan b = plan_bwd_ws(D, f32, flags, a->B, a->Hq, a->Hkv, (int)a->Sq, (int)a->q_split, q_pos0, chunk, a->n_chunks, work_bytes);
+    const bool shared = b.split.n > 1;
     out->compute_units = device_cus();
     out->fwd_rows = f.rows;
     out->fwd_paired = f.n_slots != f.n_qtiles;

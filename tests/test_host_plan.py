@@ -133,3 +133,14 @@ def test_one_round_of_shares_stays(B, Hq, Hkv, S):
     plan = la.attn_plan(B, Hq, Hkv, 128, S, [S], [0], 0, None, True)
     if plan["compute_units"] == 256:
         assert plan["fwd"]["kernel"] == "fwd_bf16_shares_kernel<128, 2>" and plan["dq"]["kernel"] == "bwd_dq_shares_kernel<128, 2>"
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,causal", [(1, 1, 1, 500, True), (1, 2, 1, 200, False), (1, 2, 1, 500, True), (4, 32, 8, 1000, True), (1, 8, 4, 2000, False)])
+def test_a_workspace_that_is_too_small_is_none(B, Hq, Hkv, S, causal):
+    """Head dim 64, where shared key tiles take another kernel than tiles of one block: one byte short is the launch without a workspace."""
+    a = _args(64, B, Hq, Hkv, S, [(S, 0)], L.LTR_CAUSAL if causal else 0)
+    need, short, full = ctypes.c_int64(0), L.AttnPlanWs(), L.AttnPlanWs()
+    assert L.load().ltr_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(need)) == 0 and need.value > 0
+    assert L.load().ltr_attn_plan_ws(ctypes.byref(a), need.value - 1, ctypes.byref(short)) == 0
+    assert L.load().ltr_attn_plan_ws(ctypes.byref(a), need.value, ctypes.byref(full)) == 0 and full.blocks_per_tile > 1
+    assert bytes(short.plan) == bytes(_plan(a)[1]) and short.blocks_per_tile == 1
