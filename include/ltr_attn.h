@@ -58,7 +58,8 @@ extern "C" {
 #define LTR_DKDV_BF16 64u /* backward: chunk[c].dk / dv are bf16 tensors that RECEIVE dK / dV of this call (no accumulation) */
 #define LTR_ROPE_Q 128u   /* forward: q is un-rotated; RoPE is applied to it in the kernel's prologue (rope_freqs) */
 #define LTR_ROPE_DQ 256u  /* backward: dQ leaves the dQ kernel rotated by the conjugate angles (gradient of LTR_ROPE_Q) */
-#define LTR_DKDV_KEYS_128 512u  /* backward, tuning hint: the dK/dV kernel's blocks own 128 keys (the default choice is the library's) */
+#define LTR_DKDV_KEYS_128 512u  /* backward, tuning hint: the dK/dV kernel's blocks own 128 keys (the default choice is the library's, as
+                                   is that among the kernels with 128 keys) */
 #define LTR_DKDV_KEYS_256 1024u /* backward, tuning hint: they own 256 keys (bf16, head dim 64 only: LTR_EUNSUP otherwise); results
                                    do not depend on the hint beyond the order of fp32 additions inside a block */
 #define LTR_DQ_ROWS_256 2048u /* backward, tuning hint: the dQ kernel's blocks own 256 query rows (the default choice is the library's) */

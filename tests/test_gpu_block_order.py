@@ -35,6 +35,9 @@ def _reference(q, k, v, do):
     (128, 8, 32, 8, 1000),    # four q heads per pair
     (128, 11, 16, 8, 2100),   # groups of several sizes, two q heads per pair
     (128, 1, 8, 8, 1100),     # one pair per XCD
+    (96, 13, 8, 8, 2300),     # padded head dims: groups of 7 + 6 and 5 + 5 + 3 pairs, places of the last one empty
+    (40, 13, 8, 8, 2300),
+    (128, 5, 8, 8, 2500),     # 3 + 2
 ])
 def test_every_block_runs_once(ltr, D, B, Hq, Hkv, S):
     g = torch.Generator(device="cuda").manual_seed(S)

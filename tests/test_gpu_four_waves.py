@@ -59,3 +59,42 @@ def test_four_waves(ltr, D, B, Hq, Hkv, Sq, q_pos, split, chunks, causal):
     assert (dq32 - dq1.cpu()).norm() <= 1e-5 * dq1.cpu().norm()
     # bf16 rounding (2^-8 of the value) and the cancellation of the accumulator's start value (2^-23 of 0.5 + |dQ|)
     assert ((dq16.cpu().float() - dq32).abs() <= dq32.abs() / 256 + 1e-6).all()
+
+
+@pytest.mark.parametrize("D,B,Hq,Hkv,Sq,q_pos,split", [
+    (64, 40, 16, 16, 140, 0, None),
+    (64, 24, 24, 12, 150, (40, 300), 33),        # two segments: a wave's rows from both
+    (128, 24, 16, 16, 300, 0, None),
+    (128, 19, 24, 12, 290, 7, None),
+])
+def test_four_waves_with_rope(ltr, D, B, Hq, Hkv, Sq, q_pos, split):
+    """q rotated in the prologue (into a copy and in place) and dQ rotated back in the epilogue, against launches of the same kernels on q rotated
+    beforehand."""
+    qp = q_pos if isinstance(q_pos, tuple) else (q_pos, q_pos)
+    total = max(qp) + Sq
+    plan = ltr.attn_plan(B, Hq, Hkv, D, Sq, [total], [0], q_pos, split, True)
+    assert plan["fwd"]["kernel"] == "fwd_bf16_w4_kernel<%d>" % D and plan["dq"]["kernel"] == "bwd_dq_w4_kernel<%d>" % D
+    g = torch.Generator(device="cuda").manual_seed(Sq)
+    q, do, k, v = (torch.randn(B, s, h, D, generator=g, device="cuda").to(torch.bfloat16) for s, h in ((Sq, Hq), (Sq, Hq), (total, Hkv), (total, Hkv)))
+    freqs = orc.precompute_freqs_cis(D, total)
+    rows = torch.arange(Sq)
+    at = freqs[rows + qp[0] if split is None else torch.where(rows < split, rows + qp[0], rows - split + qp[1])]
+    q_in = orc.apply_rotary_emb(q.cpu(), q.cpu(), at)[0].cuda()
+    table = ltr.rope_table(freqs.cuda())
+    o_ref, lse_ref = ltr.attn_fwd(q_in, [k], [v], [0], q_pos, split, True)
+    rot, inplace = torch.full_like(q, float("nan")), q.clone()
+    for src, dst in ((q, rot), (inplace, inplace), (q, None)):
+        o, lse = ltr.attn_fwd(src, [k], [v], [0], q_pos, split, True, q_rope=table, q_rot_out=dst)
+        assert torch.equal(o, o_ref) and torch.equal(lse, lse_ref)
+        assert dst is None or torch.equal(dst, q_in)
+    delta = torch.empty(lse.shape, dtype=torch.float32, device="cuda")
+    sink = torch.zeros(k.shape, dtype=torch.float32, device="cuda")
+    plain, turned = (torch.full(q.shape, start, dtype=torch.float32, device="cuda") for start in (0.0, 0.5))
+    turned16 = torch.empty_like(q)
+    for dq, kw in ((plain, {}), (turned, dict(dq_rope=table)), (turned16, dict(dq_rope=table))):
+        ltr.attn_bwd_accumulate(rot, do, lse, delta, [k], [v], [0], dq, [sink], [sink], q_pos, split, True, do_dkdv=False, o=o, **kw)
+    want = orc.apply_rotary_emb(plain.cpu(), plain.cpu(), at.conj())[0]
+    got = turned.cpu() - 0.5
+    # four fp32 products per pair of columns, and the cancellation of the accumulator's start value (2^-23 of 0.5 + |dQ|)
+    assert ((got - want).abs() <= 2e-6 * (0.5 + want.abs())).all()
+    assert ((turned16.cpu().float() - want).abs() <= want.abs() / 256 + 2e-6).all()

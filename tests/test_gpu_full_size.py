@@ -279,12 +279,12 @@ def test_config5_full_ulysses_layout(ltr):
     assert qd.grad[0][:, :, :r * (H // W)].abs().max() == 0
 
 
-@pytest.mark.parametrize("keys,rows", [(256, 512), (128, 256)])
+@pytest.mark.parametrize("keys,rows", [(256, 512), (128, 256), (None, None)])
 def test_head_dim_64_ring_share_both_block_sizes(ltr, keys, rows):
-    """Head dim 64 at a size where the 256-key dK/dV blocks and 512-row dQ blocks are what the library runs: one zig-zag rank
+    """Head dim 64 at full size, both block sizes and the library's own choice (128-row blocks of two key shares, 128 keys): one zig-zag rank
     share (rank 2 of 4: half-chunks 2 and 5 of 8 x 2048 positions) of a causal GQA 8/2 sequence of 16384, B = 2, against all
-    8 KV half-chunks in ring order, fp32 dK / dV accumulators, bf16 dQ with DELTA from O.  Both block sizes of all three
-    kernels forced through the hint flags (the forward with the dQ kernel's rows per block); sampled rows (O, LSE, dQ) and sampled keys (dK, dV) against the oracle's closed form."""
+    8 KV half-chunks in ring order, fp32 dK / dV accumulators, bf16 dQ with DELTA from O.  The sizes are
+    forced through the hint flags (the forward with the dQ kernel's rows per block); sampled rows (O, LSE, dQ) and sampled keys (dK, dV) against the oracle's closed form."""
     g = torch.Generator().manual_seed(5)
     B, Hq, Hkv, D, S, W = 2, 8, 2, 64, 16384, 4
     hc = S // (2 * W)
@@ -303,6 +303,11 @@ def test_head_dim_64_ring_share_both_block_sizes(ltr, keys, rows):
     vs = [vd[:, i * hc:(i + 1) * hc] for i in order]
     pos0 = [i * hc for i in order]
     qp = (r * hc, (2 * W - 1 - r) * hc)
+    plan = ltr.attn_plan(B, Hq, Hkv, D, 2 * hc, [hc] * len(order), pos0, qp, hc, True, fwd_rows=rows, dq_rows=rows, dkdv_keys=keys)
+    if plan["compute_units"] == 256:
+        want = {512: ("fwd_bf16_kernel<64, 2>", "bwd_dq_kernel<64, 2>", "bwd_dkdv_kernel<64, 2>"), 256: ("fwd_bf16_kernel<64, 1>", "bwd_dq_kernel<64, 1>", None),
+                None: ("fwd_bf16_shares_kernel<64, 2>", "bwd_dq_shares_kernel<64, 2>", None)}[rows]
+        assert all(plan[k]["kernel"] == w for k, w in zip(("fwd", "dq", "dkdv"), want) if w) and plan["dkdv"]["keys"] == (keys or 128)
     ol, lsel = ltr.attn_fwd(ql, ks, vs, pos0, qp, hc, True, fwd_rows=rows)     # the forward's block follows the dQ kernel's
     dk = torch.zeros(kd.shape, dtype=torch.float32, device="cuda")
     dv = torch.zeros(vd.shape, dtype=torch.float32, device="cuda")
@@ -323,8 +328,8 @@ def test_head_dim_64_ring_share_both_block_sizes(ltr, keys, rows):
 def test_head_dim_64_paired_512_row_blocks(ltr, Sq):
     """Head dim 64, one causal chunk, enough (batch, head) pairs that the 512-row blocks of the forward and dQ kernels are
     handed out in pairs (late q tile + early counterpart: 4 tiles -> 2 slots x 128 pairs = 256 blocks, one per CU), with a
-    ragged last tile in the second case.  512 rows forced through the hint flags (the library's own choice at 2048); sampled
-    rows and keys against the oracle's closed form."""
+    ragged last tile in the second case.  512 rows forced through the hint flags; the library's own choice (four-wave forward; paired 256-row
+    dQ blocks at 2048, four waves at 1900) beside them.  Sampled rows and keys against the oracle's closed form."""
     g = torch.Generator().manual_seed(11 + Sq)
     B, Hq, Hkv, D = 4, 32, 8, 64
     q = torch.randn(B, Sq, Hq, D, generator=g).to(torch.bfloat16)
@@ -341,7 +346,16 @@ def test_head_dim_64_paired_512_row_blocks(ltr, Sq):
     delta_ws = torch.empty(B, Hq, Sq, dtype=torch.float32, device="cuda")
     ltr.attn_bwd_accumulate(qd, dod, lse, delta_ws, [kd], [vd], [0], dq, [dk], [dv], 0, None, True, do_dkdv=False, o=o, dq_rows=512)
     ltr.attn_bwd_accumulate(qd, dod, lse, delta_ws, [kd], [vd], [0], dq, [dk], [dv], 0, None, True, do_dq=False)
+    own = ltr.attn_plan(B, Hq, Hkv, D, Sq, [Sq], [0], 0, None, True)
+    if own["compute_units"] == 256:
+        assert own["fwd"]["kernel"] == "fwd_bf16_w4_kernel<64>"
+        assert own["dq"]["kernel"] == ("bwd_dq_kernel<64, 1>" if Sq == 2048 else "bwd_dq_w4_kernel<64>") and own["dq"]["paired"] == (Sq == 2048)
+    o_own, lse_own = ltr.attn_fwd(qd, [kd], [vd], [0], 0, None, True)
+    dq_own = torch.empty_like(dq)
+    ltr.attn_bwd_accumulate(qd, dod, lse_own, torch.empty_like(delta_ws), [kd], [vd], [0], dq_own, [dk], [dv], 0, None, True, do_dkdv=False, o=o_own)
     pos = torch.arange(Sq)
+    edges = [512, Sq - Sq % 512 or Sq]
+    _check_rows(q, k, v, pos, pos, True, o_own.cpu(), lse_own.cpu(), do, dq_own.cpu(), n=30, edge_rows=edges + [128, Sq - Sq % 128 or Sq])
     oc, lsec = o.cpu(), lse.cpu()
-    _check_rows(q, k, v, pos, pos, True, oc, lsec, do, dq.cpu(), n=30, edge_rows=[512, Sq - Sq % 512 or Sq])
+    _check_rows(q, k, v, pos, pos, True, oc, lsec, do, dq.cpu(), n=30, edge_rows=edges)
     _check_keys(q, k, v, oc, lsec, do, pos, pos, True, dk.float().cpu(), dv.float().cpu(), n=8, edge_keys=[256, Sq - 63])

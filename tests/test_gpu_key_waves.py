@@ -1,8 +1,11 @@
 """bwd_dkdv_keywave_kernel (head dim 64, one wave per 32 keys), which launches with many key tiles take: against the dense oracle, at
 the edges of its tiles (128 keys per block, 32 per wave, 64 rows per step in two halves)."""
+import ctypes
+
 import pytest
 import torch
 
+from lightron_amd import _lib as L
 from oracle import ring_attention_oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -53,3 +56,43 @@ def test_key_waves(ltr, B, Hq, Hkv, Sq, q_pos, split, chunks, causal, share):
         assert (x[~seen].abs() < 1e-6).all() and (y[~seen] == 0).all()
         # bf16 rounding (2^-8 of the value) and the cancellation of the accumulator's start value (2^-23 of 0.5 + |x|)
         assert ((y - x).abs() <= x.abs() / 256 + 1e-6).all()
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,q_pos,split,chunks,causal", [
+    (24, 16, 16, 140, 0, None, [(140, 0)], True),
+    (20, 16, 16, 97, (40, 300), 33, [(31, 0), (130, 31), (64, 500)], True),
+    (20, 16, 16, 65, 0, None, [(129, 0)], False),
+    (16, 16, 8, 1000, 0, None, [(1000, 0)], True),
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_key_waves_have_the_sums_of_the_two_wave_kernel(ltr, B, Hq, Hkv, Sq, q_pos, split, chunks, causal, dtype):
+    """Heads of 56 columns run in bwd_dkdv_pad_kernel<64> (two waves per 32 keys); the same heads with eight columns of zeros run here: the
+    same sums in the same order, bit for bit."""
+    lens, pos = [n for n, _ in chunks], [p for _, p in chunks]
+    kernel = lambda D: ltr.attn_plan(B, Hq, Hkv, D, Sq, lens, pos, q_pos, split, causal)["dkdv"]["kernel"]
+    assert (kernel(64), kernel(56)) == ("bwd_dkdv_keywave_kernel<64>", "bwd_dkdv_pad_kernel<64>")
+    total, at = sum(lens), [sum(lens[:i]) for i in range(len(lens))]
+    g = torch.Generator(device="cuda").manual_seed(Sq)
+    narrow = [torch.randn(B, s, h, 56, generator=g, device="cuda").to(torch.bfloat16) for s, h in ((Sq, Hq), (Sq, Hq), (total, Hkv), (total, Hkv))]
+    wide = [torch.nn.functional.pad(t, (0, 8)) for t in narrow]
+    cut = lambda t: [t[:, a:a + n] for a, n in zip(at, lens)]
+    o, lse = ltr.attn_fwd(wide[0], cut(wide[2]), cut(wide[3]), pos, q_pos, split, causal, scale=56 ** -0.5)
+    delta = ltr.attn_delta(o, wide[1])
+    qp = q_pos if isinstance(q_pos, tuple) else (q_pos, q_pos)
+    out = []
+    for q, do, k, v in (narrow, wide):
+        dk, dv = (torch.full(k.shape, 0.5, dtype=dtype, device="cuda") for _ in range(2))
+        a = L.BwdArgs()
+        a.q, a.d_o, a.lse, a.delta = q.data_ptr(), do.data_ptr(), lse.data_ptr(), delta.data_ptr()
+        a.B, a.Hq, a.Hkv, a.D, a.Sq, a.n_chunks = B, Hq, Hkv, q.shape[3], Sq, len(chunks)
+        a.q_pos0[:], a.q_split, a.scale, a.io_dtype = qp, Sq if split is None else split, 56 ** -0.5, L.LTR_BF16
+        a.flags = L.LTR_NO_DQ | L.LTR_HEAD_COLS | (L.LTR_CAUSAL if causal else 0) | (L.LTR_DKDV_BF16 if dtype == torch.bfloat16 else 0)
+        for name, t in (("q", q), ("do", do), ("k", k), ("v", v), ("dk", dk), ("dv", dv)):
+            getattr(a, name + "_stride")[:] = t.stride()[:3]
+        for i, (kc, vc, dkc, dvc) in enumerate(zip(cut(k), cut(v), cut(dk), cut(dv))):
+            c = a.chunk[i]
+            c.k, c.v, c.dk, c.dv, c.sk, c.pos0 = kc.data_ptr(), vc.data_ptr(), dkc.data_ptr(), dvc.data_ptr(), lens[i], pos[i]
+        L.check(L.load().ltr_attn_bwd(ctypes.byref(a), torch.cuda.current_stream().cuda_stream), "ltr_attn_bwd")
+        out.append((dk[..., :56], dv[..., :56]))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert out[0][0].float().abs().max() > 0.6
