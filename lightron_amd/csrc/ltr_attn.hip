@@ -1035,6 +1035,8 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
 //   16 x 12 heads D=64 S=1024   56 / 65 -> 43 / 58       7 x 32 heads D=64 S=2214  210 / 273 -> 185 / 251
 //   4 x 16 heads D=128 S=1024   35 / 46 -> 32 / 42      13 x 16 heads D=128 S=1800  241 / 317 -> 229 / 308
 //   4 x 32 heads D=128 S=8192 2046 / 2844 -> 2173 / 2925 (long blocks: the tile traffic shows)
+// Bound at head dim 64 by vector instructions: 13.6 / 10.2 per MFMA in the first of these launches, the vector pipe active 59 / 52 % and the
+// matrix pipe 30 / 36 % of a SIMD's time.
 template <int D>
 struct FourWaves {
     static constexpr int BN = 64, PER_CU = D == 64 ? 3 : 2;
@@ -1448,8 +1450,9 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
 // A wave's 32 keys of a step are two sub-tiles whose chains alternate.  Operand layout (lane l, i = l % 16, g = l / 16): A[i][g], B[g][i],
 // C[4g + r][i] for accumulator register r.  As in the 32-row kernels both contractions choose their order: step 4s + j of S^T contracts d = 16s + 4g + j (K: one 128-bit read for four steps), step r of O^T / dQ^T the keys 4g + r of a
 // sub-tile, whose P^T / dS^T is the accumulator register r as it is.  f32_swz serves both reads (rows 4 apart land 4 chunks apart).
-// Each wave ends up with 16 of the 64 columns of all shares and writes 16 bytes per lane.  Bound by the wave's chain of MFMAs
-// and its LDS reads (one block per CU).  Kernel us, 32 -> 16 rows, forward and dQ, 2 x 8 heads of 256 rows against 256, 768, 1024 keys:
+// Each wave ends up with 16 of the 64 columns of all shares and writes 16 bytes per lane.  Bound by latency, one wave per SIMD (one block per
+// CU): forward / dQ wait 35 / 43 % of the time for data and barriers, matrix pipe 29 / 33 % busy, vector 21 / 15, LDS 10 / 9 (a third of it bank
+// conflicts).  Kernel us, 32 -> 16 rows, forward and dQ, 2 x 8 heads of 256 rows against 256, 768, 1024 keys:
 // 10.8 -> 7.5, 22.0 -> 14.6, 27.7 -> 18.1 and 15.0 -> 9.4, 29.9 -> 18.7, 37.3 -> 23.3; one head of 8 rows and 64 keys 7.1 -> 5.0, 9.2 -> 6.2.
 struct F32Rows16 {
     static constexpr int D = 64, KS = 4, BM = 16;
@@ -2376,7 +2379,8 @@ __global__ __launch_bounds__(512) void bwd_dkdv_pad_kernel(const BwdParams p) {
 // handed over between waves, a block of four waves owns 128 keys in 51 KB of LDS, and two blocks share a CU: one's start, end and barriers run
 // under the other's matrix work, which is what bounds bwd_dkdv_kernel<64, 1> on short rows of blocks (16 x 12 heads, causal S=1024:
 // 115 us there, 97 here, 82 with the blocks longest first; 32 x 4 heads S=4096: 680 -> 579; the same sums in the same order, bit for
-// bit).  Bound: matrix and vector pipe taking turns, 1.06 PFLOP/s without a mask at S=4096.  Three blocks per CU would need 168 registers:
+// bit).  1.06 PFLOP/s without a mask at S=4096.  Bound by two waves per SIMD that fill neither pipe: vector active 40 %, matrix 31 % of a
+// SIMD's time at S=1024, a wave waits a third of its time for data and barriers and a third for issue.  Three blocks per CU would need 168 registers:
 // 21 and more spill, 83 -> 88 us.  Every (row, key) sub-tile of 32 x 32: S and dP in two alternating chains, P and dS in registers,
 // dV^T += dO^T P, dK^T += Q^T dS.
 template <int D>
