@@ -61,7 +61,8 @@ extern "C" {
 #define LTR_DKDV_KEYS_128 512u  /* backward, tuning hint: the dK/dV kernel's blocks own 128 keys (the default choice is the library's, as
                                    is that among the kernels with 128 keys) */
 #define LTR_DKDV_KEYS_256 1024u /* backward, tuning hint: they own 256 keys (bf16, head dim 64 only: LTR_EUNSUP otherwise); results
-                                   do not depend on the hint beyond the order of fp32 additions inside a block */
+                                   do not depend on the hint beyond the order of fp32 additions inside a block.  Tiles with a mask or a tail
+                                   are slow in it (registers spill): the library takes it for launches without any */
 #define LTR_DQ_ROWS_256 2048u /* backward, tuning hint: the dQ kernel's blocks own 256 query rows (the default choice is the library's) */
 #define LTR_DQ_ROWS_512 4096u /* backward, tuning hint: they own 512 rows (bf16, head dim 64 only: LTR_EUNSUP otherwise); same results */
 #define LTR_FWD_ROWS_256 8192u  /* forward, tuning hint: the kernel's blocks own 256 query rows (the default choice is the library's) */

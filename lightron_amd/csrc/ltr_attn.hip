@@ -4235,7 +4235,9 @@ RowChoice choose_rows(const RowCosts &costs, unsigned allowed, int D, bool causa
         // 8 x 32 heads, 1100 rows against 1000 + 400 keys 140 - 93, 16 x 16 heads S=1024 72 - 57), but the model makes them too short in one full
         // round of pairs, four of their blocks on a CU that runs three (4 x 16 heads S=2048 forward 50.0 - 52.7, modelled 0.98 of the pairs), and
         // for zig-zag shares with long blocks, where some CUs get one more of the late segment's than others (4 x 8 heads, 3612 rows of 7224
-        // 138 - 160, 0.91; 2 x 32 heads, 3618 of 28944 1043 - 1122, 0.98)
+        // 138 - 160, 0.91; 2 x 32 heads, 3618 of 28944 1043 - 1122, 0.98).  Padded heads have no four-wave form and take two shares for some
+        // zig-zag shares (heads of 40, forward / forward and backward: 4 x 128 heads S=820 of 1640 278 / 913 - 246 / 824, 8 x 24 heads 4028 of 8056
+        // 1082 / 4257 - 1104 / 4239, 8 x 64 heads 3934 of 15736 5508 / 22407 - 5551 / 21818)
         const int n = (Sq + 255) / 256, slots = (n + 1) / 2;
         if (n > 1 && BH * slots % cus == 0 && q_tiles_uneven(Sq, 256, q_split, q_pos0, chunk, n_chunks)) {
             if (D == 128) return first;
