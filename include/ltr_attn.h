@@ -82,6 +82,10 @@ extern "C" {
                                     dQ kernel: LTR_DQ_BF16 | LTR_DELTA_FROM_O for fp32.  LTR_EUNSUP with bf16 or LTR_BWD_F32_SCALAR */
 
 /* error codes */
+#define LTR_BWD_JOINT 524288u /* backward: dQ and dK/dV blocks may run side by side in one launch, where the library finds that faster (bf16; DELTA then
+                                  comes from a launch of its own before it); no output may overlap an input.  Without the flag the dQ kernel has
+                                  ended before the dK/dV kernel starts */
+
 #define LTR_OK 0
 #define LTR_EINVAL (-1)   /* null pointer, bad size, bad flag */
 #define LTR_EUNSUP (-2)   /* unsupported head dim / dtype combination */
@@ -212,7 +216,7 @@ typedef struct ltr_attn_bwd_args {
     float scale;
     uint32_t flags;       /* LTR_CAUSAL | LTR_NO_DQ | LTR_NO_DKDV | LTR_DQ_BF16 | LTR_DELTA_FROM_O | LTR_DKDV_BF16 | LTR_ROPE_DQ |
                              LTR_DKDV_KEYS_128 | LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR |
-                             LTR_HEAD_COLS | LTR_DQ_F32_RESULT */
+                             LTR_HEAD_COLS | LTR_DQ_F32_RESULT | LTR_BWD_JOINT */
     int32_t io_dtype;     /* LTR_BF16 or LTR_F32, of q/k/v/dO (LTR_F32: fp32 kernels on v_mfma_f32_32x32x2_f32 for the 1e-4 cases;
                              LTR_DQ_BF16, LTR_DELTA_FROM_O and LTR_DKDV_BF16 are bf16 only and return LTR_EUNSUP with it) */
     int32_t n_chunks;
@@ -317,7 +321,7 @@ int ltr_copy_strided(const ltr_copy_args *args, void *stream);
  * behind F.scaled_dot_product_attention, model/model.py:193); it is for benchmarks and profiles that must name the kernel
  * they measured, and for tests of the size hints.  The sizes, strides' owner shapes, positions, chunk lengths, dtype and
  * flags of args are read; flags may also carry the forward's hints (LTR_FWD_ROWS_256 / LTR_FWD_ROWS_512 / LTR_FWD_F32_SCALAR) and
- * LTR_HEAD_COLS.  The library's launches and this answer come from one function, so they cannot drift apart (a forward that
+ * LTR_HEAD_COLS.  With LTR_BWD_JOINT dq_kernel and dkdv_kernel are the same name where one launch holds the blocks of both.  The library's launches and this answer come from one function, so they cannot drift apart (a forward that
  * rotates q in place, see q_rot, takes one wave per row group where the plan may name key shares).  Kernel names are those a
  * profiler shows.  ltr_attn_plan_ws is the plan of ltr_attn_fwd and of ltr_attn_bwd_ws with a workspace of workspace_bytes: dkdv_blocks
  * then counts the blocks that share key tiles, and the kernel that sums their partial results is named beside them.

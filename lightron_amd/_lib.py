@@ -21,6 +21,7 @@ LTR_FWD_F32_SCALAR = 32768
 LTR_BWD_F32_SCALAR = 65536
 LTR_HEAD_COLS = 131072
 LTR_DQ_F32_RESULT = 262144
+LTR_BWD_JOINT = 524288
 
 EXPORTS = ("ltr_attn_fwd", "ltr_attn_bwd_delta", "ltr_attn_bwd", "ltr_attn_bwd_ws", "ltr_attn_bwd_workspace", "ltr_attn_bwd_noalloc", "ltr_attn_plan", "ltr_attn_plan_ws", "ltr_cast_f32_to_bf16",
            "ltr_rope_apply", "ltr_copy_strided", "ltr_abi_version", "ltr_strerror")

@@ -210,7 +210,7 @@ def _partials(lib, ref, device):
 
 def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_accs, q_pos0=0, q_split=None,
                         causal=False, scale=None, do_dq=True, do_dkdv=True, o=None, library_scratch=False, dq_rope=None,
-                        dkdv_keys=None, dq_rows=None, f32_scalar=False, share_keys=False):
+                        dkdv_keys=None, dq_rows=None, f32_scalar=False, share_keys=False, joint=False):
     """Adds this Q chunk's contribution into the fp32 accumulators dq_acc / dk_accs / dv_accs.
     do_dq / do_dkdv select which of the two backward kernels are enqueued.  dq_acc may instead be a bf16
     tensor: it then RECEIVES dQ (LTR_DQ_BF16), which is only right when ks / vs hold every KV chunk these
@@ -228,7 +228,8 @@ def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_a
     dq_rows: None, 256 or 512 query rows per block of the dQ kernel (512: bf16 with head dim 64 only).
     f32_scalar: fp32 inputs only - the scalar fp32 kernels instead of the matrix-pipe ones (LTR_BWD_F32_SCALAR).
     share_keys: launches with few key tiles may let several dK/dV blocks share a tile and sum their partials from a workspace
-    allocated here (ltr_attn_bwd_ws); dK / dV then differ from the unshared ones in the order of fp32 additions."""
+    allocated here (ltr_attn_bwd_ws); dK / dV then differ from the unshared ones in the order of fp32 additions.
+    joint: dQ and dK/dV blocks may run side by side in one launch (LTR_BWD_JOINT); no output may then overlap an input."""
     lib = _lib.load()
     if library_scratch and (o is None or not do_dq):
         raise RuntimeError("library_scratch needs o (DELTA is computed from it) and do_dq")
@@ -270,7 +271,8 @@ def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_a
     a.scale = float(scale if scale is not None else 1.0 / math.sqrt(D))
     a.flags = ((_lib.LTR_CAUSAL if causal else 0) | (0 if do_dq else _lib.LTR_NO_DQ)
                | (0 if do_dkdv else _lib.LTR_NO_DKDV) | (_lib.LTR_DQ_BF16 if dq_direct else 0)
-               | (_lib.LTR_DKDV_BF16 if dkdv_direct else 0) | (_lib.LTR_BWD_F32_SCALAR if f32_scalar else 0))
+               | (_lib.LTR_DKDV_BF16 if dkdv_direct else 0) | (_lib.LTR_BWD_F32_SCALAR if f32_scalar else 0)
+               | (_lib.LTR_BWD_JOINT if joint else 0))
     a.io_dtype = _DT[q.dtype]
     if dkdv_keys is not None:
         if dkdv_keys not in (128, 256):
@@ -316,12 +318,13 @@ def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_a
 
 def attn_plan(B: int, Hq: int, Hkv: int, D: int, Sq: int, chunk_lens: Sequence[int], k_pos0: Sequence[int], q_pos0=0,
               q_split: Optional[int] = None, causal: bool = False, dtype: torch.dtype = torch.bfloat16, fwd_rows=None,
-              dq_rows=None, dkdv_keys=None, f32_scalar: bool = False, share_keys: bool = False) -> dict:
+              dq_rows=None, dkdv_keys=None, f32_scalar: bool = False, share_keys: bool = False, joint: bool = False) -> dict:
     """Which kernels the library would launch for this problem on the current device (ltr_attn_plan: a host call, no
     tensors needed; at most 32 chunks = one launch): block sizes, block counts and the kernels' names as a profiler
     shows them.  fwd_rows / dq_rows / dkdv_keys force a size like the arguments of attn_fwd / attn_bwd_accumulate.
     share_keys: the backward gets the workspace it asks for, as in block_attention's backward: "dkdv" then also names the
-    blocks that share a key tile and, where any do, the kernel that sums their partial dK / dV."""
+    blocks that share a key tile and, where any do, the kernel that sums their partial dK / dV.
+    joint: with LTR_BWD_JOINT, as there; "dq" and "dkdv" name the same kernel where one launch holds the blocks of both."""
     lib = _lib.load()
     a = _lib.BwdArgs()
     a.B, a.Hq, a.Hkv, a.D, a.Sq, a.n_chunks = B, Hq, Hkv, D, Sq, len(chunk_lens)
@@ -330,6 +333,8 @@ def attn_plan(B: int, Hq: int, Hkv: int, D: int, Sq: int, chunk_lens: Sequence[i
     a.flags = (_lib.LTR_CAUSAL if causal else 0) | ((_lib.LTR_FWD_F32_SCALAR | _lib.LTR_BWD_F32_SCALAR) if f32_scalar else 0)
     if D not in (64, 128) and dtype == torch.bfloat16:
         a.flags |= _lib.LTR_HEAD_COLS
+    if joint:   # of a backward that writes bf16 results
+        a.flags |= _lib.LTR_BWD_JOINT | ((_lib.LTR_DELTA_FROM_O | _lib.LTR_DQ_BF16 | _lib.LTR_DKDV_BF16) if dtype == torch.bfloat16 else 0)
     for val, lo, hi, name in ((fwd_rows, _lib.LTR_FWD_ROWS_256, _lib.LTR_FWD_ROWS_512, "fwd_rows"),
                               (dq_rows, _lib.LTR_DQ_ROWS_256, _lib.LTR_DQ_ROWS_512, "dq_rows"),
                               (dkdv_keys, _lib.LTR_DKDV_KEYS_128, _lib.LTR_DKDV_KEYS_256, "dkdv_keys")):
@@ -420,7 +425,7 @@ class BlockAttentionFunction(torch.autograd.Function):
             # accumulators and cast once at the end, instead of one bf16 rounding per node: nothing flows to k, v here
             dk_accs, dv_accs = ctx.kv_grad_acc
             attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_accs, q_pos0, q_split, causal,
-                                scale, o=o if fuse else None, dq_rope=ctx.q_rope, share_keys=True)
+                                scale, o=o if fuse else None, dq_rope=ctx.q_rope, share_keys=True, joint=True)
             dq = dq_acc if (direct or f32) else cast_to_bf16(dq_acc)
             return (dq, None, None, None, None, None, None, None, None, None, None) + (None,) * (2 * n_chunks)
         lens = [k.shape[1] for k in ks]
@@ -435,7 +440,7 @@ class BlockAttentionFunction(torch.autograd.Function):
         dk_accs = [dk_buf[:, o_:o_ + n_] for o_, n_ in zip(offs, lens)]
         dv_accs = [dv_buf[:, o_:o_ + n_] for o_, n_ in zip(offs, lens)]
         attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_accs, q_pos0, q_split, causal, scale,
-                            o=o if fuse else None, dq_rope=ctx.q_rope, share_keys=True)
+                            o=o if fuse else None, dq_rope=ctx.q_rope, share_keys=True, joint=True)
         dq = dq_acc if (direct or f32) else cast_to_bf16(dq_acc)
         dk16, dv16 = dk_buf, dv_buf
         dks = [dk16[:, o_:o_ + n_] for o_, n_ in zip(offs, lens)]
@@ -547,7 +552,7 @@ class SingleChunkAttentionFunction(torch.autograd.Function):
             a.n_chunks = 1
             # one call holds every key these rows see and every row that sees these keys: the kernels write bf16 results
             a.flags = ((_lib.LTR_CAUSAL if causal else 0) | _lib.LTR_DQ_BF16 | _lib.LTR_DKDV_BF16 | _lib.LTR_DELTA_FROM_O
-                       | (_lib.LTR_ROPE_DQ if q_rope is not None else 0))
+                       | (_lib.LTR_ROPE_DQ if q_rope is not None else 0) | _lib.LTR_BWD_JOINT)
             ch = a.chunk[0]
             ch.sk, ch.pos0 = k.shape[1], int(k_pos0)
             if q_rope is not None:

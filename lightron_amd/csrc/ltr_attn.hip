@@ -122,6 +122,7 @@ struct BwdParams {
     void *dq;          // fp32 accumulator, or bf16 result with LTR_DQ_BF16
     int B, Hq, Hkv, n_rep;
     BlockMap q_map, kv_map;   // of the dQ and the dK/dV kernel
+    JointMap joint;    // of bwd_joint_kernel, which holds the blocks of both
     int cols;          // head dim of the tensors (the kernel's own width, or less: PAD kernels)
     int Sq, n_qtiles;
     long long qs[3], dos[3], dqs[3], ks[3], vs[3], dks[3], dvs[3];
@@ -1927,7 +1928,7 @@ __device__ __forceinline__ void write_key_rows(unsigned char *stage, int lane, c
 }
 
 template <int D, int KW, bool PAD>
-__device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
+__device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockItem item) {
     const int cols = PAD ? p.cols : D;
     using L = BwdLds<D, KW>;   // KW = 32-key halves per wave
     constexpr int BN = L::BN, BM = L::BM;
@@ -1945,24 +1946,6 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
 
     // block -> (batch, kv head, chunk, key tile); same XCD grouping as the forward.  Blocks that share a key tile follow each
     // other: each takes n_reps of the q heads and, of a head's visible q tiles, every 2^share_log2-th
-    BlockItem item;
-    const int P = p.B * p.Hkv;
-    if constexpr (KW == 1) {
-        item = block_item(p.kv_map, P);
-        if (item.pair >= P) return;
-    } else {   // pair after pair on a linear grid: this kernel runs without a mask, and has no scalar registers left for a map (6 % slower)
-        int idx = blockIdx.x, rest;
-        if ((P & 7) == 0) {
-            const int n = p.tiles_seen << p.split_log2;
-            item.pair = (idx >> 3) / n * 8 + (idx & 7);
-            rest = (idx >> 3) % n;
-        } else {
-            item.pair = idx % P;
-            rest = idx / P;
-        }
-        item.sub = rest & ((1 << p.split_log2) - 1);
-        item.item = rest >> p.split_log2;
-    }
     const int pair = item.pair, split = item.sub, tile = item.item;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
     int c = 0, kt = tile;
@@ -2368,11 +2351,30 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p) {
 
 template <int D, int KW>
 __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
-    bwd_dkdv_body<D, KW, false>(p);
+    const int P = p.B * p.Hkv;
+    BlockItem item;
+    if constexpr (KW == 1) {
+        item = block_item(p.kv_map, P);
+        if (item.pair >= P) return;
+    } else {   // pair after pair on a linear grid: this kernel runs without a mask, and has no scalar registers left for a map (6 % slower)
+        int idx = blockIdx.x, rest;
+        if ((P & 7) == 0) {
+            const int n = p.tiles_seen << p.split_log2;
+            item.pair = (idx >> 3) / n * 8 + (idx & 7);
+            rest = (idx >> 3) % n;
+        } else {
+            item.pair = idx % P;
+            rest = idx / P;
+        }
+        item.sub = rest & ((1 << p.split_log2) - 1);
+        item.item = rest >> p.split_log2;
+    }
+    bwd_dkdv_body<D, KW, false>(p, item);
 }
 template <int D>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_dkdv_pad_kernel(const BwdParams p) {
-    bwd_dkdv_body<D, 1, true>(p);
+    const BlockItem item = block_item(p.kv_map, p.B * p.Hkv);
+    if (item.pair < p.B * p.Hkv) bwd_dkdv_body<D, 1, true>(p, item);
 }
 
 // dK/dV at head dim 64, one wave per 32-key slice: K and V operands (32 registers) and both accumulators (64) fit one wave, so nothing is
@@ -2395,7 +2397,7 @@ struct KeyWaveLds {
     static_assert(2 * TOTAL <= 160 * 1024, "two blocks per CU");
 };
 template <int D>
-__global__ __launch_bounds__(256, 2) void bwd_dkdv_keywave_kernel(const BwdParams p) {
+__device__ __forceinline__ void bwd_dkdv_keywave_body(const BwdParams &p, const BlockItem item) {
     using L = KeyWaveLds<D>;
     constexpr int BN = L::BN, BM = L::BM;
     constexpr int CPR = D / 8;
@@ -2407,7 +2409,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_keywave_kernel(const BwdParam
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool causal = p.flags & LTR_CAUSAL;
     // block -> (batch, kv head, chunk, key tile), shares of a key tile: as in bwd_dkdv_body
-    const BlockItem item = block_item(p.kv_map, p.B * p.Hkv);
     const int pair = item.pair, split = item.sub, tile = item.item;
     if (pair >= p.B * p.Hkv) return;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
@@ -2655,6 +2656,10 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_keywave_kernel(const BwdParam
     write_key_rows<D, false>(stage, lane, dvacc, 1.f, as_bf16, p.chunk[c].dv, b * p.dvs[0] + hkv * p.dvs[2], p.dvs[1], key0 + 32 * w, sk, D);
     write_key_rows<D, false>(stage, lane, dkacc, p.scale, as_bf16, p.chunk[c].dk, b * p.dks[0] + hkv * p.dks[2], p.dks[1], key0 + 32 * w, sk, D);
 }
+template <int D>
+__global__ __launch_bounds__(256, 2) void bwd_dkdv_keywave_kernel(const BwdParams p) {
+    bwd_dkdv_keywave_body<D>(p, block_item(p.kv_map, p.B * p.Hkv));
+}
 
 // Sum of the partial dK / dV that the blocks sharing a key tile left in p.part (bf16 and fp32 kernels alike), in the order of
 // the shares: results do not depend on which block finished first.  A wave takes 64 columns of one 32-key slice of dK or dV
@@ -2791,7 +2796,7 @@ __device__ __forceinline__ void lds_tr_gemm_at_rb(const unsigned (&addr)[D / 32]
 
 // RB = 32-row blocks per wave: a lane owns RB query rows, a block 256 * RB / KS; KS = key shares per row group as in the forward
 template <int D, int RB, int KS, bool PAD, int NW = 8, int BN = FwdTile<D, 1, KS>::BN>
-__device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
+__device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem item) {
     const int cols = PAD ? p.cols : D;
     constexpr int RG = NW / KS, BM = 32 * RB * RG;   // the NW waves of the block share every K / V tile
     constexpr int BNT = BN * KS;                     // BN keys per wave, BNT per tile
@@ -2807,7 +2812,6 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
     const int rg = w / KS, ks = w % KS;      // row group and key share of the wave
     const bool causal = p.flags & LTR_CAUSAL;
 
-    const BlockItem item = block_item(p.q_map, p.B * p.Hkv);
     const int pair = item.pair, rep = item.sub, slot = item.item;
     if (pair >= p.B * p.Hkv) return;
     const int n_qt = (p.Sq + BM - 1) / BM;
@@ -3107,19 +3111,42 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p) {
 
 template <int D>   // see FourWaves
 __global__ __launch_bounds__(256, FourWaves<D>::PER_CU) void bwd_dq_w4_kernel(const BwdParams p) {
-    bwd_dq_body<D, 1, 1, false, 4, FourWaves<D>::BN>(p);
+    bwd_dq_body<D, 1, 1, false, 4, FourWaves<D>::BN>(p, block_item(p.q_map, p.B * p.Hkv));
 }
 template <int D, int RB>
 __global__ __launch_bounds__(512) void bwd_dq_kernel(const BwdParams p) {
-    bwd_dq_body<D, RB, 1, false>(p);
+    bwd_dq_body<D, RB, 1, false>(p, block_item(p.q_map, p.B * p.Hkv));
 }
 template <int D, int KS>
 __global__ __launch_bounds__(512) void bwd_dq_shares_kernel(const BwdParams p) {
-    bwd_dq_body<D, 1, KS, false>(p);
+    bwd_dq_body<D, 1, KS, false>(p, block_item(p.q_map, p.B * p.Hkv));
 }
 template <int D, int KS>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_dq_pad_kernel(const BwdParams p) {
-    bwd_dq_body<D, 1, KS, true>(p);
+    bwd_dq_body<D, 1, KS, true>(p, block_item(p.q_map, p.B * p.Hkv));
+}
+
+// dQ and dK/dV blocks in one launch (LTR_BWD_JOINT).  Given DELTA, neither kind needs anything of the other; in launches of their own each ends with
+// CUs idle and the next begins with all of them waiting for their first tiles, which is what a pass of few blocks spends its time on.  DELTA
+// comes from delta_kernel then.  Taken where the modelled time is shorter (joint_launch).  us of the backward, apart -> joint:
+//   4 x 12 heads D=64 S=128   17.2 -> 12.0       2 x 16 heads D=96 S=777   57.8 -> 42.5       1 x 32 heads on 8 D=128 S=1237   94.8 -> 78
+//   1 x 16 heads D=128 S=4096  257 -> 242        1 x 12 heads D=128 S=3418  181 -> 145        3 x 8 heads D=128 S=926   61 -> 42
+// Registers are those of the dK/dV kernel, LDS the larger of both: one block per CU, as for either kind alone.
+template <int D, int KS, bool PAD>
+__device__ __forceinline__ void bwd_joint_body(const BwdParams &p) {
+    const int P = p.B * p.Hkv;
+    const JointItem j = joint_item_at(p.joint, p.q_map, p.kv_map, P, blockIdx.x);
+    if (j.item.pair >= P) return;
+    if (j.keys) bwd_dkdv_body<D, 1, PAD>(p, j.item);
+    else bwd_dq_body<D, 1, KS, PAD>(p, j.item);
+}
+template <int D, int KS>
+__global__ __launch_bounds__(512) void bwd_joint_kernel(const BwdParams p) {
+    bwd_joint_body<D, KS, false>(p);
+}
+template <int D, int KS>   // head dims below D
+__global__ __launch_bounds__(512) void bwd_joint_pad_kernel(const BwdParams p) {
+    bwd_joint_body<D, KS, true>(p);
 }
 
 // ------------------------------------------------------------------------------ backward, fp32
@@ -3937,6 +3964,12 @@ constexpr int shares_lds_bytes() {   // forward and dQ kernels with key shares: 
 static_assert(shares_lds_bytes<128, 2>() <= 160 * 1024 && shares_lds_bytes<128, 4>() <= 160 * 1024 && shares_lds_bytes<64, 4>() <= 160 * 1024, "LDS of one CU");
 static_assert(8 * WaveStage<64>::BYTES <= shares_lds_bytes<128, 2>() && 8 * WaveStage<32>::BYTES <= shares_lds_bytes<64, 2>(), "staging areas");
 
+template <int D, int KS>
+constexpr int joint_lds_bytes() {
+    constexpr int dq = KS == 1 ? dq_lds_bytes<D>() : shares_lds_bytes<D, KS>();
+    return dq > BwdLds<D, 1>::TOTAL ? dq : BwdLds<D, 1>::TOTAL;
+}
+
 int enable_large_lds() {
     int dev = 0;
     if (current_device(&dev)) return LTR_EDEVICE;
@@ -3992,6 +4025,14 @@ int enable_large_lds() {
         {(const void *)bwd_dq_shares_kernel<128, 4>, shares_lds_bytes<128, 4>()},
         {(const void *)bwd_dq_shares_kernel<64, 2>, shares_lds_bytes<64, 2>()},
         {(const void *)bwd_dq_shares_kernel<64, 4>, shares_lds_bytes<64, 4>()},
+        {(const void *)bwd_joint_kernel<64, 1>, joint_lds_bytes<64, 1>()},
+        {(const void *)bwd_joint_kernel<64, 2>, joint_lds_bytes<64, 2>()},
+        {(const void *)bwd_joint_pad_kernel<64, 1>, joint_lds_bytes<64, 1>()},
+        {(const void *)bwd_joint_pad_kernel<64, 2>, joint_lds_bytes<64, 2>()},
+        {(const void *)bwd_joint_kernel<128, 1>, joint_lds_bytes<128, 1>()},
+        {(const void *)bwd_joint_kernel<128, 2>, joint_lds_bytes<128, 2>()},
+        {(const void *)bwd_joint_pad_kernel<128, 1>, joint_lds_bytes<128, 1>()},
+        {(const void *)bwd_joint_pad_kernel<128, 2>, joint_lds_bytes<128, 2>()},
     };
     bool ok = true;
     for (const auto &k : large) ok = ok && hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, k.bytes) == hipSuccess;
@@ -4351,23 +4392,31 @@ int f32_rows(int D, long long pairs, int Sq, int cus, int &ks) {
     return ks == F32Rows16::KS && blocks(F32Rows16::BM) <= cus ? F32Rows16::BM : 128 / ks;
 }
 // The kernels of these choices, for the launches and for the plans: a plan's name is that of the kernel a launch takes.
-struct F32Kernel {
+struct KernelChoice {
     const void *fn;
     const char *name;
     int lds;
 };
 #define LTR_KERNEL(...) (const void *)__VA_ARGS__, #__VA_ARGS__
-F32Kernel f32_fwd_kernel(int D, int ks, int rows) {
-    if (D == 128) return ks == 1 ? F32Kernel{LTR_KERNEL(fwd_f32_mfma_kernel<128, 1>), F32Mfma<128, 1>::LDS} : F32Kernel{LTR_KERNEL(fwd_f32_mfma_kernel<128, 2>), F32Mfma<128, 2>::LDS};
+KernelChoice f32_fwd_kernel(int D, int ks, int rows) {
+    if (D == 128) return ks == 1 ? KernelChoice{LTR_KERNEL(fwd_f32_mfma_kernel<128, 1>), F32Mfma<128, 1>::LDS} : KernelChoice{LTR_KERNEL(fwd_f32_mfma_kernel<128, 2>), F32Mfma<128, 2>::LDS};
     if (ks == 1) return {LTR_KERNEL(fwd_f32_mfma_kernel<64, 1>), F32Mfma<64, 1>::LDS};
     if (ks == 2) return {LTR_KERNEL(fwd_f32_mfma_kernel<64, 2>), F32Mfma<64, 2>::LDS};
-    return rows == F32Rows16::BM ? F32Kernel{LTR_KERNEL(fwd_f32_mfma_kernel<64, 4>), F32Mfma<64, 4>::LDS} : F32Kernel{LTR_KERNEL(fwd_f32_rows32_kernel<64, 4>), F32Mfma<64, 4>::LDS};
+    return rows == F32Rows16::BM ? KernelChoice{LTR_KERNEL(fwd_f32_mfma_kernel<64, 4>), F32Mfma<64, 4>::LDS} : KernelChoice{LTR_KERNEL(fwd_f32_rows32_kernel<64, 4>), F32Mfma<64, 4>::LDS};
 }
-F32Kernel f32_dq_kernel(int D, int ks, int rows) {
-    if (D == 128) return ks == 1 ? F32Kernel{LTR_KERNEL(bwd_dq_f32_mfma_kernel<128, 1>), F32Mfma<128, 1>::LDS} : F32Kernel{LTR_KERNEL(bwd_dq_f32_mfma_kernel<128, 2>), F32Mfma<128, 2>::LDS};
+KernelChoice f32_dq_kernel(int D, int ks, int rows) {
+    if (D == 128) return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_dq_f32_mfma_kernel<128, 1>), F32Mfma<128, 1>::LDS} : KernelChoice{LTR_KERNEL(bwd_dq_f32_mfma_kernel<128, 2>), F32Mfma<128, 2>::LDS};
     if (ks == 1) return {LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 1>), F32Mfma<64, 1>::LDS};
     if (ks == 2) return {LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 2>), F32Mfma<64, 2>::LDS};
-    return rows == F32Rows16::BM ? F32Kernel{LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 4>), F32Mfma<64, 4>::LDS} : F32Kernel{LTR_KERNEL(bwd_dq_f32_rows32_kernel<64, 4>), F32Mfma<64, 4>::LDS};
+    return rows == F32Rows16::BM ? KernelChoice{LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 4>), F32Mfma<64, 4>::LDS} : KernelChoice{LTR_KERNEL(bwd_dq_f32_rows32_kernel<64, 4>), F32Mfma<64, 4>::LDS};
+}
+KernelChoice joint_kernel(int D, bool pad, int ks) {
+    if (pad) {
+        if (D == 128) return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<128, 1>), joint_lds_bytes<128, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<128, 2>), joint_lds_bytes<128, 2>()};
+        return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<64, 1>), joint_lds_bytes<64, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<64, 2>), joint_lds_bytes<64, 2>()};
+    }
+    if (D == 128) return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_kernel<128, 1>), joint_lds_bytes<128, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_kernel<128, 2>), joint_lds_bytes<128, 2>()};
+    return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_kernel<64, 1>), joint_lds_bytes<64, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_kernel<64, 2>), joint_lds_bytes<64, 2>()};
 }
 #undef LTR_KERNEL
 
@@ -4490,7 +4539,171 @@ struct BwdPlan {
     int dq_rows, dq_qtiles, dq_slots;
     int dq_group, kv_group;   // see pair_group
     long long dq_blocks;
+    bool joint, keys_first;   // one launch for both kinds of blocks (bwd_joint_kernel), and which of them go first
 };
+// Does a bf16 backward run its dQ and dK/dV blocks in one launch, with how many key shares per row group and blocks per key tile, and which kind
+// first?  Both ways are priced by launch_us over classes of blocks (up to 8 evenly spaced tiles stand for all): the plan as it is, one launch after
+// the other, and every joint one.  Constants fitted to 21000 launches of 2200 random problems (calls, ring and zig-zag ranks, single ring steps;
+// 4 - 32 heads, 45 - 5800 rows; rms error 9 - 12 %).  Of 5600 other launches that were joined, the backward takes 1 / 1.31 of the time, geometric
+// mean: 1.48 times faster where it took up to 25 us, 1.37 up to 50, 1.24 up to 100, 1.10 past 200.
+struct JointCost {
+    double q_step_us[2], q_fixed_us[2];   // dQ blocks of one and two key shares: per K / V tile and per block
+    double shares4_step_us, shares4_fixed_us;
+    double kv_step_us, kv_fixed_us;       // dK/dV blocks: per 64 q rows of a head and per block
+    double q_acc_us, kv_acc_us;           // more per block where the results are added to fp32 accumulators
+    double launch_us, delta_us, delta_bytes_per_us, reduce_us, reduce_bytes_per_us;
+};
+constexpr JointCost JOINT_128{{2.13, 2.56}, {8.1, 8.5}, 1.33, 8.5, 1.68, 8.9, 2.8, 2.4, 1.4, 2.0, 3.3e6, 5.2, 18e6},
+    JOINT_64{{2.90, 1.35}, {4.6, 5.7}, 1.33, 6.5, 0.99, 5.8, 1.0, 2.3, 3.3, 1.8, 2.7e6, 4.6, 23e6};
+constexpr KvSplitCost KEY_WAVES_64{64, 1.43, 6.7, 0.82, 3.4, 1.35, 3.5, 19e6};
+void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
+                  int n_chunks, bool may_split, int cus) {
+    constexpr int CLASSES = 8;
+    const JointCost &cost = D == 128 ? JOINT_128 : JOINT_64;
+    const bool causal = (flags & LTR_CAUSAL) != 0;
+    const long long pairs = (long long)B * Hkv, q_pairs = (long long)B * Hq;
+    // key tiles by position, as the launch sorts them
+    int order[LTR_MAX_CHUNKS];
+    for (int i = 0; i < n_chunks; i++) {
+        int k = i;
+        for (; causal && k > 0 && chunk[order[k - 1]].pos0 > chunk[i].pos0; k--) order[k] = order[k - 1];
+        order[k] = i;
+    }
+    const int q_last = !causal ? 0x7fffffff
+                               : std::max(q_split > 0 ? q_pos0[0] + q_split - 1 : (int)0x80000000, Sq > q_split ? q_pos0[1] + (Sq - q_split) - 1 : (int)0x80000000);
+    long long tiles_seen = 0;
+    for (int i = 0; i < n_chunks; i++) tiles_seen += seen_tiles(chunk[i].sk, chunk[i].pos0, q_last, 128);
+    // few blocks only: past some hundred rounds nothing is left to gain
+    if (tiles_seen == 0 || pl.kv_tiles > GRID_YZ_MAX || pairs > 8LL * GRID_YZ_MAX || pl.dq_blocks + pl.kv_blocks > 1 << 18) return;
+    struct List {
+        BlockClass c[CLASSES];
+        int k;
+        long long n;
+        double total_us() const {
+            double t = 0;
+            for (int i = 0; i < k; i++) t += c[i].us * c[i].n;
+            return t;
+        }
+    };
+    auto dq_blocks = [&](int rows, int key_log2, double step_us, double fixed_us, bool paired) {
+        List l;
+        const int n = (Sq + rows - 1) / rows, slots = paired ? (n + 1) / 2 : n;
+        auto us = [&](int t) {   // 1: a block that sees nothing
+            long long tiles = 0;
+            const int r0 = t * rows, r1 = std::min(Sq, r0 + rows) - 1;
+            int hi = r1 < q_split ? q_pos0[0] + r1 : q_pos0[1] + (r1 - q_split);
+            if (r0 < q_split && r1 >= q_split) hi = std::max(hi, q_pos0[0] + q_split - 1);
+            for (int c = 0; c < n_chunks; c++) {
+                const long long seen = causal ? std::min<long long>(std::max<long long>((long long)hi - chunk[c].pos0 + 1, 0), chunk[c].sk) : chunk[c].sk;
+                tiles += (seen + (1 << key_log2) - 1) >> key_log2;
+            }
+            return tiles ? tiles * step_us + fixed_us + (flags & LTR_DQ_BF16 ? 0 : cost.q_acc_us) : 1.0;
+        };
+        l.n = q_pairs * slots;
+        l.k = causal ? std::min(slots, CLASSES) : 1;
+        for (int j = 0; j < l.k; j++) {
+            const int slot = l.k > 1 ? (int)((long long)j * (slots - 1) / (l.k - 1)) : 0, late = n - 1 - slot;
+            l.c[j] = {us(late) + (paired && slot < late ? us(slot) : 0), l.n * (j + 1) / l.k - l.n * j / l.k};
+        }
+        return l;
+    };
+    auto kv_blocks = [&](int n_split, double step_us, double fixed_us) {
+        List l;
+        const long long n = n_split > 1 ? tiles_seen : pl.kv_tiles;
+        l.n = pairs * n * n_split;
+        l.k = causal ? (int)std::min<long long>(n, CLASSES) : 1;
+        for (int j = 0; j < l.k; j++) {
+            long long t = l.k > 1 ? j * (n - 1) / (l.k - 1) : 0;
+            int i = 0;
+            for (; i < n_chunks - 1; i++) {
+                const int in_chunk = seen_tiles(chunk[order[i]].sk, chunk[order[i]].pos0, n_split > 1 ? q_last : 0x7fffffff, 128);
+                if (t < in_chunk) break;
+                t -= in_chunk;
+            }
+            long long rows = Sq;
+            const long long kpos = chunk[order[i]].pos0 + t * 128;
+            if (causal)
+                rows = std::min<long long>(std::max<long long>(q_pos0[0] + (long long)q_split - kpos, 0), q_split) +
+                       std::min<long long>(std::max<long long>(q_pos0[1] + (long long)(Sq - q_split) - kpos, 0), Sq - q_split);
+            const long long steps = ((rows + 63) / 64 * (Hq / Hkv) + n_split - 1) / n_split;
+            l.c[j] = {rows > 0 ? steps * step_us + fixed_us + (n_split > 1 || (flags & LTR_DKDV_BF16) ? 0 : cost.kv_acc_us) : 1.0, l.n * (j + 1) / l.k - l.n * j / l.k};
+        }
+        return l;
+    };
+    auto both_us = [&](const List &first, const List &second) {
+        BlockClass c[2 * CLASSES];
+        std::copy(first.c, first.c + first.k, c);
+        std::copy(second.c, second.c + second.k, c + first.k);
+        return launch_us(c, first.k + second.k, cus);
+    };
+    auto reduce_us = [&](int n_split) { return n_split > 1 ? cost.reduce_us + (double)pl.kv_tiles * pairs * n_split * 128 * D * 8 / cost.reduce_bytes_per_us : 0.0; };
+
+    // the plan as it is
+    double apart = 2 * cost.launch_us + reduce_us(pl.split.n);
+    if (pl.dq_four_waves) {
+        const TileCost &c = (D == 128 ? DQ_ROWS_128 : DQ_ROWS_64).kernel[FOUR_WAVES];
+        const int per_cu = (int)std::min<long long>(D == 128 ? FourWaves<128>::PER_CU : FourWaves<64>::PER_CU, (pl.dq_blocks + cus - 1) / cus);
+        const List l = dq_blocks(128, 6, per_cu == 1 ? c.alone_us : per_cu * c.step_us, per_cu == 1 ? c.alone_fixed_us : per_cu * c.fixed_us, false);
+        apart += launch_us(l.c, l.k, per_cu * cus);
+    } else {
+        const int i = pl.dq_ks == 4 ? SHARES_4 : pl.dq_ks == 2 ? SHARES_2 : ROWS_256;
+        const RowKernel k = row_kernel(i, D);
+        const List l = dq_blocks(k.rows, k.key_log2, i == SHARES_4 ? cost.shares4_step_us : cost.q_step_us[i == SHARES_2], i == SHARES_4 ? cost.shares4_fixed_us : cost.q_fixed_us[i == SHARES_2],
+                                 pl.dq_slots != pl.dq_qtiles);
+        apart += launch_us(l.c, l.k, cus);
+    }
+    if (pl.key_waves) {
+        const int per_cu = pairs * pl.kv_tiles * pl.split.n > cus ? 2 : 1;
+        const List l = kv_blocks(pl.split.n, per_cu == 1 ? KEY_WAVES_64.alone_us : 2 * KEY_WAVES_64.step_us, per_cu == 1 ? KEY_WAVES_64.alone_fixed_us : 2 * KEY_WAVES_64.fixed_us);
+        apart += launch_us(l.c, l.k, per_cu * cus);
+    } else {
+        const List l = kv_blocks(pl.split.n, cost.kv_step_us, cost.kv_fixed_us);
+        apart += launch_us(l.c, l.k, cus);
+    }
+    // where the plan has several blocks on a CU the model takes it for slower than it is, most of all at head dim 64 with both kernels of that
+    // kind: of 5600 random launches joined at 0.96, 100 lost more than 1 %, 80 of them there; of 5400 with about these factors 50
+    double best = apart * (D == 128 ? pl.dq_four_waves ? 0.92 : 0.98
+                                    : pl.key_waves && pl.dq_four_waves ? 0.78 : pl.key_waves || pl.dq_four_waves || pl.dq_blocks + pl.kv_blocks > 8 * cus ? 0.88 : 0.96);
+    const double common = cost.launch_us + (flags & LTR_DELTA_FROM_O ? cost.delta_us + (double)q_pairs * Sq * D * 4 / cost.delta_bytes_per_us : 0.0);
+    int best_ks = 0, best_n = 1;
+    bool keys_first = false;
+    // dQ blocks of one and two shares; the blocks of both kinds are looked at in both orders, unless all run at once or even spread evenly over
+    // the CUs they take longer than the best so far
+    List q[2];
+    for (int ks = 1; ks <= 2; ks++) {
+        const RowKernel k = row_kernel(ks == 2 ? SHARES_2 : ROWS_256, D);
+        q[ks - 1] = dq_blocks(k.rows, k.key_log2, cost.q_step_us[ks - 1], cost.q_fixed_us[ks - 1], false);
+    }
+    for (int n = 1; n <= 16; n *= 2) {
+        if (n > 1 && (!may_split || pairs * tiles_seen * n > 5LL * cus || (double)pairs * tiles_seen * n * 128 * D * 8 > MAX_PART_BYTES)) break;
+        if (n > 1 && n > (long long)(Sq + 63) / 64 * (Hq / Hkv)) break;
+        const List kv = kv_blocks(n, cost.kv_step_us, cost.kv_fixed_us);
+        for (int ks = 1; ks <= 2; ks++) {
+            const double rest = common + reduce_us(n);
+            if (rest + (q[ks - 1].total_us() + kv.total_us()) / cus >= best) continue;
+            const bool one_round = q[ks - 1].n + kv.n <= cus;
+            for (int first = 0; first < (one_round ? 1 : 2); first++) {
+                const double us = rest + (first ? both_us(kv, q[ks - 1]) : both_us(q[ks - 1], kv));
+                if (us < best) {
+                    best = us;
+                    best_ks = ks;
+                    best_n = n;
+                    keys_first = first;
+                }
+            }
+        }
+    }
+    if (!best_ks) return;
+    pl.joint = true;
+    pl.keys_first = keys_first;
+    pl.key_waves = pl.dq_four_waves = false;
+    pl.dq_ks = best_ks;
+    pl.dq_rows = 256 / best_ks;
+    pl.dq_qtiles = pl.dq_slots = (Sq + pl.dq_rows - 1) / pl.dq_rows;
+    pl.dq_blocks = (long long)pl.dq_slots * B * Hq;
+    pl.split = {best_n, 1, best_n > 1 ? q_last : 0x7fffffff, best_n > 1 ? tiles_seen : pl.kv_tiles, 0};
+    while (pl.split.reps * 2 <= best_n && Hq / Hkv % (pl.split.reps * 2) == 0) pl.split.reps *= 2;
+}
 BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
                  int n_chunks, bool may_split = false) {
     BwdPlan pl;
@@ -4499,7 +4712,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.part_bytes = 0;
     pl.dq_ks = 1;
     pl.dq_group = pl.kv_group = 1;
-    pl.dq_four_waves = false;
+    pl.dq_four_waves = pl.joint = pl.keys_first = false;
     may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
     pl.key_waves = false;
     const int cus = device_cus();
@@ -4563,13 +4776,12 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     } else {
         // head dim 64: one wave per 32 keys (two blocks per CU) or two (one block).  A block alone on its CU is faster with eight
         // waves, a CU is faster with two blocks of four.  Constants fitted to 195 launches each (60 shapes, n = 1 .. 32; rms 7 %)
-        split_keys(KvSplitCost{64, 1.43, 6.7, 0.82, 3.4, 1.35, 3.5, 19e6});
+        split_keys(KEY_WAVES_64);
         const KvSplit one_wave = pl.split;
         split_keys(KvSplitCost{64, 1.14, 7.0, 1.01, 5.8, 0.6, 4.0, 17e6});
         pl.key_waves = one_wave.us < 0.96 * pl.split.us;
         if (pl.key_waves) pl.split = one_wave;
     }
-    size_parts();
     const RowChoice choice = flags & LTR_NO_DQ
                                  ? RowChoice{flags & LTR_DQ_ROWS_512 ? ROWS_512 : ROWS_256, false}
                                  : choose_rows(D == 128 ? DQ_ROWS_128 : DQ_ROWS_64,
@@ -4580,9 +4792,15 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.dq_ks = choice.kernel == SHARES_2 ? 2 : choice.kernel == SHARES_4 ? 4 : 1;
     pl.dq_rows = row_kernel(choice.kernel, D).rows;
     pl.dq_qtiles = (Sq + pl.dq_rows - 1) / pl.dq_rows;
-    const bool uneven = causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks);
+    bool uneven = causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks);
     pl.dq_slots = choice.paired ? (pl.dq_qtiles + 1) / 2 : pl.dq_ks > 1 || pl.dq_four_waves ? pl.dq_qtiles : q_tile_slots(pl.dq_qtiles, (long long)B * Hq, uneven, cus);
     pl.dq_blocks = (long long)pl.dq_slots * B * Hq;
+    constexpr unsigned NOT_JOINT = LTR_NO_DQ | LTR_NO_DKDV | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_DKDV_KEYS_128 | LTR_DKDV_KEYS_256;
+    if ((flags & LTR_BWD_JOINT) && !(flags & NOT_JOINT) && !pl.wide_q && !pl.wide_kv) {
+        joint_launch(pl, D, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split, cus);
+        if (pl.joint) uneven = causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks);
+    }
+    size_parts();
     const long long pairs = (long long)B * Hkv;
     const int slots = cus / 8;
     pl.dq_group = pair_group(pairs, (long long)pl.dq_slots * (Hq / Hkv), slots * (pl.dq_four_waves ? D == 64 ? FourWaves<64>::PER_CU : FourWaves<128>::PER_CU : 1),
@@ -4768,7 +4986,7 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
     if (pl.f32_ks) {   // fp32 on the matrix pipe; the chunk offsets of its LDS-direct loads are 64-bit, nothing more to check
         rc = enable_large_lds();
         if (rc) return rc;
-        const F32Kernel k = f32_fwd_kernel(a->D, pl.f32_ks, pl.rows);
+        const KernelChoice k = f32_fwd_kernel(a->D, pl.f32_ks, pl.rows);
         return launch(k.fn, pl.blocks, 256, k.lds, st, p);
     }
     if (a->D == 128) return launch((const void *)fwd_f32_kernel<128>, pl.blocks, 64, 0, st, p);
@@ -4818,7 +5036,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     if (a->B <= 0 || a->Hq <= 0 || a->Hkv <= 0 || a->Sq <= 0 || a->Hq % a->Hkv) return LTR_EINVAL;
     if (a->n_chunks < 1 || a->n_chunks > LTR_MAX_CHUNKS) return LTR_EINVAL;
     if (flags & ~(LTR_CAUSAL | LTR_NO_DQ | LTR_NO_DKDV | LTR_DQ_BF16 | LTR_DELTA_FROM_O | LTR_DKDV_BF16 | LTR_ROPE_DQ | LTR_DKDV_KEYS_128 |
-                  LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR | LTR_HEAD_COLS | LTR_DQ_F32_RESULT))
+                  LTR_DKDV_KEYS_256 | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_BWD_F32_SCALAR | LTR_HEAD_COLS | LTR_DQ_F32_RESULT | LTR_BWD_JOINT))
         return LTR_EINVAL;
     if ((flags & LTR_BWD_F32_SCALAR) && a->io_dtype != LTR_F32) return LTR_EUNSUP;
     if ((flags & LTR_DQ_F32_RESULT) && (a->io_dtype != LTR_F32 || (flags & LTR_BWD_F32_SCALAR))) return LTR_EUNSUP;
@@ -4932,7 +5150,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
         rc = enable_large_lds();
         if (rc) return rc;
         if (do_dq) {
-            const F32Kernel k = f32_dq_kernel(a->D, pl.f32_ks, pl.dq_rows);
+            const KernelChoice k = f32_dq_kernel(a->D, pl.f32_ks, pl.dq_rows);
             rc = launch(k.fn, pl.dq_blocks, 256, k.lds, st, p);
             if (rc) return rc;
         }
@@ -4962,6 +5180,35 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     }
     rc = enable_large_lds();
     if (rc) return rc;
+    if (pl.joint) {
+        if (fused_delta) {
+            ltr_attn_delta_args d{};
+            d.o = a->o;
+            d.d_o = a->d_o;
+            d.delta = delta;
+            d.B = a->B;
+            d.Hq = a->Hq;
+            d.D = a->D;
+            d.Sq = a->Sq;
+            for (int i = 0; i < 3; i++) {
+                d.o_stride[i] = a->o_stride[i];
+                d.do_stride[i] = a->do_stride[i];
+            }
+            d.o_dtype = d.do_dtype = LTR_BF16;
+            rc = ltr_attn_bwd_delta(&d, stream);
+            if (rc) return rc;
+            p.flags &= ~LTR_DELTA_FROM_O;
+        }
+        if (flags & LTR_CAUSAL)   // longest dK/dV blocks first, as below
+            std::stable_sort(p.chunk, p.chunk + p.n_chunks, [](const ChunkDev &x, const ChunkDev &y) { return x.pos0 < y.pos0; });
+        const unsigned n_q = map_blocks(p.q_map, p.B * p.Hkv), n_kv = map_blocks(p.kv_map, p.B * p.Hkv);
+        p.joint = {pl.keys_first ? n_kv : n_q, pl.keys_first};
+        const KernelChoice k = joint_kernel(D, pad, pl.dq_ks);
+        rc = launch(k.fn, (long long)n_q + n_kv, 512, k.lds, st, p);
+        return rc || pl.split.n == 1 ? rc
+               : D == 128            ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
+                                     : launch((const void *)bwd_dkdv_reduce_kernel<64, 1>, reduce_grid, 256, 0, st, p);
+    }
     // the dQ kernel goes first: with LTR_DELTA_FROM_O it produces the DELTA that the dK/dV kernel reads
     if (do_dq) {
         if (pad) {
@@ -5104,6 +5351,11 @@ int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work
         if (b.key_waves) snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_keywave_kernel<%d>", D);
         else snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);
     }
+    if (b.joint) {   // one kernel for both
+        const char *name = joint_kernel(D, pad, b.dq_ks).name;
+        snprintf(out->dq_kernel, sizeof(out->dq_kernel), "%s", name);
+        snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "%s", name);
+    }
     if (ws) {
         ws->blocks_per_tile = shared ? b.split.n : 1;
         ws->reduce_blocks = shared ? reduce_blocks(b, D) : 0;
@@ -5129,7 +5381,7 @@ extern "C" int ltr_attn_bwd_noalloc(const ltr_attn_bwd_args *a, void *stream) {
     if (a->Sq > LTR_NOALLOC_MAX_ROWS || (long long)a->B * a->Hq > LTR_NOALLOC_MAX_ROWS ||
         (long long)a->B * a->Hq * a->Sq > LTR_NOALLOC_MAX_ROWS)
         return LTR_ETOOBIG;
-    return bwd_launch(a, a->flags | LTR_DELTA_FROM_O, true, stream);
+    return bwd_launch(a, (a->flags | LTR_DELTA_FROM_O) & ~LTR_BWD_JOINT, true, stream);
 }
 
 extern "C" int ltr_cast_f32_to_bf16(const float *src, void *dst, int64_t n, void *stream) {

@@ -255,7 +255,7 @@ struct ChunksFunction {
             }
             // this node holds every key these rows see and every row of it that sees these keys: the kernels write bf16 results
             a.flags = cols | (c.causal ? LTR_CAUSAL : 0u) | (direct ? LTR_DQ_BF16 : 0u) | (!f32 && !own_acc ? LTR_DKDV_BF16 : 0u) |
-                      (direct32 ? LTR_DQ_F32_RESULT : delta_from_o && first == 0 ? LTR_DELTA_FROM_O : 0u) | (rope.defined() ? LTR_ROPE_DQ : 0u);
+                      (direct32 ? LTR_DQ_F32_RESULT : delta_from_o && first == 0 ? LTR_DELTA_FROM_O : 0u) | (rope.defined() ? LTR_ROPE_DQ : 0u) | LTR_BWD_JOINT;   // the results are fresh tensors or the ring's accumulators
             // few key tiles: blocks share them and leave partial sums in a workspace (from torch's caching allocator)
             int64_t part_bytes = 0;
             check_rc(ltr_attn_bwd_workspace(&a, &part_bytes), "ltr_attn_bwd_workspace");

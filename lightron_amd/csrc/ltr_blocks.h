@@ -91,3 +91,77 @@ inline BlockGrid block_grid(long long pairs, long long items, long long inner, l
     }
     return {{0, (int)items, 1, (int)inner}, (unsigned)(pairs * items * inner), 1, 1};
 }
+
+// Blocks of two kinds in one launch (bwd_joint_kernel): all blocks of one kind, each in its own order, then all of the other, on a linear grid.
+// The hardware hands blocks out in that order, so the second kind fills the CUs that the first leaves idle, at its end and, where there are
+// fewer blocks than CUs, from the start.
+struct JointMap {
+    unsigned first;    // blocks of the kind that goes first
+    int keys_first;    // which that is: dK/dV, or dQ
+};
+LTR_HOST_DEVICE unsigned map_blocks(const BlockMap &m, int pairs) {   // places of a map, the empty ones of a last group among them
+    return m.group ? 8u * m.inner * m.group * m.groups * m.items : (unsigned)pairs * m.items * m.inner;
+}
+struct JointItem {
+    BlockItem item;
+    bool keys;         // a dK/dV block
+};
+LTR_HOST_DEVICE JointItem joint_item_at(const JointMap &j, const BlockMap &q, const BlockMap &kv, int pairs, unsigned id) {
+    const bool second = id >= j.first;   // the first kind has a multiple of 8 places where there are groups: the XCD stays id % 8
+    if (second) id -= j.first;
+    JointItem r;
+    r.keys = second != (j.keys_first != 0);
+    const BlockMap &m = r.keys ? kv : q;
+    if (m.group) {
+        const unsigned i = id >> 3, t = i / (unsigned)m.inner, z = t / (unsigned)m.group;
+        r.item = block_item_at(m, pairs, (i - t * m.inner) << 3 | (id & 7), t - z * m.group, z);
+    } else {
+        r.item = block_item_at(m, pairs, id, 0, 0);
+    }
+    return r;
+}
+
+// Time of a launch whose blocks go, in this order, each to the slot (a CU's place for a block) that is free first: what the hardware's in-order
+// dispatch comes to.  Blocks come as classes of equal length.  Slots that are free at the same time are counted together; to keep their
+// list short, times that differ by less than 3 % of a block are the same.
+struct BlockClass {
+    double us;
+    long long n;
+};
+inline double launch_us(const BlockClass *classes, int n_classes, int slots) {
+    constexpr int MOST = 48;
+    struct Run {
+        double at;
+        long long n;
+    } run[MOST];
+    int runs = 1;
+    run[0] = {0, slots};
+    double end = 0;
+    for (int c = 0; c < n_classes; c++) {
+        const double eps = std::max(0.3, 0.03 * classes[c].us);
+        // whole rounds of equal blocks move all slots alike
+        const long long rounds = std::max(0LL, classes[c].n / slots - 1);
+        for (int i = 0; i < runs; i++) run[i].at += rounds * classes[c].us;
+        if (rounds > 0) end = std::max(end, run[runs - 1].at);
+        for (long long left = classes[c].n - rounds * slots; left > 0;) {
+            const long long n = std::min(left, run[0].n);
+            const double at = run[0].at + classes[c].us;
+            left -= n;
+            run[0].n -= n;
+            if (run[0].n == 0) {
+                runs--;
+                for (int i = 0; i < runs; i++) run[i] = run[i + 1];
+            }
+            end = std::max(end, at);
+            int i = 0;
+            while (i < runs && run[i].at < at - eps) i++;
+            if (i < runs && run[i].at <= at + eps) run[i].n += n;
+            else if (runs == MOST) run[std::min(i, runs - 1)].n += n;
+            else {
+                for (int k = runs++; k > i; k--) run[k] = run[k - 1];
+                run[i] = {at, n};
+            }
+        }
+    }
+    return end;
+}

@@ -1,0 +1,104 @@
+"""bwd_joint_kernel (dQ and dK/dV blocks in one launch) against the dense oracle and against the two launches it takes the place of, at the
+edges of both kinds' tiles (128 or 256 rows, 64-row sub-tiles, 128 keys)."""
+import pytest
+import torch
+
+from oracle import ring_attention_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,B,Hq,Hkv,Sq,q_pos,split,chunks,causal", [
+    (64, 2, 12, 12, 1, 0, None, [(1, 0)], True),                                   # one row, one key
+    (64, 4, 12, 12, 128, 0, None, [(128, 0)], True),
+    (64, 1, 8, 2, 321, 0, None, [(321, 0)], True),                                 # grouped heads, pairs that do not divide among the XCDs
+    (64, 3, 16, 16, 193, (40, 300), 33, [(31, 0), (130, 31), (64, 500)], True),    # two segments, chunk tails, keys no row sees
+    (128, 2, 8, 8, 257, 0, None, [(257, 0)], True),                                # one row and key past two tiles
+    (128, 1, 32, 8, 700, 0, None, [(700, 0)], True),                               # shared key tiles
+    (128, 1, 16, 16, 500, 37, None, [(300, 0), (129, 300)], False),
+    (128, 5, 8, 8, 450, 0, None, [(450, 0)], True),
+    (128, 5, 32, 32, 240, 0, None, [(240, 0)], False),                             # more blocks than CUs
+    (96, 2, 16, 16, 391, 0, None, [(391, 0)], True),
+    (40, 1, 8, 4, 130, 3, None, [(133, 0)], True),
+])
+def test_joint(ltr, D, B, Hq, Hkv, Sq, q_pos, split, chunks, causal):
+    total, pos = sum(n for n, _ in chunks), [p for _, p in chunks]
+    plan = ltr.attn_plan(B, Hq, Hkv, D, Sq, [n for n, _ in chunks], pos, q_pos, split, causal, share_keys=True, joint=True)
+    assert plan["dq"]["kernel"] == plan["dkdv"]["kernel"] and plan["dq"]["kernel"].startswith("bwd_joint")
+    g = torch.Generator().manual_seed(Sq)
+    mk = lambda s, h: torch.randn(B, s, h, D, generator=g).to(torch.bfloat16)
+    q, do, k, v = mk(Sq, Hq), mk(Sq, Hq), mk(total, Hkv), mk(total, Hkv)
+    at = [sum(n for n, _ in chunks[:i]) for i in range(len(chunks))]
+    cut = lambda t: [t[:, a:a + n] for a, (n, _) in zip(at, chunks)]
+    qp = q_pos if isinstance(q_pos, tuple) else (q_pos, q_pos)
+    rows = torch.arange(Sq)
+    qpos = rows + qp[0] if split is None else torch.where(rows < split, rows + qp[0], rows - split + qp[1])
+    kpos = torch.cat([torch.arange(p, p + n) for n, p in chunks])
+    _, _, *ref = orc.dense_attention_grads(q.float(), k.float(), v.float(), do.float(), qpos, kpos, causal, dtype=torch.float32)
+    qd, kd, vd, dod = q.cuda(), k.cuda(), v.cuda(), do.cuda()
+    o, lse = (t.detach() for t in ltr.block_attention(qd, cut(kd), cut(vd), pos, q_pos, split, causal))
+
+    def run(joint, dtype, fill):
+        delta = torch.full(lse.shape, 3.0, dtype=torch.float32, device="cuda") if dtype == torch.bfloat16 else ltr.attn_delta(o, dod)
+        if D not in (64, 128):   # the padded kernels are reached through block_attention only
+            leaves = [t.clone().requires_grad_(True) for t in (qd, kd, vd)]
+            ltr.block_attention(leaves[0], cut(leaves[1]), cut(leaves[2]), pos, q_pos, split, causal)[0].backward(dod)
+            return [t.grad for t in leaves], None
+        out = [torch.full(t.shape, fill, dtype=dtype, device="cuda") for t in (qd, kd, vd)]
+        ltr.attn_bwd_accumulate(qd, dod, lse, delta, cut(kd), cut(vd), pos, out[0], cut(out[1]), cut(out[2]), q_pos, split, causal,
+                                o=o if dtype == torch.bfloat16 else None, share_keys=True, joint=joint)
+        return out, delta
+
+    # bf16 P, dS, products and results: 2e-3 .. 3.1e-3 of the norm.  With one key dS = dP - DELTA is zero but for the rounding of two fp32 sums of
+    # size 8 (1e-6), times a key and 1 / sqrt(D): 1e-6 per element.  Results where no query sees a key are zeros
+    results, delta = run(True, torch.bfloat16, 7.0)
+    for name, got, want in zip(("dq", "dk", "dv"), results, ref):
+        assert (got.cpu().float() - want).norm() <= 1e-2 * want.norm() + 1e-6 * want.numel() ** 0.5, name
+    seen = torch.ones(total, dtype=torch.bool) if not causal else kpos <= qpos.max()
+    assert not results[1].cpu()[:, ~seen].any() and not results[2].cpu()[:, ~seen].any()
+    if delta is None:
+        return
+    want_delta = (do.float() * o.cpu().float()).sum(-1).transpose(1, 2)
+    assert (delta.cpu() - want_delta).abs().max() <= 1e-5 * D + 1e-5 * want_delta.abs().max()
+    again, _ = run(True, torch.bfloat16, 7.0)
+    assert all(torch.equal(a, b) for a, b in zip(results, again))
+    # fp32 accumulators with DELTA given: the sums of the two launches in another order, added to what was there
+    joint, apart = run(True, torch.float32, 0.5)[0], run(False, torch.float32, 0.5)[0]
+    for a, b in zip(joint, apart):
+        a, b = a.cpu() - 0.5, b.cpu() - 0.5
+        assert (a - b).norm() <= 2e-5 * b.norm() + 1e-6 * b.numel() ** 0.5
+    for got, want in zip(joint, ref):
+        assert (got.cpu() - 0.5 - want).norm() <= 1e-2 * want.norm() + 1e-6 * want.numel() ** 0.5
+
+
+def test_joint_backward_under_rope_and_replays(ltr):
+    """RoPE's gradient in the dQ blocks, and a captured backward replayed between eager calls."""
+    g = torch.Generator().manual_seed(5)
+    q, do, k, v = (torch.randn(2, 300, 8, 128, generator=g).to(torch.bfloat16).cuda() for _ in range(4))
+    freqs = ltr.precompute_freqs_cis(128, 300)
+    table = ltr.rope_table(freqs).cuda()
+    assert ltr.attn_plan(2, 8, 8, 128, 300, [300], [0], causal=True, joint=True)["dq"]["kernel"].startswith("bwd_joint")
+    def grads(rope):
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        x = leaves[0] if rope else ltr.apply_rotary_emb(leaves[0], leaves[0], freqs.cuda())[0]
+        ltr.block_attention(x, [leaves[1]], [leaves[2]], [0], causal=True, **(dict(q_rope=table) if rope else {}))[0].backward(do)
+        return [t.grad for t in leaves]
+    for a, b in zip(grads(True), grads(False)):   # dQ rounded before its rotation, or after
+        assert (a.float() - b.float()).norm() <= 5e-3 * b.float().norm()
+    with torch.no_grad():
+        o, lse = ltr.block_attention(q, [k], [v], [0], causal=True)
+    delta, out = torch.empty_like(lse), [torch.empty_like(t) for t in (q, k, v)]
+    call = lambda: ltr.attn_bwd_accumulate(q, do, lse, delta, [k], [v], [0], out[0], [out[1]], [out[2]], 0, None, True, o=o, joint=True)
+    call()
+    want = [t.clone() for t in out]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(3):
+        for t in out:
+            t.fill_(3.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, want))
+        call()
+        assert all(torch.equal(a, b) for a, b in zip(out, want))

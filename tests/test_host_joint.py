@@ -1,0 +1,148 @@
+"""CPU tests of the backward in one launch (LTR_BWD_JOINT): the block order of its two kinds (csrc/ltr_blocks.h, compiled with the host
+compiler), the launch times it is chosen by, and its plans."""
+import ctypes
+import heapq
+import os
+import random
+import shutil
+import subprocess
+
+import pytest
+import torch
+
+import lightron_amd as la
+from lightron_amd import _lib as L
+
+CSRC = os.path.join(os.path.dirname(la.__file__), "csrc")
+PROGRAM = r"""
+#include "ltr_blocks.h"
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+// "order" pairs q_items q_inner q_group kv_items kv_inner kv_group keys_first -> "ok"; "time" slots (us n)... -> launch_us
+int main(int argc, char **argv) {
+    if (argv[1][0] == 't') {
+        std::vector<BlockClass> c;
+        for (int i = 3; i < argc; i += 2) c.push_back({atof(argv[i]), atoll(argv[i + 1])});
+        printf("%.6f\n", launch_us(c.data(), (int)c.size(), atoi(argv[2])));
+        return 0;
+    }
+    long long a[10];
+    for (int i = 2; i < argc; i++) a[i] = atoll(argv[i]);
+    const int pairs = (int)a[2], keys_first = (int)a[9];
+    const BlockMap m[2] = {block_grid(pairs, a[3], a[4], a[5]).map, block_grid(pairs, a[6], a[7], a[8]).map};
+    const long long n[2] = {(long long)pairs * a[3] * a[4], (long long)pairs * a[6] * a[7]};
+    const unsigned places[2] = {map_blocks(m[0], pairs), map_blocks(m[1], pairs)};
+    const JointMap j = {places[keys_first], keys_first};
+    std::vector<unsigned char> seen[2] = {std::vector<unsigned char>(n[0]), std::vector<unsigned char>(n[1])};
+    long long got[2] = {};
+    std::vector<int> order[2] = {std::vector<int>(8), std::vector<int>(8)};
+    for (unsigned id = 0; id < places[0] + places[1]; id++) {
+        const JointItem b = joint_item_at(j, m[0], m[1], pairs, id);
+        const int kv = b.keys, items = (int)(kv ? a[6] : a[3]), inner = (int)(kv ? a[7] : a[4]);
+        if ((id < j.first) != (b.keys == (keys_first != 0))) return printf("kind\n"), 1;
+        if (b.item.pair >= pairs) continue;
+        if (b.item.pair < 0 || b.item.item < 0 || b.item.item >= items || b.item.sub < 0 || b.item.sub >= inner) return printf("range\n"), 1;
+        if (pairs % 8 == 0 && (b.item.pair & 7) != (int)(id & 7)) return printf("xcd\n"), 1;
+        if (seen[kv][((long long)b.item.pair * items + b.item.item) * inner + b.item.sub]++) return printf("twice\n"), 1;
+        got[kv]++;
+    }
+    if (got[0] != n[0] || got[1] != n[1]) return printf("missing\n"), 1;
+    printf("ok\n");
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    cxx = os.environ.get("CXX", "g++")
+    if not shutil.which(cxx):
+        pytest.skip("no host compiler")
+    d = tmp_path_factory.mktemp("joint")
+    (d / "joint.cpp").write_text(PROGRAM)
+    subprocess.run([cxx, "-O2", "-std=c++17", "-I", CSRC, str(d / "joint.cpp"), "-o", str(d / "joint")], check=True)
+    return lambda *a: subprocess.run([str(d / "joint")] + [str(x) for x in a], capture_output=True, text=True).stdout.strip()
+
+
+@pytest.mark.parametrize("pairs,q,kv", [
+    (8, (1, 1, 1), (1, 1, 1)), (8, (5, 4, 1), (10, 4, 1)), (40, (7, 2, 5), (9, 1, 3)), (104, (3, 1, 7), (6, 2, 13)),   # last groups with empty places
+    (7, (9, 4, 1), (5, 2, 1)), (1, (3, 8, 1), (2, 16, 1)), (12, (4, 3, 1), (1, 1, 1)),                                   # pairs that do not divide among the XCDs
+])
+@pytest.mark.parametrize("keys_first", [0, 1])
+def test_every_block_of_both_kinds_once(program, pairs, q, kv, keys_first):
+    assert program("order", pairs, *q, *kv, keys_first) == "ok"
+
+
+def _dispatch(classes, slots):
+    free, end = [0.0] * slots, 0.0
+    for us, n in classes:
+        for _ in range(n):
+            t = heapq.heappop(free) + us
+            end = max(end, t)
+            heapq.heappush(free, t)
+    return end
+
+
+def test_launch_time_is_that_of_in_order_dispatch(program):
+    """Against the slots one by one: times within 3 % of a block count as one, which moves the end by a few such steps at most."""
+    rng = random.Random(3)
+    for _ in range(60):
+        slots = rng.choice([1, 7, 32, 256])
+        classes = [(rng.uniform(2, 60), rng.randrange(1, 3 * slots + 2)) for _ in range(rng.randrange(1, 17))]
+        want = _dispatch(classes, slots)
+        got = float(program("time", slots, *[x for c in classes for x in c]))
+        assert abs(got - want) <= 0.06 * max(us for us, _ in classes) + 0.02 * want, (slots, classes, got, want)
+
+
+def _args(D, B, Hq, Hkv, Sq, chunks, flags, dtype=L.LTR_BF16):
+    a = L.BwdArgs()
+    a.B, a.Hq, a.Hkv, a.D, a.Sq, a.q_split, a.n_chunks, a.flags, a.io_dtype = B, Hq, Hkv, D, Sq, Sq, len(chunks), flags, dtype
+    for i, (sk, pos0) in enumerate(chunks):
+        a.chunk[i].sk, a.chunk[i].pos0 = sk, pos0
+    return a
+
+
+def test_only_with_the_flag_and_without_size_hints():
+    case = dict(B=2, Hq=16, Hkv=16, D=128, Sq=600, chunk_lens=[600], k_pos0=[0], causal=True)
+    both = la.attn_plan(**case, joint=True)
+    assert both["dq"]["kernel"] == both["dkdv"]["kernel"] and both["dq"]["kernel"].startswith("bwd_joint_kernel<128, ")
+    for kw in ({}, dict(share_keys=True), dict(joint=True, dq_rows=256), dict(joint=True, dkdv_keys=128), dict(joint=True, dtype=torch.float32)):
+        p = la.attn_plan(**case, **kw)
+        assert p["dq"]["kernel"] != p["dkdv"]["kernel"], kw
+    f = L.LTR_BWD_JOINT | L.LTR_CAUSAL
+    for skip in (L.LTR_NO_DQ, L.LTR_NO_DKDV):   # one kind of blocks only
+        p = L.AttnPlan()
+        assert L.load().ltr_attn_plan(ctypes.byref(_args(128, 2, 16, 16, 600, [(600, 0)], f | skip)), ctypes.byref(p)) == 0
+        assert p.dq_kernel != p.dkdv_kernel
+
+
+def test_plans_of_joint_launches_hold_together():
+    """Workspace, blocks and rows of random problems belong to each other; past several rounds of blocks nothing is joined."""
+    rng = random.Random(1)
+    joint = 0
+    for _ in range(400):
+        n_rep, Hkv, D = rng.choice([1, 2, 4]), rng.choice([1, 4, 8, 12, 16]), rng.choice([64, 128, 96, 40])
+        B, S, n, causal = rng.choice([1, 2, 5, 16]), rng.randrange(1, 5000), rng.choice([1, 1, 3]), rng.random() < 0.7
+        chunks = [(rng.randrange(1, S + 1), i * S) for i in range(n)]
+        f = L.LTR_BWD_JOINT | L.LTR_HEAD_COLS | (L.LTR_CAUSAL if causal else 0) | rng.choice([0, L.LTR_DELTA_FROM_O | L.LTR_DQ_BF16 | L.LTR_DKDV_BF16])
+        a = _args(D, B, n_rep * Hkv, Hkv, S, chunks, f)
+        need, ws = ctypes.c_int64(0), L.AttnPlanWs()
+        assert L.load().ltr_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(need)) == 0
+        assert L.load().ltr_attn_plan_ws(ctypes.byref(a), need.value, ctypes.byref(ws)) == 0
+        if ws.plan.dq_kernel != ws.plan.dkdv_kernel:
+            continue
+        joint += 1
+        width = 64 if D <= 64 else 128
+        assert ws.plan.dq_kernel.decode() == "bwd_joint%s_kernel<%d, %d>" % ("" if D in (64, 128) else "_pad", width, 256 // ws.plan.dq_rows)
+        assert ws.plan.dq_rows in (128, 256) and not ws.plan.dq_paired and ws.plan.dkdv_keys == 128
+        assert ws.plan.dq_blocks == -(-S // ws.plan.dq_rows) * B * n_rep * Hkv
+        tiles = sum(-(-(min(sk, S - p) if causal else sk) // 128) for sk, p in chunks if not causal or p < S)
+        t = ws.blocks_per_tile
+        assert need.value == (tiles * B * Hkv * t * 128 * width * 8 if t > 1 else 0)
+        assert ws.plan.dkdv_blocks == (tiles if t > 1 else sum(-(-sk // 128) for sk, _ in chunks)) * B * Hkv * t
+        if need.value:   # one byte short: no shared tiles
+            assert L.load().ltr_attn_plan_ws(ctypes.byref(a), need.value - 1, ctypes.byref(ws)) == 0 and ws.blocks_per_tile == 1
+    assert joint > 100
+    big = la.attn_plan(8, 32, 32, 128, 4096, [4096], [0], causal=True, joint=True)
+    assert big["dq"]["kernel"] == "bwd_dq_kernel<128, 1>" and big["dkdv"]["kernel"] == "bwd_dkdv_kernel<128, 1>"
