@@ -171,6 +171,15 @@ __device__ __forceinline__ void q_pos_range(int r0, int r1, int split, int p0, i
     }
 }
 
+// Masked tiles of the forward and dQ kernels: a key of the chunk is visible to a row up to the chunk's end and, under a causal mask, up to the
+// row's position.  The last visible one, counted from `first` (keys of the chunk; this lane's first of the tile): one compare with a constant and
+// one select per score.  (With the two comparisons per score it was six instructions, and 32 registers of the forward held the keys.)
+__device__ __forceinline__ int last_key(bool causal, int row_pos, int chunk_pos0, int chunk_keys, int first) {
+    int last = chunk_keys - 1;
+    if (causal) last = min(last, __builtin_elementwise_sub_sat(row_pos, chunk_pos0));
+    return __builtin_elementwise_sub_sat(last, first);
+}
+
 __device__ __forceinline__ BlockItem block_item(const BlockMap &m, int pairs) { return block_item_at(m, pairs, blockIdx.x, blockIdx.y, blockIdx.z); }
 
 // both halves of the wave end up with combine(x[l], x[l ^ 32])
@@ -216,12 +225,15 @@ __device__ __forceinline__ int lds_swz_off(int row, int chunk) {   // element of
 // (tile = swizzled tile, see lds_swz)
 template <int D>
 __device__ __forceinline__ bf16x8 lds_operand_tr_swz(const __bf16 *tile, int k0, int n_base, int lane) {
+    // k0 is a multiple of 16, which the swizzle of a row does not see: it is an immediate beside the lane's address, and one pair of addresses
+    // per column block serves every k0 (left to the compiler each k0 had its own: 24 registers of the forward and dK/dV kernels)
     const int li = lane & 15, g = lane >> 4;
     const int hh = g >> 1;
     const int col = n_base + ((g & 1) << 4) + ((li & 3) << 2);
-    const int row = k0 + 4 * hh + (li >> 2);
-    i16x4 lo = lds_read_tr16(tile + lds_swz_off<D>(row, col >> 3) + (col & 7));
-    i16x4 hi = lds_read_tr16(tile + lds_swz_off<D>(row + 8, col >> 3) + (col & 7));
+    const int row = 4 * hh + (li >> 2);
+    const __bf16 *const block = tile + k0 * D;
+    i16x4 lo = lds_read_tr16(block + lds_swz_off<D>(row, col >> 3) + (col & 7));
+    i16x4 hi = lds_read_tr16(block + lds_swz_off<D>(row + 8, col >> 3) + (col & 7));
     union {
         struct { i16x4 a, b; } s;
         bf16x8 v;
@@ -324,93 +336,19 @@ __device__ __forceinline__ bf16x8 operand_of(const PackedTile &t, int kb) {
     return c.v;
 }
 
-// Two independent 32x32 accumulation chains over the head dimension (added to ra / rb as passed in), A operands from rows of swizzled LDS tiles
-// (row pointers rowa / rowb, swizzle words swa / swb of those rows, already XOR-ed with the lane's half),
-// B operands from registers.  The chains alternate so no MFMA waits for its predecessor, and the operand reads
-// run PF steps ahead of the MFMAs that use them; sched_barrier pins that order (left alone, the scheduler sinks
-// each read to just before its use and the full LDS latency is exposed at every step).
-template <int D>
-__device__ __forceinline__ void lds_gemm_pair(const __bf16 *rowa, int swa, const __bf16 *rowb, int swb,
-                                              const bf16x8 (&ba)[D / 16], const bf16x8 (&bb)[D / 16],
-                                              f32x16 &ra, f32x16 &rb) {
-    constexpr int NK = D / 16, PF = 2;
-    bf16x8 xa[PF + 1], xb[PF + 1];
-#pragma unroll
-    for (int i = 0; i < PF; i++) {
-        xa[i] = *(const bf16x8 *)(rowa + (((2 * i) ^ swa) << 3));
-        xb[i] = *(const bf16x8 *)(rowb + (((2 * i) ^ swb) << 3));
-    }
-#pragma unroll
-    for (int kb = 0; kb < NK; kb++) {
-        if (kb + PF < NK) {
-            xa[(kb + PF) % (PF + 1)] = *(const bf16x8 *)(rowa + (((2 * (kb + PF)) ^ swa) << 3));
-            xb[(kb + PF) % (PF + 1)] = *(const bf16x8 *)(rowb + (((2 * (kb + PF)) ^ swb) << 3));
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        ra = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[kb % (PF + 1)], ba[kb], ra, 0, 0, 0);
-        rb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xb[kb % (PF + 1)], bb[kb], rb, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-struct NoHook {
-    __device__ __forceinline__ void operator()(int) const {}
-};
-
-// One 32x32 accumulation chain over the head dimension (added to r as passed in): A operands from row `row` of a
-// swizzled LDS tile (sw = swizzle word of the row XOR the lane's half), B operands from registers.  hook(kb)
-// is placed right after MFMA kb: independent arithmetic of the same wave written there issues while the matrix
-// pipe works on that MFMA (a wave issues one instruction per ~5 clocks, an MFMA occupies the pipe for 32).
-template <int D, class Hook = NoHook>
-__device__ __forceinline__ void lds_gemm_chain(const __bf16 *row, int sw, const bf16x8 (&b)[D / 16], f32x16 &r,
-                                               Hook hook = Hook()) {
-    constexpr int NK = D / 16, PF = 2;
-    bf16x8 x[PF + 1];
-#pragma unroll
-    for (int i = 0; i < PF; i++) x[i] = *(const bf16x8 *)(row + (((2 * i) ^ sw) << 3));
-#pragma unroll
-    for (int kb = 0; kb < NK; kb++) {
-        if (kb + PF < NK) x[(kb + PF) % (PF + 1)] = *(const bf16x8 *)(row + (((2 * (kb + PF)) ^ sw) << 3));
-        __builtin_amdgcn_sched_barrier(0);
-        r = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[kb % (PF + 1)], b[kb], r, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        hook(kb);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-// acc[db] (32 x 32 tiles over the head dimension) += T^T-operand x B for NKB blocks of 16 tile rows starting at
-// row0: the A operands are transpose reads of the swizzled LDS tile T (rows = contraction index), the B
-// operands b[kb] come from registers.  Reads run PF MFMAs ahead, order pinned as in lds_gemm_pair; hook(step)
-// is placed right after MFMA `step` (see lds_gemm_chain).
-template <int D, int NKB, class Hook = NoHook>
-__device__ __forceinline__ void lds_tr_gemm(const __bf16 *T, int row0, int lane, const bf16x8 (&b)[NKB],
-                                            f32x16 (&acc)[D / 32], Hook hook = Hook()) {
-    constexpr int ND = D / 32, N = NKB * ND, PF = 3;
-    bf16x8 a[PF + 1];
-#pragma unroll
-    for (int i = 0; i < PF && i < N; i++) a[i] = lds_operand_tr_swz<D>(T, row0 + (i / ND) * 16, (i % ND) * 32, lane);
-#pragma unroll
-    for (int step = 0; step < N; step++) {
-        if (step + PF < N)
-            a[(step + PF) % (PF + 1)] = lds_operand_tr_swz<D>(T, row0 + ((step + PF) / ND) * 16, ((step + PF) % ND) * 32, lane);
-        __builtin_amdgcn_sched_barrier(0);
-        acc[step % ND] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[step % (PF + 1)], b[step / ND], acc[step % ND], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        hook(step);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-// The same two GEMM loops with the LDS byte addresses of the lane's operands passed in (one per head-dimension block:
-// the swizzle makes them differ per lane, not by a constant) plus an immediate: a kernel that has no registers left to
-// unroll its tile loop over the LDS buffers keeps these addresses in registers and flips them between the buffers with one
-// XOR each per tile, instead of rebuilding every address from pointer + swizzle before each read.
 typedef __attribute__((address_space(3))) const bf16x8 *lds_bf16x8_ptr;
 typedef __attribute__((address_space(3))) i16x4 *lds_i16x4_ptr;
 typedef __attribute__((address_space(3))) const f32x4 *lds_f32x4_ptr;
 typedef __attribute__((address_space(3))) const i32x4 *lds_i32x4_ptr;
 
+// GEMM loops of the kernels whose LDS addresses of the lane's operands are in registers (one per 16 columns of a tile's rows, or a pair per
+// head-dimension block: the swizzle makes them differ per lane, not by a constant), plus an immediate for the rows and the buffer.
+// A kernel that does not unroll its tile loop over the LDS buffers flips them between the buffers with one XOR each per tile.
+
+// Two independent 32x32 accumulation chains over the head dimension (added to ra / rb as passed in), A operands from rows of swizzled LDS tiles,
+// B operands from registers.  The chains alternate so no MFMA waits for its predecessor, and the operand reads
+// run PF steps ahead of the MFMAs that use them; sched_barrier pins that order (left alone, the scheduler sinks
+// each read to just before its use and the full LDS latency is exposed at every step).
 template <int D>
 __device__ __forceinline__ void lds_gemm_pair_at(const unsigned (&addr)[D / 16], int imm_a, int imm_b,
                                                  const bf16x8 (&ba)[D / 16], const bf16x8 (&bb)[D / 16], f32x16 &ra, f32x16 &rb) {
@@ -434,6 +372,24 @@ __device__ __forceinline__ void lds_gemm_pair_at(const unsigned (&addr)[D / 16],
     }
 }
 
+// one such chain
+template <int D>
+__device__ __forceinline__ void lds_gemm_chain_at(const unsigned (&addr)[D / 16], int imm, const bf16x8 (&b)[D / 16], f32x16 &r) {
+    constexpr int NK = D / 16, PF = 2;
+    bf16x8 x[PF + 1];
+#pragma unroll
+    for (int i = 0; i < PF; i++) x[i] = *(lds_bf16x8_ptr)(uintptr_t)(addr[i] + imm);
+#pragma unroll
+    for (int kb = 0; kb < NK; kb++) {
+        if (kb + PF < NK) x[(kb + PF) % (PF + 1)] = *(lds_bf16x8_ptr)(uintptr_t)(addr[kb + PF] + imm);
+        __builtin_amdgcn_sched_barrier(0);
+        r = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[kb % (PF + 1)], b[kb], r, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// acc[db] (32 x 32 tiles over the head dimension) += T^T-operand x B for NKB blocks of 16 tile rows: the A operands are transpose reads of
+// the swizzled LDS tile T (rows = contraction index), the B operands b[kb] come from registers; reads run PF MFMAs ahead.
 // addr[j][h]: byte address of the lane's transpose-read element for head-dimension block j, rows +0 (h = 0) / +8 (h = 1)
 template <int D, int NKB>
 __device__ __forceinline__ void lds_tr_gemm_at(const unsigned (&addr)[D / 32][2], int imm, const bf16x8 (&b)[NKB], f32x16 (&acc)[D / 32]) {
@@ -499,8 +455,14 @@ __device__ __forceinline__ void wave_tile_rowmajor(unsigned char *stage, int lan
     }
 }
 
-// lds_gemm_chain / lds_tr_gemm for a wave that owns KW 32-key halves (dK/dV kernel) or KW 32-row blocks (forward): every operand
-// read from LDS feeds one MFMA per half (b[k], r[k] / acc[k] belong to half k); hook(step) follows the MFMAs of operand `step`.
+struct NoHook {
+    __device__ __forceinline__ void operator()(int) const {}
+};
+
+// The chain and the transpose GEMM for a wave that owns KW 32-key halves (dK/dV kernel) or KW 32-row blocks (forward): every operand
+// read from LDS feeds one MFMA per half (b[k], r[k] / acc[k] belong to half k).  row: the lane's row of a swizzled tile, sw = the row's
+// swizzle word XOR the lane's half.  hook(step) follows the MFMAs of operand `step`: independent arithmetic of the same wave
+// written there issues while the matrix pipe works (a wave issues one instruction per ~5 clocks, an MFMA occupies the pipe for 32).
 template <int D, int KW, class Hook = NoHook>
 __device__ __forceinline__ void lds_gemm_chain_kw(const __bf16 *row, int sw, const bf16x8 (&b)[KW][D / 16], f32x16 (&r)[KW],
                                                   Hook hook = Hook()) {
@@ -609,7 +571,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     constexpr int CPR = D / 8;   // 16-byte chunks per row
     constexpr int RPI = 64 / CPR;            // rows filled by one wave-wide 16-byte-per-lane LDS-direct load (1 KB)
     constexpr int NI = BNT / (RPI * NW);      // such loads per wave, per tensor and per tile
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // two {K tile, V tile} buffers,
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // two K tiles, two V tiles,
     constexpr int TILE = BNT * D;            // rows unpadded, 16-byte chunks XOR-swizzled (lds_swz)
     constexpr int BUF_ELEMS = 2 * TILE;
 
@@ -735,7 +697,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     // transfer j of the tile in flight (ti, into buffer buf): j < NI are this wave's K rows, the rest its V rows
     auto gload_one = [&](int j, int ti, int buf) {
         const int i = j % NI;
-        const unsigned dst = lds_address(smem) + buf * BUF_ELEMS * 2 + (j / NI) * TILE * 2 + RPI * (NI * w + i) * D * 2;
+        const unsigned dst = lds_address(smem) + buf * TILE * 2 + (j / NI) * BUF_ELEMS * 2 + RPI * (NI * w + i) * D * 2;
         const int row = RPI * (NI * w + i) + st_row;
         const int key = min(ti * BNT + row, ld_sk - 1);
         const int chunk = st_pc ^ lds_swz<D>(row);
@@ -763,11 +725,33 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     }
     tile_barrier();
     // One tile; the loop below is unrolled over the two LDS buffers so that every LDS address is a loop-invariant
-    // per-lane register plus an immediate offset (no address arithmetic between the MFMAs).
+    // per-lane register plus an immediate offset (no address arithmetic between the MFMAs).  The registers are spelled out and opaque:
+    // the K tiles and the V tiles each lie in one window of 64 KB, which the offsets reach, and 16 registers address all of it.
+    static_assert(2 * TILE * 2 <= 65536, "offsets of an LDS read end at 65535");
+    unsigned ka[D / 16], va[D / 32][2];
+    if constexpr (RB == 1) {
+        const unsigned lds0 = lds_address(smem) + (KS > 1 ? ks * BN * D * 2 : 0);
+        const int sw = lds_swz<D>(l32) ^ hh;        // rows l32 + 32 n share the swizzle word of row l32
+#pragma unroll
+        for (int kb = 0; kb < D / 16; kb++) {
+            ka[kb] = lds0 + ((l32 * D + (((2 * kb) ^ sw) << 3)) << 1);
+            asm volatile("" : "+v"(ka[kb]));
+        }
+        const int li = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < D / 32; i++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int col = i * 32 + ((g & 1) << 4) + ((li & 3) << 2), row = 4 * (g >> 1) + (li >> 2) + 8 * e;
+                va[i][e] = lds0 + 2 * TILE * 2 + ((lds_swz_off<D>(row, col >> 3) + (col & 7)) << 1);
+                asm volatile("" : "+v"(va[i][e]));
+            }
+    }
     auto tile_step = [&](auto par_tag) {
         constexpr int par = decltype(par_tag)::value;
         const int sk = nx_sk, pos0 = nx_pos0, key0 = nx_key0 + (KS > 1 ? ks * BN : 0);
-        const __bf16 *Ks = (const __bf16 *)smem + par * BUF_ELEMS + (KS > 1 ? ks * BN * D : 0), *Vs = Ks + TILE;
+        constexpr int at = par * TILE * 2;                                                        // RB == 1: offset of ka, va
+        const __bf16 *const Ks = (const __bf16 *)smem + par * TILE, *const Vs = Ks + BUF_ELEMS;   // RB == 2
         t++;
         settle();
         const bool have_next = c < p.n_chunks;
@@ -792,12 +776,11 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
             for (int nb = 0; nb + 1 < NB; nb += 2) {
                 s[nb][0] = zero16;
                 s[nb + 1][0] = zero16;
-                lds_gemm_pair<D>(Ks + (nb * 32 + l32) * D, lds_swz<D>(nb * 32 + l32) ^ hh, Ks + (nb * 32 + 32 + l32) * D,
-                                 lds_swz<D>(nb * 32 + 32 + l32) ^ hh, qreg[0], qreg[0], s[nb][0], s[nb + 1][0]);
+                lds_gemm_pair_at<D>(ka, at + nb * 32 * D * 2, at + (nb + 1) * 32 * D * 2, qreg[0], qreg[0], s[nb][0], s[nb + 1][0]);
             }
             if constexpr (NB == 1) {
                 s[0][0] = zero16;
-                lds_gemm_chain<D>(Ks + l32 * D, lds_swz<D>(l32) ^ hh, qreg[0], s[0][0]);
+                lds_gemm_chain_at<D>(ka, at, qreg[0], s[0][0]);
             }
         } else {
 #pragma unroll
@@ -812,15 +795,13 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
         const bool need_mask = (key0 + BN > sk) || (causal && (pos0 + key0 + BN - 1 > w_lo));
         if (need_mask) {
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++)
+            for (int rb = 0; rb < RB; rb++) {
+                const int last = last_key(causal, my_pos[rb], pos0, sk, key0 + 4 * hh);
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int key = key0 + nb * 32 + 8 * (r / 4) + 4 * hh + (r % 4);
-                        const bool vis = key < sk && (!causal || pos0 + key <= my_pos[rb]);
-                        s[nb][rb][r] = vis ? s[nb][rb][r] : -INFINITY;
-                    }
+                    for (int r = 0; r < 16; r++) s[nb][rb][r] = nb * 32 + 8 * (r / 4) + r % 4 <= last ? s[nb][rb][r] : -INFINITY;
+            }
         }
         // t = s*c2 - reference (exp2 domain), P = exp2(t) rounded to bf16, row sum of the rounded P (what PV uses)
 #pragma unroll
@@ -894,7 +875,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
             bf16x8 pb[2 * NB];
 #pragma unroll
             for (int kb = 0; kb < 2 * NB; kb++) pb[kb] = operand_of(pt[0][kb >> 1], kb & 1);
-            lds_tr_gemm<D, 2 * NB>(Vs, 0, lane, pb, oacc[0]);   // 16 keys per MFMA
+            lds_tr_gemm_at<D, 2 * NB>(va, at, pb, oacc[0]);   // 16 keys per MFMA
         } else {
             bf16x8 pb[RB][2 * NB];
 #pragma unroll
@@ -2997,13 +2978,11 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
             // an invisible entry gets S = -inf, so P = 0 and dS = 0
             if (need_mask) {
 #pragma unroll
-                for (int rb = 0; rb < RB; rb++)
+                for (int rb = 0; rb < RB; rb++) {
+                    const int last = row_ok[rb] ? last_key(causal, my_pos[rb], pos0, sk, key0 + nb * 32 + 4 * hh) : -1;
 #pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int key = key0 + nb * 32 + 8 * (r / 4) + 4 * hh + (r % 4);
-                        const bool vis = key < sk && row_ok[rb] && (!causal || pos0 + key <= my_pos[rb]);
-                        s[rb][r] = vis ? s[rb][r] : -INFINITY;
-                    }
+                    for (int r = 0; r < 16; r++) s[rb][r] = 8 * (r / 4) + r % 4 <= last ? s[rb][r] : -INFINITY;
+                }
             }
             bf16x8 dsb[RB][2];
 #pragma unroll
