@@ -1908,7 +1908,41 @@ __device__ __forceinline__ void write_key_rows(unsigned char *stage, int lane, c
     });
 }
 
-template <int D, int KW, bool PAD>
+// DELTA = rowsum(dO * O) of every row of the q heads that a dK/dV block walks, by the block itself (into LDS: [head][row]), for launches of few rows:
+// the additions are delta_kernel's, whose launch costs more than these rows' bytes.
+template <int D, bool PAD>
+__device__ __forceinline__ void own_delta(const BwdParams &p, int b, int h_first, float *out) {
+    constexpr int LANES = D / 8, ROWS = 512 / LANES, FLIGHT = 4;   // lanes per row, rows per pass, passes in flight
+    const int d = 8 * (threadIdx.x % LANES), first = threadIdx.x / LANES, n = p.n_reps * p.Sq;
+    const bool in = !PAD || d < p.cols;
+    for (int base = first; base < n; base += FLIGHT * ROWS) {
+        bf16x8 o[FLIGHT], g[FLIGHT];
+#pragma unroll
+        for (int i = 0; i < FLIGHT; i++) {
+            const int idx = base + i * ROWS, rep = idx / p.Sq, row = idx - rep * p.Sq;
+            o[i] = g[i] = as_bf16x8(make_uint4(0, 0, 0, 0));
+            if (idx < n && in) {
+                o[i] = as_bf16x8(*(const uint4 *)((const __bf16 *)p.o + b * p.os_[0] + (long long)row * p.os_[1] + (h_first + rep) * p.os_[2] + d));
+                g[i] = as_bf16x8(*(const uint4 *)((const __bf16 *)p.d_o + b * p.dos[0] + (long long)row * p.dos[1] + (h_first + rep) * p.dos[2] + d));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < FLIGHT; i++) {
+            float acc = 0.f, acc_hi = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                acc = fmaf((float)o[i][e], (float)g[i][e], acc);
+                acc_hi = fmaf((float)o[i][4 + e], (float)g[i][4 + e], acc_hi);
+            }
+            acc += acc_hi;
+#pragma unroll
+            for (int off = LANES / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, LANES);
+            if (base + i * ROWS < n && d == 0) out[base + i * ROWS] = acc;
+        }
+    }
+}
+
+template <int D, int KW, bool PAD, bool OWN_DELTA = false>
 __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockItem item) {
     const int cols = PAD ? p.cols : D;
     using L = BwdLds<D, KW>;   // KW = 32-key halves per wave
@@ -1994,7 +2028,10 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
 
     unsigned short *const tlist = (unsigned short *)(smem + L::LIST_OFF);     // [2][MAX_QTILES]
     int *const tcount = (int *)(smem + L::LIST_OFF + 2 * L::MAX_QTILES * 2);
+    const int h_first = hkv * p.n_rep + (split >> p.share_log2) * p.n_reps;   // first of the n_reps q heads this block walks
+    float *const dlt = (float *)(smem + L::TOTAL);                            // OWN_DELTA: [n_reps][Sq]
     if (w == 0) list_q_tiles<BM, L::MAX_QTILES>(p, lane, split, tile_kpos_lo, tile_kpos_hi, key_tail, tlist, tcount);
+    if constexpr (OWN_DELTA) own_delta<D, PAD>(p, b, h_first, dlt);
     __syncthreads();
 
     const int st_row = lane / CPR, st_pc = lane % CPR;   // this lane's place inside a 1 KB LDS-direct load
@@ -2011,7 +2048,6 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
     }
     const __bf16 *qp_head = nullptr, *dop_head = nullptr;
     const float *sp_head = nullptr;   // LSE (wave 0) or DELTA - BM (wave 1) of the head's rows, indexed by row0 + tid
-    const int h_first = hkv * p.n_rep + (split >> p.share_log2) * p.n_reps;   // first of the n_reps q heads this block walks
     auto set_head = [&](int rep) __attribute__((always_inline)) {
         const int h = h_first + rep;
         qp_head = (const __bf16 *)p.q + b * p.qs[0] + h * p.qs[2];
@@ -2074,13 +2110,11 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
             }
             if (tid < 2 * BM) {
                 const float *sp = sp_head + row0;
-                if (!MASK) {
-                    sld = sp[tid];
-                } else {
-                    const int r = tid < BM ? tid : tid - BM;
-                    sld_ok = row0 + r < p.Sq;
-                    sld = sp[sld_ok ? tid : (tid < BM ? 0 : BM)];
-                }
+                const int r = tid < BM ? tid : tid - BM;
+                if (MASK) sld_ok = row0 + r < p.Sq;
+                if (OWN_DELTA && w == 1) sld = dlt[rep * p.Sq + (!MASK || sld_ok ? row0 + r : 0)];
+                else if (!MASK) sld = sp[tid];
+                else sld = sp[sld_ok ? tid : (tid < BM ? 0 : BM)];
             }
         };
         auto lds_store = [&](int buf) {   // the LSE / DELTA values fetched by gload
@@ -3111,12 +3145,12 @@ __global__ __launch_bounds__(512) void bwd_dq_pad_kernel(const BwdParams p) {
 //   4 x 12 heads D=64 S=128   17.2 -> 12.0       2 x 16 heads D=96 S=777   57.8 -> 42.5       1 x 32 heads on 8 D=128 S=1237   94.8 -> 78
 //   1 x 16 heads D=128 S=4096  257 -> 242        1 x 12 heads D=128 S=3418  181 -> 145        3 x 8 heads D=128 S=926   61 -> 42
 // Registers are those of the dK/dV kernel, LDS the larger of both: one block per CU, as for either kind alone.
-template <int D, int KS, bool PAD>
+template <int D, int KS, bool PAD, bool OWN_DELTA = false>
 __device__ __forceinline__ void bwd_joint_body(const BwdParams &p) {
     const int P = p.B * p.Hkv;
     const JointItem j = joint_item_at(p.joint, p.q_map, p.kv_map, P, blockIdx.x);
     if (j.item.pair >= P) return;
-    if (j.keys) bwd_dkdv_body<D, 1, PAD>(p, j.item);
+    if (j.keys) bwd_dkdv_body<D, 1, PAD, OWN_DELTA>(p, j.item);
     else bwd_dq_body<D, 1, KS, PAD>(p, j.item);
 }
 template <int D, int KS>
@@ -3126,6 +3160,16 @@ __global__ __launch_bounds__(512) void bwd_joint_kernel(const BwdParams p) {
 template <int D, int KS>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_joint_pad_kernel(const BwdParams p) {
     bwd_joint_body<D, KS, true>(p);
+}
+
+// the same with DELTA computed by the dK/dV blocks for themselves (own_delta), as the dQ blocks compute theirs: launches of few rows (own_delta_rows)
+template <int D>
+__global__ __launch_bounds__(512) void bwd_joint_delta_kernel(const BwdParams p) {
+    bwd_joint_body<D, 2, false, true>(p);
+}
+template <int D>
+__global__ __launch_bounds__(512) void bwd_joint_delta_pad_kernel(const BwdParams p) {
+    bwd_joint_body<D, 2, true, true>(p);
 }
 
 // ------------------------------------------------------------------------------ backward, fp32
@@ -3949,6 +3993,18 @@ constexpr int joint_lds_bytes() {
     return dq > BwdLds<D, 1>::TOTAL ? dq : BwdLds<D, 1>::TOTAL;
 }
 
+// Rows (q heads x rows) of a dK/dV block that computes DELTA itself: what they cost a block against delta_kernel's launch.  Backward in a graph, faster
+// than with that launch, one round of blocks (means of 10000 random launches; a launch by the host less besides):
+//   head dims up to 64    up to 128 rows 1.08 - 1.14     256 rows 1.05 - 1.09     384 rows 1.01     512 rows 0.99 - 1.01     768 rows 0.96
+//   up to 128             up to 128 rows 1.05 - 1.07     256 rows 0.99 - 1.00     384 rows 0.94     more than a round of blocks: 0.94 and less
+constexpr int own_delta_rows(int D) { return D == 64 ? 320 : 144; }
+template <int D>
+constexpr int joint_delta_lds_bytes() {
+    constexpr int kv = BwdLds<D, 1>::TOTAL + own_delta_rows(D) * 4;
+    return joint_lds_bytes<D, 2>() > kv ? joint_lds_bytes<D, 2>() : kv;
+}
+static_assert(joint_delta_lds_bytes<128>() <= 160 * 1024, "LDS of one CU");
+
 int enable_large_lds() {
     int dev = 0;
     if (current_device(&dev)) return LTR_EDEVICE;
@@ -4004,6 +4060,10 @@ int enable_large_lds() {
         {(const void *)bwd_dq_shares_kernel<128, 4>, shares_lds_bytes<128, 4>()},
         {(const void *)bwd_dq_shares_kernel<64, 2>, shares_lds_bytes<64, 2>()},
         {(const void *)bwd_dq_shares_kernel<64, 4>, shares_lds_bytes<64, 4>()},
+        {(const void *)bwd_joint_delta_kernel<64>, joint_delta_lds_bytes<64>()},
+        {(const void *)bwd_joint_delta_pad_kernel<64>, joint_delta_lds_bytes<64>()},
+        {(const void *)bwd_joint_delta_kernel<128>, joint_delta_lds_bytes<128>()},
+        {(const void *)bwd_joint_delta_pad_kernel<128>, joint_delta_lds_bytes<128>()},
         {(const void *)bwd_joint_kernel<64, 1>, joint_lds_bytes<64, 1>()},
         {(const void *)bwd_joint_kernel<64, 2>, joint_lds_bytes<64, 2>()},
         {(const void *)bwd_joint_pad_kernel<64, 1>, joint_lds_bytes<64, 1>()},
@@ -4389,7 +4449,11 @@ KernelChoice f32_dq_kernel(int D, int ks, int rows) {
     if (ks == 2) return {LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 2>), F32Mfma<64, 2>::LDS};
     return rows == F32Rows16::BM ? KernelChoice{LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 4>), F32Mfma<64, 4>::LDS} : KernelChoice{LTR_KERNEL(bwd_dq_f32_rows32_kernel<64, 4>), F32Mfma<64, 4>::LDS};
 }
-KernelChoice joint_kernel(int D, bool pad, int ks) {
+KernelChoice joint_kernel(int D, bool pad, int ks, bool own_delta) {
+    if (own_delta) {
+        if (pad) return D == 128 ? KernelChoice{LTR_KERNEL(bwd_joint_delta_pad_kernel<128>), joint_delta_lds_bytes<128>()} : KernelChoice{LTR_KERNEL(bwd_joint_delta_pad_kernel<64>), joint_delta_lds_bytes<64>()};
+        return D == 128 ? KernelChoice{LTR_KERNEL(bwd_joint_delta_kernel<128>), joint_delta_lds_bytes<128>()} : KernelChoice{LTR_KERNEL(bwd_joint_delta_kernel<64>), joint_delta_lds_bytes<64>()};
+    }
     if (pad) {
         if (D == 128) return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<128, 1>), joint_lds_bytes<128, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<128, 2>), joint_lds_bytes<128, 2>()};
         return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<64, 1>), joint_lds_bytes<64, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<64, 2>), joint_lds_bytes<64, 2>()};
@@ -4519,6 +4583,7 @@ struct BwdPlan {
     int dq_group, kv_group;   // see pair_group
     long long dq_blocks;
     bool joint, keys_first;   // one launch for both kinds of blocks (bwd_joint_kernel), and which of them go first
+    bool own_delta;           // and its dK/dV blocks compute DELTA for themselves (own_delta)
 };
 // Does a bf16 backward run its dQ and dK/dV blocks in one launch, with how many key shares per row group and blocks per key tile, and which kind
 // first?  Both ways are priced by launch_us over classes of blocks (up to 8 evenly spaced tiles stand for all): the plan as it is, one launch after
@@ -4643,7 +4708,7 @@ void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, in
     // kind: of 5600 random launches joined at 0.96, 100 lost more than 1 %, 80 of them there; of 5400 with about these factors 50
     double best = apart * (D == 128 ? pl.dq_four_waves ? 0.92 : 0.98
                                     : pl.key_waves && pl.dq_four_waves ? 0.78 : pl.key_waves || pl.dq_four_waves || pl.dq_blocks + pl.kv_blocks > 8 * cus ? 0.88 : 0.96);
-    const double common = cost.launch_us + (flags & LTR_DELTA_FROM_O ? cost.delta_us + (double)q_pairs * Sq * D * 4 / cost.delta_bytes_per_us : 0.0);
+    const double delta_us = flags & LTR_DELTA_FROM_O ? cost.delta_us + (double)q_pairs * Sq * D * 4 / cost.delta_bytes_per_us : 0.0;
     int best_ks = 0, best_n = 1;
     bool keys_first = false;
     // dQ blocks of one and two shares; the blocks of both kinds are looked at in both orders, unless all run at once or even spread evenly over
@@ -4657,10 +4722,13 @@ void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, in
         if (n > 1 && (!may_split || pairs * tiles_seen * n > 5LL * cus || (double)pairs * tiles_seen * n * 128 * D * 8 > MAX_PART_BYTES)) break;
         if (n > 1 && n > (long long)(Sq + 63) / 64 * (Hq / Hkv)) break;
         const List kv = kv_blocks(n, cost.kv_step_us, cost.kv_fixed_us);
+        int reps = 1;
+        while (reps * 2 <= n && Hq / Hkv % (reps * 2) == 0) reps *= 2;
         for (int ks = 1; ks <= 2; ks++) {
-            const double rest = common + reduce_us(n);
-            if (rest + (q[ks - 1].total_us() + kv.total_us()) / cus >= best) continue;
             const bool one_round = q[ks - 1].n + kv.n <= cus;
+            const bool own = ks == 2 && one_round && (flags & LTR_DELTA_FROM_O) && (long long)Hq / Hkv / reps * Sq <= own_delta_rows(D);
+            const double rest = cost.launch_us + (own ? 0.5 : delta_us) + reduce_us(n);
+            if (rest + (q[ks - 1].total_us() + kv.total_us()) / cus >= best) continue;
             for (int first = 0; first < (one_round ? 1 : 2); first++) {
                 const double us = rest + (first ? both_us(kv, q[ks - 1]) : both_us(q[ks - 1], kv));
                 if (us < best) {
@@ -4668,6 +4736,7 @@ void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, in
                     best_ks = ks;
                     best_n = n;
                     keys_first = first;
+                    pl.own_delta = own;
                 }
             }
         }
@@ -4691,7 +4760,7 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.part_bytes = 0;
     pl.dq_ks = 1;
     pl.dq_group = pl.kv_group = 1;
-    pl.dq_four_waves = pl.joint = pl.keys_first = false;
+    pl.dq_four_waves = pl.joint = pl.keys_first = pl.own_delta = false;
     may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
     pl.key_waves = false;
     const int cus = device_cus();
@@ -5160,7 +5229,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     rc = enable_large_lds();
     if (rc) return rc;
     if (pl.joint) {
-        if (fused_delta) {
+        if (fused_delta && !pl.own_delta) {
             ltr_attn_delta_args d{};
             d.o = a->o;
             d.d_o = a->d_o;
@@ -5182,7 +5251,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
             std::stable_sort(p.chunk, p.chunk + p.n_chunks, [](const ChunkDev &x, const ChunkDev &y) { return x.pos0 < y.pos0; });
         const unsigned n_q = map_blocks(p.q_map, p.B * p.Hkv), n_kv = map_blocks(p.kv_map, p.B * p.Hkv);
         p.joint = {pl.keys_first ? n_kv : n_q, pl.keys_first};
-        const KernelChoice k = joint_kernel(D, pad, pl.dq_ks);
+        const KernelChoice k = joint_kernel(D, pad, pl.dq_ks, pl.own_delta);
         rc = launch(k.fn, (long long)n_q + n_kv, 512, k.lds, st, p);
         return rc || pl.split.n == 1 ? rc
                : D == 128            ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
@@ -5331,7 +5400,7 @@ int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work
         else snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);
     }
     if (b.joint) {   // one kernel for both
-        const char *name = joint_kernel(D, pad, b.dq_ks).name;
+        const char *name = joint_kernel(D, pad, b.dq_ks, b.own_delta).name;
         snprintf(out->dq_kernel, sizeof(out->dq_kernel), "%s", name);
         snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "%s", name);
     }

@@ -13,6 +13,10 @@ pytestmark = pytest.mark.gpu
     (64, 4, 12, 12, 128, 0, None, [(128, 0)], True),
     (64, 1, 8, 2, 321, 0, None, [(321, 0)], True),                                 # grouped heads, pairs that do not divide among the XCDs
     (64, 3, 16, 16, 193, (40, 300), 33, [(31, 0), (130, 31), (64, 500)], True),    # two segments, chunk tails, keys no row sees
+    (64, 2, 16, 8, 160, 5, None, [(165, 0)], True),                                # DELTA by the blocks: 2 heads x 160 rows, their most
+    (128, 1, 16, 16, 144, 0, None, [(144, 0)], True),                              # one head of 144
+    (128, 2, 8, 8, 97, 0, None, [(97, 0)], False),
+    (120, 1, 8, 8, 101, 0, None, [(101, 0)], True),
     (128, 2, 8, 8, 257, 0, None, [(257, 0)], True),                                # one row and key past two tiles
     (128, 1, 32, 8, 700, 0, None, [(700, 0)], True),                               # shared key tiles
     (128, 1, 16, 16, 500, 37, None, [(300, 0), (129, 300)], False),

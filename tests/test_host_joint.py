@@ -120,10 +120,10 @@ def test_only_with_the_flag_and_without_size_hints():
 def test_plans_of_joint_launches_hold_together():
     """Workspace, blocks and rows of random problems belong to each other; past several rounds of blocks nothing is joined."""
     rng = random.Random(1)
-    joint = 0
+    joint = own = 0
     for _ in range(400):
         n_rep, Hkv, D = rng.choice([1, 2, 4]), rng.choice([1, 4, 8, 12, 16]), rng.choice([64, 128, 96, 40])
-        B, S, n, causal = rng.choice([1, 2, 5, 16]), rng.randrange(1, 5000), rng.choice([1, 1, 3]), rng.random() < 0.7
+        B, S, n, causal = rng.choice([1, 2, 5, 16]), rng.randrange(1, rng.choice([200, 5000])), rng.choice([1, 1, 3]), rng.random() < 0.7
         chunks = [(rng.randrange(1, S + 1), i * S) for i in range(n)]
         f = L.LTR_BWD_JOINT | L.LTR_HEAD_COLS | (L.LTR_CAUSAL if causal else 0) | rng.choice([0, L.LTR_DELTA_FROM_O | L.LTR_DQ_BF16 | L.LTR_DKDV_BF16])
         a = _args(D, B, n_rep * Hkv, Hkv, S, chunks, f)
@@ -134,7 +134,13 @@ def test_plans_of_joint_launches_hold_together():
             continue
         joint += 1
         width = 64 if D <= 64 else 128
-        assert ws.plan.dq_kernel.decode() == "bwd_joint%s_kernel<%d, %d>" % ("" if D in (64, 128) else "_pad", width, 256 // ws.plan.dq_rows)
+        pad = "" if D in (64, 128) else "_pad"
+        if ws.plan.dq_kernel.startswith(b"bwd_joint_delta"):   # DELTA by the blocks themselves: few rows, one round, nothing given
+            assert ws.plan.dq_kernel.decode() == "bwd_joint_delta%s_kernel<%d>" % (pad, width) and ws.plan.dq_rows == 128
+            assert f & L.LTR_DELTA_FROM_O and S <= (320 if width == 64 else 144) and ws.plan.dq_blocks + ws.plan.dkdv_blocks <= 256
+            own += 1
+        else:
+            assert ws.plan.dq_kernel.decode() == "bwd_joint%s_kernel<%d, %d>" % (pad, width, 256 // ws.plan.dq_rows)
         assert ws.plan.dq_rows in (128, 256) and not ws.plan.dq_paired and ws.plan.dkdv_keys == 128
         assert ws.plan.dq_blocks == -(-S // ws.plan.dq_rows) * B * n_rep * Hkv
         tiles = sum(-(-(min(sk, S - p) if causal else sk) // 128) for sk, p in chunks if not causal or p < S)
@@ -143,6 +149,6 @@ def test_plans_of_joint_launches_hold_together():
         assert ws.plan.dkdv_blocks == (tiles if t > 1 else sum(-(-sk // 128) for sk, _ in chunks)) * B * Hkv * t
         if need.value:   # one byte short: no shared tiles
             assert L.load().ltr_attn_plan_ws(ctypes.byref(a), need.value - 1, ctypes.byref(ws)) == 0 and ws.blocks_per_tile == 1
-    assert joint > 100
+    assert joint > 100 and own > 3
     big = la.attn_plan(8, 32, 32, 128, 4096, [4096], [0], causal=True, joint=True)
     assert big["dq"]["kernel"] == "bwd_dq_kernel<128, 1>" and big["dkdv"]["kernel"] == "bwd_dkdv_kernel<128, 1>"
