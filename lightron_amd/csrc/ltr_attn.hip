@@ -172,12 +172,18 @@ __device__ __forceinline__ void q_pos_range(int r0, int r1, int split, int p0, i
 }
 
 // Masked tiles of the forward and dQ kernels: a key of the chunk is visible to a row up to the chunk's end and, under a causal mask, up to the
-// row's position.  The last visible one, counted from `first` (keys of the chunk; this lane's first of the tile): one compare with a constant and
-// one select per score.  (With the two comparisons per score it was six instructions, and 32 registers of the forward held the keys.)
-__device__ __forceinline__ int last_key(bool causal, int row_pos, int chunk_pos0, int chunk_keys, int first) {
+// row's position.  Which of the 32 keys from `first` on (keys of the chunk) are, as bits: a score then costs a bit-field extract and a bit-field
+// insert.  (With the two comparisons per score it was six instructions, and 32 registers of the forward held the keys; a comparison with a
+// constant and a select wait for each other through VCC.)
+__device__ __forceinline__ unsigned visible_bits(bool causal, int row_pos, int chunk_pos0, int chunk_keys, int first) {
     int last = chunk_keys - 1;
     if (causal) last = min(last, __builtin_elementwise_sub_sat(row_pos, chunk_pos0));
-    return __builtin_elementwise_sub_sat(last, first);
+    const int n = min(max(__builtin_elementwise_sub_sat(last, first), -1), 31) + 1;
+    return (unsigned)((1ull << n) - 1);
+}
+__device__ __forceinline__ float visible_score(unsigned bits, int key, float s) {   // s, or -inf
+    const unsigned keep = (unsigned)__builtin_amdgcn_sbfe((int)bits, key, 1);
+    return __uint_as_float((keep & __float_as_uint(s)) | (~keep & 0xff800000u));
 }
 
 __device__ __forceinline__ BlockItem block_item(const BlockMap &m, int pairs) { return block_item_at(m, pairs, blockIdx.x, blockIdx.y, blockIdx.z); }
@@ -795,13 +801,13 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
         const bool need_mask = (key0 + BN > sk) || (causal && (pos0 + key0 + BN - 1 > w_lo));
         if (need_mask) {
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++) {
-                const int last = last_key(causal, my_pos[rb], pos0, sk, key0 + 4 * hh);
+            for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++)
+                for (int nb = 0; nb < NB; nb++) {
+                    const unsigned bits = visible_bits(causal, my_pos[rb], pos0, sk, key0 + nb * 32 + 4 * hh);
 #pragma unroll
-                    for (int r = 0; r < 16; r++) s[nb][rb][r] = nb * 32 + 8 * (r / 4) + r % 4 <= last ? s[nb][rb][r] : -INFINITY;
-            }
+                    for (int r = 0; r < 16; r++) s[nb][rb][r] = visible_score(bits, 8 * (r / 4) + r % 4, s[nb][rb][r]);
+                }
         }
         // t = s*c2 - reference (exp2 domain), P = exp2(t) rounded to bf16, row sum of the rounded P (what PV uses)
 #pragma unroll
@@ -2638,6 +2644,7 @@ __device__ __forceinline__ void bwd_dkdv_keywave_body(const BwdParams &p, const 
                             p1 = kpos <= qpos[2 * (j & 1) + 1] ? p1 : 0.f;
                         }
                         pt.u[j] = pack2_bf16(p0, p1);
+                        asm("" : "+v"(pt.u[j]));   // or one half of the pair is rounded a second time for dS
                         ds.u[j] = bwd_ds_pair(pt.u[j], dp, j);
                     }
                 }
@@ -2992,13 +2999,17 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
         const bool have_next = c < p.n_chunks;
         if (have_next) gload(t, par ^ 1);
 
-        const bool need_mask = (key0 + BN > sk) || (causal && (pos0 + key0 + BN - 1 > w_lo));
         // 32 keys at a time, one block after the other: one live (S^T, dP^T) tile pair keeps the kernel at two
         // waves per SIMD, and the other wave's MFMAs cover this wave's softmax arithmetic.  A wave whose rows all
         // precede the tile's first key has nothing to add (see the forward kernel).
         if ((!causal || pos0 + key0 <= w_hi) && (KS == 1 || key0 < sk)) {
 #pragma unroll
         for (int nb = 0; nb < BN / 32; nb++) {
+            // with two row blocks per wave (64 rows) the rest of a diagonal or last tile is left out and whole blocks of one go without a mask: 4 x 16
+            // heads of 64, causal S=4096 211 -> 198 us; with one it is 1 - 3 % slower
+            if (RB == 2 && nb > 0 && ((causal && pos0 + key0 + nb * 32 > w_hi) || key0 + nb * 32 >= sk)) break;
+            const int mask_end = key0 + (RB == 2 ? nb * 32 + 32 : BN);
+            const bool need_mask = mask_end > sk || (causal && pos0 + mask_end - 1 > w_lo);
             f32x16 s[RB], dp[RB];
 #pragma unroll
             for (int rb = 0; rb < RB; rb++) {
@@ -3013,9 +3024,9 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
             if (need_mask) {
 #pragma unroll
                 for (int rb = 0; rb < RB; rb++) {
-                    const int last = row_ok[rb] ? last_key(causal, my_pos[rb], pos0, sk, key0 + nb * 32 + 4 * hh) : -1;
+                    const unsigned bits = row_ok[rb] ? visible_bits(causal, my_pos[rb], pos0, sk, key0 + nb * 32 + 4 * hh) : 0u;
 #pragma unroll
-                    for (int r = 0; r < 16; r++) s[rb][r] = 8 * (r / 4) + r % 4 <= last ? s[rb][r] : -INFINITY;
+                    for (int r = 0; r < 16; r++) s[rb][r] = visible_score(bits, 8 * (r / 4) + r % 4, s[rb][r]);
                 }
             }
             bf16x8 dsb[RB][2];
