@@ -278,6 +278,10 @@ __device__ __forceinline__ void tile_barrier() {
 // transfer leaves its lanes out), so the padding costs neither memory traffic nor passes over the tensors.  Measured beside
 // zero-padding q, k, v and slicing the results (B=2, 16 heads, D=96, S=777, forward + backward): 163 us with 11 pad, fill and slice
 // launches (47 us of them), 80 us without.
+// The kernels of width 128 skip the fourth block of 32 columns where the tensors end by column 96 (DC = 96 columns computed; tiles, swizzle and
+// addresses stay those of the width): a quarter of the matrix work and of the LDS reads.  Kernel us, all four blocks -> three, forward / dQ / dK/dV:
+//   2 x 16 heads of 96 S=777   18.8 / 25.6 / 31.1 -> 17.6 / 24.6 / 28.3     8 x 32 on 8 of 96 S=2048   280 / 416 / 510 -> 253 / 372 / 453
+//   6 x 8 heads of 80 S=3000    114 / 159 / 218 -> 103 / 141 / 195          1 x 32 of 72, S=1000, no mask   23.0 / 31.5 / 38.9 -> 21.5 / 29.7 / 34.7
 template <int BYTES>
 __device__ __forceinline__ void clear_lds(unsigned char *smem) {   // followed by a barrier: the fill covers the columns that transfers write
     for (int i = threadIdx.x * 16; i < BYTES; i += 512 * 16) *(uint4 *)(smem + i) = make_uint4(0, 0, 0, 0);
@@ -355,10 +359,10 @@ typedef __attribute__((address_space(3))) const i32x4 *lds_i32x4_ptr;
 // B operands from registers.  The chains alternate so no MFMA waits for its predecessor, and the operand reads
 // run PF steps ahead of the MFMAs that use them; sched_barrier pins that order (left alone, the scheduler sinks
 // each read to just before its use and the full LDS latency is exposed at every step).
-template <int D>
+template <int D, int DC = D>
 __device__ __forceinline__ void lds_gemm_pair_at(const unsigned (&addr)[D / 16], int imm_a, int imm_b,
                                                  const bf16x8 (&ba)[D / 16], const bf16x8 (&bb)[D / 16], f32x16 &ra, f32x16 &rb) {
-    constexpr int NK = D / 16, PF = 2;
+    constexpr int NK = DC / 16, PF = 2;
     bf16x8 xa[PF + 1], xb[PF + 1];
 #pragma unroll
     for (int i = 0; i < PF; i++) {
@@ -379,9 +383,9 @@ __device__ __forceinline__ void lds_gemm_pair_at(const unsigned (&addr)[D / 16],
 }
 
 // one such chain
-template <int D>
+template <int D, int DC = D>
 __device__ __forceinline__ void lds_gemm_chain_at(const unsigned (&addr)[D / 16], int imm, const bf16x8 (&b)[D / 16], f32x16 &r) {
-    constexpr int NK = D / 16, PF = 2;
+    constexpr int NK = DC / 16, PF = 2;
     bf16x8 x[PF + 1];
 #pragma unroll
     for (int i = 0; i < PF; i++) x[i] = *(lds_bf16x8_ptr)(uintptr_t)(addr[i] + imm);
@@ -397,9 +401,9 @@ __device__ __forceinline__ void lds_gemm_chain_at(const unsigned (&addr)[D / 16]
 // acc[db] (32 x 32 tiles over the head dimension) += T^T-operand x B for NKB blocks of 16 tile rows: the A operands are transpose reads of
 // the swizzled LDS tile T (rows = contraction index), the B operands b[kb] come from registers; reads run PF MFMAs ahead.
 // addr[j][h]: byte address of the lane's transpose-read element for head-dimension block j, rows +0 (h = 0) / +8 (h = 1)
-template <int D, int NKB>
+template <int D, int NKB, int DC = D>
 __device__ __forceinline__ void lds_tr_gemm_at(const unsigned (&addr)[D / 32][2], int imm, const bf16x8 (&b)[NKB], f32x16 (&acc)[D / 32]) {
-    constexpr int ND = D / 32, N = NKB * ND, PF = 3;
+    constexpr int ND = DC / 32, N = NKB * ND, PF = 3;
     auto operand = [&](int i) {
         const int off = imm + (i / ND) * 16 * D * 2;
         union {
@@ -469,10 +473,10 @@ struct NoHook {
 // read from LDS feeds one MFMA per half (b[k], r[k] / acc[k] belong to half k).  row: the lane's row of a swizzled tile, sw = the row's
 // swizzle word XOR the lane's half.  hook(step) follows the MFMAs of operand `step`: independent arithmetic of the same wave
 // written there issues while the matrix pipe works (a wave issues one instruction per ~5 clocks, an MFMA occupies the pipe for 32).
-template <int D, int KW, class Hook = NoHook>
+template <int D, int KW, int DC = D, class Hook = NoHook>
 __device__ __forceinline__ void lds_gemm_chain_kw(const __bf16 *row, int sw, const bf16x8 (&b)[KW][D / 16], f32x16 (&r)[KW],
                                                   Hook hook = Hook()) {
-    constexpr int NK = D / 16, PF = 2;
+    constexpr int NK = DC / 16, PF = 2;
     bf16x8 x[PF + 1];
 #pragma unroll
     for (int i = 0; i < PF; i++) x[i] = *(const bf16x8 *)(row + (((2 * i) ^ sw) << 3));
@@ -487,10 +491,10 @@ __device__ __forceinline__ void lds_gemm_chain_kw(const __bf16 *row, int sw, con
         __builtin_amdgcn_sched_barrier(0);
     }
 }
-template <int D, int NKB, int KW, class Hook = NoHook>
+template <int D, int NKB, int KW, int DC = D, class Hook = NoHook>
 __device__ __forceinline__ void lds_tr_gemm_kw(const __bf16 *T, int row0, int lane, const bf16x8 (&b)[KW][NKB],
                                                f32x16 (&acc)[KW][D / 32], Hook hook = Hook()) {
-    constexpr int ND = D / 32, N = NKB * ND, PF = 3;
+    constexpr int ND = DC / 32, N = NKB * ND, PF = 3;
     bf16x8 a[PF + 1];
 #pragma unroll
     for (int i = 0; i < PF && i < N; i++) a[i] = lds_operand_tr_swz<D>(T, row0 + (i / ND) * 16, (i % ND) * 32, lane);
@@ -569,7 +573,7 @@ __device__ __forceinline__ void collect_shares(unsigned char *smem, int w, int k
 // KS = waves that share a 32-row group: each takes its own BN keys of every tile of KS * BN keys, and their partial (reference, row
 // sum, O) are merged through LDS at the end.  For launches with too few query rows to give every CU a block (see FwdPlan).
 // NW = waves: eight (one block per CU, two waves per SIMD), or four with 64-key tiles (FourWaves), where several blocks share a CU.
-template <int D, int RB, int KS, bool PAD, int NW = 8, int BN = FwdTile<D, RB, KS>::BN>
+template <int D, int RB, int KS, bool PAD, int NW = 8, int BN = FwdTile<D, RB, KS>::BN, int DC = D>
 __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     const int cols = PAD ? p.cols : D;
     constexpr int RG = NW / KS, BM = 32 * RB * RG;   // the NW waves of the block share every K / V tile
@@ -630,7 +634,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
     for (int rb = 0; rb < RB; rb++) {
         const __bf16 *qp = (const __bf16 *)p.q + b * p.qs[0] + (long long)my_row[rb] * p.qs[1] + h * p.qs[2];
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++) {
+        for (int kb = 0; kb < DC / 16; kb++) {
             uint4 x = make_uint4(0, 0, 0, 0);
             if (row_ok[rb] && (!PAD || kb * 16 + 8 * hh < cols)) x = *(const uint4 *)(qp + kb * 16 + 8 * hh);
             qreg[rb][kb] = as_bf16x8(x);
@@ -641,7 +645,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
             const float *fr = p.rope + (long long)(my_pos[rb] - p.rope_pos0) * cols + 8 * hh;
             __bf16 *qr = p.q_rot && ks == 0 ? (__bf16 *)p.q_rot + b * p.qrs[0] + (long long)my_row[rb] * p.qrs[1] + h * p.qrs[2] + 8 * hh : nullptr;
 #pragma unroll
-            for (int kb = 0; kb < D / 16; kb++) {
+            for (int kb = 0; kb < DC / 16; kb++) {
                 if (PAD && kb * 16 + 8 * hh >= cols) continue;
                 qreg[rb][kb] = rope_rotate8(qreg[rb][kb], *(const f32x4 *)(fr + 16 * kb), *(const f32x4 *)(fr + 16 * kb + 4));
                 if (qr) *(bf16x8 *)(qr + 16 * kb) = qreg[rb][kb];
@@ -739,13 +743,13 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
         const unsigned lds0 = lds_address(smem) + (KS > 1 ? ks * BN * D * 2 : 0);
         const int sw = lds_swz<D>(l32) ^ hh;        // rows l32 + 32 n share the swizzle word of row l32
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++) {
+        for (int kb = 0; kb < DC / 16; kb++) {
             ka[kb] = lds0 + ((l32 * D + (((2 * kb) ^ sw) << 3)) << 1);
             asm volatile("" : "+v"(ka[kb]));
         }
         const int li = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int i = 0; i < D / 32; i++)
+        for (int i = 0; i < DC / 32; i++)
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 const int col = i * 32 + ((g & 1) << 4) + ((li & 3) << 2), row = 4 * (g >> 1) + (li >> 2) + 8 * e;
@@ -782,11 +786,11 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
             for (int nb = 0; nb + 1 < NB; nb += 2) {
                 s[nb][0] = zero16;
                 s[nb + 1][0] = zero16;
-                lds_gemm_pair_at<D>(ka, at + nb * 32 * D * 2, at + (nb + 1) * 32 * D * 2, qreg[0], qreg[0], s[nb][0], s[nb + 1][0]);
+                lds_gemm_pair_at<D, DC>(ka, at + nb * 32 * D * 2, at + (nb + 1) * 32 * D * 2, qreg[0], qreg[0], s[nb][0], s[nb + 1][0]);
             }
             if constexpr (NB == 1) {
                 s[0][0] = zero16;
-                lds_gemm_chain_at<D>(ka, at, qreg[0], s[0][0]);
+                lds_gemm_chain_at<D, DC>(ka, at, qreg[0], s[0][0]);
             }
         } else {
 #pragma unroll
@@ -863,7 +867,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
                 const float alpha = l_row > 0.f ? __builtin_amdgcn_exp2f(-shift) : 1.f;
                 l_run[rb] *= alpha;
 #pragma unroll
-                for (int i = 0; i < D / 32; i++)
+                for (int i = 0; i < DC / 32; i++)
 #pragma unroll
                     for (int r = 0; r < 16; r++) oacc[rb][i][r] *= alpha;
 #pragma unroll
@@ -881,7 +885,7 @@ __device__ __forceinline__ void fwd_bf16_body(const FwdParams &p) {
             bf16x8 pb[2 * NB];
 #pragma unroll
             for (int kb = 0; kb < 2 * NB; kb++) pb[kb] = operand_of(pt[0][kb >> 1], kb & 1);
-            lds_tr_gemm_at<D, 2 * NB>(va, at, pb, oacc[0]);   // 16 keys per MFMA
+            lds_tr_gemm_at<D, 2 * NB, DC>(va, at, pb, oacc[0]);   // 16 keys per MFMA
         } else {
             bf16x8 pb[RB][2 * NB];
 #pragma unroll
@@ -1045,7 +1049,8 @@ __global__ __launch_bounds__(512) void fwd_bf16_shares_kernel(const FwdParams p)
 }
 template <int D, int KS>   // head dims below D
 __global__ __launch_bounds__(512) void fwd_bf16_pad_kernel(const FwdParams p) {
-    fwd_bf16_body<D, 1, KS, true>(p);
+    if (D == 128 && p.cols <= 96) fwd_bf16_body<D, 1, KS, true, 8, FwdTile<D, 1, KS>::BN, D == 128 ? 96 : D>(p);   // three column blocks, see below
+    else fwd_bf16_body<D, 1, KS, true>(p);
 }
 
 // ------------------------------------------------------------------------------ forward, fp32
@@ -1948,7 +1953,7 @@ __device__ __forceinline__ void own_delta(const BwdParams &p, int b, int h_first
     }
 }
 
-template <int D, int KW, bool PAD, bool OWN_DELTA = false>
+template <int D, int KW, bool PAD, bool OWN_DELTA = false, int DC = D>
 __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockItem item) {
     const int cols = PAD ? p.cols : D;
     using L = BwdLds<D, KW>;   // KW = 32-key halves per wave
@@ -2013,7 +2018,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
         for (int k = 0; k < KW; k++) {
             const int ksafe = min(my_key[k], sk - 1);
 #pragma unroll
-            for (int kb = 0; kb < D / 16; kb++) {
+            for (int kb = 0; kb < DC / 16; kb++) {
                 uint4 x = make_uint4(0, 0, 0, 0);
                 if (!PAD || kb * 16 + 8 * hh < cols) x = *(const uint4 *)(base + (long long)ksafe * rs + kb * 16 + 8 * hh);
                 if (!key_ok[k]) x = make_uint4(0, 0, 0, 0);
@@ -2204,15 +2209,15 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
                     }
                 }
                 PackedTile ppa[KW], ppb[KW];
-                constexpr int NK = D / 16, ND = D / 32;
+                constexpr int NK = DC / 16, NS = 2 * (DC / 32);   // MFMAs of a chain, of a half of dV / dK
                 __builtin_amdgcn_s_setprio(1);
                 // every Q / dO operand read from LDS feeds the MFMAs of both halves
-                lds_gemm_chain_kw<D, KW>(Qs + l32 * D, lds_swz<D>(l32) ^ hh, kvreg, sa);
-                lds_gemm_chain_kw<D, KW>(Qs + (32 + l32) * D, lds_swz<D>(32 + l32) ^ hh, kvreg, sb, [&](int kb) {
+                lds_gemm_chain_kw<D, KW, DC>(Qs + l32 * D, lds_swz<D>(l32) ^ hh, kvreg, sa);
+                lds_gemm_chain_kw<D, KW, DC>(Qs + (32 + l32) * D, lds_swz<D>(32 + l32) ^ hh, kvreg, sb, [&](int kb) {
 #pragma unroll
                     for (int k = 0; k < KW; k++)
 #pragma unroll
-                        for (int j = kb * (8 / NK); j < (kb + 1) * (8 / NK); j++) ppa[k].u[j] = bwd_p_pair<MASK>(sa[k], j, c2, kpos[k], qa);
+                        for (int j = kb * 8 / NK; j < (kb + 1) * 8 / NK; j++) ppa[k].u[j] = bwd_p_pair<MASK>(sa[k], j, c2, kpos[k], qa);
                 });
                 bf16x8 pba[KW][2], pbb[KW][2];
 #pragma unroll
@@ -2221,11 +2226,11 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
                     pba[k][0] = operand_of(ppa[k], 0);
                     pba[k][1] = operand_of(ppa[k], 1);
                 }
-                lds_tr_gemm_kw<D, 2, KW>(dOs, 0, lane, pba, acc, [&](int step) {
+                lds_tr_gemm_kw<D, 2, KW, DC>(dOs, 0, lane, pba, acc, [&](int step) {
 #pragma unroll
                     for (int k = 0; k < KW; k++)
 #pragma unroll
-                        for (int j = step * (4 / ND); j < (step + 1) * (4 / ND); j++) ppb[k].u[j] = bwd_p_pair<MASK>(sb[k], j, c2, kpos[k], qb);
+                        for (int j = step * 8 / NS; j < (step + 1) * 8 / NS; j++) ppb[k].u[j] = bwd_p_pair<MASK>(sb[k], j, c2, kpos[k], qb);
                 });
 #pragma unroll
                 for (int k = 0; k < KW; k++) {
@@ -2233,7 +2238,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
                     pbb[k][0] = operand_of(ppb[k], 0);
                     pbb[k][1] = operand_of(ppb[k], 1);
                 }
-                lds_tr_gemm_kw<D, 2, KW>(dOs, 32, lane, pbb, acc);
+                lds_tr_gemm_kw<D, 2, KW, DC>(dOs, 32, lane, pbb, acc);
                 __builtin_amdgcn_s_setprio(0);
                 if (more) lds_store(nbuf);
                 tile_barrier();
@@ -2289,9 +2294,9 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
                         }
                 }
                 PackedTile dsa[KW], dsb[KW];
-                constexpr int NK = D / 16, ND = D / 32;
+                constexpr int NK = DC / 16, NS = 2 * (DC / 32);   // MFMAs of a chain, of a half of dV / dK
                 __builtin_amdgcn_s_setprio(1);
-                lds_gemm_chain_kw<D, KW>(dOs + l32 * D, lds_swz<D>(l32) ^ hh, kvreg, dpa);
+                lds_gemm_chain_kw<D, KW, DC>(dOs + l32 * D, lds_swz<D>(l32) ^ hh, kvreg, dpa);
                 unsigned pua[KW][8], pub[KW][8];
 #pragma unroll
                 for (int k = 0; k < KW; k++) {
@@ -2300,11 +2305,11 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
                     pua[k][0] = pa0.x; pua[k][1] = pa0.y; pua[k][2] = pa0.z; pua[k][3] = pa0.w;
                     pua[k][4] = pa1.x; pua[k][5] = pa1.y; pua[k][6] = pa1.z; pua[k][7] = pa1.w;
                 }
-                lds_gemm_chain_kw<D, KW>(dOs + (32 + l32) * D, lds_swz<D>(32 + l32) ^ hh, kvreg, dpb, [&](int kb) {
+                lds_gemm_chain_kw<D, KW, DC>(dOs + (32 + l32) * D, lds_swz<D>(32 + l32) ^ hh, kvreg, dpb, [&](int kb) {
 #pragma unroll
                     for (int k = 0; k < KW; k++)
 #pragma unroll
-                        for (int j = kb * (8 / NK); j < (kb + 1) * (8 / NK); j++) dsa[k].u[j] = bwd_ds_pair(pua[k][j], dpa[k], j);
+                        for (int j = kb * 8 / NK; j < (kb + 1) * 8 / NK; j++) dsa[k].u[j] = bwd_ds_pair(pua[k][j], dpa[k], j);
                 });
                 bf16x8 dba[KW][2], dbb[KW][2];
 #pragma unroll
@@ -2316,18 +2321,18 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams &p, const BlockIte
                     dba[k][0] = operand_of(dsa[k], 0);
                     dba[k][1] = operand_of(dsa[k], 1);
                 }
-                lds_tr_gemm_kw<D, 2, KW>(Qs, 0, lane, dba, acc, [&](int step) {
+                lds_tr_gemm_kw<D, 2, KW, DC>(Qs, 0, lane, dba, acc, [&](int step) {
 #pragma unroll
                     for (int k = 0; k < KW; k++)
 #pragma unroll
-                        for (int j = step * (4 / ND); j < (step + 1) * (4 / ND); j++) dsb[k].u[j] = bwd_ds_pair(pub[k][j], dpb[k], j);
+                        for (int j = step * 8 / NS; j < (step + 1) * 8 / NS; j++) dsb[k].u[j] = bwd_ds_pair(pub[k][j], dpb[k], j);
                 });
 #pragma unroll
                 for (int k = 0; k < KW; k++) {
                     dbb[k][0] = operand_of(dsb[k], 0);
                     dbb[k][1] = operand_of(dsb[k], 1);
                 }
-                lds_tr_gemm_kw<D, 2, KW>(Qs, 32, lane, dbb, acc);
+                lds_tr_gemm_kw<D, 2, KW, DC>(Qs, 32, lane, dbb, acc);
                 __builtin_amdgcn_s_setprio(0);
                 tile_barrier();
                 par ^= 1;
@@ -2395,7 +2400,9 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
 template <int D>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_dkdv_pad_kernel(const BwdParams p) {
     const BlockItem item = block_item(p.kv_map, p.B * p.Hkv);
-    if (item.pair < p.B * p.Hkv) bwd_dkdv_body<D, 1, true>(p, item);
+    if (item.pair >= p.B * p.Hkv) return;
+    if (D == 128 && p.cols <= 96) bwd_dkdv_body<D, 1, true, false, D == 128 ? 96 : D>(p, item);
+    else bwd_dkdv_body<D, 1, true>(p, item);
 }
 
 // dK/dV at head dim 64, one wave per 32-key slice: K and V operands (32 registers) and both accumulators (64) fit one wave, so nothing is
@@ -2763,10 +2770,10 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const BwdParams p)
 // registers as the B operand of dQ^T += K^T dS^T, whose A operand is the K tile read by transpose loads.
 // lds_gemm_pair_at / lds_tr_gemm_at for a wave that owns RB 32-row blocks: every operand read from LDS feeds one MFMA per row
 // block (ba[rb], bb[rb], ra[rb], rb_[rb] / b[rb], acc[rb] belong to row block rb).
-template <int D, int RB>
+template <int D, int RB, int DC>
 __device__ __forceinline__ void lds_gemm_pair_at_rb(const unsigned (&addr)[D / 16], int imm_a, int imm_b, const bf16x8 (&ba)[RB][D / 16],
                                                     const bf16x8 (&bb)[RB][D / 16], f32x16 (&ra)[RB], f32x16 (&rb_)[RB]) {
-    constexpr int NK = D / 16, PF = 2;
+    constexpr int NK = DC / 16, PF = 2;
     bf16x8 xa[PF + 1], xb[PF + 1];
 #pragma unroll
     for (int i = 0; i < PF; i++) {
@@ -2788,10 +2795,10 @@ __device__ __forceinline__ void lds_gemm_pair_at_rb(const unsigned (&addr)[D / 1
         __builtin_amdgcn_sched_barrier(0);
     }
 }
-template <int D, int NKB, int RB>
+template <int D, int NKB, int RB, int DC>
 __device__ __forceinline__ void lds_tr_gemm_at_rb(const unsigned (&addr)[D / 32][2], int imm, const bf16x8 (&b)[RB][NKB],
                                                   f32x16 (&acc)[RB][D / 32]) {
-    constexpr int ND = D / 32, N = NKB * ND, PF = 3;
+    constexpr int ND = DC / 32, N = NKB * ND, PF = 3;
     auto operand = [&](int i) {
         const int off = imm + (i / ND) * 16 * D * 2;
         union {
@@ -2817,7 +2824,7 @@ __device__ __forceinline__ void lds_tr_gemm_at_rb(const unsigned (&addr)[D / 32]
 }
 
 // RB = 32-row blocks per wave: a lane owns RB query rows, a block 256 * RB / KS; KS = key shares per row group as in the forward
-template <int D, int RB, int KS, bool PAD, int NW = 8, int BN = FwdTile<D, 1, KS>::BN>
+template <int D, int RB, int KS, bool PAD, int NW = 8, int BN = FwdTile<D, 1, KS>::BN, int DC = D>
 __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem item) {
     const int cols = PAD ? p.cols : D;
     constexpr int RG = NW / KS, BM = 32 * RB * RG;   // the NW waves of the block share every K / V tile
@@ -2877,7 +2884,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
         const __bf16 *qp = (const __bf16 *)p.q + b * p.qs[0] + (long long)rsafe * p.qs[1] + h * p.qs[2];
         const __bf16 *dop = (const __bf16 *)p.d_o + b * p.dos[0] + (long long)rsafe * p.dos[1] + h * p.dos[2];
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++) {
+        for (int kb = 0; kb < DC / 16; kb++) {
             if (PAD && kb * 16 + 8 * hh >= cols) {
                 qreg[rb][kb] = doreg[rb][kb] = as_bf16x8(make_uint4(0, 0, 0, 0));
                 continue;
@@ -2890,7 +2897,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
             const __bf16 *op = (const __bf16 *)p.o + b * p.os_[0] + (long long)rsafe * p.os_[1] + h * p.os_[2];
             float part = 0.f;
 #pragma unroll
-            for (int kb = 0; kb < D / 16; kb++) {
+            for (int kb = 0; kb < DC / 16; kb++) {
                 if (PAD && kb * 16 + 8 * hh >= cols) continue;
                 const bf16x8 ov = as_bf16x8(*(const uint4 *)(op + kb * 16 + 8 * hh));
 #pragma unroll
@@ -2981,10 +2988,10 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
         const unsigned lds0 = lds_address(smem) + (KS > 1 ? ks * BN * D * 2 : 0);   // the only LDS object of the kernel: aligned far beyond the buffer size
         const int sw = lds_swz<D>(l32) ^ hh;        // rows l32 + 32 n share the swizzle word of row l32
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++) pa[kb] = lds0 + ((l32 * D + (((2 * kb) ^ sw) << 3)) << 1);
+        for (int kb = 0; kb < DC / 16; kb++) pa[kb] = lds0 + ((l32 * D + (((2 * kb) ^ sw) << 3)) << 1);
         const int li = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int j = 0; j < D / 32; j++)
+        for (int j = 0; j < DC / 32; j++)
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 const int col = j * 32 + ((g & 1) << 4) + ((li & 3) << 2), row = 4 * (g >> 1) + (li >> 2) + 8 * e;
@@ -3017,7 +3024,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
                 dp[rb] = ndlt[rb];
             }
             __builtin_amdgcn_s_setprio(1);   // MFMA sections run at raised priority, see the forward kernel
-            lds_gemm_pair_at_rb<D, RB>(pa, nb * 32 * D * 2, TILE * 2 + nb * 32 * D * 2, qreg, doreg, s, dp);
+            lds_gemm_pair_at_rb<D, RB, DC>(pa, nb * 32 * D * 2, TILE * 2 + nb * 32 * D * 2, qreg, doreg, s, dp);
             __builtin_amdgcn_s_setprio(0);
             // mask fix-up (tail of the chunk, diagonal tiles, rows past the end): wave-uniform branch touching S only;
             // an invisible entry gets S = -inf, so P = 0 and dS = 0
@@ -3048,15 +3055,15 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
                 dsb[rb][1] = operand_of(ds, 1);
             }
             __builtin_amdgcn_s_setprio(1);
-            lds_tr_gemm_at_rb<D, 2, RB>(ta, nb * 32 * D * 2, dsb, dqacc);   // every K^T operand feeds one MFMA per row block
+            lds_tr_gemm_at_rb<D, 2, RB, DC>(ta, nb * 32 * D * 2, dsb, dqacc);   // every K^T operand feeds one MFMA per row block
             __builtin_amdgcn_s_setprio(0);
         }
         }
         tile_barrier();
 #pragma unroll
-        for (int kb = 0; kb < D / 16; kb++) pa[kb] ^= BUF_ELEMS * 2;
+        for (int kb = 0; kb < DC / 16; kb++) pa[kb] ^= BUF_ELEMS * 2;
 #pragma unroll
-        for (int j = 0; j < D / 32; j++) {
+        for (int j = 0; j < DC / 32; j++) {
             ta[j][0] ^= BUF_ELEMS * 2;
             ta[j][1] ^= BUF_ELEMS * 2;
         }
@@ -3147,7 +3154,9 @@ __global__ __launch_bounds__(512) void bwd_dq_shares_kernel(const BwdParams p) {
 }
 template <int D, int KS>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_dq_pad_kernel(const BwdParams p) {
-    bwd_dq_body<D, 1, KS, true>(p, block_item(p.q_map, p.B * p.Hkv));
+    const BlockItem item = block_item(p.q_map, p.B * p.Hkv);
+    if (D == 128 && p.cols <= 96) bwd_dq_body<D, 1, KS, true, 8, FwdTile<D, 1, KS>::BN, D == 128 ? 96 : D>(p, item);
+    else bwd_dq_body<D, 1, KS, true>(p, item);
 }
 
 // dQ and dK/dV blocks in one launch (LTR_BWD_JOINT).  Given DELTA, neither kind needs anything of the other; in launches of their own each ends with
@@ -3156,13 +3165,13 @@ __global__ __launch_bounds__(512) void bwd_dq_pad_kernel(const BwdParams p) {
 //   4 x 12 heads D=64 S=128   17.2 -> 12.0       2 x 16 heads D=96 S=777   57.8 -> 42.5       1 x 32 heads on 8 D=128 S=1237   94.8 -> 78
 //   1 x 16 heads D=128 S=4096  257 -> 242        1 x 12 heads D=128 S=3418  181 -> 145        3 x 8 heads D=128 S=926   61 -> 42
 // Registers are those of the dK/dV kernel, LDS the larger of both: one block per CU, as for either kind alone.
-template <int D, int KS, bool PAD, bool OWN_DELTA = false>
+template <int D, int KS, bool PAD, bool OWN_DELTA = false, int DC = D>
 __device__ __forceinline__ void bwd_joint_body(const BwdParams &p) {
     const int P = p.B * p.Hkv;
     const JointItem j = joint_item_at(p.joint, p.q_map, p.kv_map, P, blockIdx.x);
     if (j.item.pair >= P) return;
-    if (j.keys) bwd_dkdv_body<D, 1, PAD, OWN_DELTA>(p, j.item);
-    else bwd_dq_body<D, 1, KS, PAD>(p, j.item);
+    if (j.keys) bwd_dkdv_body<D, 1, PAD, OWN_DELTA, DC>(p, j.item);
+    else bwd_dq_body<D, 1, KS, PAD, 8, FwdTile<D, 1, KS>::BN, DC>(p, j.item);
 }
 template <int D, int KS>
 __global__ __launch_bounds__(512) void bwd_joint_kernel(const BwdParams p) {
@@ -3170,7 +3179,8 @@ __global__ __launch_bounds__(512) void bwd_joint_kernel(const BwdParams p) {
 }
 template <int D, int KS>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_joint_pad_kernel(const BwdParams p) {
-    bwd_joint_body<D, KS, true>(p);
+    if (D == 128 && p.cols <= 96) bwd_joint_body<D, KS, true, false, D == 128 ? 96 : D>(p);
+    else bwd_joint_body<D, KS, true>(p);
 }
 
 // the same with DELTA computed by the dK/dV blocks for themselves (own_delta), as the dQ blocks compute theirs: launches of few rows (own_delta_rows)
@@ -3180,7 +3190,8 @@ __global__ __launch_bounds__(512) void bwd_joint_delta_kernel(const BwdParams p)
 }
 template <int D>
 __global__ __launch_bounds__(512) void bwd_joint_delta_pad_kernel(const BwdParams p) {
-    bwd_joint_body<D, 2, true, true>(p);
+    if (D == 128 && p.cols <= 96) bwd_joint_body<D, 2, true, true, D == 128 ? 96 : D>(p);
+    else bwd_joint_body<D, 2, true, true>(p);
 }
 
 // ------------------------------------------------------------------------------ backward, fp32
