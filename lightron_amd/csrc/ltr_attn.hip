@@ -61,6 +61,7 @@
 #include <stdint.h>
 #include <math.h>
 #include <stdio.h>
+#include <string.h>
 #include <type_traits>
 #include <atomic>
 #include <algorithm>
@@ -4423,6 +4424,100 @@ constexpr RowCosts FWD_ROWS_64{FWD_SHARES_64, {{1.83, 6.9, 2.01, 7.2, 0.16}, {0.
 constexpr RowCosts FWD_ROWS_128{FWD_SHARES_128, {{1.52, 7.3, 1.70, 7.5, 0.26}, {1.77, 8.6, 1.98, 6.9, 0.72}, {1.03, 8.5, 1.18, 6.8, 0.44}, {1.16, 7.8, 0.92, 4.5, 0.57}, {}}};
 constexpr RowCosts DQ_ROWS_64{DQ_SHARES_64, {{2.17, 7.7, 2.61, 7.2, 0.43}, {1.26, 7.9, 1.43, 6.3, 0.54}, {1.33, 8.9, 1.69, 6.7, 0.57}, {1.04, 6.9, 0.75, 3.5, 0.59}, {1.93, 15.4, 2.51, 6.5, 0.48}}};
 constexpr RowCosts DQ_ROWS_128{DQ_SHARES_128, {{2.02, 9.5, 2.45, 6.7, 0.52}, {2.32, 10.4, 2.65, 8.5, 0.69}, {1.33, 11.3, 1.51, 9.1, 0.44}, {1.63, 8.3, 1.30, 5.4, 0.56}, {}}};
+// The blocks of a launch as classes for launch_us: neighbours that differ by less than 3 % are one class.
+struct BlockList {
+    static constexpr int MOST = 64;   // tiles looked at: all of up to 64, else 64 evenly spaced ones
+    BlockClass c[MOST];
+    int k = 0;
+    long long n = 0;
+    void add(double us, long long blocks) {
+        n += blocks;
+        if (k > 0 && std::abs(c[k - 1].us - us) < 0.03 * us) {
+            c[k - 1].us = (c[k - 1].us * c[k - 1].n + us * blocks) / (double)(c[k - 1].n + blocks);
+            c[k - 1].n += blocks;
+        } else {
+            c[k++] = {us, blocks};
+        }
+    }
+    double total_us() const {
+        double t = 0;
+        for (int i = 0; i < k; i++) t += c[i].us * c[i].n;
+        return t;
+    }
+};
+// Blocks of a forward or dQ launch, late tiles first: a block takes step_us per K / V tile and fixed_us besides, one that sees nothing 1 us.
+BlockList q_tile_blocks(RowKernel kernel, double step_us, double fixed_us, bool paired, bool causal, long long BH, int Sq, int q_split, const int *q_pos0,
+                        const ChunkDev *chunk, int n_chunks) {
+    BlockList l;
+    const int n = (Sq + kernel.rows - 1) / kernel.rows, slots = paired ? (n + 1) / 2 : n, k = causal ? std::min(slots, BlockList::MOST) : 1;
+    auto us = [&](int t) {
+        long long tiles = 0;
+        const int r0 = t * kernel.rows, r1 = std::min(Sq, r0 + kernel.rows) - 1;
+        int hi = r1 < q_split ? q_pos0[0] + r1 : q_pos0[1] + (r1 - q_split);
+        if (r0 < q_split && r1 >= q_split) hi = std::max(hi, q_pos0[0] + q_split - 1);
+        for (int c = 0; c < n_chunks; c++) {
+            const long long seen = causal ? std::min<long long>(std::max<long long>((long long)hi - chunk[c].pos0 + 1, 0), chunk[c].sk) : chunk[c].sk;
+            tiles += (seen + (1 << kernel.key_log2) - 1) >> kernel.key_log2;
+        }
+        return tiles ? tiles * step_us + fixed_us : 1.0;
+    };
+    const long long blocks = BH * slots;
+    for (int j = 0; j < k; j++) {
+        const int slot = k == slots ? j : k > 1 ? (int)((long long)j * (slots - 1) / (k - 1)) : 0, late = n - 1 - slot;
+        l.add(us(late) + (paired && slot < late ? us(slot) : 0), blocks * (j + 1) / k - blocks * j / k);
+    }
+    return l;
+}
+
+// A second look at the choice of a forward launch, by launch_us: choose_rows knows a launch by its longest and average block, which is wrong by up to 40 %
+// where whole rounds decide (a zig-zag share whose late half is one round of two shares, taken for a round and a half: 1 x 32 heads,
+// 1194 rows of 9552, D=128 194 us with four shares, 140 with two).  Constants fitted to 5500 random launches of every kernel (rms 6 - 10 %);
+// another kernel is taken where it is 6 % faster by them, but never for four waves, whose blocks share a CU better than the constants say.  Of those
+// launches a quarter change: all of them together become 3.3 % (head dim 64) and 1.5 % (128) shorter, one in a hundred loses more than 2 %.
+struct LaunchCost {
+    double step_us[N_ROW_KERNELS], fixed_us[N_ROW_KERNELS];   // four waves: of a block among others, as a share of its CU
+    double alone_us, alone_fixed_us;                          // four waves, alone on a CU
+    double paired_us, paired_fixed_us;                        // two shares in pairs
+};
+constexpr LaunchCost FWD_LAUNCH_64{{1.92, 1.125, 1.35, 0.447, 1.76}, {4.8, 5.1, 5.45, 2.5, 6.2}, 0.78, 4.7, 1.09, 4.8},
+    FWD_LAUNCH_128{{1.565, 1.84, 1.2, 0.816, 0}, {5.8, 6.5, 6.6, 4.0, 0}, 1.09, 6.2, 1.76, 6.1};
+RowChoice faster_rows(const LaunchCost &cost, RowChoice chosen, unsigned allowed, int D, bool causal, long long BH, int Sq, int q_split, const int *q_pos0,
+                      const ChunkDev *chunk, int n_chunks, int cus) {
+    // a hint; four waves; past 32 rounds nothing decides but the step
+    if ((allowed & (allowed - 1)) == 0 || chosen.kernel == FOUR_WAVES || BH * ((Sq + 255) / 256) > 32LL * cus) return chosen;
+    auto launch = [&](int i, bool shares_paired) {
+        const RowKernel k = row_kernel(i, D);
+        const int n = (Sq + k.rows - 1) / k.rows;
+        int per_cu = 1;
+        double step = shares_paired ? cost.paired_us : cost.step_us[i], fixed = shares_paired ? cost.paired_fixed_us : cost.fixed_us[i];
+        bool paired = shares_paired;
+        if (i == FOUR_WAVES) {
+            per_cu = (int)std::min<long long>(D == 64 ? FourWaves<64>::PER_CU : FourWaves<128>::PER_CU, (BH * n + cus - 1) / cus);
+            step = per_cu == 1 ? cost.alone_us : per_cu * step;
+            fixed = per_cu == 1 ? cost.alone_fixed_us : per_cu * fixed;
+        } else if (i == ROWS_256 || i == ROWS_512) {
+            paired = q_tile_slots(n, BH, causal && q_tiles_uneven(Sq, k.rows, q_split, q_pos0, chunk, n_chunks), cus) != n;
+        }
+        const BlockList l = q_tile_blocks(k, step, fixed, paired, causal, BH, Sq, q_split, q_pos0, chunk, n_chunks);
+        return launch_us(l.c, l.k, per_cu * cus);
+    };
+    const double now = launch(chosen.kernel, chosen.paired);
+    if (now < 14) return chosen;   // a call of that length waits for its host side
+    RowChoice better = chosen;
+    double best = 0.94 * now;
+    for (int i = 0; i < N_ROW_KERNELS; i++) {
+        if (!(allowed >> i & 1) || i == chosen.kernel) continue;
+        // four waves: not alone on a CU, and not for 256 rows without a mask (11 of 22 such launches 3 - 13 % slower)
+        if (i == FOUR_WAVES && (BH * ((Sq + 127) / 128) <= cus || (!causal && chosen.kernel == ROWS_256))) continue;
+        const double us = launch(i, false);
+        if (us < best && (i != FOUR_WAVES || us < 0.9 * now)) {
+            best = us;
+            better = {i, false};
+        }
+    }
+    return better;
+}
+
 // rows_256, rows_512: the caller's hints; shares: a row group's keys may be shared
 unsigned allowed_rows(bool rows_256, bool rows_512, bool shares, bool pad, int D) {
     if (rows_512) return 1u << ROWS_512;
@@ -4506,9 +4601,10 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     }
     const bool causal_ = (flags & LTR_CAUSAL) != 0;
     const int cus = device_cus();
-    const RowChoice choice = choose_rows(D == 128 ? FWD_ROWS_128 : FWD_ROWS_64,
-                                         allowed_rows(flags & LTR_FWD_ROWS_256, flags & LTR_FWD_ROWS_512, may_share, flags & LTR_HEAD_COLS, D), D, causal_,
-                                         (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk, n_chunks, cus);
+    const unsigned allowed = allowed_rows(flags & LTR_FWD_ROWS_256, flags & LTR_FWD_ROWS_512, may_share, flags & LTR_HEAD_COLS, D);
+    const RowChoice first = choose_rows(D == 128 ? FWD_ROWS_128 : FWD_ROWS_64, allowed, D, causal_, (long long)B * Hq, (long long)B * Hkv, Sq, q_split, q_pos0, chunk,
+                                        n_chunks, cus);
+    const RowChoice choice = faster_rows(D == 128 ? FWD_LAUNCH_128 : FWD_LAUNCH_64, first, allowed, D, causal_, (long long)B * Hq, Sq, q_split, q_pos0, chunk, n_chunks, cus);
     pl.wide = choice.kernel == ROWS_512;
     pl.four_waves = choice.kernel == FOUR_WAVES;
     pl.ks = choice.kernel == SHARES_2 ? 2 : choice.kernel == SHARES_4 ? 4 : 1;
@@ -4608,7 +4704,7 @@ struct BwdPlan {
     bool own_delta;           // and its dK/dV blocks compute DELTA for themselves (own_delta)
 };
 // Does a bf16 backward run its dQ and dK/dV blocks in one launch, with how many key shares per row group and blocks per key tile, and which kind
-// first?  Both ways are priced by launch_us over classes of blocks (up to 8 evenly spaced tiles stand for all): the plan as it is, one launch after
+// first?  Both ways are priced by launch_us over classes of blocks (BlockList): the plan as it is, one launch after
 // the other, and every joint one.  Constants fitted to 21000 launches of 2200 random problems (calls, ring and zig-zag ranks, single ring steps;
 // 4 - 32 heads, 45 - 5800 rows; rms error 9 - 12 %).  Of 5600 other launches that were joined, the backward takes 1 / 1.31 of the time, geometric
 // mean: 1.48 times faster where it took up to 25 us, 1.37 up to 50, 1.24 up to 100, 1.10 past 200.
@@ -4624,7 +4720,6 @@ constexpr JointCost JOINT_128{{2.13, 2.56}, {8.1, 8.5}, 1.33, 8.5, 1.68, 8.9, 2.
 constexpr KvSplitCost KEY_WAVES_64{64, 1.43, 6.7, 0.82, 3.4, 1.35, 3.5, 19e6};
 void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
                   int n_chunks, bool may_split, int cus) {
-    constexpr int CLASSES = 8;
     const JointCost &cost = D == 128 ? JOINT_128 : JOINT_64;
     const bool causal = (flags & LTR_CAUSAL) != 0;
     const long long pairs = (long long)B * Hkv, q_pairs = (long long)B * Hq;
@@ -4641,45 +4736,17 @@ void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, in
     for (int i = 0; i < n_chunks; i++) tiles_seen += seen_tiles(chunk[i].sk, chunk[i].pos0, q_last, 128);
     // few blocks only: past some hundred rounds nothing is left to gain
     if (tiles_seen == 0 || pl.kv_tiles > GRID_YZ_MAX || pairs > 8LL * GRID_YZ_MAX || pl.dq_blocks + pl.kv_blocks > 1 << 18) return;
-    struct List {
-        BlockClass c[CLASSES];
-        int k;
-        long long n;
-        double total_us() const {
-            double t = 0;
-            for (int i = 0; i < k; i++) t += c[i].us * c[i].n;
-            return t;
-        }
-    };
+    using List = BlockList;
     auto dq_blocks = [&](int rows, int key_log2, double step_us, double fixed_us, bool paired) {
-        List l;
-        const int n = (Sq + rows - 1) / rows, slots = paired ? (n + 1) / 2 : n;
-        auto us = [&](int t) {   // 1: a block that sees nothing
-            long long tiles = 0;
-            const int r0 = t * rows, r1 = std::min(Sq, r0 + rows) - 1;
-            int hi = r1 < q_split ? q_pos0[0] + r1 : q_pos0[1] + (r1 - q_split);
-            if (r0 < q_split && r1 >= q_split) hi = std::max(hi, q_pos0[0] + q_split - 1);
-            for (int c = 0; c < n_chunks; c++) {
-                const long long seen = causal ? std::min<long long>(std::max<long long>((long long)hi - chunk[c].pos0 + 1, 0), chunk[c].sk) : chunk[c].sk;
-                tiles += (seen + (1 << key_log2) - 1) >> key_log2;
-            }
-            return tiles ? tiles * step_us + fixed_us + (flags & LTR_DQ_BF16 ? 0 : cost.q_acc_us) : 1.0;
-        };
-        l.n = q_pairs * slots;
-        l.k = causal ? std::min(slots, CLASSES) : 1;
-        for (int j = 0; j < l.k; j++) {
-            const int slot = l.k > 1 ? (int)((long long)j * (slots - 1) / (l.k - 1)) : 0, late = n - 1 - slot;
-            l.c[j] = {us(late) + (paired && slot < late ? us(slot) : 0), l.n * (j + 1) / l.k - l.n * j / l.k};
-        }
-        return l;
+        return q_tile_blocks({rows, key_log2}, step_us, fixed_us + (flags & LTR_DQ_BF16 ? 0 : cost.q_acc_us), paired, causal, q_pairs, Sq, q_split, q_pos0, chunk, n_chunks);
     };
     auto kv_blocks = [&](int n_split, double step_us, double fixed_us) {
         List l;
         const long long n = n_split > 1 ? tiles_seen : pl.kv_tiles;
-        l.n = pairs * n * n_split;
-        l.k = causal ? (int)std::min<long long>(n, CLASSES) : 1;
-        for (int j = 0; j < l.k; j++) {
-            long long t = l.k > 1 ? j * (n - 1) / (l.k - 1) : 0;
+        const long long blocks = pairs * n * n_split;
+        const int k = causal ? (int)std::min<long long>(n, List::MOST) : 1;
+        for (int j = 0; j < k; j++) {
+            long long t = k == n ? j : k > 1 ? j * (n - 1) / (k - 1) : 0;
             int i = 0;
             for (; i < n_chunks - 1; i++) {
                 const int in_chunk = seen_tiles(chunk[order[i]].sk, chunk[order[i]].pos0, n_split > 1 ? q_last : 0x7fffffff, 128);
@@ -4692,12 +4759,12 @@ void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, in
                 rows = std::min<long long>(std::max<long long>(q_pos0[0] + (long long)q_split - kpos, 0), q_split) +
                        std::min<long long>(std::max<long long>(q_pos0[1] + (long long)(Sq - q_split) - kpos, 0), Sq - q_split);
             const long long steps = ((rows + 63) / 64 * (Hq / Hkv) + n_split - 1) / n_split;
-            l.c[j] = {rows > 0 ? steps * step_us + fixed_us + (n_split > 1 || (flags & LTR_DKDV_BF16) ? 0 : cost.kv_acc_us) : 1.0, l.n * (j + 1) / l.k - l.n * j / l.k};
+            l.add(rows > 0 ? steps * step_us + fixed_us + (n_split > 1 || (flags & LTR_DKDV_BF16) ? 0 : cost.kv_acc_us) : 1.0, blocks * (j + 1) / k - blocks * j / k);
         }
         return l;
     };
     auto both_us = [&](const List &first, const List &second) {
-        BlockClass c[2 * CLASSES];
+        BlockClass c[2 * List::MOST];
         std::copy(first.c, first.c + first.k, c);
         std::copy(second.c, second.c + second.k, c + first.k);
         return launch_us(c, first.k + second.k, cus);
@@ -4774,8 +4841,8 @@ void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, in
     pl.split = {best_n, 1, best_n > 1 ? q_last : 0x7fffffff, best_n > 1 ? tiles_seen : pl.kv_tiles, 0};
     while (pl.split.reps * 2 <= best_n && Hq / Hkv % (pl.split.reps * 2) == 0) pl.split.reps *= 2;
 }
-BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
-                 int n_chunks, bool may_split = false) {
+BwdPlan make_bwd_plan(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
+                      int n_chunks, bool may_split) {
     BwdPlan pl;
     pl.f32_ks = 0;
     pl.split = KvSplit{1, 1, 0x7fffffff, 0, 0};
@@ -4878,6 +4945,31 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.kv_group = pair_group(pairs, (pl.split.n > 1 ? pl.split.tiles : pl.kv_tiles) * pl.split.n, pl.key_waves ? 2 * slots : slots,
                              causal_ && key_tiles_uneven(Sq, pl.keys_per_block, q_split, q_pos0, chunk, n_chunks));
     return pl;
+}
+// The plan of a problem, a function of these numbers alone.  One with LTR_BWD_JOINT prices up to 20 launches (2 - 6 us) and is asked for twice by a
+// backward, for its workspace and for its launch: a thread keeps the last one.
+BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
+                 int n_chunks, bool may_split = false) {
+    if (!(flags & LTR_BWD_JOINT) || f32) return make_bwd_plan(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split);
+    struct Problem {
+        int head[12];
+        int keys[LTR_MAX_CHUNKS][2];
+    };
+    static thread_local Problem last{};   // no problem has 0 chunks
+    static thread_local BwdPlan plan;
+    Problem now;
+    const int head[12] = {n_chunks, D, (int)flags, B, Hq, Hkv, Sq, q_split, q_pos0[0], q_pos0[1], may_split, device_cus()};
+    std::copy(head, head + 12, now.head);
+    for (int c = 0; c < n_chunks; c++) {
+        now.keys[c][0] = chunk[c].sk;
+        now.keys[c][1] = chunk[c].pos0;
+    }
+    const size_t used = sizeof(now.head) + n_chunks * sizeof(now.keys[0]);
+    if (memcmp(&now, &last, used) != 0) {
+        plan = make_bwd_plan(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split);
+        memcpy(&last, &now, used);
+    }
+    return plan;
 }
 // The plan with a workspace of that many bytes: shared key tiles if their partial sums fit, else the launch without a workspace (whose kernel
 // and block order are other ones than those chosen for sharing).

@@ -6,6 +6,7 @@ import os
 import random
 import shutil
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 import torch
@@ -152,3 +153,26 @@ def test_plans_of_joint_launches_hold_together():
     assert joint > 100 and own > 3
     big = la.attn_plan(8, 32, 32, 128, 4096, [4096], [0], causal=True, joint=True)
     assert big["dq"]["kernel"] == "bwd_dq_kernel<128, 1>" and big["dkdv"]["kernel"] == "bwd_dkdv_kernel<128, 1>"
+
+
+def test_the_plan_kept_is_that_of_the_problem():
+    """A thread keeps its last plan: problems that differ in one number each, asked for in turn, in both orders and on several threads."""
+    base = dict(B=2, Hq=16, Hkv=4, D=128, Sq=700, chunks=[(700, 0), (300, 700)], flags=L.LTR_BWD_JOINT | L.LTR_CAUSAL | L.LTR_HEAD_COLS)
+    variants = [base] + [dict(base, **kw) for kw in (dict(B=3), dict(Hq=8), dict(Hkv=16), dict(D=96), dict(Sq=900), dict(chunks=[(700, 0)]),
+                                                     dict(chunks=[(700, 0), (301, 700)]), dict(chunks=[(700, 0), (300, 600)]),
+                                                     dict(flags=base["flags"] & ~L.LTR_CAUSAL), dict(flags=base["flags"] | L.LTR_DELTA_FROM_O))]
+
+    def ask(v):
+        a, need, ws = _args(**v), ctypes.c_int64(0), L.AttnPlanWs()
+        assert L.load().ltr_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(need)) == 0
+        assert L.load().ltr_attn_plan_ws(ctypes.byref(a), need.value, ctypes.byref(ws)) == 0
+        p = ws.plan
+        return need.value, ws.blocks_per_tile, p.dq_kernel, p.dkdv_kernel, p.dq_blocks, p.dkdv_blocks, p.dq_rows
+
+    alone = [ask(v) for v in variants]
+    assert len(set(alone)) > 6
+    for order in (range(len(variants)), reversed(range(len(variants)))):
+        for i in order:
+            assert ask(variants[i]) == alone[i] == ask(variants[i])
+    with ThreadPoolExecutor(4) as pool:
+        assert list(pool.map(ask, variants * 20)) == alone * 20
