@@ -80,12 +80,11 @@ extern "C" {
 
 #define LTR_DQ_F32_RESULT 262144u /* backward, fp32: dq RECEIVES dQ of this call (no accumulation) and delta is computed from the fp32 o by the
                                     dQ kernel: LTR_DQ_BF16 | LTR_DELTA_FROM_O for fp32.  LTR_EUNSUP with bf16 or LTR_BWD_F32_SCALAR */
+#define LTR_BWD_JOINT 524288u /* backward: dQ and dK/dV blocks may run side by side in one launch, where the library finds that faster (bf16; DELTA comes
+                                    from a launch of its own before it, or in launches of few rows from the blocks that use it); no output
+                                    may overlap an input.  Without the flag the dQ kernel has ended before the dK/dV kernel starts */
 
 /* error codes */
-#define LTR_BWD_JOINT 524288u /* backward: dQ and dK/dV blocks may run side by side in one launch, where the library finds that faster (bf16; DELTA then
-                                  comes from a launch of its own before it); no output may overlap an input.  Without the flag the dQ kernel has
-                                  ended before the dK/dV kernel starts */
-
 #define LTR_OK 0
 #define LTR_EINVAL (-1)   /* null pointer, bad size, bad flag */
 #define LTR_EUNSUP (-2)   /* unsupported head dim / dtype combination */
@@ -321,7 +320,8 @@ int ltr_copy_strided(const ltr_copy_args *args, void *stream);
  * behind F.scaled_dot_product_attention, model/model.py:193); it is for benchmarks and profiles that must name the kernel
  * they measured, and for tests of the size hints.  The sizes, strides' owner shapes, positions, chunk lengths, dtype and
  * flags of args are read; flags may also carry the forward's hints (LTR_FWD_ROWS_256 / LTR_FWD_ROWS_512 / LTR_FWD_F32_SCALAR) and
- * LTR_HEAD_COLS.  With LTR_BWD_JOINT dq_kernel and dkdv_kernel are the same name where one launch holds the blocks of both.  The library's launches and this answer come from one function, so they cannot drift apart (a forward that
+ * LTR_HEAD_COLS.  With LTR_BWD_JOINT dq_kernel and dkdv_kernel are the same name where one launch holds the blocks of both.
+ * The library's launches and this answer come from one function, so they cannot drift apart (a forward that
  * rotates q in place, see q_rot, takes one wave per row group where the plan may name key shares).  Kernel names are those a
  * profiler shows.  ltr_attn_plan_ws is the plan of ltr_attn_fwd and of ltr_attn_bwd_ws with a workspace of workspace_bytes: dkdv_blocks
  * then counts the blocks that share key tiles, and the kernel that sums their partial results is named beside them.

@@ -42,6 +42,8 @@
 //                        bitwise reproducible.  bwd_dq_kernel<64, 2>: two 32-row blocks per wave (a lane owns two
 //                        query rows): every K / V operand read from LDS feeds two MFMAs; head dim 64 only, chosen by the
 //                        host when the wider blocks still fill the device (or forced with LTR_DQ_ROWS_512).
+//   bwd_joint_kernel<D, KS>  the blocks of bwd_dq_kernel (KS = 2: of two key shares) and of bwd_dkdv_kernel<D, 1> in one launch, where
+//                        they are few (LTR_BWD_JOINT); bwd_joint_delta_kernel<D>: with DELTA by the blocks themselves.
 //   bwd_dq_f32_mfma_kernel<D, KS>, bwd_dkdv_f32_mfma_kernel<D>
 //                        the fp32 backward on v_mfma_f32_32x32x2_f32 (see there).
 //   bwd_dq_f32_kernel<D>, bwd_dkdv_f32_kernel<D, DV>
@@ -4472,8 +4474,9 @@ BlockList q_tile_blocks(RowKernel kernel, double step_us, double fixed_us, bool 
 // A second look at the choice of a forward launch, by launch_us: choose_rows knows a launch by its longest and average block, which is wrong by up to 40 %
 // where whole rounds decide (a zig-zag share whose late half is one round of two shares, taken for a round and a half: 1 x 32 heads,
 // 1194 rows of 9552, D=128 194 us with four shares, 140 with two).  Constants fitted to 5500 random launches of every kernel (rms 6 - 10 %);
-// another kernel is taken where it is 6 % faster by them, but never for four waves, whose blocks share a CU better than the constants say.  Of those
-// launches a quarter change: all of them together become 3.3 % (head dim 64) and 1.5 % (128) shorter, one in a hundred loses more than 2 %.
+// another kernel is taken where it is 6 % faster by them (four waves: 10 %), but none in place of four waves, whose blocks share a CU better
+// than they say.  Of those launches a quarter change: all of them together become 3.3 % (head dim 64) and 1.5 % (128) shorter, one in a
+// hundred loses more than 2 %.
 struct LaunchCost {
     double step_us[N_ROW_KERNELS], fixed_us[N_ROW_KERNELS];   // four waves: of a block among others, as a share of its CU
     double alone_us, alone_fixed_us;                          // four waves, alone on a CU
@@ -4580,8 +4583,53 @@ KernelChoice joint_kernel(int D, bool pad, int ks, bool own_delta) {
 }
 #undef LTR_KERNEL
 
-FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
-                 int n_chunks, bool may_share = true) {
+// What a bf16 plan depends on, and the plans that a thread keeps: pricing launches takes 1 - 10 us, as long as queueing them, and a program asks for the
+// same few problems again and again (layers, steps, the ranks of a ring).  32 pairs of places by a hash of the sizes, nothing of a tensor among them;
+// a new problem takes the place of its pair that was not used last.
+struct Problem {
+    int head[12];
+    int keys[LTR_MAX_CHUNKS][2];
+    size_t used;   // bytes of the above
+    Problem() : head{}, used(0) {}   // no problem has 0 chunks
+    Problem(int D, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks, bool may)
+        : head{n_chunks, D, (int)flags, B, Hq, Hkv, Sq, q_split, q_pos0[0], q_pos0[1], may, device_cus()}, used(sizeof(head) + n_chunks * sizeof(keys[0])) {
+        for (int c = 0; c < n_chunks; c++) {
+            keys[c][0] = chunk[c].sk;
+            keys[c][1] = chunk[c].pos0;
+        }
+    }
+    bool operator==(const Problem &o) const { return head[0] == o.head[0] && memcmp(this, &o, used) == 0; }
+    unsigned hash() const {
+        uint64_t h = 0;
+        for (int i : head) h = (h ^ (unsigned)i) * 0x9e3779b97f4a7c15ull, h ^= h >> 29;
+        for (int c = 0; c < head[0]; c++)
+            for (int i : keys[c]) h = (h ^ (unsigned)i) * 0x9e3779b97f4a7c15ull, h ^= h >> 29;
+        return (unsigned)(h >> 32) % 32;
+    }
+};
+template <class Plan>
+struct KeptPlans {
+    Problem problem[32][2];
+    Plan plan[32][2];
+    unsigned char used_last[32] = {};
+    template <class Make>
+    Plan get(const Problem &now, Make make) {
+        const unsigned h = now.hash();
+        unsigned i = used_last[h];
+        if (!(problem[h][i] == now)) {
+            i ^= 1;
+            if (!(problem[h][i] == now)) {
+                plan[h][i] = make();
+                problem[h][i] = now;
+            }
+            used_last[h] = i;
+        }
+        return plan[h][i];
+    }
+};
+
+FwdPlan make_fwd_plan(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
+                      int n_chunks, bool may_share) {
     FwdPlan pl;
     pl.f32_ks = 0;
     pl.ks = 1;
@@ -4616,6 +4664,13 @@ FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     pl.group = pair_group((long long)B * Hkv, (long long)pl.n_slots * (Hq / Hkv), cus / 8 * (pl.four_waves ? D == 64 ? FourWaves<64>::PER_CU : FourWaves<128>::PER_CU : 1),
                           uneven && pl.n_slots == pl.n_qtiles);   // paired tiles are equal blocks
     return pl;
+}
+FwdPlan plan_fwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
+                 int n_chunks, bool may_share = true) {
+    auto make = [&] { return make_fwd_plan(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_share); };
+    if (f32) return make();
+    static thread_local KeptPlans<FwdPlan> kept;
+    return kept.get(Problem(D, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_share), make);
 }
 
 // Blocks that share one key tile of the dK/dV kernel.  A launch with fewer key tiles than the device has CUs (few kv heads, a
@@ -4946,30 +5001,14 @@ BwdPlan make_bwd_plan(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, i
                              causal_ && key_tiles_uneven(Sq, pl.keys_per_block, q_split, q_pos0, chunk, n_chunks));
     return pl;
 }
-// The plan of a problem, a function of these numbers alone.  One with LTR_BWD_JOINT prices up to 20 launches (2 - 6 us) and is asked for twice by a
-// backward, for its workspace and for its launch: a thread keeps the last one.
+// The plan of a problem.  One with LTR_BWD_JOINT prices up to 20 launches (1 - 10 us), and a backward asks with a workspace in mind and, where that
+// plan needs none, once more without.
 BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
                  int n_chunks, bool may_split = false) {
-    if (!(flags & LTR_BWD_JOINT) || f32) return make_bwd_plan(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split);
-    struct Problem {
-        int head[12];
-        int keys[LTR_MAX_CHUNKS][2];
-    };
-    static thread_local Problem last{};   // no problem has 0 chunks
-    static thread_local BwdPlan plan;
-    Problem now;
-    const int head[12] = {n_chunks, D, (int)flags, B, Hq, Hkv, Sq, q_split, q_pos0[0], q_pos0[1], may_split, device_cus()};
-    std::copy(head, head + 12, now.head);
-    for (int c = 0; c < n_chunks; c++) {
-        now.keys[c][0] = chunk[c].sk;
-        now.keys[c][1] = chunk[c].pos0;
-    }
-    const size_t used = sizeof(now.head) + n_chunks * sizeof(now.keys[0]);
-    if (memcmp(&now, &last, used) != 0) {
-        plan = make_bwd_plan(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split);
-        memcpy(&last, &now, used);
-    }
-    return plan;
+    auto make = [&] { return make_bwd_plan(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split); };
+    if (!(flags & LTR_BWD_JOINT) || f32) return make();
+    static thread_local KeptPlans<BwdPlan> kept;
+    return kept.get(Problem(D, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split), make);
 }
 // The plan with a workspace of that many bytes: shared key tiles if their partial sums fit, else the launch without a workspace (whose kernel
 // and block order are other ones than those chosen for sharing).

@@ -156,7 +156,8 @@ def test_plans_of_joint_launches_hold_together():
 
 
 def test_the_plan_kept_is_that_of_the_problem():
-    """A thread keeps its last plan: problems that differ in one number each, asked for in turn, in both orders and on several threads."""
+    """A thread keeps plans: problems that differ in one number each, asked for in turn, in both orders and on several threads, and more of them
+    than places."""
     base = dict(B=2, Hq=16, Hkv=4, D=128, Sq=700, chunks=[(700, 0), (300, 700)], flags=L.LTR_BWD_JOINT | L.LTR_CAUSAL | L.LTR_HEAD_COLS)
     variants = [base] + [dict(base, **kw) for kw in (dict(B=3), dict(Hq=8), dict(Hkv=16), dict(D=96), dict(Sq=900), dict(chunks=[(700, 0)]),
                                                      dict(chunks=[(700, 0), (301, 700)]), dict(chunks=[(700, 0), (300, 600)]),
@@ -167,7 +168,7 @@ def test_the_plan_kept_is_that_of_the_problem():
         assert L.load().ltr_attn_bwd_workspace(ctypes.byref(a), ctypes.byref(need)) == 0
         assert L.load().ltr_attn_plan_ws(ctypes.byref(a), need.value, ctypes.byref(ws)) == 0
         p = ws.plan
-        return need.value, ws.blocks_per_tile, p.dq_kernel, p.dkdv_kernel, p.dq_blocks, p.dkdv_blocks, p.dq_rows
+        return need.value, ws.blocks_per_tile, p.dq_kernel, p.dkdv_kernel, p.dq_blocks, p.dkdv_blocks, p.dq_rows, p.fwd_rows, p.fwd_blocks, p.fwd_kernel
 
     alone = [ask(v) for v in variants]
     assert len(set(alone)) > 6
@@ -176,3 +177,11 @@ def test_the_plan_kept_is_that_of_the_problem():
             assert ask(variants[i]) == alone[i] == ask(variants[i])
     with ThreadPoolExecutor(4) as pool:
         assert list(pool.map(ask, variants * 20)) == alone * 20
+    many = [dict(base, Sq=S, chunks=[(S, 0)]) for S in range(130, 130 * 121, 130)]   # one key tile more each
+
+    def ask_anew(v):   # on a thread of its own, which keeps nothing yet
+        with ThreadPoolExecutor(1) as one:
+            return one.submit(ask, v).result()
+
+    new = [ask_anew(v) for v in many]
+    assert len(set(new)) == len(many) and [ask(v) for v in many] == new == [ask(v) for v in many]
