@@ -42,3 +42,18 @@ def test_delta_error_is_that_of_sixteen_sums(ltr, D):
     a.chunk[0].k, a.chunk[0].v, a.chunk[0].sk = k.data_ptr(), v.data_ptr(), S
     L.check(L.load().ltr_attn_bwd(ctypes.byref(a), torch.cuda.current_stream().cuda_stream), "ltr_attn_bwd")
     assert rms(delta) <= bound
+
+
+@pytest.mark.parametrize("D", [8, 40, 64, 72, 128])
+@pytest.mark.parametrize("B,S,H", [(1, 1, 1), (2, 31, 1), (1, 33, 3), (3, 65, 5)])   # rows on both sides of a block's 32 or 64
+def test_delta_of_aligned_bf16_is_that_of_the_general_kernel(ltr, D, B, S, H):
+    g = torch.Generator(device="cuda").manual_seed(D + S)
+    wide = torch.randn(2, B, S, H + 1, D, device="cuda", generator=g).to(torch.bfloat16)
+    o, do = wide[0, :, :, 1:], wide[1, :, :, :H]              # strides of their own
+    shifted = torch.empty(o.numel() + 1, device="cuda", dtype=torch.bfloat16)[1:].view(o.shape)   # 2 bytes off: the general kernel
+    shifted.copy_(o)
+    got = ltr.attn_delta(o, do)
+    assert torch.equal(got, ltr.attn_delta(shifted, do))
+    want = (o.double() * do.double()).sum(-1).transpose(1, 2)
+    bound = D * 2.0 ** -24 * (o.double() * do.double()).abs().sum(-1).transpose(1, 2)   # D roundings of fp32, each of at most the sum of sizes
+    assert ((got.double() - want).abs() <= bound).all()
