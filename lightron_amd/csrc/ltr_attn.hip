@@ -65,6 +65,7 @@
 #include <stdio.h>
 #include <string.h>
 #include <type_traits>
+#include <optional>
 #include <atomic>
 #include <algorithm>
 #include "ltr_attn.h"
@@ -4480,10 +4481,29 @@ struct BlockList {
             c[k++] = {us, blocks};
         }
     }
+    // the least that the launch can take: its blocks spread evenly, or the longest of them
+    double least_us(int slots) const { return std::max(total_us() / slots, longest_us()); }
     double total_us() const {
         double t = 0;
         for (int i = 0; i < k; i++) t += c[i].us * c[i].n;
         return t;
+    }
+    double longest_us() const {
+        double t = 0;
+        for (int i = 0; i < k; i++) t = std::max(t, c[i].us);
+        return t;
+    }
+};
+// 0, then n / d more each time, in whole numbers: floor(j n / d) for j = 0, 1, 2 ... with one division in all
+struct EvenSteps {
+    long long at = 0, whole, rest, d, over = 0;
+    EvenSteps(long long n, long long d_) : whole(d_ > 0 ? n / d_ : 0), rest(d_ > 0 ? n - whole * d_ : 0), d(d_) {}
+    long long next() {   // by how much it grew
+        over += rest;
+        const long long grew = whole + (over >= d);
+        if (over >= d) over -= d;
+        at += grew;
+        return grew;
     }
 };
 // Blocks of a forward or dQ launch, late tiles first: a block takes step_us per K / V tile and fixed_us besides, one that sees nothing 1 us.
@@ -4502,10 +4522,10 @@ BlockList q_tile_blocks(RowKernel kernel, double step_us, double fixed_us, bool 
         }
         return tiles ? tiles * step_us + fixed_us : 1.0;
     };
-    const long long blocks = BH * slots;
-    for (int j = 0; j < k; j++) {
-        const int slot = k == slots ? j : k > 1 ? (int)((long long)j * (slots - 1) / (k - 1)) : 0, late = n - 1 - slot;
-        l.add(us(late) + (paired && slot < late ? us(slot) : 0), blocks * (j + 1) / k - blocks * j / k);
+    EvenSteps blocks(BH * slots, k), tile(slots - 1, k - 1);
+    for (int j = 0; j < k; j++, tile.next()) {
+        const int slot = (int)tile.at, late = n - 1 - slot;
+        l.add(us(late) + (paired && slot < late ? us(slot) : 0), blocks.next());
     }
     return l;
 }
@@ -4527,7 +4547,7 @@ RowChoice faster_rows(const LaunchCost &cost, RowChoice chosen, unsigned allowed
                       const ChunkDev *chunk, int n_chunks, int cus) {
     // a hint; four waves; past 32 rounds nothing decides but the step
     if ((allowed & (allowed - 1)) == 0 || chosen.kernel == FOUR_WAVES || BH * ((Sq + 255) / 256) > 32LL * cus) return chosen;
-    auto launch = [&](int i, bool shares_paired) {
+    auto launch = [&](int i, bool shares_paired, double most) {   // `most` or more is not worth a closer look
         const RowKernel k = row_kernel(i, D);
         const int n = (Sq + k.rows - 1) / k.rows;
         int per_cu = 1;
@@ -4541,9 +4561,11 @@ RowChoice faster_rows(const LaunchCost &cost, RowChoice chosen, unsigned allowed
             paired = q_tile_slots(n, BH, causal && q_tiles_uneven(Sq, k.rows, q_split, q_pos0, chunk, n_chunks), cus) != n;
         }
         const BlockList l = q_tile_blocks(k, step, fixed, paired, causal, BH, Sq, q_split, q_pos0, chunk, n_chunks);
-        return launch_us(l.c, l.k, per_cu * cus);
+        if (l.least_us(per_cu * cus) >= most) return most;
+        Dispatch d(per_cu * cus);
+        return d.add(l.c, l.k, most) ? d.end : most;
     };
-    const double now = launch(chosen.kernel, chosen.paired);
+    const double now = launch(chosen.kernel, chosen.paired, 1e30);
     if (now < 14) return chosen;   // a call of that length waits for its host side
     RowChoice better = chosen;
     double best = 0.94 * now;
@@ -4551,7 +4573,7 @@ RowChoice faster_rows(const LaunchCost &cost, RowChoice chosen, unsigned allowed
         if (!(allowed >> i & 1) || i == chosen.kernel) continue;
         // four waves: not alone on a CU, and not for 256 rows without a mask (11 of 22 such launches 3 - 13 % slower)
         if (i == FOUR_WAVES && (BH * ((Sq + 127) / 128) <= cus || (!causal && chosen.kernel == ROWS_256))) continue;
-        const double us = launch(i, false);
+        const double us = launch(i, false, best);
         if (us < best && (i != FOUR_WAVES || us < 0.9 * now)) {
             best = us;
             better = {i, false};
@@ -4812,11 +4834,14 @@ struct JointCost {
 constexpr JointCost JOINT_128{{2.13, 2.56}, {8.1, 8.5}, 1.33, 8.5, 1.68, 8.9, 2.8, 2.4, 1.4, 2.0, 3.3e6, 5.2, 18e6},
     JOINT_64{{2.90, 1.35}, {4.6, 5.7}, 1.33, 6.5, 0.99, 5.8, 1.0, 2.3, 3.3, 1.8, 2.7e6, 4.6, 23e6};
 constexpr KvSplitCost KEY_WAVES_64{64, 1.43, 6.7, 0.82, 3.4, 1.35, 3.5, 19e6};
-void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
+// pl: the launches apart; alone: those that share no key tiles, which a joint launch that shares none has to be faster than as well (it is also the plan
+// of a call without a workspace)
+void joint_launch(BwdPlan &pl, const BwdPlan &alone, int D, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
                   int n_chunks, bool may_split, int cus) {
     const JointCost &cost = D == 128 ? JOINT_128 : JOINT_64;
     const bool causal = (flags & LTR_CAUSAL) != 0;
     const long long pairs = (long long)B * Hkv, q_pairs = (long long)B * Hq;
+    const int n_rep = Hq / Hkv;
     // key tiles by position, as the launch sorts them
     int order[LTR_MAX_CHUNKS];
     for (int i = 0; i < n_chunks; i++) {
@@ -4834,86 +4859,109 @@ void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, in
     auto dq_blocks = [&](int rows, int key_log2, double step_us, double fixed_us, bool paired) {
         return q_tile_blocks({rows, key_log2}, step_us, fixed_us + (flags & LTR_DQ_BF16 ? 0 : cost.q_acc_us), paired, causal, q_pairs, Sq, q_split, q_pos0, chunk, n_chunks);
     };
-    auto kv_blocks = [&](int n_split, double step_us, double fixed_us) {
-        List l;
-        const long long n = n_split > 1 ? tiles_seen : pl.kv_tiles;
-        const long long blocks = pairs * n * n_split;
-        const int k = causal ? (int)std::min<long long>(n, List::MOST) : 1;
-        for (int j = 0; j < k; j++) {
-            long long t = k == n ? j : k > 1 ? j * (n - 1) / (k - 1) : 0;
-            int i = 0;
-            for (; i < n_chunks - 1; i++) {
-                const int in_chunk = seen_tiles(chunk[order[i]].sk, chunk[order[i]].pos0, n_split > 1 ? q_last : 0x7fffffff, 128);
-                if (t < in_chunk) break;
-                t -= in_chunk;
+    // rows that see each of the key tiles looked at, tiles by position: of all tiles, and of those that some row sees (the launches that share)
+    struct KeyTiles {
+        long long n = 0;
+        int k = 0;
+        int rows[List::MOST];
+    } key_tiles[2];
+    auto look_at = [&](KeyTiles &t, long long n, int last) {
+        t.n = n;
+        t.k = causal ? (int)std::min<long long>(n, List::MOST) : 1;
+        EvenSteps tile(n - 1, t.k - 1);
+        long long before = 0;   // tiles of the chunks before chunk i
+        int i = 0, in_chunk = seen_tiles(chunk[order[0]].sk, chunk[order[0]].pos0, last, 128);
+        for (int j = 0; j < t.k; j++, tile.next()) {
+            while (i < n_chunks - 1 && tile.at - before >= in_chunk) {
+                before += in_chunk;
+                i++;
+                in_chunk = seen_tiles(chunk[order[i]].sk, chunk[order[i]].pos0, last, 128);
             }
             long long rows = Sq;
-            const long long kpos = chunk[order[i]].pos0 + t * 128;
+            const long long kpos = chunk[order[i]].pos0 + (tile.at - before) * 128;
             if (causal)
                 rows = std::min<long long>(std::max<long long>(q_pos0[0] + (long long)q_split - kpos, 0), q_split) +
                        std::min<long long>(std::max<long long>(q_pos0[1] + (long long)(Sq - q_split) - kpos, 0), Sq - q_split);
-            const long long steps = ((rows + 63) / 64 * (Hq / Hkv) + n_split - 1) / n_split;
-            l.add(rows > 0 ? steps * step_us + fixed_us + (n_split > 1 || (flags & LTR_DKDV_BF16) ? 0 : cost.kv_acc_us) : 1.0, blocks * (j + 1) / k - blocks * j / k);
+            t.rows[j] = (int)rows;
+        }
+    };
+    auto kv_blocks = [&](int n_split, double step_us, double fixed_us) {   // n_split: a power of two
+        KeyTiles &t = key_tiles[n_split > 1];
+        if (t.k == 0) look_at(t, n_split > 1 ? tiles_seen : pl.kv_tiles, n_split > 1 ? q_last : 0x7fffffff);
+        List l;
+        const double acc_us = n_split > 1 || (flags & LTR_DKDV_BF16) ? 0 : cost.kv_acc_us;
+        EvenSteps blocks(pairs * t.n * n_split, t.k);
+        for (int j = 0; j < t.k; j++) {
+            const long long steps = ((t.rows[j] + 63LL) / 64 * n_rep + n_split - 1) >> __builtin_ctz(n_split);
+            l.add(t.rows[j] > 0 ? steps * step_us + fixed_us + acc_us : 1.0, blocks.next());
         }
         return l;
     };
-    auto both_us = [&](const List &first, const List &second) {
-        BlockClass c[2 * List::MOST];
-        std::copy(first.c, first.c + first.k, c);
-        std::copy(second.c, second.c + second.k, c + first.k);
-        return launch_us(c, first.k + second.k, cus);
-    };
     auto reduce_us = [&](int n_split) { return n_split > 1 ? cost.reduce_us + (double)pl.kv_tiles * pairs * n_split * 128 * D * 8 / cost.reduce_bytes_per_us : 0.0; };
 
-    // the plan as it is
-    double apart = 2 * cost.launch_us + reduce_us(pl.split.n);
-    if (pl.dq_four_waves) {
-        const TileCost &c = (D == 128 ? DQ_ROWS_128 : DQ_ROWS_64).kernel[FOUR_WAVES];
-        const int per_cu = (int)std::min<long long>(D == 128 ? FourWaves<128>::PER_CU : FourWaves<64>::PER_CU, (pl.dq_blocks + cus - 1) / cus);
-        const List l = dq_blocks(128, 6, per_cu == 1 ? c.alone_us : per_cu * c.step_us, per_cu == 1 ? c.alone_fixed_us : per_cu * c.fixed_us, false);
-        apart += launch_us(l.c, l.k, per_cu * cus);
-    } else {
-        const int i = pl.dq_ks == 4 ? SHARES_4 : pl.dq_ks == 2 ? SHARES_2 : ROWS_256;
-        const RowKernel k = row_kernel(i, D);
-        const List l = dq_blocks(k.rows, k.key_log2, i == SHARES_4 ? cost.shares4_step_us : cost.q_step_us[i == SHARES_2], i == SHARES_4 ? cost.shares4_fixed_us : cost.q_fixed_us[i == SHARES_2],
-                                 pl.dq_slots != pl.dq_qtiles);
-        apart += launch_us(l.c, l.k, cus);
-    }
-    if (pl.key_waves) {
-        const int per_cu = pairs * pl.kv_tiles * pl.split.n > cus ? 2 : 1;
-        const List l = kv_blocks(pl.split.n, per_cu == 1 ? KEY_WAVES_64.alone_us : 2 * KEY_WAVES_64.step_us, per_cu == 1 ? KEY_WAVES_64.alone_fixed_us : 2 * KEY_WAVES_64.fixed_us);
-        apart += launch_us(l.c, l.k, per_cu * cus);
-    } else {
-        const List l = kv_blocks(pl.split.n, cost.kv_step_us, cost.kv_fixed_us);
-        apart += launch_us(l.c, l.k, cus);
-    }
-    // where the plan has several blocks on a CU the model takes it for slower than it is, most of all at head dim 64 with both kernels of that
-    // kind: of 5600 random launches joined at 0.96, 100 lost more than 1 %, 80 of them there; of 5400 with about these factors 50
-    double best = apart * (D == 128 ? pl.dq_four_waves ? 0.92 : 0.98
-                                    : pl.key_waves && pl.dq_four_waves ? 0.78 : pl.key_waves || pl.dq_four_waves || pl.dq_blocks + pl.kv_blocks > 8 * cus ? 0.88 : 0.96);
+    // the launches of a plan one after the other, and what a joint one has to be shorter than
+    auto apart_us = [&](const BwdPlan &x) {
+        double us = 2 * cost.launch_us + reduce_us(x.split.n);
+        if (x.dq_four_waves) {
+            const TileCost &c = (D == 128 ? DQ_ROWS_128 : DQ_ROWS_64).kernel[FOUR_WAVES];
+            const int per_cu = (int)std::min<long long>(D == 128 ? FourWaves<128>::PER_CU : FourWaves<64>::PER_CU, (x.dq_blocks + cus - 1) / cus);
+            const List l = dq_blocks(128, 6, per_cu == 1 ? c.alone_us : per_cu * c.step_us, per_cu == 1 ? c.alone_fixed_us : per_cu * c.fixed_us, false);
+            us += launch_us(l.c, l.k, per_cu * cus);
+        } else {
+            const int i = x.dq_ks == 4 ? SHARES_4 : x.dq_ks == 2 ? SHARES_2 : ROWS_256;
+            const RowKernel k = row_kernel(i, D);
+            const List l = dq_blocks(k.rows, k.key_log2, i == SHARES_4 ? cost.shares4_step_us : cost.q_step_us[i == SHARES_2], i == SHARES_4 ? cost.shares4_fixed_us : cost.q_fixed_us[i == SHARES_2],
+                                     x.dq_slots != x.dq_qtiles);
+            us += launch_us(l.c, l.k, cus);
+        }
+        if (x.key_waves) {
+            const int per_cu = pairs * x.kv_tiles * x.split.n > cus ? 2 : 1;
+            const List l = kv_blocks(x.split.n, per_cu == 1 ? KEY_WAVES_64.alone_us : 2 * KEY_WAVES_64.step_us, per_cu == 1 ? KEY_WAVES_64.alone_fixed_us : 2 * KEY_WAVES_64.fixed_us);
+            us += launch_us(l.c, l.k, per_cu * cus);
+        } else {
+            const List l = kv_blocks(x.split.n, cost.kv_step_us, cost.kv_fixed_us);
+            us += launch_us(l.c, l.k, cus);
+        }
+        // where the plan has several blocks on a CU the model takes it for slower than it is, most of all at head dim 64 with both kernels of that
+        // kind: of 5600 random launches joined at 0.96, 100 lost more than 1 %, 80 of them there; of 5400 with about these factors 50
+        return us * (D == 128 ? x.dq_four_waves ? 0.92 : 0.98
+                              : x.key_waves && x.dq_four_waves ? 0.78 : x.key_waves || x.dq_four_waves || x.dq_blocks + x.kv_blocks > 8 * cus ? 0.88 : 0.96);
+    };
+    double best = apart_us(pl);
     const double delta_us = flags & LTR_DELTA_FROM_O ? cost.delta_us + (double)q_pairs * Sq * D * 4 / cost.delta_bytes_per_us : 0.0;
     int best_ks = 0, best_n = 1;
     bool keys_first = false;
     // dQ blocks of one and two shares; the blocks of both kinds are looked at in both orders, unless all run at once or even spread evenly over
-    // the CUs they take longer than the best so far
+    // the CUs they take longer than the best so far.  The kind that goes first is dispatched once, for all that may follow
     List q[2];
+    double q_total[2], q_longest[2];
+    std::optional<Dispatch> after_q[2];
     for (int ks = 1; ks <= 2; ks++) {
         const RowKernel k = row_kernel(ks == 2 ? SHARES_2 : ROWS_256, D);
         q[ks - 1] = dq_blocks(k.rows, k.key_log2, cost.q_step_us[ks - 1], cost.q_fixed_us[ks - 1], false);
+        q_total[ks - 1] = q[ks - 1].total_us();
+        q_longest[ks - 1] = q[ks - 1].longest_us();
     }
     for (int n = 1; n <= 16; n *= 2) {
         if (n > 1 && (!may_split || pairs * tiles_seen * n > 5LL * cus || (double)pairs * tiles_seen * n * 128 * D * 8 > MAX_PART_BYTES)) break;
-        if (n > 1 && n > (long long)(Sq + 63) / 64 * (Hq / Hkv)) break;
+        if (n > 1 && n > (long long)(Sq + 63) / 64 * n_rep) break;
         const List kv = kv_blocks(n, cost.kv_step_us, cost.kv_fixed_us);
+        const double kv_total = kv.total_us(), kv_longest = kv.longest_us();
+        std::optional<Dispatch> after_kv;
         int reps = 1;
-        while (reps * 2 <= n && Hq / Hkv % (reps * 2) == 0) reps *= 2;
+        while (reps * 2 <= n && n_rep % (reps * 2) == 0) reps *= 2;
         for (int ks = 1; ks <= 2; ks++) {
             const bool one_round = q[ks - 1].n + kv.n <= cus;
-            const bool own = ks == 2 && one_round && (flags & LTR_DELTA_FROM_O) && (long long)Hq / Hkv / reps * Sq <= own_delta_rows(D);
+            const bool own = ks == 2 && one_round && (flags & LTR_DELTA_FROM_O) && (long long)n_rep / reps * Sq <= own_delta_rows(D);
             const double rest = cost.launch_us + (own ? 0.5 : delta_us) + reduce_us(n);
-            if (rest + (q[ks - 1].total_us() + kv.total_us()) / cus >= best) continue;
+            if (rest + std::max((q_total[ks - 1] + kv_total) / cus, std::max(q_longest[ks - 1], kv_longest)) >= best) continue;
             for (int first = 0; first < (one_round ? 1 : 2); first++) {
-                const double us = rest + (first ? both_us(kv, q[ks - 1]) : both_us(q[ks - 1], kv));
+                const List &one = first ? kv : q[ks - 1], &other = first ? q[ks - 1] : kv;
+                std::optional<Dispatch> &after_one = first ? after_kv : after_q[ks - 1];
+                if (!after_one) after_one.emplace(cus).add(one.c, one.k);
+                Dispatch both(*after_one);
+                if (!both.add(other.c, other.k, best - rest)) continue;
+                const double us = rest + both.end;
                 if (us < best) {
                     best = us;
                     best_ks = ks;
@@ -4925,6 +4973,10 @@ void joint_launch(BwdPlan &pl, int D, unsigned flags, int B, int Hq, int Hkv, in
         }
     }
     if (!best_ks) return;
+    if (best_n == 1 && pl.split.n > 1 && best >= apart_us(alone)) {
+        pl = alone;
+        return;
+    }
     pl.joint = true;
     pl.keys_first = keys_first;
     pl.key_waves = pl.dq_four_waves = false;
@@ -4947,8 +4999,8 @@ BwdPlan make_bwd_plan(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, i
     may_split = may_split && !(flags & (LTR_NO_DKDV | LTR_BWD_F32_SCALAR));
     pl.key_waves = false;
     const int cus = device_cus();
-    auto split_keys = [&](const KvSplitCost &cost) {
-        pl.split = kv_split(cost, may_split ? 32 : 1, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks, cus);
+    auto split_keys = [&](const KvSplitCost &cost, int max_n) {
+        return kv_split(cost, max_n, D, pl.keys_per_block, (flags & LTR_CAUSAL) != 0, B, Hkv, Hq / Hkv, Sq, q_split, q_pos0, chunk, n_chunks, cus);
     };
     auto size_parts = [&]() {
         if (pl.split.n > 1) pl.part_bytes = (int64_t)pl.split.tiles * B * Hkv * pl.split.n * pl.keys_per_block * D * 2 * 4;
@@ -4972,7 +5024,8 @@ BwdPlan make_bwd_plan(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, i
         // 27064), but they would move single elements by the whole sum's error, which from about here on exceeds 1e-4 of them:
         // the tolerance to which results of this path are to stay the same
         may_split = may_split && (long long)(Hq / Hkv) * Sq <= 4096;
-        split_keys(D == 128 ? KvSplitCost{32, 9.0, 18.0, 9.0, 18.0, 0.25, 2.0, 6e6} : KvSplitCost{32, 4.5, 6.75, 4.5, 6.75, 0.25, 2.0, 6e6});
+        pl.split = split_keys(D == 128 ? KvSplitCost{32, 9.0, 18.0, 9.0, 18.0, 0.25, 2.0, 6e6} : KvSplitCost{32, 4.5, 6.75, 4.5, 6.75, 0.25, 2.0, 6e6},
+                              may_split ? 32 : 1);
         size_parts();
         pl.dq_qtiles = pl.dq_slots = (Sq + pl.dq_rows - 1) / pl.dq_rows;
         pl.dq_blocks = (long long)pl.dq_qtiles * B * Hq;
@@ -5001,18 +5054,21 @@ BwdPlan make_bwd_plan(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, i
     pl.kv_tiles = 0;
     for (int c = 0; c < n_chunks; c++) pl.kv_tiles += (chunk[c].sk + pl.keys_per_block - 1) / pl.keys_per_block;
     pl.kv_blocks = pl.kv_tiles * B * Hkv;
-    if (D == 128 || (flags & LTR_HEAD_COLS) || wide) {
-        split_keys(D == 128 ? KvSplitCost{64, 1.4, 11.2, 1.4, 11.2, 0.25, 2.0, 8e6}
-                            : wide ? KvSplitCost{64, 1.9, 11.4, 1.9, 11.4, 0.25, 2.0, 6e6} : KvSplitCost{64, 1.0, 8.0, 1.0, 8.0, 0.25, 2.0, 6e6});
-    } else {
+    auto choose_kv = [&](BwdPlan &x, int max_n) {   // the kernel of whole or shared key tiles
+        x.key_waves = false;
+        if (D == 128 || (flags & LTR_HEAD_COLS) || wide) {
+            x.split = split_keys(D == 128 ? KvSplitCost{64, 1.4, 11.2, 1.4, 11.2, 0.25, 2.0, 8e6}
+                                          : wide ? KvSplitCost{64, 1.9, 11.4, 1.9, 11.4, 0.25, 2.0, 6e6} : KvSplitCost{64, 1.0, 8.0, 1.0, 8.0, 0.25, 2.0, 6e6}, max_n);
+            return;
+        }
         // head dim 64: one wave per 32 keys (two blocks per CU) or two (one block).  A block alone on its CU is faster with eight
         // waves, a CU is faster with two blocks of four.  Constants fitted to 195 launches each (60 shapes, n = 1 .. 32; rms 7 %)
-        split_keys(KEY_WAVES_64);
-        const KvSplit one_wave = pl.split;
-        split_keys(KvSplitCost{64, 1.14, 7.0, 1.01, 5.8, 0.6, 4.0, 17e6});
-        pl.key_waves = one_wave.us < 0.96 * pl.split.us;
-        if (pl.key_waves) pl.split = one_wave;
-    }
+        const KvSplit one_wave = split_keys(KEY_WAVES_64, max_n);
+        x.split = split_keys(KvSplitCost{64, 1.14, 7.0, 1.01, 5.8, 0.6, 4.0, 17e6}, max_n);
+        x.key_waves = one_wave.us < 0.96 * x.split.us;
+        if (x.key_waves) x.split = one_wave;
+    };
+    choose_kv(pl, may_split ? 32 : 1);
     const RowChoice choice = flags & LTR_NO_DQ
                                  ? RowChoice{flags & LTR_DQ_ROWS_512 ? ROWS_512 : ROWS_256, false}
                                  : choose_rows(D == 128 ? DQ_ROWS_128 : DQ_ROWS_64,
@@ -5028,7 +5084,9 @@ BwdPlan make_bwd_plan(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, i
     pl.dq_blocks = (long long)pl.dq_slots * B * Hq;
     constexpr unsigned NOT_JOINT = LTR_NO_DQ | LTR_NO_DKDV | LTR_DQ_ROWS_256 | LTR_DQ_ROWS_512 | LTR_DKDV_KEYS_128 | LTR_DKDV_KEYS_256;
     if ((flags & LTR_BWD_JOINT) && !(flags & NOT_JOINT) && !pl.wide_q && !pl.wide_kv) {
-        joint_launch(pl, D, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split, cus);
+        BwdPlan alone = pl;
+        if (pl.split.n > 1) choose_kv(alone, 1);
+        joint_launch(pl, alone, D, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split, cus);
         if (pl.joint) uneven = causal_ && q_tiles_uneven(Sq, pl.dq_rows, q_split, q_pos0, chunk, n_chunks);
     }
     size_parts();
@@ -5040,8 +5098,7 @@ BwdPlan make_bwd_plan(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, i
                              causal_ && key_tiles_uneven(Sq, pl.keys_per_block, q_split, q_pos0, chunk, n_chunks));
     return pl;
 }
-// The plan of a problem.  One with LTR_BWD_JOINT prices up to 20 launches (1 - 10 us), and a backward asks with a workspace in mind and, where that
-// plan needs none, once more without.
+// The plan of a problem.  One with LTR_BWD_JOINT prices up to 20 launches (1 - 8 us), and a backward asks twice, for the workspace and for the launch.
 BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk,
                  int n_chunks, bool may_split = false) {
     auto make = [&] { return make_bwd_plan(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split); };
@@ -5050,10 +5107,10 @@ BwdPlan plan_bwd(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq
     return kept.get(Problem(D, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, may_split), make);
 }
 // The plan with a workspace of that many bytes: shared key tiles if their partial sums fit, else the launch without a workspace (whose kernel
-// and block order are other ones than those chosen for sharing).
+// and block order are other ones than those chosen for sharing).  A joint plan that shares no tiles fits no workspace as well: it is not priced again.
 BwdPlan plan_bwd_ws(int D, bool f32, unsigned flags, int B, int Hq, int Hkv, int Sq, int q_split, const int *q_pos0, const ChunkDev *chunk, int n_chunks,
                     int64_t work_bytes) {
-    if (work_bytes > 0) {
+    if (work_bytes > 0 || (flags & LTR_BWD_JOINT)) {
         const BwdPlan pl = plan_bwd(D, f32, flags, B, Hq, Hkv, Sq, q_split, q_pos0, chunk, n_chunks, true);
         if (pl.part_bytes <= work_bytes) return pl;
     }

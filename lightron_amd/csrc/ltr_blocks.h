@@ -128,40 +128,59 @@ struct BlockClass {
     double us;
     long long n;
 };
-inline double launch_us(const BlockClass *classes, int n_classes, int slots) {
-    constexpr int MOST = 48;
+struct Dispatch {
+    static constexpr int MOST = 48;
     struct Run {
         double at;
         long long n;
-    } run[MOST];
-    int runs = 1;
-    run[0] = {0, slots};
-    double end = 0;
-    for (int c = 0; c < n_classes; c++) {
-        const double eps = std::max(0.3, 0.03 * classes[c].us);
-        // whole rounds of equal blocks move all slots alike
-        const long long rounds = std::max(0LL, classes[c].n / slots - 1);
-        for (int i = 0; i < runs; i++) run[i].at += rounds * classes[c].us;
-        if (rounds > 0) end = std::max(end, run[runs - 1].at);
-        for (long long left = classes[c].n - rounds * slots; left > 0;) {
-            const long long n = std::min(left, run[0].n);
-            const double at = run[0].at + classes[c].us;
-            left -= n;
-            run[0].n -= n;
-            if (run[0].n == 0) {
-                runs--;
-                for (int i = 0; i < runs; i++) run[i] = run[i + 1];
+    } place[2 * MOST], *run = place;   // slots by the time they are free; the list moves up in its place as runs leave at its front
+    int runs = 1, slots;
+    double end = 0;                    // of the last block
+    explicit Dispatch(int slots_) : slots(slots_) { run[0] = {0, slots_}; }
+    Dispatch(const Dispatch &o) : runs(o.runs), slots(o.slots), end(o.end) { std::copy(o.run, o.run + o.runs, place); }
+    Dispatch &operator=(const Dispatch &) = delete;
+    // more blocks, after those before them; false as soon as one of them ends at `most` or later: `end` is then less than it would have been
+    bool add(const BlockClass *classes, int n_classes, double most = 1e300) {
+        for (int c = 0; c < n_classes; c++) {
+            const double us = classes[c].us, eps = std::max(0.3, 0.03 * us);
+            long long left = classes[c].n;
+            // whole rounds of equal blocks move all slots alike
+            if (left >= 2LL * slots) {
+                const long long rounds = left / slots - 1;
+                for (int i = 0; i < runs; i++) run[i].at += rounds * us;
+                end = std::max(end, run[runs - 1].at);
+                left -= rounds * slots;
             }
-            end = std::max(end, at);
-            int i = 0;
-            while (i < runs && run[i].at < at - eps) i++;
-            if (i < runs && run[i].at <= at + eps) run[i].n += n;
-            else if (runs == MOST) run[std::min(i, runs - 1)].n += n;
-            else {
-                for (int k = runs++; k > i; k--) run[k] = run[k - 1];
-                run[i] = {at, n};
+            while (left > 0) {
+                const long long n = std::min(left, run[0].n);
+                const double at = run[0].at + us;
+                left -= n;
+                run[0].n -= n;
+                if (run[0].n == 0) {
+                    runs--;
+                    run++;
+                }
+                end = std::max(end, at);
+                int i = runs;   // the first run that is free at `at` or later: near the end, for the blocks of a launch are much alike
+                while (i > 0 && run[i - 1].at >= at - eps) i--;
+                if (i < runs && run[i].at <= at + eps) run[i].n += n;
+                else if (runs == MOST) run[std::min(i, runs - 1)].n += n;
+                else {
+                    if (run + runs == place + 2 * MOST) {
+                        std::copy(run, run + runs, place);
+                        run = place;
+                    }
+                    for (int k = runs++; k > i; k--) run[k] = run[k - 1];
+                    run[i] = {at, n};
+                }
             }
+            if (end >= most) return false;
         }
+        return true;
     }
-    return end;
+};
+inline double launch_us(const BlockClass *classes, int n_classes, int slots) {
+    Dispatch d(slots);
+    d.add(classes, n_classes);
+    return d.end;
 }
