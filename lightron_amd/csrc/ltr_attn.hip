@@ -286,6 +286,11 @@ __device__ __forceinline__ void tile_barrier() {
 // addresses stay those of the width): a quarter of the matrix work and of the LDS reads.  Kernel us, all four blocks -> three, forward / dQ / dK/dV:
 //   2 x 16 heads of 96 S=777   18.8 / 25.6 / 31.1 -> 17.6 / 24.6 / 28.3     8 x 32 on 8 of 96 S=2048   280 / 416 / 510 -> 253 / 372 / 453
 //   6 x 8 heads of 80 S=3000    114 / 159 / 218 -> 103 / 141 / 195          1 x 32 of 72, S=1000, no mask   23.0 / 31.5 / 38.9 -> 21.5 / 29.7 / 34.7
+// Those are kernels of their own, told apart by the type of their argument: with both bodies in one kernel each had the registers of the larger
+// and twice the spilled scalars (bwd_joint_pad_kernel<128, 2> 115 for 40, 256 vector registers for 215), head dims above 96 too.  In time
+// it is 1 % at most (2 x 16 heads of 96, S=777, joint 37.3 -> 36.8 us; 8 x 32 on 8 of 96, S=2048 the same).
+template <class Params>
+struct Columns96 : Params {};   // the same bytes
 template <int BYTES>
 __device__ __forceinline__ void clear_lds(unsigned char *smem) {   // followed by a barrier: the fill covers the columns that transfers write
     for (int i = threadIdx.x * 16; i < BYTES; i += 512 * 16) *(uint4 *)(smem + i) = make_uint4(0, 0, 0, 0);
@@ -1053,8 +1058,12 @@ __global__ __launch_bounds__(512) void fwd_bf16_shares_kernel(const FwdParams p)
 }
 template <int D, int KS>   // head dims below D
 __global__ __launch_bounds__(512) void fwd_bf16_pad_kernel(const FwdParams p) {
-    if (D == 128 && p.cols <= 96) fwd_bf16_body<D, 1, KS, true, 8, FwdTile<D, 1, KS>::BN, D == 128 ? 96 : D>(p);   // three column blocks, see below
-    else fwd_bf16_body<D, 1, KS, true>(p);
+    fwd_bf16_body<D, 1, KS, true>(p);
+}
+template <int D, int KS>
+__global__ __launch_bounds__(512) void fwd_bf16_pad_kernel(const Columns96<FwdParams> p) {
+    static_assert(D == 128);
+    fwd_bf16_body<D, 1, KS, true, 8, FwdTile<D, 1, KS>::BN, 96>(p);
 }
 
 // ------------------------------------------------------------------------------ forward, fp32
@@ -2440,9 +2449,13 @@ __global__ __launch_bounds__(512) void bwd_dkdv_kernel(const BwdParams p) {
 template <int D>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_dkdv_pad_kernel(const BwdParams p) {
     const BlockItem item = block_item(p.kv_map, p.B * p.Hkv);
-    if (item.pair >= p.B * p.Hkv) return;
-    if (D == 128 && p.cols <= 96) bwd_dkdv_body<D, 1, true, false, D == 128 ? 96 : D>(p, item);
-    else bwd_dkdv_body<D, 1, true>(p, item);
+    if (item.pair < p.B * p.Hkv) bwd_dkdv_body<D, 1, true>(p, item);
+}
+template <int D>
+__global__ __launch_bounds__(512) void bwd_dkdv_pad_kernel(const Columns96<BwdParams> p) {
+    static_assert(D == 128);
+    const BlockItem item = block_item(p.kv_map, p.B * p.Hkv);
+    if (item.pair < p.B * p.Hkv) bwd_dkdv_body<D, 1, true, false, 96>(p, item);
 }
 
 // dK/dV at head dim 64, one wave per 32-key slice: K and V operands (32 registers) and both accumulators (64) fit one wave, so nothing is
@@ -3197,9 +3210,12 @@ __global__ __launch_bounds__(512) void bwd_dq_shares_kernel(const BwdParams p) {
 }
 template <int D, int KS>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_dq_pad_kernel(const BwdParams p) {
-    const BlockItem item = block_item(p.q_map, p.B * p.Hkv);
-    if (D == 128 && p.cols <= 96) bwd_dq_body<D, 1, KS, true, 8, FwdTile<D, 1, KS>::BN, D == 128 ? 96 : D>(p, item);
-    else bwd_dq_body<D, 1, KS, true>(p, item);
+    bwd_dq_body<D, 1, KS, true>(p, block_item(p.q_map, p.B * p.Hkv));
+}
+template <int D, int KS>
+__global__ __launch_bounds__(512) void bwd_dq_pad_kernel(const Columns96<BwdParams> p) {
+    static_assert(D == 128);
+    bwd_dq_body<D, 1, KS, true, 8, FwdTile<D, 1, KS>::BN, 96>(p, block_item(p.q_map, p.B * p.Hkv));
 }
 
 // dQ and dK/dV blocks in one launch (LTR_BWD_JOINT).  Given DELTA, neither kind needs anything of the other; in launches of their own each ends with
@@ -3222,8 +3238,12 @@ __global__ __launch_bounds__(512) void bwd_joint_kernel(const BwdParams p) {
 }
 template <int D, int KS>   // head dims below D
 __global__ __launch_bounds__(512) void bwd_joint_pad_kernel(const BwdParams p) {
-    if (D == 128 && p.cols <= 96) bwd_joint_body<D, KS, true, false, D == 128 ? 96 : D>(p);
-    else bwd_joint_body<D, KS, true>(p);
+    bwd_joint_body<D, KS, true>(p);
+}
+template <int D, int KS>
+__global__ __launch_bounds__(512) void bwd_joint_pad_kernel(const Columns96<BwdParams> p) {
+    static_assert(D == 128);
+    bwd_joint_body<D, KS, true, false, 96>(p);
 }
 
 // the same with DELTA computed by the dK/dV blocks for themselves (own_delta), as the dQ blocks compute theirs: launches of few rows (own_delta_rows)
@@ -3233,8 +3253,12 @@ __global__ __launch_bounds__(512) void bwd_joint_delta_kernel(const BwdParams p)
 }
 template <int D>
 __global__ __launch_bounds__(512) void bwd_joint_delta_pad_kernel(const BwdParams p) {
-    if (D == 128 && p.cols <= 96) bwd_joint_body<D, 2, true, true, D == 128 ? 96 : D>(p);
-    else bwd_joint_body<D, 2, true, true>(p);
+    bwd_joint_body<D, 2, true, true>(p);
+}
+template <int D>
+__global__ __launch_bounds__(512) void bwd_joint_delta_pad_kernel(const Columns96<BwdParams> p) {
+    static_assert(D == 128);
+    bwd_joint_body<D, 2, true, true, 96>(p);
 }
 
 // ------------------------------------------------------------------------------ backward, fp32
@@ -4070,6 +4094,10 @@ constexpr int joint_delta_lds_bytes() {
 }
 static_assert(joint_delta_lds_bytes<128>() <= 160 * 1024, "LDS of one CU");
 
+// address of a kernel that takes this argument (the padded kernels of width 128 exist for two)
+template <class Params>
+const void *kernel_of(void (*kernel)(Params)) { return (const void *)kernel; }
+
 int enable_large_lds() {
     int dev = 0;
     if (current_device(&dev)) return LTR_EDEVICE;
@@ -4103,20 +4131,27 @@ int enable_large_lds() {
         {(const void *)bwd_dq_f32_rows32_kernel<64, 4>, F32Mfma<64, 4>::LDS},
         {(const void *)bwd_dkdv_f32_mfma_kernel<128>, F32DkdvLds<128>::LDS},
         {(const void *)bwd_dkdv_f32_mfma_kernel<64>, F32DkdvLds<64>::LDS},
-        {(const void *)bwd_dkdv_pad_kernel<128>, BwdLds<128, 1>::TOTAL},
-        {(const void *)fwd_bf16_pad_kernel<128, 1>, fwd_lds_bytes<128>()},
-        {(const void *)fwd_bf16_pad_kernel<128, 2>, shares_lds_bytes<128, 2>()},
-        {(const void *)fwd_bf16_pad_kernel<128, 4>, shares_lds_bytes<128, 4>()},
-        {(const void *)bwd_dq_pad_kernel<128, 1>, dq_lds_bytes<128>()},
-        {(const void *)bwd_dq_pad_kernel<128, 2>, shares_lds_bytes<128, 2>()},
-        {(const void *)bwd_dq_pad_kernel<128, 4>, shares_lds_bytes<128, 4>()},
-        {(const void *)bwd_dkdv_pad_kernel<64>, BwdLds<64, 1>::TOTAL},
-        {(const void *)fwd_bf16_pad_kernel<64, 1>, fwd_lds_bytes<64>()},
-        {(const void *)fwd_bf16_pad_kernel<64, 2>, shares_lds_bytes<64, 2>()},
-        {(const void *)fwd_bf16_pad_kernel<64, 4>, shares_lds_bytes<64, 4>()},
-        {(const void *)bwd_dq_pad_kernel<64, 1>, dq_lds_bytes<64>()},
-        {(const void *)bwd_dq_pad_kernel<64, 2>, shares_lds_bytes<64, 2>()},
-        {(const void *)bwd_dq_pad_kernel<64, 4>, shares_lds_bytes<64, 4>()},
+        {kernel_of<BwdParams>(bwd_dkdv_pad_kernel<128>), BwdLds<128, 1>::TOTAL},
+        {kernel_of<Columns96<BwdParams>>(bwd_dkdv_pad_kernel<128>), BwdLds<128, 1>::TOTAL},
+        {kernel_of<FwdParams>(fwd_bf16_pad_kernel<128, 1>), fwd_lds_bytes<128>()},
+        {kernel_of<Columns96<FwdParams>>(fwd_bf16_pad_kernel<128, 1>), fwd_lds_bytes<128>()},
+        {kernel_of<FwdParams>(fwd_bf16_pad_kernel<128, 2>), shares_lds_bytes<128, 2>()},
+        {kernel_of<Columns96<FwdParams>>(fwd_bf16_pad_kernel<128, 2>), shares_lds_bytes<128, 2>()},
+        {kernel_of<FwdParams>(fwd_bf16_pad_kernel<128, 4>), shares_lds_bytes<128, 4>()},
+        {kernel_of<Columns96<FwdParams>>(fwd_bf16_pad_kernel<128, 4>), shares_lds_bytes<128, 4>()},
+        {kernel_of<BwdParams>(bwd_dq_pad_kernel<128, 1>), dq_lds_bytes<128>()},
+        {kernel_of<Columns96<BwdParams>>(bwd_dq_pad_kernel<128, 1>), dq_lds_bytes<128>()},
+        {kernel_of<BwdParams>(bwd_dq_pad_kernel<128, 2>), shares_lds_bytes<128, 2>()},
+        {kernel_of<Columns96<BwdParams>>(bwd_dq_pad_kernel<128, 2>), shares_lds_bytes<128, 2>()},
+        {kernel_of<BwdParams>(bwd_dq_pad_kernel<128, 4>), shares_lds_bytes<128, 4>()},
+        {kernel_of<Columns96<BwdParams>>(bwd_dq_pad_kernel<128, 4>), shares_lds_bytes<128, 4>()},
+        {kernel_of<BwdParams>(bwd_dkdv_pad_kernel<64>), BwdLds<64, 1>::TOTAL},
+        {kernel_of<FwdParams>(fwd_bf16_pad_kernel<64, 1>), fwd_lds_bytes<64>()},
+        {kernel_of<FwdParams>(fwd_bf16_pad_kernel<64, 2>), shares_lds_bytes<64, 2>()},
+        {kernel_of<FwdParams>(fwd_bf16_pad_kernel<64, 4>), shares_lds_bytes<64, 4>()},
+        {kernel_of<BwdParams>(bwd_dq_pad_kernel<64, 1>), dq_lds_bytes<64>()},
+        {kernel_of<BwdParams>(bwd_dq_pad_kernel<64, 2>), shares_lds_bytes<64, 2>()},
+        {kernel_of<BwdParams>(bwd_dq_pad_kernel<64, 4>), shares_lds_bytes<64, 4>()},
         {(const void *)fwd_bf16_shares_kernel<128, 2>, shares_lds_bytes<128, 2>()},
         {(const void *)fwd_bf16_shares_kernel<128, 4>, shares_lds_bytes<128, 4>()},
         {(const void *)fwd_bf16_shares_kernel<64, 2>, shares_lds_bytes<64, 2>()},
@@ -4126,17 +4161,20 @@ int enable_large_lds() {
         {(const void *)bwd_dq_shares_kernel<64, 2>, shares_lds_bytes<64, 2>()},
         {(const void *)bwd_dq_shares_kernel<64, 4>, shares_lds_bytes<64, 4>()},
         {(const void *)bwd_joint_delta_kernel<64>, joint_delta_lds_bytes<64>()},
-        {(const void *)bwd_joint_delta_pad_kernel<64>, joint_delta_lds_bytes<64>()},
+        {kernel_of<BwdParams>(bwd_joint_delta_pad_kernel<64>), joint_delta_lds_bytes<64>()},
         {(const void *)bwd_joint_delta_kernel<128>, joint_delta_lds_bytes<128>()},
-        {(const void *)bwd_joint_delta_pad_kernel<128>, joint_delta_lds_bytes<128>()},
+        {kernel_of<BwdParams>(bwd_joint_delta_pad_kernel<128>), joint_delta_lds_bytes<128>()},
+        {kernel_of<Columns96<BwdParams>>(bwd_joint_delta_pad_kernel<128>), joint_delta_lds_bytes<128>()},
         {(const void *)bwd_joint_kernel<64, 1>, joint_lds_bytes<64, 1>()},
         {(const void *)bwd_joint_kernel<64, 2>, joint_lds_bytes<64, 2>()},
-        {(const void *)bwd_joint_pad_kernel<64, 1>, joint_lds_bytes<64, 1>()},
-        {(const void *)bwd_joint_pad_kernel<64, 2>, joint_lds_bytes<64, 2>()},
+        {kernel_of<BwdParams>(bwd_joint_pad_kernel<64, 1>), joint_lds_bytes<64, 1>()},
+        {kernel_of<BwdParams>(bwd_joint_pad_kernel<64, 2>), joint_lds_bytes<64, 2>()},
         {(const void *)bwd_joint_kernel<128, 1>, joint_lds_bytes<128, 1>()},
         {(const void *)bwd_joint_kernel<128, 2>, joint_lds_bytes<128, 2>()},
-        {(const void *)bwd_joint_pad_kernel<128, 1>, joint_lds_bytes<128, 1>()},
-        {(const void *)bwd_joint_pad_kernel<128, 2>, joint_lds_bytes<128, 2>()},
+        {kernel_of<BwdParams>(bwd_joint_pad_kernel<128, 1>), joint_lds_bytes<128, 1>()},
+        {kernel_of<Columns96<BwdParams>>(bwd_joint_pad_kernel<128, 1>), joint_lds_bytes<128, 1>()},
+        {kernel_of<BwdParams>(bwd_joint_pad_kernel<128, 2>), joint_lds_bytes<128, 2>()},
+        {kernel_of<Columns96<BwdParams>>(bwd_joint_pad_kernel<128, 2>), joint_lds_bytes<128, 2>()},
     };
     bool ok = true;
     for (const auto &k : large) ok = ok && hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, k.bytes) == hipSuccess;
@@ -4630,18 +4668,24 @@ KernelChoice f32_dq_kernel(int D, int ks, int rows) {
     if (ks == 2) return {LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 2>), F32Mfma<64, 2>::LDS};
     return rows == F32Rows16::BM ? KernelChoice{LTR_KERNEL(bwd_dq_f32_mfma_kernel<64, 4>), F32Mfma<64, 4>::LDS} : KernelChoice{LTR_KERNEL(bwd_dq_f32_rows32_kernel<64, 4>), F32Mfma<64, 4>::LDS};
 }
-KernelChoice joint_kernel(int D, bool pad, int ks, bool own_delta) {
+#define LTR_PAD_KERNEL(params, ...) kernel_of<params>(__VA_ARGS__), #__VA_ARGS__
+KernelChoice joint_kernel(int D, bool pad, int ks, bool own_delta, int cols) {
+    const bool three = cols <= 96;   // blocks of 32 columns, width 128
     if (own_delta) {
-        if (pad) return D == 128 ? KernelChoice{LTR_KERNEL(bwd_joint_delta_pad_kernel<128>), joint_delta_lds_bytes<128>()} : KernelChoice{LTR_KERNEL(bwd_joint_delta_pad_kernel<64>), joint_delta_lds_bytes<64>()};
+        if (pad && D == 128)
+            return three ? KernelChoice{LTR_PAD_KERNEL(Columns96<BwdParams>, bwd_joint_delta_pad_kernel<128>), joint_delta_lds_bytes<128>()} : KernelChoice{LTR_PAD_KERNEL(BwdParams, bwd_joint_delta_pad_kernel<128>), joint_delta_lds_bytes<128>()};
+        if (pad) return {LTR_PAD_KERNEL(BwdParams, bwd_joint_delta_pad_kernel<64>), joint_delta_lds_bytes<64>()};
         return D == 128 ? KernelChoice{LTR_KERNEL(bwd_joint_delta_kernel<128>), joint_delta_lds_bytes<128>()} : KernelChoice{LTR_KERNEL(bwd_joint_delta_kernel<64>), joint_delta_lds_bytes<64>()};
     }
     if (pad) {
-        if (D == 128) return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<128, 1>), joint_lds_bytes<128, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<128, 2>), joint_lds_bytes<128, 2>()};
-        return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<64, 1>), joint_lds_bytes<64, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_pad_kernel<64, 2>), joint_lds_bytes<64, 2>()};
+        if (D == 128 && three) return ks == 1 ? KernelChoice{LTR_PAD_KERNEL(Columns96<BwdParams>, bwd_joint_pad_kernel<128, 1>), joint_lds_bytes<128, 1>()} : KernelChoice{LTR_PAD_KERNEL(Columns96<BwdParams>, bwd_joint_pad_kernel<128, 2>), joint_lds_bytes<128, 2>()};
+        if (D == 128) return ks == 1 ? KernelChoice{LTR_PAD_KERNEL(BwdParams, bwd_joint_pad_kernel<128, 1>), joint_lds_bytes<128, 1>()} : KernelChoice{LTR_PAD_KERNEL(BwdParams, bwd_joint_pad_kernel<128, 2>), joint_lds_bytes<128, 2>()};
+        return ks == 1 ? KernelChoice{LTR_PAD_KERNEL(BwdParams, bwd_joint_pad_kernel<64, 1>), joint_lds_bytes<64, 1>()} : KernelChoice{LTR_PAD_KERNEL(BwdParams, bwd_joint_pad_kernel<64, 2>), joint_lds_bytes<64, 2>()};
     }
     if (D == 128) return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_kernel<128, 1>), joint_lds_bytes<128, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_kernel<128, 2>), joint_lds_bytes<128, 2>()};
     return ks == 1 ? KernelChoice{LTR_KERNEL(bwd_joint_kernel<64, 1>), joint_lds_bytes<64, 1>()} : KernelChoice{LTR_KERNEL(bwd_joint_kernel<64, 2>), joint_lds_bytes<64, 2>()};
 }
+#undef LTR_PAD_KERNEL
 #undef LTR_KERNEL
 
 // What a bf16 plan depends on, and the plans that a thread keeps: pricing launches takes 1 - 10 us, as long as queueing them, and a program asks for the
@@ -5260,12 +5304,14 @@ extern "C" int ltr_attn_fwd(const ltr_attn_fwd_args *a, void *stream) {
         if (rc) return rc;
         if (pad) {
             const int i = pl.ks >> 1;
-            const void *const kernels[2][3] = {
-                {(const void *)fwd_bf16_pad_kernel<64, 1>, (const void *)fwd_bf16_pad_kernel<64, 2>, (const void *)fwd_bf16_pad_kernel<64, 4>},
-                {(const void *)fwd_bf16_pad_kernel<128, 1>, (const void *)fwd_bf16_pad_kernel<128, 2>, (const void *)fwd_bf16_pad_kernel<128, 4>}};
+            using Three = Columns96<FwdParams>;
+            const void *const kernels[3][3] = {
+                {kernel_of<FwdParams>(fwd_bf16_pad_kernel<64, 1>), kernel_of<FwdParams>(fwd_bf16_pad_kernel<64, 2>), kernel_of<FwdParams>(fwd_bf16_pad_kernel<64, 4>)},
+                {kernel_of<FwdParams>(fwd_bf16_pad_kernel<128, 1>), kernel_of<FwdParams>(fwd_bf16_pad_kernel<128, 2>), kernel_of<FwdParams>(fwd_bf16_pad_kernel<128, 4>)},
+                {kernel_of<Three>(fwd_bf16_pad_kernel<128, 1>), kernel_of<Three>(fwd_bf16_pad_kernel<128, 2>), kernel_of<Three>(fwd_bf16_pad_kernel<128, 4>)}};
             const int lds[2][3] = {{fwd_lds_bytes<64>(), shares_lds_bytes<64, 2>(), shares_lds_bytes<64, 4>()},
                                    {fwd_lds_bytes<128>(), shares_lds_bytes<128, 2>(), shares_lds_bytes<128, 4>()}};
-            return launch(kernels[D == 128][i], dims(grid), 512, lds[D == 128][i], st, p);
+            return launch(kernels[D == 64 ? 0 : a->D > 96 ? 1 : 2][i], dims(grid), 512, lds[D == 128][i], st, p);
         }
         if (pl.four_waves)
             return a->D == 128 ? launch((const void *)fwd_bf16_w4_kernel<128>, dims(grid), 256, FourWaves<128>::LDS, st, p)
@@ -5504,7 +5550,7 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
             std::stable_sort(p.chunk, p.chunk + p.n_chunks, [](const ChunkDev &x, const ChunkDev &y) { return x.pos0 < y.pos0; });
         const unsigned n_q = map_blocks(p.q_map, p.B * p.Hkv), n_kv = map_blocks(p.kv_map, p.B * p.Hkv);
         p.joint = {pl.keys_first ? n_kv : n_q, pl.keys_first};
-        const KernelChoice k = joint_kernel(D, pad, pl.dq_ks, pl.own_delta);
+        const KernelChoice k = joint_kernel(D, pad, pl.dq_ks, pl.own_delta, a->D);
         rc = launch(k.fn, (long long)n_q + n_kv, 512, k.lds, st, p);
         return rc || pl.split.n == 1 ? rc
                : D == 128            ? launch((const void *)bwd_dkdv_reduce_kernel<128, 1>, reduce_grid, 256, 0, st, p)
@@ -5514,12 +5560,14 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
     if (do_dq) {
         if (pad) {
             const int i = pl.dq_ks >> 1;
-            const void *const kernels[2][3] = {
-                {(const void *)bwd_dq_pad_kernel<64, 1>, (const void *)bwd_dq_pad_kernel<64, 2>, (const void *)bwd_dq_pad_kernel<64, 4>},
-                {(const void *)bwd_dq_pad_kernel<128, 1>, (const void *)bwd_dq_pad_kernel<128, 2>, (const void *)bwd_dq_pad_kernel<128, 4>}};
+            using Three = Columns96<BwdParams>;
+            const void *const kernels[3][3] = {
+                {kernel_of<BwdParams>(bwd_dq_pad_kernel<64, 1>), kernel_of<BwdParams>(bwd_dq_pad_kernel<64, 2>), kernel_of<BwdParams>(bwd_dq_pad_kernel<64, 4>)},
+                {kernel_of<BwdParams>(bwd_dq_pad_kernel<128, 1>), kernel_of<BwdParams>(bwd_dq_pad_kernel<128, 2>), kernel_of<BwdParams>(bwd_dq_pad_kernel<128, 4>)},
+                {kernel_of<Three>(bwd_dq_pad_kernel<128, 1>), kernel_of<Three>(bwd_dq_pad_kernel<128, 2>), kernel_of<Three>(bwd_dq_pad_kernel<128, 4>)}};
             const int lds[2][3] = {{dq_lds_bytes<64>(), shares_lds_bytes<64, 2>(), shares_lds_bytes<64, 4>()},
                                    {dq_lds_bytes<128>(), shares_lds_bytes<128, 2>(), shares_lds_bytes<128, 4>()}};
-            rc = launch(kernels[D == 128][i], dims(q_grid), 512, lds[D == 128][i], st, p);
+            rc = launch(kernels[D == 64 ? 0 : a->D > 96 ? 1 : 2][i], dims(q_grid), 512, lds[D == 128][i], st, p);
         } else if (pl.dq_four_waves)
             rc = a->D == 128 ? launch((const void *)bwd_dq_w4_kernel<128>, dims(q_grid), 256, FourWaves<128>::LDS, st, p)
                              : launch((const void *)bwd_dq_w4_kernel<64>, dims(q_grid), 256, FourWaves<64>::LDS, st, p);
@@ -5541,8 +5589,9 @@ int bwd_launch(const ltr_attn_bwd_args *a, unsigned flags, bool use_scratch, voi
         // the tail (the sums inside a block do not depend on the table's order).
         if (flags & LTR_CAUSAL)
             std::stable_sort(p.chunk, p.chunk + p.n_chunks, [](const ChunkDev &x, const ChunkDev &y) { return x.pos0 < y.pos0; });
-        if (pad) rc = D == 128 ? launch((const void *)bwd_dkdv_pad_kernel<128>, dims(key_grid), BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p)
-                               : launch((const void *)bwd_dkdv_pad_kernel<64>, dims(key_grid), BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p);
+        if (pad) rc = D == 64     ? launch(kernel_of<BwdParams>(bwd_dkdv_pad_kernel<64>), dims(key_grid), BwdLds<64, 1>::NT, BwdLds<64, 1>::TOTAL, st, p)
+                      : a->D > 96 ? launch(kernel_of<BwdParams>(bwd_dkdv_pad_kernel<128>), dims(key_grid), BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p)
+                                  : launch(kernel_of<Columns96<BwdParams>>(bwd_dkdv_pad_kernel<128>), dims(key_grid), BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
         else if (a->D == 128) rc = launch((const void *)bwd_dkdv_kernel<128, 1>, dims(key_grid), BwdLds<128, 1>::NT, BwdLds<128, 1>::TOTAL, st, p);
         else if (pl.wide_kv) rc = launch((const void *)bwd_dkdv_kernel<64, 2>, kv_grid, BwdLds<64, 2>::NT, BwdLds<64, 2>::TOTAL, st, p);
         else if (pl.key_waves) rc = launch((const void *)bwd_dkdv_keywave_kernel<64>, dims(key_grid), KeyWaveLds<64>::NT, KeyWaveLds<64>::TOTAL, st, p);
@@ -5653,7 +5702,7 @@ int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work
         else snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "bwd_dkdv_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);
     }
     if (b.joint) {   // one kernel for both
-        const char *name = joint_kernel(D, pad, b.dq_ks, b.own_delta).name;
+        const char *name = joint_kernel(D, pad, b.dq_ks, b.own_delta, a->D).name;
         snprintf(out->dq_kernel, sizeof(out->dq_kernel), "%s", name);
         snprintf(out->dkdv_kernel, sizeof(out->dkdv_kernel), "%s", name);
     }
