@@ -2478,7 +2478,7 @@ struct KeyWaveLds {
     static_assert(2 * TOTAL <= 160 * 1024, "two blocks per CU");
 };
 template <int D>
-__device__ __forceinline__ void bwd_dkdv_keywave_body(const BwdParams &p, const BlockItem item) {
+__global__ __launch_bounds__(256, 2) void bwd_dkdv_keywave_kernel(const BwdParams p) {
     using L = KeyWaveLds<D>;
     constexpr int BN = L::BN, BM = L::BM;
     constexpr int CPR = D / 8;
@@ -2490,6 +2490,7 @@ __device__ __forceinline__ void bwd_dkdv_keywave_body(const BwdParams &p, const 
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool causal = p.flags & LTR_CAUSAL;
     // block -> (batch, kv head, chunk, key tile), shares of a key tile: as in bwd_dkdv_body
+    const BlockItem item = block_item(p.kv_map, p.B * p.Hkv);
     const int pair = item.pair, split = item.sub, tile = item.item;
     if (pair >= p.B * p.Hkv) return;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
@@ -2737,10 +2738,6 @@ __device__ __forceinline__ void bwd_dkdv_keywave_body(const BwdParams &p, const 
     const bool as_bf16 = uniform32(p.flags & LTR_DKDV_BF16);
     write_key_rows<D, false>(stage, lane, dvacc, 1.f, as_bf16, p.chunk[c].dv, b * p.dvs[0] + hkv * p.dvs[2], p.dvs[1], key0 + 32 * w, sk, D);
     write_key_rows<D, false>(stage, lane, dkacc, p.scale, as_bf16, p.chunk[c].dk, b * p.dks[0] + hkv * p.dks[2], p.dks[1], key0 + 32 * w, sk, D);
-}
-template <int D>
-__global__ __launch_bounds__(256, 2) void bwd_dkdv_keywave_kernel(const BwdParams p) {
-    bwd_dkdv_keywave_body<D>(p, block_item(p.kv_map, p.B * p.Hkv));
 }
 
 // Sum of the partial dK / dV that the blocks sharing a key tile left in p.part (bf16 and fp32 kernels alike), in the order of
