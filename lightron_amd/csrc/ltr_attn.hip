@@ -3065,8 +3065,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
             // with two row blocks per wave (64 rows) the rest of a diagonal or last tile is left out and whole blocks of one go without a mask: 4 x 16
             // heads of 64, causal S=4096 211 -> 198 us; with one it is 1 - 3 % slower
             if (RB == 2 && nb > 0 && ((causal && pos0 + key0 + nb * 32 > w_hi) || key0 + nb * 32 >= sk)) break;
-            int mask_end = key0 + (RB == 2 ? nb * 32 + 32 : BN);
-            asm volatile("" : "+s"(mask_end));   // asked again for each block: the answer kept would be two vector instructions per tile
+            const int mask_end = key0 + (RB == 2 ? nb * 32 + 32 : BN);
             const bool need_mask = mask_end > sk || (causal && pos0 + mask_end - 1 > w_lo);
             f32x16 s[RB], dp[RB];
 #pragma unroll
@@ -3082,9 +3081,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams &p, const BlockItem 
             if (need_mask) {
 #pragma unroll
                 for (int rb = 0; rb < RB; rb++) {
-                    int row_pos = my_pos[rb], chunk_keys = sk, half = 4 * hh;
-                    asm volatile("" : "+v"(row_pos), "+s"(chunk_keys), "+v"(half));   // or the bits' beginning moves before the branch, into every tile
-                    const unsigned bits = row_ok[rb] ? visible_bits(causal, row_pos, pos0, chunk_keys, key0 + nb * 32 + half) : 0u;
+                    const unsigned bits = row_ok[rb] ? visible_bits(causal, my_pos[rb], pos0, sk, key0 + nb * 32 + 4 * hh) : 0u;
 #pragma unroll
                     for (int r = 0; r < 16; r++) s[rb][r] = visible_score(bits, 8 * (r / 4) + r % 4, s[rb][r]);
                 }
