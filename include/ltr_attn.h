@@ -342,6 +342,7 @@ int ltr_attn_plan(const ltr_attn_bwd_args *args, ltr_attn_plan_t *out);
 typedef struct ltr_attn_plan_ws_t {
     ltr_attn_plan_t plan;
     int32_t blocks_per_tile;  /* dK/dV blocks that share a key tile; 1: none do, and no reduction runs */
+    int32_t keys_first;       /* one launch for both kinds of blocks (LTR_BWD_JOINT): 1 where the dK/dV blocks go first; else 0 */
     int64_t reduce_blocks;
     char reduce_kernel[48];   /* empty without a reduction */
 } ltr_attn_plan_ws_t;

@@ -96,7 +96,7 @@ class AttnPlan(ctypes.Structure):
 
 
 class AttnPlanWs(ctypes.Structure):
-    _fields_ = [("plan", AttnPlan), ("blocks_per_tile", ctypes.c_int32), ("reduce_blocks", ctypes.c_int64), ("reduce_kernel", ctypes.c_char * 48)]
+    _fields_ = [("plan", AttnPlan), ("blocks_per_tile", ctypes.c_int32), ("keys_first", ctypes.c_int32), ("reduce_blocks", ctypes.c_int64), ("reduce_kernel", ctypes.c_char * 48)]
 
 
 LTR_PROBE_MIN_WORKSPACE = 8192 + 65536

@@ -5702,6 +5702,7 @@ int describe_plan(const ltr_attn_bwd_args *a, ltr_attn_plan_t *out, int64_t work
     }
     if (ws) {
         ws->blocks_per_tile = shared ? b.split.n : 1;
+        ws->keys_first = b.joint && b.keys_first;
         ws->reduce_blocks = shared ? reduce_blocks(b, D) : 0;
         ws->reduce_kernel[0] = 0;
         if (shared) snprintf(ws->reduce_kernel, sizeof(ws->reduce_kernel), "bwd_dkdv_reduce_kernel<%d, %d>", D, b.wide_kv ? 2 : 1);

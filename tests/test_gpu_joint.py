@@ -1,14 +1,15 @@
 """bwd_joint_kernel (dQ and dK/dV blocks in one launch) against the dense oracle and against the two launches it takes the place of, at the
-edges of both kinds' tiles (128 or 256 rows, 64-row sub-tiles, 128 keys)."""
+edges of both kinds' tiles (128 or 256 rows, 64-row sub-tiles, 128 keys), dQ blocks first and dK/dV blocks first."""
 import pytest
 import torch
 
+from attn_abi import backward
 from oracle import ring_attention_oracle as orc
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("D,B,Hq,Hkv,Sq,q_pos,split,chunks,causal", [
+DQ_FIRST = [
     (64, 2, 12, 12, 1, 0, None, [(1, 0)], True),                                   # one row, one key
     (64, 4, 12, 12, 128, 0, None, [(128, 0)], True),
     (64, 1, 8, 2, 321, 0, None, [(321, 0)], True),                                 # grouped heads, pairs that do not divide among the XCDs
@@ -24,11 +25,27 @@ pytestmark = pytest.mark.gpu
     (128, 5, 32, 32, 240, 0, None, [(240, 0)], False),                             # more blocks than CUs
     (96, 2, 16, 16, 391, 0, None, [(391, 0)], True),
     (40, 1, 8, 4, 130, 3, None, [(133, 0)], True),
-])
-def test_joint(ltr, D, B, Hq, Hkv, Sq, q_pos, split, chunks, causal):
+]
+ZIGZAG = lambda h: [(h, 0), (h, h), (h, 2 * h), (h, 3 * h)]
+KEYS_FIRST = [
+    (64, 5, 48, 12, 110, 0, None, [(110, 0)], True),                               # pairs that do not divide among the XCDs
+    (64, 3, 64, 16, 72, (36, 72), 36, ZIGZAG(36), True),                           # grouped block order, keys no row sees
+    (64, 2, 128, 32, 134, 0, None, [(134, 0)], True),                              # 256-row dQ blocks
+    (64, 3, 32, 8, 265, 0, None, [(265, 0)], True),                                # shared key tiles
+    (128, 5, 16, 8, 264, 0, None, [(264, 0)], True),
+    (128, 5, 48, 12, 132, 0, None, [(132, 0)], True),
+    (128, 3, 32, 8, 271, 0, None, [(271, 0)], True),                               # shared key tiles
+    (128, 5, 32, 8, 90, (45, 90), 45, ZIGZAG(45), True),
+    (96, 3, 64, 32, 112, 0, None, [(112, 0)], False),
+    (120, 5, 32, 8, 66, (33, 66), 33, ZIGZAG(33), True),
+    (40, 5, 16, 4, 307, 0, None, [(307, 0)], False),
+]
+
+
+@pytest.mark.parametrize("D,B,Hq,Hkv,Sq,q_pos,split,chunks,causal,keys_first", [(*c, False) for c in DQ_FIRST] + [(*c, True) for c in KEYS_FIRST])
+def test_joint(ltr, D, B, Hq, Hkv, Sq, q_pos, split, chunks, causal, keys_first):
+    """bf16 results with DELTA from o, and fp32 accumulators with DELTA given: each in the joint launch that its own plan names, in this order."""
     total, pos = sum(n for n, _ in chunks), [p for _, p in chunks]
-    plan = ltr.attn_plan(B, Hq, Hkv, D, Sq, [n for n, _ in chunks], pos, q_pos, split, causal, share_keys=True, joint=True)
-    assert plan["dq"]["kernel"] == plan["dkdv"]["kernel"] and plan["dq"]["kernel"].startswith("bwd_joint")
     g = torch.Generator().manual_seed(Sq)
     mk = lambda s, h: torch.randn(B, s, h, D, generator=g).to(torch.bfloat16)
     q, do, k, v = mk(Sq, Hq), mk(Sq, Hq), mk(total, Hkv), mk(total, Hkv)
@@ -42,37 +59,34 @@ def test_joint(ltr, D, B, Hq, Hkv, Sq, q_pos, split, chunks, causal):
     qd, kd, vd, dod = q.cuda(), k.cuda(), v.cuda(), do.cuda()
     o, lse = (t.detach() for t in ltr.block_attention(qd, cut(kd), cut(vd), pos, q_pos, split, causal))
 
-    def run(joint, dtype, fill):
-        delta = torch.full(lse.shape, 3.0, dtype=torch.float32, device="cuda") if dtype == torch.bfloat16 else ltr.attn_delta(o, dod)
-        if D not in (64, 128):   # the padded kernels are reached through block_attention only
-            leaves = [t.clone().requires_grad_(True) for t in (qd, kd, vd)]
-            ltr.block_attention(leaves[0], cut(leaves[1]), cut(leaves[2]), pos, q_pos, split, causal)[0].backward(dod)
-            return [t.grad for t in leaves], None
-        out = [torch.full(t.shape, fill, dtype=dtype, device="cuda") for t in (qd, kd, vd)]
-        ltr.attn_bwd_accumulate(qd, dod, lse, delta, cut(kd), cut(vd), pos, out[0], cut(out[1]), cut(out[2]), q_pos, split, causal,
-                                o=o if dtype == torch.bfloat16 else None, share_keys=True, joint=joint)
-        return out, delta
+    def run(joint, results, fill, delta=None):
+        got = backward(qd, dod, o, lse, cut(kd), cut(vd), pos, q_pos, split, causal, joint, results, fill, delta)
+        pad = "" if D in (64, 128) else "_pad"
+        names = {"bwd_joint%s_kernel<%d, %d>" % (pad, 64 if D <= 64 else 128, 256 // got.plan.rows)}
+        if delta is None:
+            names.add("bwd_joint_delta%s_kernel<%d>" % (pad, 64 if D <= 64 else 128))
+        assert (got.plan.dq in names and got.plan.dkdv == got.plan.dq) if joint else not names & {got.plan.dq, got.plan.dkdv}
+        assert got.plan.keys_first == (joint and keys_first)
+        return got
 
     # bf16 P, dS, products and results: 2e-3 .. 3.1e-3 of the norm.  With one key dS = dP - DELTA is zero but for the rounding of two fp32 sums of
     # size 8 (1e-6), times a key and 1 / sqrt(D): 1e-6 per element.  Results where no query sees a key are zeros
-    results, delta = run(True, torch.bfloat16, 7.0)
-    for name, got, want in zip(("dq", "dk", "dv"), results, ref):
-        assert (got.cpu().float() - want).norm() <= 1e-2 * want.norm() + 1e-6 * want.numel() ** 0.5, name
+    direct = run(True, torch.bfloat16, 7.0)
+    for name, want in zip(("dq", "dk", "dv"), ref):
+        assert (getattr(direct, name).cpu().float() - want).norm() <= 1e-2 * want.norm() + 1e-6 * want.numel() ** 0.5, name
     seen = torch.ones(total, dtype=torch.bool) if not causal else kpos <= qpos.max()
-    assert not results[1].cpu()[:, ~seen].any() and not results[2].cpu()[:, ~seen].any()
-    if delta is None:
-        return
+    assert not direct.dk.cpu()[:, ~seen].any() and not direct.dv.cpu()[:, ~seen].any()
     want_delta = (do.float() * o.cpu().float()).sum(-1).transpose(1, 2)
-    assert (delta.cpu() - want_delta).abs().max() <= 1e-5 * D + 1e-5 * want_delta.abs().max()
-    again, _ = run(True, torch.bfloat16, 7.0)
-    assert all(torch.equal(a, b) for a, b in zip(results, again))
+    assert (direct.delta.cpu() - want_delta).abs().max() <= 1e-5 * D + 1e-5 * want_delta.abs().max()
+    again = run(True, torch.bfloat16, 7.0)
+    assert all(torch.equal(getattr(direct, n), getattr(again, n)) for n in ("dq", "dk", "dv", "delta"))
     # fp32 accumulators with DELTA given: the sums of the two launches in another order, added to what was there
-    joint, apart = run(True, torch.float32, 0.5)[0], run(False, torch.float32, 0.5)[0]
-    for a, b in zip(joint, apart):
-        a, b = a.cpu() - 0.5, b.cpu() - 0.5
-        assert (a - b).norm() <= 2e-5 * b.norm() + 1e-6 * b.numel() ** 0.5
-    for got, want in zip(joint, ref):
-        assert (got.cpu() - 0.5 - want).norm() <= 1e-2 * want.norm() + 1e-6 * want.numel() ** 0.5
+    delta = ltr.attn_delta(o, dod)
+    joint, apart = (run(j, torch.float32, 0.5, delta) for j in (True, False))
+    for name, want in zip(("dq", "dk", "dv"), ref):
+        a, b = getattr(joint, name).cpu() - 0.5, getattr(apart, name).cpu() - 0.5
+        assert (a - b).norm() <= 2e-5 * b.norm() + 1e-6 * b.numel() ** 0.5, name
+        assert (a - want).norm() <= 1e-2 * want.norm() + 1e-6 * want.numel() ** 0.5, name
 
 
 def test_joint_backward_under_rope_and_replays(ltr):
