@@ -9,8 +9,14 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("D", [72, 88, 96, 104])
-@pytest.mark.parametrize("B,Hq,Hkv,S,causal", [(1, 8, 2, 193, True), (2, 8, 8, 260, False), (8, 32, 8, 300, True)])
-def test_columns(ltr, D, B, Hq, Hkv, S, causal):
+@pytest.mark.parametrize("B,Hq,Hkv,S,causal,kernels", [
+    (1, 8, 2, 193, True, ("fwd_bf16_pad_kernel<128, 2>", "bwd_joint_pad_kernel<128, 2>", "bwd_joint_pad_kernel<128, 2>", 8)),
+    (2, 8, 8, 260, False, ("fwd_bf16_pad_kernel<128, 2>", "bwd_joint_pad_kernel<128, 2>", "bwd_joint_pad_kernel<128, 2>", 1)),
+    (8, 32, 8, 300, True, ("fwd_bf16_pad_kernel<128, 1>", "bwd_dq_pad_kernel<128, 1>", "bwd_dkdv_pad_kernel<128>", 1)),
+])
+def test_columns(ltr, D, B, Hq, Hkv, S, causal, kernels):
+    plan = ltr.attn_plan(B, Hq, Hkv, D, S, [S], [0], causal=causal, share_keys=True, joint=True)
+    assert (plan["fwd"]["kernel"], plan["dq"]["kernel"], plan["dkdv"]["kernel"], plan["dkdv"]["blocks_per_tile"]) == kernels
     g = torch.Generator().manual_seed(D)
     mk = lambda h: torch.randn(B, S, h, D, generator=g).to(torch.bfloat16)
     q, k, v, do = mk(Hq), mk(Hkv), mk(Hkv), mk(Hq)
