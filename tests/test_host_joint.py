@@ -112,9 +112,10 @@ def test_launch_time_is_that_of_in_order_dispatch(program):
         assert abs(got - want) <= 0.06 * max(us for us, _ in classes) + 0.02 * want, (slots, classes, got, want)
 
 
-def _args(D, B, Hq, Hkv, Sq, chunks, flags, dtype=L.LTR_BF16):
+def _args(D, B, Hq, Hkv, Sq, chunks, flags, dtype=L.LTR_BF16, q_pos0=(0, 0), q_split=None):
     a = L.BwdArgs()
-    a.B, a.Hq, a.Hkv, a.D, a.Sq, a.q_split, a.n_chunks, a.flags, a.io_dtype = B, Hq, Hkv, D, Sq, Sq, len(chunks), flags, dtype
+    a.B, a.Hq, a.Hkv, a.D, a.Sq, a.q_split, a.n_chunks, a.flags, a.io_dtype = B, Hq, Hkv, D, Sq, Sq if q_split is None else q_split, len(chunks), flags, dtype
+    a.q_pos0 = (ctypes.c_int64 * 2)(*q_pos0)
     for i, (sk, pos0) in enumerate(chunks):
         a.chunk[i].sk, a.chunk[i].pos0 = sk, pos0
     return a
@@ -186,8 +187,17 @@ def test_the_plan_kept_is_that_of_the_problem():
         p = ws.plan
         return need.value, ws.blocks_per_tile, p.dq_kernel, p.dkdv_kernel, p.dq_blocks, p.dkdv_blocks, p.dq_rows, p.fwd_rows, p.fwd_blocks, p.fwd_kernel
 
+    # ranks of a ring differ in where their rows stand, and zig-zag shares from contiguous ones in where the rows are cut: other key tiles are seen
+    ring = dict(base, Sq=512, chunks=[(256, i * 256) for i in range(8)], q_pos0=(256, 256), q_split=256)
+    ranks = [ring, dict(ring, q_pos0=(256, 1024)), dict(ring, q_pos0=(1536, 256)), dict(ring, q_split=128), dict(ring, q_split=128, q_pos0=(256, 1024))]
+    assert len({ask(v)[5] for v in ranks}) == len(ranks), [ask(v) for v in ranks]
+    variants += ranks
     alone = [ask(v) for v in variants]
-    assert len(set(alone)) > 6
+    assert len(set(alone)) > 6 + len(ranks)
+    # a problem with its workspace and without one
+    a, ws = _args(**base), L.AttnPlanWs()
+    for need, shared in ((alone[0][0], True), (0, False), (alone[0][0], True)):
+        assert alone[0][0] > 0 and L.load().ltr_attn_plan_ws(ctypes.byref(a), need, ctypes.byref(ws)) == 0 and (ws.blocks_per_tile > 1) == shared
     for order in (range(len(variants)), reversed(range(len(variants)))):
         for i in order:
             assert ask(variants[i]) == alone[i] == ask(variants[i])
