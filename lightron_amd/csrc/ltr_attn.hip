@@ -3214,7 +3214,7 @@ __global__ __launch_bounds__(512) void bwd_dq_pad_kernel(const Columns96<BwdPara
 
 // dQ and dK/dV blocks in one launch (LTR_BWD_JOINT).  Given DELTA, neither kind needs anything of the other; in launches of their own each ends with
 // CUs idle and the next begins with all of them waiting for their first tiles, which is what a pass of few blocks spends its time on.  DELTA
-// comes from delta_kernel then.  Taken where the modelled time is shorter (joint_launch).  us of the backward, apart -> joint:
+// comes from ltr_attn_bwd_delta's launch then (delta_bf16_kernel).  Taken where the modelled time is shorter (joint_launch).  us of the backward, apart -> joint:
 //   4 x 12 heads D=64 S=128   17.2 -> 12.0       2 x 16 heads D=96 S=777   57.8 -> 42.5       1 x 32 heads on 8 D=128 S=1237   94.8 -> 78
 //   1 x 16 heads D=128 S=4096  257 -> 242        1 x 12 heads D=128 S=3418  181 -> 145        3 x 8 heads D=128 S=926   61 -> 42
 // Registers are those of the dK/dV kernel, LDS the larger of both: one block per CU, as for either kind alone.
@@ -4564,10 +4564,8 @@ BlockList q_tile_blocks(RowKernel kernel, double step_us, double fixed_us, bool 
 
 // A second look at the choice of a forward launch, by launch_us: choose_rows knows a launch by its longest and average block, which is wrong by up to 40 %
 // where whole rounds decide (a zig-zag share whose late half is one round of two shares, taken for a round and a half: 1 x 32 heads,
-// 1194 rows of 9552, D=128 194 us with four shares, 140 with two).  Constants fitted to 5500 random launches of every kernel (rms 6 - 10 %);
-// another kernel is taken where it is 6 % faster by them (four waves: 10 %), but none in place of four waves, whose blocks share a CU better
-// than they say.  Of those launches a quarter change: all of them together become 3.3 % (head dim 64) and 1.5 % (128) shorter, one in a
-// hundred loses more than 2 %.
+// 1194 rows of 9552, D=128 194 us with four shares, 140 with two).  Constants fitted to 5500 random launches of every kernel (rms 6 - 10 %).
+// How much shorter another kernel has to be by them depends on what changes (needed_share).
 struct LaunchCost {
     double step_us[N_ROW_KERNELS], fixed_us[N_ROW_KERNELS];   // four waves: of a block among others, as a share of its CU
     double alone_us, alone_fixed_us;                          // four waves, alone on a CU
@@ -4575,38 +4573,68 @@ struct LaunchCost {
 };
 constexpr LaunchCost FWD_LAUNCH_64{{1.92, 1.125, 1.35, 0.447, 1.76}, {4.8, 5.1, 5.45, 2.5, 6.2}, 0.78, 4.7, 1.09, 4.8},
     FWD_LAUNCH_128{{1.565, 1.84, 1.2, 0.816, 0}, {5.8, 6.5, 6.6, 4.0, 0}, 1.09, 6.2, 1.76, 6.1};
+// The share of the present launch's time that another kernel may take at most, 0: never.  rounds: of 256-row blocks.  From 15085 random launches that
+// changed with one share of 0.94 (four waves 0.9) for all, one in 13 of those looked at (calls, ring and zig-zag ranks, single steps; 55 - 4096 rows,
+// 8 - 256 heads): 1.127 times as fast in the mean, but 746 more than 2 % slower, 487 more than 5 %, the worst 1.7 times (8 x 32 heads of 128, 192 rows
+// of a zig-zag share 99 us with 256 rows, 170 with four shares).  With these and four_waves_us, chosen on those launches, 15323 of 253436 others
+// change: 1.150 times as fast in the mean, 151 more than 2 % slower, 49 more than 5 %, the worst 1.20 times.
+double needed_share(int D, double now, double rounds, int from, bool from_paired, int to, bool to_paired) {
+    switch (to) {
+        case SHARES_4: return from == ROWS_256 ? 0.0 : D == 64 ? 0.94 : now < 20.5 ? 0.75 : 0.89;
+        case SHARES_2: return D == 64 || from == SHARES_4 ? 0.94 : from_paired || rounds > 2 ? 0.88 : now < 20.5 ? 0.85 : 0.92;
+        case FOUR_WAVES: return from == SHARES_4 ? 0.85 : 0.9;
+        case ROWS_512: return to_paired ? 0.0 : from_paired ? 0.91 : 0.94;
+        default: return 0.94;
+    }
+}
 RowChoice faster_rows(const LaunchCost &cost, RowChoice chosen, unsigned allowed, int D, bool causal, long long BH, int Sq, int q_split, const int *q_pos0,
                       const ChunkDev *chunk, int n_chunks, int cus) {
     // a hint; four waves; past 32 rounds nothing decides but the step
     if ((allowed & (allowed - 1)) == 0 || chosen.kernel == FOUR_WAVES || BH * ((Sq + 255) / 256) > 32LL * cus) return chosen;
-    auto launch = [&](int i, bool shares_paired, double most) {   // `most` or more is not worth a closer look
+    // Four waves: the long blocks (0.75 of the longest and more) come in whole numbers per CU and take the step of long equal blocks, which the fitted
+    // one is 11 - 19 % below; at head dim 128 with up to 1.6 of them per CU they are slower still (4 x 16 heads on 4, 1284 rows of a zig-zag
+    // share of 20544 479 us with 256 rows, 556 with four waves; modelled 568 and 504).
+    auto four_waves_us = [&](const BlockList &l, double end, double step, double fixed) {
+        double longs = 0, tiles = 0;
+        const double least = 0.75 * (l.longest_us() - fixed);
+        for (int i = 0; i < l.k; i++)
+            if (l.c[i].us - fixed >= least) longs += l.c[i].n, tiles += (l.c[i].us - fixed) / step * l.c[i].n;
+        const TileCost &tile = (D == 128 ? FWD_ROWS_128 : FWD_ROWS_64).kernel[FOUR_WAVES];
+        return std::max(end, std::ceil(longs / cus) * (tiles / longs * tile.step_us + tile.fixed_us)) * (D == 128 && longs <= 1.6 * cus ? 1.06 : 1.0);
+    };
+    auto in_pairs = [&](int i) {   // q tiles of 256 or 512 rows
+        const int rows = row_kernel(i, D).rows, n = (Sq + rows - 1) / rows;
+        return (i == ROWS_256 || i == ROWS_512) && q_tile_slots(n, BH, causal && q_tiles_uneven(Sq, rows, q_split, q_pos0, chunk, n_chunks), cus) != n;
+    };
+    auto launch = [&](int i, bool paired, double most) {   // `most` or more is not worth a closer look
         const RowKernel k = row_kernel(i, D);
-        const int n = (Sq + k.rows - 1) / k.rows;
         int per_cu = 1;
-        double step = shares_paired ? cost.paired_us : cost.step_us[i], fixed = shares_paired ? cost.paired_fixed_us : cost.fixed_us[i];
-        bool paired = shares_paired;
+        double step = i == SHARES_2 && paired ? cost.paired_us : cost.step_us[i], fixed = i == SHARES_2 && paired ? cost.paired_fixed_us : cost.fixed_us[i];
         if (i == FOUR_WAVES) {
-            per_cu = (int)std::min<long long>(D == 64 ? FourWaves<64>::PER_CU : FourWaves<128>::PER_CU, (BH * n + cus - 1) / cus);
+            per_cu = (int)std::min<long long>(D == 64 ? FourWaves<64>::PER_CU : FourWaves<128>::PER_CU, (BH * ((Sq + k.rows - 1) / k.rows) + cus - 1) / cus);
             step = per_cu == 1 ? cost.alone_us : per_cu * step;
             fixed = per_cu == 1 ? cost.alone_fixed_us : per_cu * fixed;
-        } else if (i == ROWS_256 || i == ROWS_512) {
-            paired = q_tile_slots(n, BH, causal && q_tiles_uneven(Sq, k.rows, q_split, q_pos0, chunk, n_chunks), cus) != n;
         }
         const BlockList l = q_tile_blocks(k, step, fixed, paired, causal, BH, Sq, q_split, q_pos0, chunk, n_chunks);
         if (l.least_us(per_cu * cus) >= most) return most;
         Dispatch d(per_cu * cus);
-        return d.add(l.c, l.k, most) ? d.end : most;
+        if (!d.add(l.c, l.k, most)) return most;
+        return i == FOUR_WAVES && chosen.kernel != SHARES_4 ? four_waves_us(l, d.end, step, fixed) : d.end;
     };
-    const double now = launch(chosen.kernel, chosen.paired, 1e30);
+    const bool now_paired = chosen.paired || in_pairs(chosen.kernel);
+    const double now = launch(chosen.kernel, now_paired, 1e30);
     if (now < 14) return chosen;   // a call of that length waits for its host side
     RowChoice better = chosen;
-    double best = 0.94 * now;
+    double best = now;
     for (int i = 0; i < N_ROW_KERNELS; i++) {
         if (!(allowed >> i & 1) || i == chosen.kernel) continue;
         // four waves: not alone on a CU, and not for 256 rows without a mask (11 of 22 such launches 3 - 13 % slower)
         if (i == FOUR_WAVES && (BH * ((Sq + 127) / 128) <= cus || (!causal && chosen.kernel == ROWS_256))) continue;
-        const double us = launch(i, false, best);
-        if (us < best && (i != FOUR_WAVES || us < 0.9 * now)) {
+        const bool paired = in_pairs(i);
+        const double most = std::min(best, needed_share(D, now, (double)(BH * ((Sq + 255) / 256)) / cus, chosen.kernel, now_paired, i, paired) * now);
+        if (most <= 0) continue;
+        const double us = launch(i, paired, most);
+        if (us < most) {
             best = us;
             better = {i, false};
         }
