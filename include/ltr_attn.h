@@ -189,7 +189,7 @@ int ltr_attn_bwd_delta(const ltr_attn_delta_args *args, void *stream);
  * elements): no fp32 accumulator, no zero-fill, no final cast.  LTR_DELTA_FROM_O: delta is
  * an OUTPUT workspace; the dQ kernel computes DELTA = rowsum(dO * O) of its rows from o
  * (bf16, o_stride) and stores it, and the dK/dV kernel, enqueued after it, reads it: no
- * separate ltr_attn_bwd_delta launch.  Not combinable with LTR_NO_DQ.  LTR_DKDV_BF16: when q holds
+ * separate ltr_attn_bwd_delta launch (LTR_BWD_JOINT: see there).  Not combinable with LTR_NO_DQ.  LTR_DKDV_BF16: when q holds
  * every query row that sees the keys of this call's chunks (one rank's own backward, not a ring step whose dK/dV
  * go on to other ranks), dK / dV of those chunks are complete after the call: chunk[c].dk / dv may then be the
  * bf16 results themselves (written for every key, zeros where no query sees it; dk/dv strides in bf16 elements):
@@ -199,7 +199,7 @@ typedef struct ltr_attn_bwd_args {
     const void *q;
     const void *d_o;      /* same dtype as q */
     const float *lse;     /* [B, Hq, Sq], of the COMPLETE softmax (all chunks) */
-    float *delta;         /* [B, Hq, Sq] fp32: input, or workspace written with LTR_DELTA_FROM_O */
+    float *delta;         /* [B, Hq, Sq] fp32: input, or workspace written with LTR_DELTA_FROM_O (with LTR_BWD_JOINT too) */
     void *dq;             /* fp32 accumulator by dq strides, or the bf16 result with LTR_DQ_BF16 */
     int32_t B, Hq, Hkv, D;
     int64_t Sq;

@@ -215,7 +215,7 @@ def attn_bwd_accumulate(q, do, lse, delta, ks, vs, k_pos0, dq_acc, dk_accs, dv_a
     do_dq / do_dkdv select which of the two backward kernels are enqueued.  dq_acc may instead be a bf16
     tensor: it then RECEIVES dQ (LTR_DQ_BF16), which is only right when ks / vs hold every KV chunk these
     queries can see and fit one launch (at most 32 chunks).  With o (the bf16 forward output) given, delta is a
-    workspace: the dQ kernel of the first launch computes rowsum(dO * O) into it (LTR_DELTA_FROM_O) and no
+    workspace: the first launch computes rowsum(dO * O) into it (LTR_DELTA_FROM_O) and no
     attn_delta call is needed; this needs do_dq.  dk_accs / dv_accs may be bf16 tensors as well: they then RECEIVE
     dK / dV (LTR_DKDV_BF16; every key is written), which is only right when q holds every query row that sees
     these keys - one rank's own backward, not a ring step whose dK/dV are summed over ranks.
@@ -411,7 +411,7 @@ class BlockAttentionFunction(torch.autograd.Function):
         if do.stride(3) != 1:
             do = do.contiguous()
         do = do.to(q.dtype)
-        fuse = o.dtype == torch.bfloat16 and not f32   # DELTA computed by the dQ kernel from o
+        fuse = o.dtype == torch.bfloat16 and not f32   # DELTA computed from o by the backward
         delta = (torch.empty(lse.shape, dtype=torch.float32, device=q.device) if fuse else attn_delta(o, do))
         # one launch sees every chunk: dQ is written as bf16 by the kernel; otherwise it accumulates in fp32
         direct = n_chunks <= _lib.LTR_MAX_CHUNKS and not f32
@@ -537,7 +537,7 @@ class SingleChunkAttentionFunction(torch.autograd.Function):
         dv = torch.empty(k.shape, dtype=torch.bfloat16, device=dev)
         if Sq == 0:
             return dq, dk.zero_(), dv.zero_(), None
-        delta = torch.empty((B, Hq, Sq), dtype=torch.float32, device=dev)   # workspace: filled by the dQ kernel from o
+        delta = torch.empty((B, Hq, Sq), dtype=torch.float32, device=dev)   # workspace: filled from o
         key = _single_key(q, k, v, (do.stride(), k_pos0, q_pos0, q_split, causal, scale, None if q_rope is None else q_rope.shape[0]))
         prep = _prepared.bwd.get(key)
         if prep is None:

@@ -195,7 +195,7 @@ struct ChunksFunction {
                               (uintptr_t)o.data_ptr() % 16 == 0;
         const bool delta_from_o = direct32 || (!f32 && o.scalar_type() == at::kBFloat16);
         Tensor dq = direct || direct32 ? torch::empty({B, Sq, Hq, D}, q.options()) : torch::zeros({B, Sq, Hq, D}, q.options().dtype(at::kFloat));
-        Tensor delta = torch::empty({B, Hq, Sq}, lse.options());   // with delta_from_o a workspace: filled by the dQ kernel
+        Tensor delta = torch::empty({B, Hq, Sq}, lse.options());   // with delta_from_o a workspace: filled by the dQ kernel, or before a joint launch
         if (!delta_from_o) {
             ltr_attn_delta_args d{};
             d.o = o.data_ptr();
