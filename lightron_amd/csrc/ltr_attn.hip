@@ -4887,9 +4887,10 @@ struct BwdPlan {
 };
 // Does a bf16 backward run its dQ and dK/dV blocks in one launch, with how many key shares per row group and blocks per key tile, and which kind
 // first?  Both ways are priced by launch_us over classes of blocks (BlockList): the plan as it is, one launch after
-// the other, and every joint one.  Constants fitted to 21000 launches of 2200 random problems (calls, ring and zig-zag ranks, single ring steps;
-// 4 - 32 heads, 45 - 5800 rows; rms error 9 - 12 %).  Of 5600 other launches that were joined, the backward takes 1 / 1.31 of the time, geometric
-// mean: 1.48 times faster where it took up to 25 us, 1.37 up to 50, 1.24 up to 100, 1.10 past 200.
+// the other, and every joint one.  Constants fitted to random problems (calls, ring and zig-zag ranks, single ring steps; 4 - 32 heads, 45 - 5800
+// rows; rms error 9 - 12 %).  Of 40405 others (8 - 256 heads, 45 - 4096 rows) 25360 are joined, 1 / 1.314 of the time apart in the geometric mean:
+// 1.54 times as fast where that was up to 25 us, 1.38 up to 50, 1.27 up to 100, 1.19 up to 200, 1.08 past 1600.  75 are more than 2 % slower, 16
+// more than 5 %, the worst 1.095 times.
 struct JointCost {
     double q_step_us[2], q_fixed_us[2];   // dQ blocks of one and two key shares: per K / V tile and per block
     double shares4_step_us, shares4_fixed_us;
@@ -4989,7 +4990,8 @@ void joint_launch(BwdPlan &pl, const BwdPlan &alone, int D, unsigned flags, int 
             us += launch_us(l.c, l.k, cus);
         }
         // where the plan has several blocks on a CU the model takes it for slower than it is, most of all at head dim 64 with both kernels of that
-        // kind: of 5600 random launches joined at 0.96, 100 lost more than 1 %, 80 of them there; of 5400 with about these factors 50
+        // kind.  Of those joined with these factors, by the kernels apart: four-wave dQ at head dim 128 1455, 1.100 times as fast, 41 more than 2 %
+        // slower (at 0.86 none of 984, 1.123 times); both of that kind at 64 245, 1.078 times, 12 (at 0.74 none of 162); all others 23660, 22
         return us * (D == 128 ? x.dq_four_waves ? 0.92 : 0.98
                               : x.key_waves && x.dq_four_waves ? 0.78 : x.key_waves || x.dq_four_waves || x.dq_blocks + x.kv_blocks > 8 * cus ? 0.88 : 0.96);
     };
