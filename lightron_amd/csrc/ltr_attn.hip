@@ -4574,7 +4574,7 @@ struct LaunchCost {
 constexpr LaunchCost FWD_LAUNCH_64{{1.92, 1.125, 1.35, 0.447, 1.76}, {4.8, 5.1, 5.45, 2.5, 6.2}, 0.78, 4.7, 1.09, 4.8},
     FWD_LAUNCH_128{{1.565, 1.84, 1.2, 0.816, 0}, {5.8, 6.5, 6.6, 4.0, 0}, 1.09, 6.2, 1.76, 6.1};
 // The share of the present launch's time that another kernel may take at most, 0: never.  rounds: of 256-row blocks.  From 15085 random launches that
-// changed with one share of 0.94 (four waves 0.9) for all, one in 13 of those looked at (calls, ring and zig-zag ranks, single steps; 55 - 4096 rows,
+// changed with one share of 0.94 (four waves 0.9) for all, one in 13 of those looked at (calls, ring and zig-zag ranks, single steps; 90 - 8190 rows,
 // 8 - 256 heads): 1.127 times as fast in the mean, but 746 more than 2 % slower, 487 more than 5 %, the worst 1.7 times (8 x 32 heads of 128, 192 rows
 // of a zig-zag share 99 us with 256 rows, 170 with four shares).  With these and four_waves_us, chosen on those launches, 15323 of 253436 others
 // change: 1.150 times as fast in the mean, 151 more than 2 % slower, 49 more than 5 %, the worst 1.20 times.
@@ -4888,7 +4888,7 @@ struct BwdPlan {
 // Does a bf16 backward run its dQ and dK/dV blocks in one launch, with how many key shares per row group and blocks per key tile, and which kind
 // first?  Both ways are priced by launch_us over classes of blocks (BlockList): the plan as it is, one launch after
 // the other, and every joint one.  Constants fitted to random problems (calls, ring and zig-zag ranks, single ring steps; 4 - 32 heads, 45 - 5800
-// rows; rms error 9 - 12 %).  Of 40405 others (8 - 256 heads, 45 - 4096 rows) 25360 are joined, 1 / 1.314 of the time apart in the geometric mean:
+// rows; rms error 9 - 12 %).  Of 40405 others (8 - 256 heads, 90 - 8190 rows) 25360 are joined, 1 / 1.314 of the time apart in the geometric mean:
 // 1.54 times as fast where that was up to 25 us, 1.38 up to 50, 1.27 up to 100, 1.19 up to 200, 1.08 past 1600.  75 are more than 2 % slower, 16
 // more than 5 %, the worst 1.095 times.
 struct JointCost {
